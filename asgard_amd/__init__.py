@@ -441,7 +441,8 @@ class KronmultMatrix:
     def autotune(self, x, y):
         """Times the kernel shapes on this operator (y is overwritten) and
         keeps the fastest; returns (waves_per_row, kernel) with kernel 0 =
-        factors from global memory, 1 = LDS factor tables, 2 = matrix cores."""
+        factors from global memory, 1 = LDS factor tables, 2 = matrix cores,
+        3 = one dimension at a time (akm_create_sparse_grid)."""
         px, dx = _vec_ptr(x, self.dtype)
         py, dy = _vec_ptr(y, self.dtype)
         if not (dx and dy):

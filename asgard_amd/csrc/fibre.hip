@@ -1,0 +1,847 @@
+// Fibre-walk kernels: operators whose factors are mostly the identity, one
+// dimension at a time, with no intermediate list of cell pairs.
+//
+// A term with non-identity dimensions S (a_0 the whole-acting one, then a_1
+// .. a_{m-1}) is evaluated by the recursion
+//   Op_0 = F_{a0},   Op_i v = L_{ai} (Op_{i-1} v) + Op_{i-1} (U_{ai} v)
+// (F the whole factor, U its part from the diagonal on, L the part strictly
+// before it), which is the sum of the 2^(m-1) chains of the reference's
+// global operator (kronmult::permutes, src/device/asgard_kronmult.hpp:152-220)
+// with the products that chains share taken once: 3 * 2^(m-1) - 2 products
+// instead of m * 2^(m-1).  Products whose inputs are ready run in one launch,
+// so a term takes m launches, and terms that act in one and the same single
+// dimension are added into one factor table.
+//
+// Kernel: a workgroup holds `nslot` slots of N = n^d lanes.  A slot walks
+// pieces of one cell's connection list, up to fl_piece connections each; a
+// cell with a long list takes several slots of one workgroup, whose partials
+// are added in slot order through LDS.  Lane e reads entry e of a connected
+// cell's tensor once and multiplies it with its digit's column of the factor
+// block, which gives it a share of the n rows of its fibre; the rows are
+// summed through LDS at the end (reading row entries instead costs n loads of
+// x per connection).  Results repeat bit for bit.
+//
+// What bounds it: on the operators it is chosen for, the chain of dependent
+// loads and the launch, not bandwidth.  A piece's list entries sit in the
+// slot's record, so the chain is record, blocks, LDS, store; lists are cut
+// into pieces so that a row of 512 connections (a level-0 cell at d = 4,
+// level 7) is not the tail of the launch.  Measured (FP64, us per apply, the
+// pair kernels and the best other global layout before): d = 4 n = 2 level 7
+// advection-diffusion 7.1 (411 / 20); d = 4 n = 3 level 5 9.5 (129 / 12);
+// d = 2 n = 2 level 5 3.3 (3.9 / 6.5); d = 3 n = 3 level 6, every factor
+// dense, three stages 24 (23 / 60).
+#include "fibre.hpp"
+#include "kron_kernels.hpp"
+#include "matrix.hpp"
+
+#include <algorithm>
+#include <array>
+#include <map>
+#include <numeric>
+
+namespace akm
+{
+namespace
+{
+constexpr int fl_piece = 8; // connections of a piece: one batch of loads
+
+//! Up to fl_piece connections of one product.
+struct fl_piece_rec
+{
+  int in;     // vector: 0 the operator's input, v > 0 work vector v - 1
+  int stride; // tensor stride of the product's dimension
+  unsigned magic; // ceil(2^32 / stride), 0 for stride 1
+  int len;        // connections | last piece of its round << 16
+  // (connected cell, factor block of all tables); entries past len name the
+  // zero block
+  int2 entry[fl_piece];
+};
+static_assert(sizeof(fl_piece_rec) == 5 * sizeof(int4), "piece records are five int4");
+
+//! A slot and its first piece.
+struct fl_slot_rec
+{
+  int cell;  // output cell, -1: empty slot
+  int group; // rank within the cell's slots | slots << 16
+  int vec;   // output work vector, -1: y
+  int more;  // further pieces: more of them from `next` on
+  int next, rounds, pad[2]; // rounds: of the workgroup (the same in its slots)
+  fl_piece_rec p;
+};
+static_assert(sizeof(fl_slot_rec) == 7 * sizeof(int4), "slot records are seven int4");
+
+template<typename P>
+struct fl_args
+{
+  const int4 *slots;
+  const int4 *pieces;
+  const P *tab;
+  int n, N, nslot;
+  int64_t stride;
+  const P *x;
+  P *work;
+  P *y;
+  const P *xg;
+  const double *pc;
+  double jdt;
+  P alpha, beta, gamma;
+  int identities;
+};
+
+//! Column s of a factor block, n values.
+template<typename P, int NT>
+__device__ __forceinline__ void fl_column(const P *A, P (&v)[NT])
+{
+  constexpr int W = (NT == 3) ? 1 : ((sizeof(P) == 4) ? NT : 2); // values per read
+  typedef P vec __attribute__((ext_vector_type(W)));
+#pragma unroll
+  for (int j = 0; j < NT; j += W)
+  {
+    const vec t = *reinterpret_cast<const vec *>(A + j);
+#pragma unroll
+    for (int i = 0; i < W; i++)
+      v[j + i] = t[i];
+  }
+}
+
+//! Digit of tensor entry e at the piece's dimension.
+__device__ __forceinline__ int fl_digit(int e, unsigned magic, int n)
+{
+  return ((magic != 0) ? static_cast<int>(__umulhi(static_cast<unsigned>(e), magic)) : e) % n;
+}
+
+//! c[r] += the first U of a piece's connections: column `s` of each block
+//! times entry e of the connected cell.  All loads precede their uses.
+template<typename P, int NT, int U>
+__device__ __forceinline__ void fl_connections(const P *__restrict__ in, const P *__restrict__ tab,
+                                               int N, int len, const int4 *ent, P (&c)[NT])
+{
+  P av[U][NT], xv[U];
+#pragma unroll
+  for (int u = 0; u < U; u++)
+  {
+    const int cell = (u % 2 == 0) ? ent[u / 2].x : ent[u / 2].z;
+    const int block = (u % 2 == 0) ? ent[u / 2].y : ent[u / 2].w;
+    xv[u] = in[int64_t(cell) * N];
+    fl_column<P, NT>(tab + int64_t(block) * (NT * NT), av[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++)
+  {
+    const P xu = (u < len) ? xv[u] : P{0};
+#pragma unroll
+    for (int r = 0; r < NT; r++)
+      c[r] = fma(av[u][r], xu, c[r]);
+  }
+}
+
+//! A finished sum of entry pos of a vector: into its work vector, or into y.
+template<typename P>
+__device__ __forceinline__ void fl_store(fl_args<P> const &a, int vec, int64_t pos, P sum)
+{
+  if (vec >= 0)
+  {
+    a.work[int64_t(vec) * a.stride + pos] = sum;
+    return;
+  }
+  if (a.identities > 0)
+    sum += static_cast<P>(a.identities) * a.x[pos];
+  P out = a.alpha * sum;
+  if (a.beta != P{0})
+    out += a.beta * a.y[pos];
+  if (a.gamma != P{0})
+    out += a.gamma * a.xg[pos];
+  if (a.pc != nullptr)
+    out = static_cast<P>(static_cast<double>(out) / (1.0 - a.jdt * a.pc[pos]));
+  a.y[pos] = out;
+}
+
+//! One stage: a workgroup's slots, then each cell's slot partials added in
+//! slot order.  A slot whose pieces act in several dimensions takes a round
+//! per dimension.  LDS: NT values per thread.
+template<typename P, int NT>
+__global__ void __launch_bounds__(1024) fl_stage(fl_args<P> a, int group0)
+{
+  extern __shared__ __align__(16) unsigned char fl_smem[];
+  P *ex = reinterpret_cast<P *>(fl_smem);
+  const int tpb = blockDim.x, t = threadIdx.x, N = a.N;
+  const int slot = t / N;
+  const int e = t - slot * N;
+  const bool mine = slot < a.nslot;
+  // idle lanes read slot 0's record and store nothing
+  const int4 *rec = a.slots + (int64_t(group0 + blockIdx.x) * a.nslot + (mine ? slot : 0)) * 7;
+  const int4 head = rec[0], tail = rec[1];
+  int4 ph = rec[2];
+  int4 ent[fl_piece / 2] = {rec[3], rec[4], rec[5], rec[6]};
+  const bool live = mine && head.x >= 0;
+  int more = live ? head.w : 0;
+  const int4 *next = a.pieces + int64_t(tail.x) * 5;
+  bool have = live;
+  P acc = 0;
+  const int rounds = tail.y;
+  for (int round = 0; round < rounds; round++)
+  {
+    P c[NT];
+#pragma unroll
+    for (int r = 0; r < NT; r++)
+      c[r] = 0;
+    const int s = fl_digit(e, static_cast<unsigned>(ph.z), NT);
+    const int stride = ph.y;
+    bool open = have;
+    while (open)
+    {
+      const int len = ph.w & 0xffff;
+      open = (ph.w >> 16) == 0;
+      const P *in = ((ph.x == 0) ? a.x : a.work + int64_t(ph.x - 1) * a.stride) + e;
+      const int4 cur[fl_piece / 2] = {ent[0], ent[1], ent[2], ent[3]};
+      have = more > 0;
+      if (have)
+      {
+        ph = next[0];
+#pragma unroll
+        for (int i = 0; i < fl_piece / 2; i++)
+          ent[i] = next[1 + i];
+        next += 5;
+        more--;
+      }
+      if (__any(len > fl_piece / 2))
+        fl_connections<P, NT, fl_piece>(in, a.tab + s * NT, N, len, cur, c);
+      else
+        fl_connections<P, NT, fl_piece / 2>(in, a.tab + s * NT, N, len, cur, c);
+    }
+    // lane e holds shares of the rows of its fibre: row r's entry is e with
+    // its digit s replaced by r
+    if (mine)
+    {
+#pragma unroll
+      for (int r = 0; r < NT; r++)
+        ex[s * tpb + t + (r - s) * stride] = c[r];
+    }
+    __syncthreads();
+    if (round + 1 == rounds)
+      break;
+#pragma unroll
+    for (int r = 0; r < NT; r++)
+      acc += ex[r * tpb + t];
+    __syncthreads();
+  }
+  if (rounds > 1)
+  {
+    // earlier rounds' sums join the last round's shares
+    const P last = ex[t];
+    __syncthreads();
+    ex[t] = acc + last;
+    __syncthreads();
+  }
+  if (!live || (head.y & 0xffff) != 0)
+    return;
+  P sum = 0;
+  const int count = head.y >> 16;
+  for (int i = 0; i < count; i++)
+  {
+#pragma unroll
+    for (int r = 0; r < NT; r++)
+      sum += ex[r * tpb + t + i * N];
+  }
+  fl_store(a, head.z, int64_t(head.x) * N + e, sum);
+}
+
+//! One stage for n > 4 or N > 1024: a workgroup per job, its threads over the
+//! cell's entries, row by row.
+template<typename P>
+__global__ void __launch_bounds__(256) fl_stage_any(fl_args<P> a, int group0)
+{
+  const int4 *rec = a.slots + int64_t(group0 + blockIdx.x) * 7;
+  const int4 head = rec[0], tail = rec[1];
+  const int n = a.n;
+  for (int e = threadIdx.x; e < a.N; e += blockDim.x)
+  {
+    P sum = 0;
+    for (int i = 0; i <= head.w; i++)
+    {
+      const int4 *p = (i == 0) ? rec + 2 : a.pieces + int64_t(tail.x + i - 1) * 5;
+      const int4 ph = p[0];
+      const int s = fl_digit(e, static_cast<unsigned>(ph.z), n);
+      const P *in = ((ph.x == 0) ? a.x : a.work + int64_t(ph.x - 1) * a.stride) + e - s * ph.y;
+      const int2 *ent = reinterpret_cast<const int2 *>(p + 1);
+      for (int u = 0; u < (ph.w & 0xffff); u++)
+      {
+        const P *A = a.tab + int64_t(ent[u].y) * (int64_t(n) * n) + s;
+        const P *xin = in + int64_t(ent[u].x) * a.N;
+        for (int j = 0; j < n; j++)
+          sum = fma(A[j * n], xin[j * ph.y], sum);
+      }
+    }
+    fl_store(a, head.z, int64_t(head.x) * a.N + e, sum);
+  }
+}
+
+//! Factor tables: block q of table i is the sum over its (term, dimension)
+//! pairs of connect_1d block q (column-major, as in vA); then per 1D cell the
+//! diagonal blocks cut to the columns from the row's own on (upper) and
+//! before it (lower).  The last block of all is zero.
+template<typename P>
+__global__ void __launch_bounds__(256)
+    fl_tables(const P *__restrict__ vA, const int *__restrict__ ptr, const int *__restrict__ src,
+              const int *__restrict__ c1_diag, int ntab, int nconn, int M, int n, int d, int T,
+              P *tab)
+{
+  const int nn = n * n;
+  const int64_t per = int64_t(nconn + 2 * M) * nn;
+  for (int64_t i = blockIdx.x * int64_t(256) + threadIdx.x; i < per * ntab + nn;
+       i += int64_t(256) * gridDim.x)
+  {
+    const int t = static_cast<int>(i / per);
+    const int64_t rem = i - t * per;
+    const int b = static_cast<int>(rem / nn);
+    const int w = static_cast<int>(rem - int64_t(b) * nn);
+    const int j = w / n, s = w - j * n;
+    int q = b;
+    bool keep = t < ntab;
+    if (keep && b >= nconn)
+    {
+      const bool upper = b < nconn + M;
+      q = c1_diag[b - nconn - (upper ? 0 : M)];
+      keep = upper ? j >= s : j < s;
+    }
+    P v = 0;
+    if (keep)
+      for (int k = ptr[t]; k < ptr[t + 1]; k++)
+        v += vA[((int64_t(q) * T + src[2 * k]) * d + src[2 * k + 1]) * nn + w];
+    tab[i] = v;
+  }
+}
+
+//! One product of the plan before it is laid out.
+struct product
+{
+  int in, out; // vectors: 0 the input, v > 0 work vector v - 1; out -1: y
+  int k, fill, table, stage;
+};
+
+//! The products of all terms, in stages (see the file comment).
+struct program
+{
+  std::vector<product> prods;
+  std::vector<std::vector<std::pair<int, int>>> tables; // (term, dimension) pairs
+  int vectors = 0, stages = 0, identities = 0;
+
+  program(int T, std::vector<std::vector<int>> const &term_act)
+  {
+    std::map<int, int> single; // dimension -> table of the one-dimension terms
+    for (int t = 0; t < T; t++)
+    {
+      act = term_act[t];
+      const int m = static_cast<int>(act.size());
+      if (m == 0)
+      {
+        identities++;
+        continue;
+      }
+      stages = std::max(stages, m);
+      table_of.assign(m, -1);
+      if (m == 1)
+      {
+        auto it = single.find(act[0]);
+        if (it != single.end())
+        {
+          tables[it->second].emplace_back(t, act[0]);
+          continue;
+        }
+        single.emplace(act[0], static_cast<int>(tables.size()));
+      }
+      for (int i = 0; i < m; i++)
+      {
+        table_of[i] = static_cast<int>(tables.size());
+        tables.push_back({{t, act[i]}});
+      }
+      upper.clear();
+      partial.clear();
+      emit(m - 1, 0, -1, m - 1);
+    }
+    // a product's stage is where its output is formed; y is formed last
+    for (auto &p : prods)
+      if (p.out < 0)
+        p.stage = std::max(stages, 1) - 1;
+  }
+
+private:
+  std::vector<int> act, table_of;
+  std::map<int, int> upper;                    // set of uppers -> vector
+  std::map<std::pair<int, int>, int> partial;  // (i, set) -> vector Op_i u_set
+
+  //! u_set: the uppers of `set` (bits over act), the highest first.
+  int upper_vector(int set)
+  {
+    if (set == 0)
+      return 0;
+    auto it = upper.find(set);
+    if (it != upper.end())
+      return it->second;
+    int low = 0; // the lowest bit acts last
+    while (((set >> low) & 1) == 0)
+      low++;
+    const int rest = set & (set - 1);
+    const int in = upper_vector(rest);
+    const int v = ++vectors;
+    prods.push_back({in, v, act[low], gk_upper, table_of[low], __builtin_popcount(rest)});
+    upper.emplace(set, v);
+    return v;
+  }
+  //! Adds Op_i u_set to vector `out`, formed in stage `stage`.
+  void emit(int i, int set, int out, int stage)
+  {
+    if (i == 0)
+    {
+      prods.push_back({upper_vector(set), out, act[0], gk_full, table_of[0], stage});
+      return;
+    }
+    const std::pair<int, int> key(i - 1, set);
+    auto it = partial.find(key);
+    if (it == partial.end())
+    {
+      const int v = ++vectors;
+      it = partial.emplace(key, v).first;
+      emit(i - 1, set, v, __builtin_popcount(set) + i - 1);
+    }
+    prods.push_back({it->second, out, act[i], gk_lower, table_of[i], stage});
+    emit(i - 1, set | (1 << i), out, stage);
+  }
+};
+
+//! The part [lo, hi) of a cell's list a fill walks.
+static void fill_range(gk_lists const &l, int cell, int fill, int &lo, int &hi)
+{
+  lo = (fill == gk_upper) ? l.diag[cell] : l.ptr[cell];
+  hi = (fill == gk_lower) ? l.diag[cell] + 1 : l.ptr[cell + 1];
+}
+} // namespace
+
+void order_by_dims(int d, int64_t cells, const int *elem, std::vector<int> const &dims, int M,
+                   std::vector<int> &order)
+{
+  order.resize(cells);
+  std::iota(order.begin(), order.end(), 0);
+  if (M > 16 * cells + 1024)
+  {
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+      for (int k : dims)
+      {
+        const int ea = elem[int64_t(a) * d + k], eb = elem[int64_t(b) * d + k];
+        if (ea != eb)
+          return ea < eb;
+      }
+      return false;
+    });
+    return;
+  }
+  // stable counting sorts, the least significant dimension first
+  std::vector<int> count(M + 1), next(cells);
+  for (size_t i = dims.size(); i-- > 0;)
+  {
+    const int k = dims[i];
+    std::fill(count.begin(), count.end(), 0);
+    for (int64_t c = 0; c < cells; c++)
+      count[elem[c * d + k] + 1]++;
+    for (int v = 0; v < M; v++)
+      count[v + 1] += count[v];
+    for (int c : order)
+      next[count[elem[int64_t(c) * d + k]]++] = c;
+    order.swap(next);
+  }
+}
+
+int build_fibre_lists(int d, int64_t cells, const int *elem, int k, int M,
+                      std::vector<int> const &c1_pntr, std::vector<int> const &c1_indx,
+                      std::vector<int> const &c1_diag, gk_lists &out, std::vector<int> &order,
+                      int64_t &repeated)
+{
+  std::vector<int> dims;
+  for (int j = 0; j < d; j++)
+    if (j != k)
+      dims.push_back(j);
+  dims.push_back(k);
+  order_by_dims(d, cells, elem, dims, M, order);
+  repeated = -1;
+  // pass 0 counts every cell's connections, pass 1 writes them
+  std::vector<int> member(M, -1);
+  out.ptr.assign(cells + 1, 0);
+  out.diag.assign(cells, -1);
+  for (int pass = 0; pass < 2; pass++)
+  {
+    for (int64_t f0 = 0; f0 < cells;)
+    {
+      const int *first = elem + int64_t(order[f0]) * d;
+      int64_t f1 = f0;
+      for (; f1 < cells; f1++)
+      {
+        const int *cell = elem + int64_t(order[f1]) * d;
+        bool same = true;
+        for (int j = 0; j < d && same; j++)
+          same = (j == k) || cell[j] == first[j];
+        if (!same)
+          break;
+        if (pass == 0 && member[cell[k]] >= 0 && (repeated < 0 || order[f1] < repeated))
+          repeated = order[f1];
+        member[cell[k]] = order[f1];
+      }
+      const int last = elem[int64_t(order[f1 - 1]) * d + k];
+      for (int64_t f = f0; f < f1; f++)
+      {
+        const int c = order[f], r = elem[int64_t(c) * d + k];
+        int cnt = 0;
+        const int base = out.ptr[c];
+        for (int q = c1_pntr[r]; q < c1_pntr[r + 1]; q++)
+        {
+          const int col = c1_indx[q];
+          if (col > last)
+            break;
+          if (member[col] < 0)
+            continue;
+          if (pass == 1)
+          {
+            if (q == c1_diag[r])
+              out.diag[c] = base + cnt;
+            out.cell[base + cnt] = member[col];
+            out.q[base + cnt] = q;
+          }
+          cnt++;
+        }
+        if (pass == 0)
+          out.ptr[c + 1] = cnt;
+      }
+      for (int64_t f = f0; f < f1; f++)
+        member[elem[int64_t(order[f]) * d + k]] = -1;
+      f0 = f1;
+    }
+    if (pass == 0)
+    {
+      if (repeated >= 0)
+        return AKM_SUCCESS;
+      int64_t total = 0;
+      for (int64_t c = 0; c < cells; c++)
+      {
+        total += out.ptr[c + 1];
+        if (total > (int64_t(1) << 31) - 1)
+          return set_error(AKM_ERR_UNSUPPORTED, "global kron: connection lists too large");
+        out.ptr[c + 1] = static_cast<int>(total);
+      }
+      out.cell.resize(total);
+      out.q.resize(total);
+    }
+  }
+  for (int64_t c = 0; c < cells; c++)
+    if (out.diag[c] < 0 || out.cell[out.diag[c]] != c)
+      return set_error(AKM_ERR_INVALID, "global kron: connect_1d row without its diagonal");
+  return AKM_SUCCESS;
+}
+
+bool whole_level_grid(int d, int64_t cells, const int *elem)
+{
+  std::map<std::array<signed char, 6>, int64_t> levels;
+  std::array<signed char, 6> key{}, last{};
+  int64_t *last_count = nullptr;
+  for (int64_t c = 0; c < cells; c++)
+  {
+    for (int k = 0; k < d; k++)
+    {
+      const int e = elem[c * d + k];
+      key[k] = (e == 0) ? 0 : static_cast<signed char>(32 - __builtin_clz(unsigned(e)));
+    }
+    if (last_count == nullptr || key != last)
+    {
+      last_count = &levels[key];
+      last = key;
+    }
+    ++*last_count;
+  }
+  for (auto const &kv : levels)
+  {
+    int64_t whole = 1;
+    for (int k = 0; k < d; k++)
+    {
+      whole *= (kv.first[k] <= 1) ? 1 : int64_t(1) << (kv.first[k] - 1);
+      if (kv.first[k] > 0)
+      {
+        key = kv.first;
+        key[k]--;
+        if (levels.count(key) == 0)
+          return false;
+      }
+    }
+    if (kv.second != whole)
+      return false;
+  }
+  return true;
+}
+
+int64_t fibre_lanes(akm_matrix_s const &m, std::vector<gk_lists> const &lists,
+                    std::vector<std::vector<int>> const &term_act)
+{
+  const program prog(m.T, term_act);
+  // half of the connections lie on each side of the diagonal
+  int64_t steps = 0;
+  for (auto const &p : prog.prods)
+    steps += static_cast<int64_t>(lists[p.k].cell.size()) / (p.fill == gk_full ? 1 : 2);
+  return steps * m.N;
+}
+
+int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells, const int *elem,
+                     std::vector<gk_lists> const &lists,
+                     std::vector<std::vector<int>> const &term_act,
+                     std::vector<int> const &c1_diag, fibre_plan &plan)
+{
+  const int d = m.d, n = m.n, N = static_cast<int>(m.N);
+  const program prog(m.T, term_act);
+  // lanes share a workgroup's LDS by slot; wider tensors and larger blocks
+  // take one workgroup per cell.  Workgroups of 256 threads start sooner
+  // (d = 2, n = 2, level 5: 3.2 us an apply against 3.6 with 512 and 5.0 with
+  // 1024); from 65 entries on a cell's list needs the slots of 1024 (d = 4,
+  // n = 3, level 5: 9.4 us against 10.9 with 256 or 512)
+  plan.slots_of_lanes = n >= 2 && n <= 4 && N <= 1024;
+  plan.tpb = !plan.slots_of_lanes ? 256 : (N <= 64 ? 256 : 1024);
+  plan.nslot = plan.slots_of_lanes ? plan.tpb / N : 1;
+  plan.vectors = prog.vectors;
+  plan.identities = prog.identities;
+  plan.ntab = static_cast<int>(prog.tables.size());
+  plan.nconn = m.nconn;
+  plan.M = m.M;
+  plan.stride = cells * N;
+  const int64_t blocks = int64_t(plan.nconn) + 2 * plan.M; // of one table
+  if (blocks * plan.ntab >= (int64_t(1) << 31) - 1 || cells >= (int64_t(1) << 31))
+    return set_error(AKM_ERR_UNSUPPORTED, "fibre plan: factor tables too large");
+  const int zero_block = static_cast<int>(blocks * plan.ntab);
+
+  std::vector<int> stride(d, 1);
+  for (int k = d - 2; k >= 0; k--)
+    stride[k] = stride[k + 1] * n;
+  auto new_piece = [&](product const &p, int cell) {
+    fl_piece_rec r{};
+    r.in = p.in;
+    r.stride = stride[p.k];
+    r.magic = (r.stride == 1)
+                  ? 0
+                  : static_cast<unsigned>(((uint64_t(1) << 32) + r.stride - 1) / r.stride);
+    for (auto &en : r.entry)
+      en = make_int2(p.in == 0 && cell >= active_cells ? 0 : cell, zero_block);
+    return r;
+  };
+
+  // slots, stage by stage
+  std::vector<fl_slot_rec> slots;
+  std::vector<fl_piece_rec> pieces;
+  fl_slot_rec empty{};
+  empty.cell = -1;
+  const int S = plan.nslot;
+  const int nstages = std::max(prog.stages, 1);
+  struct job_rec
+  {
+    int first, count, length; // its slots in `made`, its connections
+  };
+  for (int st = 0; st < nstages; st++)
+  {
+    std::map<int, std::vector<int>> outs; // output vector -> its products
+    for (size_t i = 0; i < prog.prods.size(); i++)
+      if (prog.prods[i].stage == st)
+        outs[prog.prods[i].out].push_back(static_cast<int>(i));
+    if (st + 1 == nstages)
+      outs[-1]; // y is always written
+    std::vector<fl_slot_rec> made;
+    std::vector<job_rec> jobs;
+    for (auto &ov : outs)
+    {
+      // products of one dimension together: a slot's rounds are few
+      std::stable_sort(ov.second.begin(), ov.second.end(),
+                       [&](int u, int v) { return prog.prods[u].k < prog.prods[v].k; });
+      const int64_t ncell = (ov.first < 0) ? active_cells : cells;
+      for (int64_t c64 = 0; c64 < ncell; c64++)
+      {
+        const int c = static_cast<int>(c64);
+        int64_t total = 0;
+        int whole = 0; // slots with one piece each
+        for (int i : ov.second)
+        {
+          int lo, hi;
+          fill_range(lists[prog.prods[i].k], c, prog.prods[i].fill, lo, hi);
+          total += hi - lo;
+          whole += (hi - lo + fl_piece - 1) / fl_piece;
+        }
+        // slots of equal length when one-piece slots do not fit
+        const bool split = whole <= S;
+        const int64_t target = split ? fl_piece : (total + S - 1) / S;
+        const int first = static_cast<int>(made.size());
+        int64_t room = 0;
+        for (int i : ov.second)
+        {
+          product const &p = prog.prods[i];
+          gk_lists const &l = lists[p.k];
+          int lo, hi;
+          fill_range(l, c, p.fill, lo, hi);
+          if (split)
+            room = 0; // pieces do not share slots
+          while (lo < hi)
+          {
+            const bool fresh = room == 0;
+            if (fresh)
+              room = target;
+            fl_piece_rec pr = new_piece(p, c);
+            int len = 0;
+            for (; lo < hi && len < fl_piece && len < room; lo++)
+            {
+              // cells the input does not hold are zero
+              if (p.in == 0 && l.cell[lo] >= active_cells)
+                continue;
+              int q = l.q[lo];
+              if (lo == l.diag[c] && p.fill != gk_full)
+                q = plan.nconn + elem[c64 * d + p.k] + (p.fill == gk_lower ? plan.M : 0);
+              pr.entry[len++] = make_int2(l.cell[lo], static_cast<int>(p.table * blocks + q));
+            }
+            room -= len;
+            pr.len = len | (1 << 16);
+            if (fresh)
+            {
+              fl_slot_rec sr{};
+              sr.cell = c;
+              sr.group = static_cast<int>(made.size()) - first;
+              sr.vec = ov.first < 0 ? -1 : ov.first - 1;
+              sr.rounds = 1;
+              sr.p = pr;
+              made.push_back(sr);
+            }
+            else
+            {
+              fl_slot_rec &sr = made.back();
+              fl_piece_rec &before = (sr.more == 0) ? sr.p : pieces.back();
+              if (before.stride == pr.stride)
+                before.len &= 0xffff; // the same round goes on
+              else
+                sr.rounds++;
+              if (sr.more++ == 0)
+                sr.next = static_cast<int>(pieces.size());
+              pieces.push_back(pr);
+            }
+          }
+        }
+        if (static_cast<int>(made.size()) == first)
+        {
+          fl_slot_rec sr{};
+          sr.cell = c;
+          sr.vec = ov.first < 0 ? -1 : ov.first - 1;
+          sr.rounds = 1;
+          sr.p = new_piece(product{0, 0, 0, gk_full, 0, 0}, c);
+          sr.p.len = 1 << 16;
+          made.push_back(sr);
+        }
+        const int count = static_cast<int>(made.size()) - first;
+        for (int i = first; i < first + count; i++)
+          made[i].group |= count << 16;
+        jobs.push_back({first, count, static_cast<int>(std::min<int64_t>(total, 1 << 30))});
+      }
+    }
+    // jobs of many slots first, then long ones: a wavefront's pieces are
+    // alike and the long jobs start early
+    std::stable_sort(jobs.begin(), jobs.end(), [](job_rec const &u, job_rec const &v) {
+      return u.count != v.count ? u.count > v.count : u.length > v.length;
+    });
+    fibre_plan::stage rec;
+    rec.first_group = static_cast<int>(slots.size() / S);
+    for (auto const &j : jobs)
+    {
+      while (slots.size() % S != 0 && S - static_cast<int>(slots.size() % S) < j.count)
+        slots.push_back(empty);
+      slots.insert(slots.end(), made.begin() + j.first, made.begin() + j.first + j.count);
+    }
+    while (slots.size() % S != 0)
+      slots.push_back(empty);
+    rec.groups = static_cast<int>(slots.size() / S) - rec.first_group;
+    plan.stages.push_back(rec);
+  }
+  if (slots.size() > (size_t(1) << 28) || pieces.size() > (size_t(1) << 28))
+    return set_error(AKM_ERR_UNSUPPORTED, "fibre plan: too many slots");
+  for (size_t g = 0; g < slots.size(); g += S)
+  {
+    int rounds = 1;
+    for (int i = 0; i < S; i++)
+      rounds = std::max(rounds, slots[g + i].rounds);
+    for (int i = 0; i < S; i++)
+      slots[g + i].rounds = rounds;
+  }
+
+  std::vector<int> ptr(1, 0), src;
+  for (auto const &t : prog.tables)
+  {
+    for (auto const &pr : t)
+      src.insert(src.end(), {pr.first, pr.second});
+    ptr.push_back(static_cast<int>(src.size() / 2));
+  }
+  AKM_TRY(plan.slots.upload(reinterpret_cast<const int4 *>(slots.data()),
+                            int64_t(slots.size()) * 7, m.stream));
+  AKM_TRY(plan.pieces.upload(reinterpret_cast<const int4 *>(pieces.data()),
+                             int64_t(pieces.size()) * 5, m.stream));
+  AKM_TRY(plan.tab_ptr.upload(ptr.data(), int64_t(ptr.size()), m.stream));
+  AKM_TRY(plan.tab_src.upload(src.data(), int64_t(src.size()), m.stream));
+  AKM_TRY(plan.c1_diag.upload(c1_diag.data(), int64_t(c1_diag.size()), m.stream));
+  AKM_TRY(plan.work.allocate(int64_t(plan.vectors) * plan.stride * int64_t(m.esize)));
+  AKM_TRY(plan.tab.allocate((blocks * plan.ntab + 1) * n * n * int64_t(m.esize)));
+  plan.tab_valid = false;
+  plan.built = true;
+  return AKM_SUCCESS;
+}
+
+template<typename P>
+int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, P *y, P gamma,
+                const P *xg, const double *pc, double jdt)
+{
+  const int nn = m.n * m.n;
+  P *tab = reinterpret_cast<P *>(plan.tab.data());
+  if (!plan.tab_valid || plan.stamp != m.vA_stamp)
+  {
+    const int64_t count = int64_t(plan.nconn + 2 * plan.M) * nn * plan.ntab + nn;
+    const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
+    fl_tables<P><<<static_cast<unsigned>(blocks), 256, 0, m.stream>>>(
+        reinterpret_cast<const P *>(m.vA.data()), plan.tab_ptr.data(), plan.tab_src.data(),
+        plan.c1_diag.data(), plan.ntab, plan.nconn, plan.M, m.n, m.d, m.T, tab);
+    AKM_TRY(check_launch("fibre tables"));
+    plan.stamp = m.vA_stamp;
+    plan.tab_valid = true;
+  }
+  fl_args<P> a{};
+  a.slots = plan.slots.data();
+  a.pieces = plan.pieces.data();
+  a.tab = tab;
+  a.n = m.n;
+  a.N = static_cast<int>(m.N);
+  a.nslot = plan.nslot;
+  a.stride = plan.stride;
+  a.x = x;
+  a.work = reinterpret_cast<P *>(plan.work.data());
+  a.y = y;
+  a.xg = xg;
+  a.pc = pc;
+  a.jdt = jdt;
+  a.alpha = alpha;
+  a.beta = beta;
+  a.gamma = gamma;
+  a.identities = plan.identities;
+  const size_t lds = sizeof(P) * plan.tpb * m.n;
+  for (auto const &st : plan.stages)
+  {
+    const dim3 grid(static_cast<unsigned>(st.groups)), tpb(static_cast<unsigned>(plan.tpb));
+    if (!plan.slots_of_lanes)
+      fl_stage_any<P><<<grid, tpb, 0, m.stream>>>(a, st.first_group);
+    else if (m.n == 2)
+      fl_stage<P, 2><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+    else if (m.n == 3)
+      fl_stage<P, 3><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+    else
+      fl_stage<P, 4><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+    AKM_TRY(check_launch("fibre stage"));
+  }
+  return AKM_SUCCESS;
+}
+
+template int fibre_apply<double>(akm_matrix_s &, fibre_plan &, double, const double *, double,
+                                 double *, double, const double *, const double *, double);
+template int fibre_apply<float>(akm_matrix_s &, fibre_plan &, float, const float *, float,
+                                float *, float, const float *, const double *, double);
+} // namespace akm

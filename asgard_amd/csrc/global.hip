@@ -18,10 +18,12 @@
 // active ones.  For every dimension k and cell the host lists the connected
 // cells of its fibre (cells equal in all other 1D indices) with their
 // connect_1d positions.  A one-dimensional product in dimension k runs in
-// one of three layouts, which akm_autotune times: one lane per (chain, DOF),
-// the lanes of a cell reading each connected cell's tensor together; a group
-// of 8 lanes per DOF that split the list and sum by a fixed shuffle tree;
-// or one wavefront per (chain, cell) whose lane groups split the list.
+// one of these layouts, which akm_autotune times: one lane per (chain, DOF),
+// the lanes of a cell reading each connected cell's tensor together; one
+// wavefront per (chain, cell) whose lane groups split the list; the fibre
+// walk (layout 8, fibre.hip), whose slots split every list into short pieces
+// and which takes the products shared by chains once; or the slab layout
+// below.
 // Cells are taken fibre by fibre, so the cells reading the same tensors run
 // together.  The factor values are the same connect_1d blocks (vA) the pair
 // operator uses.  All chains advance together, one launch per stage, each
@@ -29,10 +31,12 @@
 // order and applies alpha/beta/gamma (and optionally the reference's Jacobi
 // scaling).
 #include "akm_internal.hpp"
+#include "fibre.hpp"
 #include "grid.hpp"
 #include "matrix.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <memory>
 #include <vector>
@@ -42,13 +46,6 @@ namespace akm
 constexpr int gk_max_dims = 6;
 constexpr int gk_threads = 256;
 constexpr int gk_group_max = 4; // chains sharing one first-stage input read
-
-enum gk_fill : int
-{
-  gk_upper = 0, // from the diagonal on (diagonal included)
-  gk_full = 1,
-  gk_lower = 2, // strictly before the diagonal
-};
 
 //! Device view of the global operator.
 struct gk_args
@@ -74,15 +71,14 @@ struct gk_args
   bool xcd_order;      // cell layouts: each XCD takes contiguous items
 };
 
-//! Lane g's share (connections g, g + LANES, ...) of one stage's product for
-//! DOF i of a chain: (fill part of A_{t,k}) applied along dimension k to
-//! `in` (padded vector, or the active-only x when `in_active_only`).  With
-//! one lane per DOF the lanes of a cell read each connected cell's tensor
-//! together (coalesced); with several, long connection lists are split.
-template<typename P, int LANES>
+//! One stage's product for DOF i of a chain: (fill part of A_{t,k}) applied
+//! along dimension k to `in` (padded vector, or the active-only x when
+//! `in_active_only`).  The lanes of a cell read each connected cell's tensor
+//! together (coalesced).
+template<typename P>
 __device__ __forceinline__ P gk_row_part(gk_args const &a, const P *__restrict__ vA, int t,
                                          int k, int fill, const P *__restrict__ in,
-                                         bool in_active_only, int64_t i, int g)
+                                         bool in_active_only, int64_t i)
 {
   const int N = a.N, n = a.n, d = a.d;
   const int64_t cell = i / N;
@@ -103,7 +99,7 @@ __device__ __forceinline__ P gk_row_part(gk_args const &a, const P *__restrict__
   const int *__restrict__ nq = a.nb_q[k];
   P acc = 0;
 #pragma unroll 4
-  for (int p = lo + g; p < hi; p += LANES)
+  for (int p = lo; p < hi; p++)
   {
     const int cj = ncell[p];
     if (in_active_only && cj >= a.active_cells)
@@ -124,29 +120,18 @@ __device__ __forceinline__ P gk_row_part(gk_args const &a, const P *__restrict__
   return acc;
 }
 
-//! Sum over the LANES lanes of a group, the same fixed tree on every run.
-template<typename P, int LANES>
-__device__ __forceinline__ P gk_group_sum(P v)
-{
-#pragma unroll
-  for (int off = LANES / 2; off > 0; off >>= 1)
-    v += __shfl_xor(v, off, LANES);
-  return v;
-}
-
-//! Stage `st` of every chain with more than st stages; one group of LANES
-//! lanes per (chain, padded DOF), cells taken fibre by fibre so that the
-//! cells reading the same connected tensors run together.
-template<typename P, int LANES>
+//! Stage `st` of every chain with more than st stages; one lane per (chain,
+//! padded DOF), cells taken fibre by fibre so that the cells reading the same
+//! connected tensors run together.
+template<typename P>
 __global__ void __launch_bounds__(gk_threads)
     gk_stage(gk_args a, const P *__restrict__ vA, const int *__restrict__ list, int nlist, int st,
              const P *__restrict__ x, P *work)
 {
   const int64_t dofs = a.cells * a.N;
-  const int64_t groups = dofs * nlist;
-  const int g = threadIdx.x % LANES;
-  for (int64_t gi = (blockIdx.x * int64_t(gk_threads) + threadIdx.x) / LANES; gi < groups;
-       gi += int64_t(gk_threads / LANES) * gridDim.x)
+  const int64_t count = dofs * nlist;
+  for (int64_t gi = blockIdx.x * int64_t(gk_threads) + threadIdx.x; gi < count;
+       gi += int64_t(gk_threads) * gridDim.x)
   {
     const int li = static_cast<int>(gi / dofs);
     const int64_t pos = gi - int64_t(li) * dofs;
@@ -157,10 +142,8 @@ __global__ void __launch_bounds__(gk_threads)
     const int64_t i = int64_t(a.order[k][pcell]) * a.N + (pos - pcell * a.N);
     const int fill = a.ch_fill[c * gk_max_dims + st];
     const P *in = (st == 0) ? x : work + (int64_t((st - 1) & 1) * a.nslots + slot) * a.stride;
-    const P v = gk_group_sum<P, LANES>(
-        gk_row_part<P, LANES>(a, vA, a.ch_term[c], k, fill, in, st == 0, i, g));
-    if (g == 0)
-      work[(int64_t(st & 1) * a.nslots + slot) * a.stride + i] = v;
+    work[(int64_t(st & 1) * a.nslots + slot) * a.stride + i] =
+        gk_row_part<P>(a, vA, a.ch_term[c], k, fill, in, st == 0, i);
   }
 }
 
@@ -986,13 +969,19 @@ static int gk_blocks_xcd(int64_t work)
 //! Host and device data of a global operator.
 struct akm_global_s
 {
+  using fibre_plan = akm::fibre_plan;
+  using gk_lists = akm::gk_lists;
   int64_t active_cells = 0, cells = 0;
   std::vector<int> elem_host; // padded cells x d
   akm::dev_buffer<int> elem;
   akm::dev_buffer<int> nb_ptr[akm::gk_max_dims], nb_cell[akm::gk_max_dims],
       nb_q[akm::gk_max_dims], nb_diag[akm::gk_max_dims], order[akm::gk_max_dims];
-  // chains
-  std::vector<int> ch_nst_host;
+  // chains: per chain its term, stages, and its stages' dimensions and fills
+  // (gk_max_dims each), and its work-buffer slot
+  struct
+  {
+    std::vector<int> term, nst, dim, fill, slot;
+  } chains_host;
   akm::dev_buffer<int> ch_term, ch_nst, ch_dim, ch_fill, ch_slot;
   std::vector<akm::dev_buffer<int>> stage_list; // per stage: the chains that have it
   std::vector<int> stage_count;
@@ -1003,9 +992,17 @@ struct akm_global_s
   bool first_grouped = false; // chosen by global_autotune
   bool xcd_order = false;     // chosen by global_autotune (cell layouts)
   int nchains = 0, nslots = 0, max_stages = 0;
-  // lanes per DOF row: 1 (coalesced tensors), 8 (split lists), or 0: one
-  // wavefront per cell (n^d <= 64)
+  // chain layouts: 1 (a lane per DOF), 0 (a wavefront per cell, n^d <= 64),
+  // or 8: the fibre walk, which has its own plan
   int lanes = 1;
+  fibre_plan fl;
+  std::vector<gk_lists> lists; // host fibre lists, per dimension
+  std::vector<std::vector<int>> term_act; // non-identity dimensions per term
+  int64_t fl_lanes = 0; // (lane, connection) steps of the fibre walk
+  // the operator of a sparse-grid (pair) handle taken one dimension at a
+  // time: no padding, no chain layouts, no Jacobi diagonal
+  bool pair = false;
+  bool slabs_built = false;
   // summation sources of gk_sum: chain layouts, and the slab layout
   akm::dev_buffer<int> src_chain, src_slab;
   int nsrc_chain = 0, nsrc_slab = 0;
@@ -1061,7 +1058,7 @@ struct akm_global_s
   akm::dev_buffer<unsigned char> work;
   akm::dev_buffer<double> pc; // Jacobi diagonal (active DOFs)
   std::vector<int> c1_pntr_h, c1_indx_h, c1_diag_h;
-  akm::dev_buffer<int> c1_diag; // device copy, made by the first device update
+  akm::dev_buffer<int> c1_diag; // device copy
   int64_t flops = 0;
 };
 
@@ -1257,6 +1254,8 @@ static int global_apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y
                                                                   jdt);
     return check_launch("global kron scale");
   }
+  if (!g.slab && g.lanes == 8)
+    return fibre_apply<P>(m, g.fl, alpha, x, beta, y, gamma, xg, pc, jdt);
   const gk_args a = global_args(m);
   const P *vA = reinterpret_cast<const P *>(m.vA.data());
   P *work = reinterpret_cast<P *>(g.work.data());
@@ -1270,7 +1269,7 @@ static int global_apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y
       continue;
     const int *list = slab ? g.stage_list_rest[st].data() : g.stage_list[st].data();
     const int blocks = (lanes == 0) ? gk_blocks_xcd(g.cells * nl * wave_size)
-                                    : gk_blocks(g.cells * m.N * nl * lanes);
+                                    : gk_blocks(g.cells * m.N * nl);
     if (!slab && lanes == 0 && st == 0 && g.first_grouped && g.first_largest > 1 && m.n >= 2 &&
         m.n <= 4)
     {
@@ -1309,10 +1308,8 @@ static int global_apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y
         gk_cell_stage<P, 0><<<blocks, gk_threads, 0, m.stream>>>(a, vA, list, nl, st, x, work);
       }
     }
-    else if (lanes == 8)
-      gk_stage<P, 8><<<blocks, gk_threads, 0, m.stream>>>(a, vA, list, nl, st, x, work);
     else
-      gk_stage<P, 1><<<blocks, gk_threads, 0, m.stream>>>(a, vA, list, nl, st, x, work);
+      gk_stage<P><<<blocks, gk_threads, 0, m.stream>>>(a, vA, list, nl, st, x, work);
     AKM_TRY(check_launch("global kron stage"));
   }
   if (slab)
@@ -1346,55 +1343,20 @@ int global_apply(akm_matrix_s &m, double alpha, const void *x, double beta, void
                                    jacobi, jdt);
 }
 
-//! The Jacobi diagonal of the reference's implicit step
-//! (build_preconditioner, src/asgard_kronmult_matrix.cpp:1016-1067): for
-//! every active DOF, the sum over terms of the product over dimensions of the
-//! 1D factors' diagonal entries (every dimension, identity factors included).
-template<typename P>
-static void jacobi_diagonal(akm_matrix_s const &m, const P *vA, std::vector<double> &pc)
-{
-  const akm_global_s &g = *m.gk;
-  const int d = m.d, n = m.n, T = m.T;
-  const int64_t N = m.N, nn = int64_t(n) * n;
-  pc.assign(g.active_cells * N, 0.0);
-  for (int64_t c = 0; c < g.active_cells; c++)
-    for (int64_t e = 0; e < N; e++)
-    {
-      double sum = 0;
-      for (int t = 0; t < T; t++)
-      {
-        double prod = 1;
-        int64_t rest = e;
-        for (int k = d - 1; k >= 0; k--)
-        {
-          const int s = static_cast<int>(rest % n);
-          rest /= n;
-          const int r1 = g.elem_host[c * d + k];
-          const int64_t q = g.c1_diag_h[r1];
-          prod *= static_cast<double>(vA[((q * T + t) * d + k) * nn + int64_t(s) * n + s]);
-        }
-        sum += prod;
-      }
-      pc[c * N + e] = sum;
-    }
-}
-
 int global_update(akm_matrix_s &m, const void *vA)
 {
   AKM_HIP(hipMemcpyAsync(m.vA.data(), vA, m.num_vA * m.esize, hipMemcpyHostToDevice, m.stream));
-  std::vector<double> pc;
-  if (m.prec == AKM_F64)
-    jacobi_diagonal(m, static_cast<const double *>(vA), pc);
-  else
-    jacobi_diagonal(m, static_cast<const float *>(vA), pc);
-  AKM_TRY(m.gk->pc.upload(pc.data(), int64_t(pc.size()), m.stream));
+  AKM_TRY(global_device_jacobi(m));
   AKM_HIP(hipStreamSynchronize(m.stream));
   return AKM_SUCCESS;
 }
 
-//! jacobi_diagonal on the device, one thread per active DOF, with the same
-//! operations in the same order (no contraction into fma), so the two agree
-//! bit for bit.
+//! The Jacobi diagonal of the reference's implicit step
+//! (build_preconditioner, src/asgard_kronmult_matrix.cpp:1016-1067): for
+//! every active DOF, the sum over terms of the product over dimensions of the
+//! 1D factors' diagonal entries (every dimension, identity factors included),
+//! one thread per DOF, products and sums rounded one by one (no contraction
+//! into fma).
 template<typename P>
 __global__ void __launch_bounds__(gk_threads)
     gk_jacobi(int64_t active_cells, int d, int n, int T, int64_t N, const int *elem,
@@ -1431,6 +1393,7 @@ int global_device_jacobi(akm_matrix_s &m)
   const int64_t work = g.active_cells * m.N;
   if (work == 0)
     return AKM_SUCCESS;
+  AKM_TRY(g.pc.allocate(work));
   if (m.prec == AKM_F64)
     gk_jacobi<double><<<gk_blocks(work), gk_threads, 0, m.stream>>>(
         g.active_cells, m.d, m.n, m.T, m.N, g.elem.data(), g.c1_diag.data(),
@@ -1440,6 +1403,17 @@ int global_device_jacobi(akm_matrix_s &m)
         g.active_cells, m.d, m.n, m.T, m.N, g.elem.data(), g.c1_diag.data(),
         reinterpret_cast<const float *>(m.vA.data()), g.pc.data());
   return check_launch("global kron Jacobi diagonal");
+}
+
+//! Builds the fibre-walk plan on first use.
+static int need_fibre_plan(akm_matrix_s &m)
+{
+  akm_global_s &g = *m.gk;
+  if (g.fl.built)
+    return AKM_SUCCESS;
+  g.fl = fibre_plan();
+  return build_fibre_plan(m, g.active_cells, g.cells, g.elem_host.data(), g.lists, g.term_act,
+                          g.c1_diag_h, g.fl);
 }
 
 int64_t global_flops(akm_matrix_s const &m) { return m.gk ? m.gk->flops : 0; }
@@ -1467,6 +1441,8 @@ int global_set_layout(akm_matrix_s &m, int layout)
   const bool cell = (layout >= 2 && layout <= 5);
   if (cell && m.N > wave_size)
     return set_error(AKM_ERR_UNSUPPORTED, "global kron: the cell layout needs n^d <= 64");
+  if (layout == 8)
+    AKM_TRY(need_fibre_plan(m));
   m.gk->slab = (layout == 6);
   if (m.gk->slab)
   {
@@ -1481,9 +1457,35 @@ int global_set_layout(akm_matrix_s &m, int layout)
   return AKM_SUCCESS;
 }
 
+//! Fibre walks of up to this many (lane, connection) steps are planned
+//! without being asked for (their slot records take about half as many
+//! bytes).
+constexpr int64_t fl_lanes_tuned = int64_t(1) << 26;
+//! The layout of a handle that is not tuned: the fibre walk up to this many
+//! (lane, connection) steps, then the slab layout.
+constexpr int64_t fl_lanes_default = int64_t(1) << 26;
+
+//! Up to this many steps the fibre walk is always the faster of the two.
+constexpr int64_t fl_lanes_small = int64_t(1) << 20;
+
+//! The layout used until akm_autotune or akm_set_tuning picks one; -1 when an
+//! operator of a pair handle has none.
+static int default_layout(akm_matrix_s const &m, akm_global_s const &g)
+{
+  if (g.fl_lanes <= fl_lanes_default)
+    return 8;
+  if (g.ngroups > 0 && (g.max_stages == 0 || g.stage_count_rest[0] == 0))
+    return 6;
+  if (g.pair)
+    return g.fl_lanes <= fl_lanes_tuned ? 8 : -1;
+  return (m.N <= wave_size) ? 2 : 1;
+}
+
+static int need_slabs(akm_matrix_s &m, akm_global_s &g);
+
 //! Times the row layouts on the operator itself (y is overwritten) and
 //! keeps the fastest.
-int global_autotune(akm_matrix_s &m, const void *x, void *y)
+int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms)
 {
   akm_global_s &g = *m.gk;
   hipEvent_t e0, e1;
@@ -1495,8 +1497,8 @@ int global_autotune(akm_matrix_s &m, const void *x, void *y)
   int rc = AKM_SUCCESS;
   bool best_xcd = false, best_slab = false;
   int best_moved = 0;
-  // layouts 1 and 8, then the cell layout with and without the grouped
-  // first stage (shared input reads against fewer, longer wavefronts), each
+  // layouts 1 and 8 (when its records stay small), then the cell layout with
+  // and without the grouped first stage (shared input reads against fewer, longer wavefronts), each
   // cell layout with and without the XCD-contiguous workgroup order, then
   // the slab layout (when some term has one or two non-identity dimensions)
   // with 0-100 % of its side-stream items moved to the main stream (100:
@@ -1513,8 +1515,24 @@ int global_autotune(akm_matrix_s &m, const void *x, void *y)
       continue;
     if (grouped && g.first_largest < 2)
       continue;
+    if (g.pair && lanes != 8 && !slab)
+      continue;
+    if (slab && g.pair && g.fl_lanes > fl_lanes_small)
+    {
+      rc = need_slabs(m, g);
+      if (rc != AKM_SUCCESS)
+        break;
+    }
     if (slab && g.ngroups == 0)
       continue;
+    if (lanes == 8)
+    {
+      if (g.fl_lanes > fl_lanes_tuned)
+        continue;
+      rc = need_fibre_plan(m);
+      if (rc != AKM_SUCCESS)
+        break;
+    }
     g.lanes = lanes;
     g.first_grouped = grouped;
     g.xcd_order = xcd;
@@ -1551,9 +1569,25 @@ int global_autotune(akm_matrix_s &m, const void *x, void *y)
   g.xcd_order = best_xcd;
   g.slab = best_slab;
   g.gs_moved = best_moved;
+  best_ms = best / 5;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return rc;
+}
+
+int factored_shape(akm_matrix_s const &m) { return global_layout(m) + 16 * m.gk->gs_moved; }
+
+int factored_set_shape(akm_matrix_s &m, int shape)
+{
+  int layout = shape % 16;
+  if (layout == 6)
+    AKM_TRY(need_slabs(m, *m.gk));
+  // the number may come from another grid of the same size
+  if (layout == 6 && m.gk->ngroups == 0)
+    layout = 8;
+  AKM_TRY(global_set_layout(m, layout));
+  m.gk->gs_moved = shape / 16;
+  return AKM_SUCCESS;
 }
 
 //! Ancestors of a 1D cell in the volume hierarchy: its parent chain down to
@@ -1581,12 +1615,6 @@ static int level_1d(int i)
   return l;
 }
 
-//! Per-dimension host copies of the fibre connection lists.
-struct gk_lists
-{
-  std::vector<int> ptr, cell, q, diag;
-};
-
 //! One bundle while the slab plan is made.
 struct gs_plan_bundle
 {
@@ -1598,12 +1626,13 @@ struct gs_plan_bundle
 //! dimensions (act[t] after the flux swap), their slabs, bundles, lists and
 //! work items.  A group whose largest slab does not fit one workgroup at
 //! one other-index combination per chunk is left to the cell-layout stages.
-static int build_slabs(akm_matrix_s &m, akm_global_s &g, std::vector<gk_lists> const &lists,
-                       std::vector<std::vector<int>> const &term_act,
-                       std::vector<int> const &ch_term, std::vector<int> const &ch_nst,
-                       std::vector<int> const &ch_dim, std::vector<int> const &ch_fill,
-                       std::vector<int> const &ch_slot)
+static int build_slabs(akm_matrix_s &m, akm_global_s &g)
 {
+  std::vector<gk_lists> const &lists = g.lists;
+  std::vector<std::vector<int>> const &term_act = g.term_act;
+  std::vector<int> const &ch_term = g.chains_host.term, &ch_nst = g.chains_host.nst,
+                         &ch_dim = g.chains_host.dim, &ch_fill = g.chains_host.fill,
+                         &ch_slot = g.chains_host.slot;
   const int d = m.d, n = m.n, T = m.T;
   const int L = m.max_level;
   const int nn = n * n;
@@ -1680,16 +1709,12 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g, std::vector<gk_lists> c
     for (int k = nd; k < d; k++)
       call *= n;
     // slabs: cells equal in every 1D index outside S, cell order kept
-    std::map<std::vector<int>, std::vector<int>> slabs;
-    std::vector<int> key;
-    for (int64_t c = 0; c < g.cells; c++)
-    {
-      key.clear();
-      for (int k = 0; k < d; k++)
-        if (std::find(S.begin(), S.end(), k) == S.end())
-          key.push_back(g.elem_host[c * d + k]);
-      slabs[key].push_back(static_cast<int>(c));
-    }
+    // (slabs in the order of those indices)
+    std::vector<int> other, by_slab;
+    for (int k = 0; k < d; k++)
+      if (std::find(S.begin(), S.end(), k) == S.end())
+        other.push_back(k);
+    order_by_dims(d, g.cells, g.elem_host.data(), other, m.M, by_slab);
     int group_chains = 0;
     for (size_t c = 0; c < ch_term.size(); c++)
       if (term_group[ch_term[c]] == static_cast<int>(gi))
@@ -1708,9 +1733,21 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g, std::vector<gk_lists> c
           lp = std::max(lp, level_1d(g.elem_host[int64_t(c) * d + k]));
       return lp;
     };
-    for (auto const &kv : slabs)
+    std::vector<int> sc;
+    for (int64_t s0 = 0; s0 < g.cells;)
     {
-      const std::vector<int> &sc = kv.second;
+      sc.clear();
+      for (; s0 < g.cells; s0++)
+      {
+        const int c = by_slab[s0];
+        bool same = true;
+        for (int k : other)
+          same = same && (sc.empty() || g.elem_host[int64_t(c) * d + k] ==
+                                            g.elem_host[int64_t(sc[0]) * d + k]);
+        if (!same)
+          break;
+        sc.push_back(c);
+      }
       const int64_t msz = static_cast<int64_t>(sc.size());
       const int64_t full = msz * ds * call;
       const int lp = slab_level(sc);
@@ -2134,61 +2171,83 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g, std::vector<gk_lists> c
   return AKM_SUCCESS;
 }
 
+//! Builds the slab layout on first use.  Chains outside its groups run in the
+//! chain layouts, which a pair handle does not have.
+static int need_slabs(akm_matrix_s &m, akm_global_s &g)
+{
+  if (g.slabs_built)
+    return AKM_SUCCESS;
+  g.slabs_built = true;
+  AKM_TRY(build_slabs(m, g));
+  if (!g.pair)
+    return AKM_SUCCESS;
+  if (g.max_stages > 0 && g.stage_count_rest[0] > 0)
+    g.ngroups = 0;
+  return (g.ngroups > 0) ? g.work.allocate(int64_t(g.ngroups) * g.cells * m.N * int64_t(m.esize))
+                         : AKM_SUCCESS;
+}
+
 //! Builds the padded cell set, the fibres, the chains and the work buffers
-//! (make_global_kron_matrix, src/asgard_kronmult_matrix.cpp:1198-1334).
+//! (make_global_kron_matrix, src/asgard_kronmult_matrix.cpp:1198-1334).  With
+//! `pair` (the operator of a sparse-grid handle, whose cells need no padding)
+//! only what the fibre walk and the slab layout use.  `repeated` = the first
+//! cell that equals an earlier one (nothing is built then), or -1.
 static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
-                        const int *active_mask, const int *flux_dim)
+                        const int *active_mask, const int *flux_dim, bool pair,
+                        int64_t &repeated)
 {
   auto g = std::unique_ptr<akm_global_s, void (*)(akm_global_s *)>(new akm_global_s(),
                                                                     destroy_global);
   const int d = m.d;
   const int64_t nact = m.rows;
   g->active_cells = nact;
+  g->pair = pair;
+  g->elem_host = elem_active;
+  repeated = -1;
 
   // ancestry completion (compute_ancestry_completion over the volume
   // hierarchy, src/asgard_indexset.cpp:243-318): add the missing ancestors
-  // in every dimension until none is missing; padding sorted
-  std::map<std::vector<int>, int64_t> index;
-  std::vector<int> key(d), anc;
-  for (int64_t c = 0; c < nact; c++)
+  // in every dimension until none is missing; padding sorted.  A grid of
+  // whole levels misses none.
+  if (!pair && !whole_level_grid(d, nact, elem_active.data()))
   {
-    key.assign(elem_active.begin() + c * d, elem_active.begin() + (c + 1) * d);
-    index.emplace(key, c);
-  }
-  std::vector<std::vector<int>> frontier, pad;
-  for (int64_t c = 0; c < nact; c++)
-    frontier.emplace_back(elem_active.begin() + c * d, elem_active.begin() + (c + 1) * d);
-  std::map<std::vector<int>, int> padset;
-  while (!frontier.empty())
-  {
-    std::vector<std::vector<int>> next;
-    for (auto const &cell : frontier)
-      for (int k = 0; k < d; k++)
-      {
-        parents_1d(cell[k], anc);
-        for (int a : anc)
+    std::map<std::vector<int>, int64_t> index;
+    std::vector<int> key(d), anc;
+    for (int64_t c = 0; c < nact; c++)
+    {
+      key.assign(elem_active.begin() + c * d, elem_active.begin() + (c + 1) * d);
+      index.emplace(key, c);
+    }
+    std::vector<std::vector<int>> frontier;
+    for (int64_t c = 0; c < nact; c++)
+      frontier.emplace_back(elem_active.begin() + c * d, elem_active.begin() + (c + 1) * d);
+    std::map<std::vector<int>, int> padset;
+    while (!frontier.empty())
+    {
+      std::vector<std::vector<int>> next;
+      for (auto const &cell : frontier)
+        for (int k = 0; k < d; k++)
         {
-          key = cell;
-          key[k] = a;
-          if (index.count(key) == 0 && padset.count(key) == 0)
+          parents_1d(cell[k], anc);
+          for (int a : anc)
           {
-            padset.emplace(key, 0);
-            next.push_back(key);
+            key = cell;
+            key[k] = a;
+            if (index.count(key) == 0 && padset.count(key) == 0)
+            {
+              padset.emplace(key, 0);
+              next.push_back(key);
+            }
           }
         }
-      }
-    frontier.swap(next);
-  }
-  g->elem_host = elem_active;
-  for (auto const &kv : padset)
-  {
-    index.emplace(kv.first, nact + static_cast<int64_t>(g->elem_host.size() / d - nact));
-    g->elem_host.insert(g->elem_host.end(), kv.first.begin(), kv.first.end());
+      frontier.swap(next);
+    }
+    for (auto const &kv : padset)
+      g->elem_host.insert(g->elem_host.end(), kv.first.begin(), kv.first.end());
   }
   g->cells = static_cast<int64_t>(g->elem_host.size() / d);
   if (g->cells * m.N > (int64_t(1) << 40))
     return set_error(AKM_ERR_UNSUPPORTED, "global kron: too many padded DOFs");
-  AKM_TRY(g->elem.upload(g->elem_host.data(), int64_t(g->elem_host.size())));
 
   // connect_1d (full hierarchy), the pattern of every 1D factor
   AKM_TRY(build_connect_1d(m.max_level, true, g->c1_pntr_h, g->c1_indx_h, g->c1_diag_h));
@@ -2196,70 +2255,33 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
   // per dimension: the fibres (cells equal in every other 1D index) and for
   // every cell its connected cells of the fibre, 1D index ascending
   std::vector<int64_t> nnz_dim(d, 0); // DOF-level pattern entries per dimension
-  std::vector<gk_lists> lists(d);
+  g->lists.resize(d);
+  std::vector<gk_lists> &lists = g->lists;
   for (int k = 0; k < d; k++)
   {
-    std::map<std::vector<int>, int> fib;
-    std::vector<int> fib_of(g->cells);
-    std::vector<std::map<int, int>> members; // 1D index -> cell
-    std::vector<int> other(d - 1);
-    for (int64_t c = 0; c < g->cells; c++)
-    {
-      for (int j = 0, o = 0; j < d; j++)
-        if (j != k)
-          other[o++] = g->elem_host[c * d + j];
-      auto it = fib.find(other);
-      if (it == fib.end())
-      {
-        it = fib.emplace(other, static_cast<int>(members.size())).first;
-        members.emplace_back();
-      }
-      fib_of[c] = it->second;
-      members[it->second].emplace(g->elem_host[c * d + k], static_cast<int>(c));
-    }
-    std::vector<int> ptr(g->cells + 1, 0), ncell, nq, ndiag(g->cells, -1);
-    for (int64_t c = 0; c < g->cells; c++)
-    {
-      const int r1 = g->elem_host[c * d + k];
-      const auto &mem = members[fib_of[c]];
-      for (int q = g->c1_pntr_h[r1]; q < g->c1_pntr_h[r1 + 1]; q++)
-      {
-        auto it = mem.find(g->c1_indx_h[q]);
-        if (it == mem.end())
-          continue;
-        if (q == g->c1_diag_h[r1])
-          ndiag[c] = static_cast<int>(ncell.size());
-        ncell.push_back(it->second);
-        nq.push_back(q);
-      }
-      if (ndiag[c] < 0 || ncell[ndiag[c]] != c)
-        return set_error(AKM_ERR_INVALID, "global kron: connect_1d row without its diagonal");
-      if (ncell.size() > (size_t(1) << 31) - 1)
-        return set_error(AKM_ERR_UNSUPPORTED, "global kron: connection lists too large");
-      ptr[c + 1] = static_cast<int>(ncell.size());
-      nnz_dim[k] += int64_t(ptr[c + 1] - ptr[c]) * m.n * m.N;
-    }
-    AKM_TRY(g->nb_ptr[k].upload(ptr.data(), int64_t(ptr.size())));
-    AKM_TRY(g->nb_cell[k].upload(ncell.data(), int64_t(ncell.size())));
-    AKM_TRY(g->nb_q[k].upload(nq.data(), int64_t(nq.size())));
-    AKM_TRY(g->nb_diag[k].upload(ndiag.data(), int64_t(ndiag.size())));
-    lists[k].ptr = std::move(ptr);
-    lists[k].cell = std::move(ncell);
-    lists[k].q = std::move(nq);
-    lists[k].diag = std::move(ndiag);
-    // processing order: fibre by fibre (fibres in key order), 1D index ascending
     std::vector<int> ord;
-    ord.reserve(g->cells);
-    for (auto const &kv : fib)
-      for (auto const &mc : members[kv.second])
-        ord.push_back(mc.second);
+    AKM_TRY(build_fibre_lists(d, g->cells, g->elem_host.data(), k, m.M, g->c1_pntr_h,
+                              g->c1_indx_h, g->c1_diag_h, lists[k], ord, repeated));
+    if (repeated >= 0)
+      return AKM_SUCCESS;
+    nnz_dim[k] = static_cast<int64_t>(lists[k].cell.size()) * m.n * m.N;
+    if (pair)
+      continue;
+    AKM_TRY(g->nb_ptr[k].upload(lists[k].ptr.data(), int64_t(lists[k].ptr.size())));
+    AKM_TRY(g->nb_cell[k].upload(lists[k].cell.data(), int64_t(lists[k].cell.size())));
+    AKM_TRY(g->nb_q[k].upload(lists[k].q.data(), int64_t(lists[k].q.size())));
+    AKM_TRY(g->nb_diag[k].upload(lists[k].diag.data(), int64_t(lists[k].diag.size())));
+    // processing order: fibre by fibre
     AKM_TRY(g->order[k].upload(ord.data(), int64_t(ord.size())));
   }
+  if (!pair)
+    AKM_TRY(g->elem.upload(g->elem_host.data(), int64_t(g->elem_host.size())));
 
   // chains (kronmult::permutes, src/device/asgard_kronmult.hpp:152-220, and
   // the active-direction order of src/asgard_kronmult_matrix.cpp:1313-1331)
-  std::vector<int> ch_term, ch_nst, ch_dim, ch_fill, ch_slot;
-  std::vector<std::vector<int>> term_act(m.T);
+  auto &[ch_term, ch_nst, ch_dim, ch_fill, ch_slot] = g->chains_host;
+  std::vector<std::vector<int>> &term_act = g->term_act;
+  term_act.resize(m.T);
   for (int t = 0; t < m.T; t++)
   {
     std::vector<int> act;
@@ -2316,11 +2338,10 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
   for (int c = 0; c < g->nchains; c++)
   {
     g->max_stages = std::max(g->max_stages, ch_nst[c]);
-    ch_slot.push_back(ch_nst[c] >= 1 ? nslots++ : -1);
+    ch_slot.push_back((ch_nst[c] >= 1 && !pair) ? nslots++ : -1);
   }
   g->nslots = nslots;
-  g->ch_nst_host = ch_nst;
-  if (g->nchains > 0)
+  if (g->nchains > 0 && !pair)
   {
     AKM_TRY(g->ch_term.upload(ch_term.data(), int64_t(ch_term.size())));
     AKM_TRY(g->ch_nst.upload(ch_nst.data(), int64_t(ch_nst.size())));
@@ -2338,10 +2359,10 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
       if (ch_nst[c] >= st + 1)
         list.push_back(c);
     g->stage_count[st] = static_cast<int>(list.size());
-    if (!list.empty())
+    if (!list.empty() && !pair)
       AKM_TRY(g->stage_list[st].upload(list.data(), int64_t(list.size())));
   }
-  if (g->max_stages > 0)
+  if (g->max_stages > 0 && !pair)
   {
     // first-stage groups: chains in order, grouped by (dimension, fill)
     std::vector<std::pair<int, int>> keys;
@@ -2375,10 +2396,13 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
     AKM_TRY(g->first_ptr.upload(gptr.data(), int64_t(gptr.size())));
     AKM_TRY(g->first_chain.upload(gchain.data(), int64_t(gchain.size())));
   }
-  AKM_TRY(build_slabs(m, *g, lists, term_act, ch_term, ch_nst, ch_dim, ch_fill, ch_slot));
-  const int64_t work_slots = int64_t(2) * nslots + g->ngroups;
-  if (work_slots > 0)
-    AKM_TRY(g->work.allocate(work_slots * g->cells * m.N * int64_t(m.esize)));
+  g->fl_lanes = fibre_lanes(m, lists, term_act);
+  // a pair handle plans slabs when it is to use or to time them
+  if (!pair || g->fl_lanes > fl_lanes_default)
+    AKM_TRY(need_slabs(m, *g));
+  if (!pair && nslots + g->ngroups > 0)
+    AKM_TRY(g->work.allocate((int64_t(2) * nslots + g->ngroups) * g->cells * m.N *
+                             int64_t(m.esize)));
   // flops as the reference counts them (src/asgard_kronmult_matrix.cpp:
   // 1389-1395): two per entry of the full DOF-level pattern of every
   // non-identity (term, dimension) on the padded set
@@ -2387,6 +2411,138 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
       if (active_mask == nullptr || active_mask[t * d + k] != 0)
         g->flops += 2 * nnz_dim[k];
   m.gk = std::move(g);
+  const int layout = default_layout(m, *m.gk);
+  if (layout < 0)
+    return AKM_SUCCESS;
+  return global_set_layout(m, layout);
+}
+
+//! Which of the T*d factors of vA are not exactly the identity (0 off the
+//! diagonal blocks, the unit matrix on them); false when a value is not
+//! finite.
+template<typename P>
+static bool active_factors(const P *vA, int T, int d, int n,
+                           std::vector<int> const &c1_pntr, std::vector<int> const &c1_diag,
+                           std::vector<int> &mask)
+{
+  const int nn = n * n, pairs = T * d;
+  mask.assign(pairs, 0);
+  bool finite = true;
+  for (size_t r = 0; r + 1 < c1_pntr.size(); r++)
+    for (int64_t q = c1_pntr[r]; q < c1_pntr[r + 1]; q++)
+      for (int td = 0; td < pairs; td++)
+      {
+        const P *b = vA + (q * pairs + td) * nn;
+        for (int i = 0; i < nn; i++)
+        {
+          const P want = (q == c1_diag[r] && i % (n + 1) == 0) ? P{1} : P{0};
+          if (b[i] != want)
+            mask[td] = 1;
+          finite = finite && std::isfinite(b[i]);
+        }
+      }
+  return finite;
+}
+
+//! active_factors of host values of the matrix's precision.
+static int active_factors_of(akm_matrix_s const &m, const void *vA, std::vector<int> &mask,
+                             bool &finite)
+{
+  std::vector<int> p1, i1, dg;
+  AKM_TRY(build_connect_1d(m.max_level, true, p1, i1, dg));
+  finite = (m.prec == AKM_F64)
+               ? active_factors(static_cast<const double *>(vA), m.T, m.d, m.n, p1, dg, mask)
+               : active_factors(static_cast<const float *>(vA), m.T, m.d, m.n, p1, dg, mask);
+  return AKM_SUCCESS;
+}
+
+int factored_build(akm_matrix_s &m, std::vector<int> const &elem, const void *vA)
+{
+  m.gk.reset();
+  m.factored = false;
+  if (m.T == 0 || m.rows == 0)
+    return AKM_SUCCESS;
+  std::vector<int> mask;
+  bool finite = false;
+  AKM_TRY(active_factors_of(m, vA, mask, finite));
+  return finite ? factored_build_mask(m, elem, mask) : AKM_SUCCESS;
+}
+
+int factored_refresh(akm_matrix_s &m, const void *values)
+{
+  if (m.T == 0 || m.rows == 0)
+    return AKM_SUCCESS;
+  std::vector<int> mask;
+  bool finite = false;
+  if (values != nullptr)
+    AKM_TRY(active_factors_of(m, values, mask, finite));
+  else
+  {
+    std::vector<unsigned char> host(m.num_vA * m.esize);
+    AKM_HIP(hipMemcpyAsync(host.data(), m.vA.data(), host.size(), hipMemcpyDeviceToHost,
+                           m.stream));
+    AKM_HIP(hipStreamSynchronize(m.stream));
+    AKM_TRY(active_factors_of(m, host.data(), mask, finite));
+  }
+  if (!finite)
+  {
+    m.factored = false;
+    return AKM_SUCCESS;
+  }
+  // a factor that became the identity may stay in the products; one that was
+  // the identity when the products were chosen may not change
+  bool covered = m.gk != nullptr;
+  for (size_t i = 0; covered && i < mask.size(); i++)
+    covered = mask[i] <= m.factored_mask[i];
+  if (covered)
+  {
+    m.factored = true;
+    return AKM_SUCCESS;
+  }
+  if (mask == m.factored_mask)
+    return AKM_SUCCESS; // no factored form for these factors
+  AKM_HIP(hipStreamSynchronize(m.stream));
+  return factored_build_mask(m, m.elem_host, mask);
+}
+
+int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem, std::vector<int> const &mask)
+{
+  m.gk.reset();
+  m.factored = false;
+  m.factored_mask = mask;
+  int widest = 0;
+  for (int t = 0; t < m.T; t++)
+    widest = std::max(widest, static_cast<int>(std::count(mask.begin() + t * m.d,
+                                                          mask.begin() + (t + 1) * m.d, 1)));
+  // one non-identity dimension per term: a product along fibres, exact on
+  // any cells; more: the chain split needs a standard grid
+  if (widest > 1 && !whole_level_grid(m.d, m.rows, elem.data()))
+    return AKM_SUCCESS;
+  int64_t repeated = -1;
+  if (build_global(m, elem, mask.data(), nullptr, true, repeated) != AKM_SUCCESS)
+  {
+    // too large for the lists or for memory: the pair kernels need neither
+    (void)hipGetLastError();
+    m.gk.reset();
+    return AKM_SUCCESS;
+  }
+  if (!m.gk)
+    return AKM_SUCCESS; // a cell is repeated
+  const akm_global_s &g = *m.gk;
+  const int layout = default_layout(m, g);
+  if (layout < 0)
+  {
+    m.gk.reset();
+    return AKM_SUCCESS;
+  }
+  // Estimated times: the pair kernels' fixed part and rate, the fibre walk's
+  // per launch and per step (the slab layout, taken only past the walk's
+  // range, is faster than that).
+  const double pair_us = 4.0 + double(m.flops()) / (m.prec == AKM_F64 ? 25e6 : 50e6);
+  const double walk_us = 1.0 + 3.0 * std::max(g.max_stages, 1) + double(g.fl_lanes) / 0.6e6;
+  m.factored = walk_us < pair_us;
+  if (!m.factored)
+    m.gk.reset();
   return AKM_SUCCESS;
 }
 } // namespace akm
@@ -2434,14 +2590,6 @@ akm_status akm_create_global_grid(int d, int n, int64_t num_cells, const int *ta
                      static_cast<long long>(expect_vA));
   std::vector<int> elem;
   cell_1d_indices(d, num_cells, table, elem);
-  {
-    std::map<std::vector<int>, int> seen;
-    for (int64_t c = 0; c < num_cells; c++)
-      if (!seen.emplace(std::vector<int>(elem.begin() + c * d, elem.begin() + (c + 1) * d), 0)
-               .second)
-        return set_error(AKM_ERR_INVALID, "global kron: cell %lld repeated",
-                         static_cast<long long>(c));
-  }
   std::unique_ptr<akm_matrix_s> m(new akm_matrix_s());
   m->prec = prec;
   m->esize = (prec == AKM_F64) ? 8 : 4;
@@ -2463,7 +2611,11 @@ akm_status akm_create_global_grid(int d, int n, int64_t num_cells, const int *ta
   m->nconn = static_cast<int>(nconn);
   if (T > 0)
     AKM_TRY(m->vA.upload(static_cast<const unsigned char *>(vA), num_vA * m->esize));
-  AKM_TRY(build_global(*m, elem, active, flux_dim));
+  int64_t repeated = -1;
+  AKM_TRY(build_global(*m, elem, active, flux_dim, false, repeated));
+  if (repeated >= 0)
+    return set_error(AKM_ERR_INVALID, "global kron: cell %lld repeated",
+                     static_cast<long long>(repeated));
   if (T > 0)
     AKM_TRY(global_update(*m, vA));
   *mat = m.release();

@@ -1345,11 +1345,11 @@ extern "C" akm_status akm_gmres_euler_mixed(akm_matrix mat, akm_matrix mat32, ak
   if (mat32 != nullptr)
   {
     saved = mat32->stream;
-    mat32->stream = mat->stream; // one stream for the whole solve
+    use_stream(*mat32, mat->stream); // one stream for the whole solve
   }
   int rc = gmres_mixed(*mat, mat32, pre, dt, x, b, restart, max_cycles, tol, inner_tol, local);
   if (mat32 != nullptr)
-    mat32->stream = saved;
+    use_stream(*mat32, saved);
   if (stats != nullptr)
     *stats = local;
   return rc;

@@ -178,6 +178,26 @@ static int apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y, P gam
                             m.stream);
 }
 
+void use_stream(akm_matrix_s &m, hipStream_t stream)
+{
+  const hipStream_t old = m.stream;
+  m.stream = stream;
+  if (old == stream || !m.gk)
+    return;
+  hipStreamCaptureStatus a = hipStreamCaptureStatusNone, b = hipStreamCaptureStatusNone;
+  hipEvent_t e = nullptr;
+  if (hipStreamIsCapturing(old, &a) == hipSuccess &&
+      hipStreamIsCapturing(stream, &b) == hipSuccess && a == hipStreamCaptureStatusNone &&
+      b == hipStreamCaptureStatusNone &&
+      hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess)
+  {
+    if (hipEventRecord(e, old) == hipSuccess)
+      (void)hipStreamWaitEvent(stream, e, 0);
+    (void)hipEventDestroy(e);
+  }
+  (void)hipGetLastError(); // a destroyed old stream has no work left
+}
+
 int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void *y,
                  double gamma, const void *xg)
 {
@@ -185,6 +205,11 @@ int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void
     return set_error(AKM_ERR_INVALID, "identity term needs a square operator");
   if (m.mode == mode_global)
     return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
+  if (m.factored && !m.pair_kernels)
+  {
+    std::lock_guard<std::mutex> lock(m.factored_mtx);
+    return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
+  }
   if (m.prec == AKM_F64)
     return apply_typed<double>(m, alpha, static_cast<const double *>(x), beta,
                                static_cast<double *>(y), gamma,
@@ -261,7 +286,7 @@ akm_status akm_set_stream(akm_matrix mat, void *stream)
 {
   if (mat == nullptr)
     return set_error(AKM_ERR_INVALID, "null matrix");
-  mat->stream = static_cast<hipStream_t>(stream);
+  use_stream(*mat, static_cast<hipStream_t>(stream));
   // tables derived from vA are rebuilt on the new stream
   mat->vA_stamp++;
   return AKM_SUCCESS;
@@ -429,6 +454,9 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
     }
   }
   AKM_TRY(build_schedule(*m));
+  m->elem_host = std::move(elem);
+  if (T > 0)
+    AKM_TRY(factored_build(*m, m->elem_host, vA));
   *mat = m.release();
   return AKM_SUCCESS;
 }
@@ -494,6 +522,8 @@ akm_status akm_update_coefficients(akm_matrix mat, const void *values)
                            hipMemcpyHostToDevice, mat->stream));
     if (mat->vAk.data() != nullptr)
       AKM_TRY(upload_vAk(*mat, values));
+    if (mat->mode == mode_grid)
+      AKM_TRY(factored_refresh(*mat, values));
   }
   AKM_HIP(hipStreamSynchronize(mat->stream));
   return AKM_SUCCESS;
@@ -561,6 +591,8 @@ akm_status akm_set_tuning(akm_matrix mat, int waves_per_row, int lds_cap_bytes,
   mat->waves = waves_per_row;
   mat->lds_cap = (lds_cap_bytes < 0) ? -1 : lds_cap_bytes;
   mat->force_generic = force_generic;
+  // a shape of the pair kernels was asked for, or everything automatic
+  mat->pair_kernels = waves_per_row != 0 || lds_cap_bytes >= 0 || force_generic != 0;
   return AKM_SUCCESS;
 }
 
@@ -594,7 +626,8 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
   if (mat->mode == mode_global)
   {
     // row layout (reported in waves_per_row as akm_set_tuning takes it)
-    AKM_TRY(global_autotune(*mat, x, y));
+    double ms = 0;
+    AKM_TRY(global_autotune(*mat, x, y, ms));
     if (waves_per_row)
       *waves_per_row = global_layout(*mat);
     if (lds_tables)
@@ -604,12 +637,15 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
   struct choice
   {
     int waves, lds, family;
+    int factored; // factored_shape, -1: the pair kernels
   };
   static std::mutex mtx;
   static std::map<std::vector<int64_t>, choice> cache;
-  const std::vector<int64_t> key = {int64_t(mat->prec), mat->d,      mat->n,  mat->T,
-                                    mat->max_level,     mat->rows,   mat->nnz, int64_t(mat->mode)};
-  choice best{0, -1, 0};
+  std::vector<int64_t> key = {int64_t(mat->prec), mat->d,      mat->n,  mat->T,
+                              mat->max_level,     mat->rows,   mat->nnz, int64_t(mat->mode)};
+  if (mat->factored)
+    key.insert(key.end(), mat->factored_mask.begin(), mat->factored_mask.end());
+  choice best{0, -1, 0, -1};
   bool cached = false;
   {
     std::lock_guard<std::mutex> lock(mtx);
@@ -622,52 +658,86 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
   }
   if (!cached)
   {
-    // enough applies per candidate for ~2 ms of timing, at most 50
-    double probe = 0;
-    mat->waves = 4;
-    mat->lds_cap = -1;
-    mat->family = 0;
-    AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, 1, &probe));
-    const int iters = std::max(1, std::min(50, int(2.0 / std::max(probe, 1e-3))));
-    double best_ms = 1e300;
-    const int lds_opts[2] = {-1, 0};
-    for (int li = 0; li < (mat->vAk.data() != nullptr ? 2 : 1); li++)
-      for (int w : {1, 2, 4, 8})
-      {
-        mat->waves = w;
-        mat->lds_cap = (mat->vAk.data() != nullptr) ? lds_opts[li] : 0;
-        double ms = 0;
-        AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, iters, &ms));
-        if (ms < best_ms)
-        {
-          best_ms = ms;
-          best = {w, mat->lds_cap, 0};
-        }
-      }
-    if (mat->prec == AKM_F64 &&
-        mfma_family_applies(mat->d, mat->n, mat->mode, mat->T, mat->epack.data() != nullptr))
+    best.factored = -1;
+    double factored_ms = 1e300;
+    mat->pair_kernels = false;
+    if (mat->factored)
     {
-      const int saved_lds = mat->lds_cap;
-      mat->family = 1;
-      for (int w : {1, 2, 4, 8, 16})
+      AKM_TRY(global_autotune(*mat, x, y, factored_ms));
+      best.factored = factored_shape(*mat);
+      mat->pair_kernels = true;
+    }
+    // the pair kernels are not timed when even twice the best rate they have
+    // reached (67 TFLOP/s FP64, 98 FP32) would be slower than that
+    const double bound = double(mat->flops()) / (mat->prec == AKM_F64 ? 140e9 : 200e9);
+    if (!(factored_ms < bound))
+    {
+      // enough applies per candidate for ~2 ms of timing, at most 50
+      double probe = 0;
+      mat->waves = 4;
+      mat->lds_cap = -1;
+      mat->family = 0;
+      AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, 1, &probe));
+      const int iters = std::max(1, std::min(50, int(2.0 / std::max(probe, 1e-3))));
+      if (best.factored >= 0)
       {
-        mat->waves = w;
-        double ms = 0;
-        AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, iters, &ms));
+        mat->pair_kernels = false;
+        AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, iters, &factored_ms));
+        mat->pair_kernels = true;
+      }
+      double best_ms = factored_ms;
+      auto take = [&](choice const &c, double ms) {
         if (ms < best_ms)
         {
           best_ms = ms;
-          best = {w, saved_lds, 1};
+          best = c;
         }
+      };
+      const int lds_opts[2] = {-1, 0};
+      for (int li = 0; li < (mat->vAk.data() != nullptr ? 2 : 1); li++)
+        for (int w : {1, 2, 4, 8})
+        {
+          mat->waves = w;
+          mat->lds_cap = (mat->vAk.data() != nullptr) ? lds_opts[li] : 0;
+          double ms = 0;
+          AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, iters, &ms));
+          take({w, mat->lds_cap, 0, -1}, ms);
+        }
+      if (mat->prec == AKM_F64 &&
+          mfma_family_applies(mat->d, mat->n, mat->mode, mat->T, mat->epack.data() != nullptr))
+      {
+        const int saved_lds = mat->lds_cap;
+        mat->family = 1;
+        for (int w : {1, 2, 4, 8, 16})
+        {
+          mat->waves = w;
+          double ms = 0;
+          AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, iters, &ms));
+          take({w, saved_lds, 1, -1}, ms);
+        }
+        mat->family = 0;
       }
-      mat->family = 0;
     }
     std::lock_guard<std::mutex> lock(mtx);
     cache[key] = best;
   }
+  if (best.factored >= 0)
+  {
+    AKM_TRY(factored_set_shape(*mat, best.factored));
+    mat->waves = 0;
+    mat->lds_cap = -1;
+    mat->family = 0;
+    mat->pair_kernels = false;
+    if (waves_per_row)
+      *waves_per_row = 1;
+    if (lds_tables)
+      *lds_tables = 3;
+    return AKM_SUCCESS;
+  }
   mat->waves = best.waves;
   mat->lds_cap = best.lds;
   mat->family = best.family;
+  mat->pair_kernels = true;
   if (waves_per_row)
     *waves_per_row = best.waves;
   if (lds_tables)
@@ -688,6 +758,7 @@ akm_status akm_set_kernel_family(akm_matrix mat, int family)
                      "kernel family 1 needs an FP64 sparse-grid matrix with d = 3, n = 3, "
                      "1 to 8 terms and max_level <= 10");
   mat->family = family;
+  mat->pair_kernels = true;
   return AKM_SUCCESS;
 }
 

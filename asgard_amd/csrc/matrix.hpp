@@ -2,6 +2,7 @@
 #pragma once
 
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "akm_internal.hpp"
@@ -70,7 +71,17 @@ struct akm_matrix_s
 
   std::unique_ptr<akm_gmres_workspace, void (*)(akm_gmres_workspace *)> gmres{nullptr,
                                                                              nullptr};
-  // global Kronecker operator (mode_global)
+  // sparse-grid handles: the operator runs one dimension at a time (gk)
+  // instead of pair by pair, because its factors allow it
+  bool factored = false;
+  bool pair_kernels = false;        // the caller asked for the pair kernels
+  // held while a factored apply is enqueued: its launches share work vectors,
+  // so two threads' applies follow each other on the stream
+  std::mutex factored_mtx;
+  std::vector<int> factored_mask;   // T x d non-identity factors gk was built for
+  std::vector<int> elem_host;       // cell 1D indices
+  // global Kronecker operator (mode_global), or the factored form of a
+  // sparse-grid operator
   std::unique_ptr<akm_global_s, void (*)(akm_global_s *)> gk{nullptr, nullptr};
 
   int64_t input_size() const { return N * cols; }
@@ -83,6 +94,11 @@ namespace akm
 //! y = alpha*A*x + beta*y + gamma*xg on device pointers (xg row-indexed).
 int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void *y,
                  double gamma, const void *xg);
+
+//! Moves the handle to `stream`.  Work of a one-dimension-at-a-time operator
+//! still running on the old stream uses the handle's work vectors, so the new
+//! stream waits for it (unless either is being captured).
+void use_stream(akm_matrix_s &m, hipStream_t stream);
 
 //! Wavefronts per row workgroup used for the matrix (explicit or automatic).
 int waves_per_row(akm_matrix_s const &m);
@@ -97,17 +113,32 @@ int global_update(akm_matrix_s &m, const void *vA);
 //! Global operator: Jacobi diagonal rebuilt on the device from the stored
 //! factor blocks (after they were written on the device).
 int global_device_jacobi(akm_matrix_s &m);
+//! Sparse-grid handle: builds the factored form of its operator (`elem`: cell
+//! 1D indices, vA: host factor blocks) when the factors allow one that is
+//! faster than the pair kernels.
+int factored_build(akm_matrix_s &m, std::vector<int> const &elem, const void *vA);
+//! After new factor values (host values, or null: the values are on the
+//! device): keeps the factored form when it still holds, else builds it anew.
+int factored_refresh(akm_matrix_s &m, const void *values);
+//! The same as factored_build for known non-identity factors (mask, T x d, all values finite).
+int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem,
+                        std::vector<int> const &mask);
 //! Global operator: flops per apply as the reference counts them.
 int64_t global_flops(akm_matrix_s const &m);
 //! Global operator: row layout in use, as akm_set_tuning takes it (1, 8, 2,
-//! 3, 4 or 5).
+//! 3, 4, 5 or 6).
 int global_layout(akm_matrix_s const &m);
-//! Global operator: times the lane layouts on the operator, keeps the faster.
-int global_autotune(akm_matrix_s &m, const void *x, void *y);
-//! Global operator: row layout 1 (lane per DOF), 8 (8 lanes per DOF), 2
-//! (wavefront per cell), 3 (wavefront per cell, chains sharing their first
+//! Global operator: times the layouts on the operator and keeps the fastest;
+//! best_ms = its time per apply.
+int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms);
+//! Factored sparse-grid operator: the layout and stream split in use, as one
+//! number, and back.
+int factored_shape(akm_matrix_s const &m);
+int factored_set_shape(akm_matrix_s &m, int shape);
+//! Global operator: row layout 1 (lane per DOF), 8 (the fibre walk, lists
+//! split over slots of lanes), 2 (wavefront per cell), 3 (wavefront per cell, chains sharing their first
 //! stage's input read it once), 4 / 5 (2 / 3 with each XCD taking contiguous
-//! cells), 0 (unchanged).
+//! cells), 6 (slabs), 0 (unchanged).
 int global_set_layout(akm_matrix_s &m, int layout);
 
 //! Kernel arguments of an FP64 matrix (vectors and scalars left empty).

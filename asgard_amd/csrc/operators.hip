@@ -175,6 +175,8 @@ akm_status akm_update_operators(akm_matrix mat, const void *const *ops, int64_t 
     AKM_TRY(update_operators_typed<double>(*mat, mat->op_ptrs.data(), lda));
   else
     AKM_TRY(update_operators_typed<float>(*mat, mat->op_ptrs.data(), lda));
+  if (mat->mode == mode_grid)
+    AKM_TRY(factored_refresh(*mat, nullptr));
   AKM_HIP(hipStreamSynchronize(mat->stream));
   return AKM_SUCCESS;
 }

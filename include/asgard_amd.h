@@ -103,7 +103,16 @@ akm_status akm_create_sparse(int d, int n, int rows, int cols, int num_terms,
  * on the fly from the cells' 1D indices and connect_1d(max_level).  vA is the
  * reference's block array: for each connect_1d(max_level) connection, for
  * each term, for each dim, one n x n column-major block (num_connections*d*T*n*n
- * values, as make_kronmult_sparse fills it at :369-393).  Host arrays. */
+ * values, as make_kronmult_sparse fills it at :369-393).  Host arrays.
+ * The operator is applied one dimension at a time, with the factors that are
+ * exactly the identity left out, where that gives the same sums faster: every
+ * term with at most one non-identity factor (any cells), or a grid of whole
+ * levels closed under lowering a level (any factors).  The products left out
+ * are exact zeros; a non-finite entry of x then reaches only the rows its
+ * non-identity factors couple.  akm_update_coefficients and
+ * akm_update_operators look at the new factors and choose again; a shape
+ * given to akm_set_tuning or akm_set_kernel_family selects the pair-by-pair
+ * kernels, akm_set_tuning(mat, 0, -1, 0) the automatic choice. */
 akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *table,
                                   int max_level, int num_terms, const void *vA,
                                   int64_t num_vA, akm_prec prec, akm_matrix *mat);
@@ -196,8 +205,9 @@ akm_status akm_matrix_info(akm_matrix mat, int64_t *tensor_size, int64_t *input_
  * (-1 = automatic, 0 = read factors from global memory) and whether to
  * force the block-wide LDS kernel (for tests).  Takes effect at the next
  * apply.  On a global operator only waves_per_row counts and picks the row
- * layout: 1 = one lane per DOF, 8 = eight lanes per DOF, 2 = one wavefront
- * per cell (n^d <= 64), 3 = as 2 with the chains whose first stage reads
+ * layout: 1 = one lane per DOF, 8 = fibre walk (each cell's connection
+ * lists cut into short pieces, one piece per group of n^d lanes; products
+ * that chains share are taken once), 2 = one wavefront per cell (n^d <= 64), 3 = as 2 with the chains whose first stage reads
  * the same input along the same dimension grouped (one read for up to four
  * chains), 4 / 5 = as 2 / 3 with the workgroups of each XCD taking
  * contiguous cells (neighbours shared in one L2), 6 = slabs: the terms
@@ -217,8 +227,9 @@ akm_status akm_set_tuning(akm_matrix mat, int waves_per_row, int lds_cap_bytes,
  * cached per (precision, d, n, terms, max level, rows, pairs) for the
  * process, so a second matrix of the same shape reuses them without timing.
  * Writes the chosen waves per row and kernel (0 = factors read from global
- * memory, 1 = LDS factor tables, 2 = matrix cores) when the pointers are not
- * NULL.  No counterpart in the reference (fixed launch shapes). */
+ * memory, 1 = LDS factor tables, 2 = matrix cores, 3 = one dimension at a
+ * time, see akm_create_sparse_grid; waves per row is then 1) when the
+ * pointers are not NULL.  No counterpart in the reference (fixed launch shapes). */
 akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_row,
                         int *lds_tables);
 

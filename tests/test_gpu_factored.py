@@ -1,0 +1,189 @@
+"""Sparse-grid operators taken one dimension at a time, against the pair
+kernels of the same handle.
+
+A handle whose factors are mostly the identity (or whose grid allows the
+split of every product) applies its operator along fibres instead of pair by
+pair.  ``set_tuning`` with a shape selects the pair kernels, which are the
+general path here.  Bars: 1e-13 of the largest result in FP64 and 1e-5 in
+FP32, the kronmult parity bars.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+import asgard_amd  # noqa: E402
+from asgard_amd import grid  # noqa: E402
+
+TOL = {np.float64: 1e-13, np.float32: 1e-5}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu_present():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+def factors(rng, d, n, level, active):
+    """Dense U[-1, 1] factors in each term's listed dimensions, identity in
+    the others."""
+    size = n << level
+    return [rng.uniform(-1, 1, (size, size)) if k in dims else np.eye(size)
+            for dims in active for k in range(d)]
+
+
+def tables(d, level, refine):
+    table, _ = grid.element_table([level] * d)
+    if refine:
+        table = grid.refine(table, 0.3, seed=7)
+    return table, int(table[:, :d].max())
+
+
+def both(m, x, alpha, beta, y0):
+    """The result of the chosen path and of the pair kernels."""
+    out = []
+    for waves in (0, 4):
+        m.set_tuning(waves_per_row=waves)
+        y = torch.from_numpy(y0.copy()).cuda()
+        m.apply(alpha, x, beta, y)
+        out.append(y.cpu().numpy().astype(np.float64))
+    m.set_tuning()
+    return out
+
+
+def close(a, b, dtype):
+    return np.abs(a - b).max() <= TOL[dtype] * max(np.abs(b).max(), 1e-300)
+
+
+CASES = [
+    # (d, n, level, refine, non-identity dimensions per term)
+    (1, 2, 5, True, [(0,)]),
+    (2, 2, 6, False, [(0,), (1,), (1,)]),           # two terms share a table
+    (2, 3, 5, True, [(1,), ()]),                    # an identity term, refined
+    (2, 4, 5, False, [(0, 1), (1,)]),               # n = 4, two stages
+    (3, 2, 6, False, [(0, 2), (0, 1, 2), ()]),
+    (3, 3, 5, False, [(0, 1, 2), (1, 2)]),
+    (3, 4, 4, True, [(0,), (2,)]),
+    (4, 2, 6, True, [(0,), (1,), (2,), (3,)]),
+    (4, 3, 4, False, [(3,), (0,)]),                 # 81 lanes: 1024-thread groups
+    (4, 4, 3, False, [(1,), (2,), (3,)]),           # 256 lanes
+    (5, 3, 3, False, [(0,), (1,), (2,), (3,), (4,)]),  # more dimensions than slots
+    (6, 2, 4, False, [(0, 3), (1, 4), (5,)]),
+    (6, 3, 2, False, [(0,), (5,)]),                 # 729 lanes: one slot
+    (2, 5, 4, False, [(0,), (1,)]),                 # n = 5: a workgroup per cell
+    (6, 4, 1, False, [(2,)]),                       # 4096 entries
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_matches_pair_kernels(case, dtype):
+    d, n, level, refine, active = case
+    rng = np.random.default_rng(11)
+    table, top = tables(d, level, refine)
+    T = len(active)
+    vA = grid.build_vA(d, n, T, top, factors(rng, d, n, top, active)).astype(dtype)
+    m = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, T, vA, dtype=dtype)
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size()).astype(dtype)).cuda()
+    y0 = rng.uniform(-1, 1, m.output_size()).astype(dtype)
+    for alpha, beta in ((1.0, 0.0), (-0.7, 0.4), (0.0, 2.0)):
+        got, want = both(m, x, alpha, beta, y0)
+        assert close(got, want, dtype), (alpha, beta)
+    if dtype == np.float64:
+        out = []
+        for waves in (0, 4):
+            m.set_tuning(waves_per_row=waves)
+            y = torch.from_numpy(y0.copy()).cuda()
+            m.apply_euler(0.01, 1.5, x, -0.5, y)
+            out.append(y.cpu().numpy())
+        assert close(out[0], out[1], dtype)
+
+
+def test_repeats_bit_for_bit_and_streams():
+    rng = np.random.default_rng(3)
+    table, top = tables(3, 5, False)
+    vA = grid.build_vA(3, 2, 1, top, factors(rng, 3, 2, top, [(0, 1, 2)]))
+    m = asgard_amd.KronmultMatrix.sparse_grid(3, 2, table, top, 1, vA)
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+    torch.cuda.synchronize()
+    outs = []
+    for i in range(6):
+        # the handle moves between streams without a wait in between
+        s = torch.cuda.Stream()
+        m.set_stream(s.cuda_stream)
+        y = torch.zeros_like(x)
+        torch.cuda.synchronize() if i % 2 else None
+        s.wait_stream(torch.cuda.current_stream())
+        m.apply(1.0, x, 0.0, y)
+        outs.append((s, y))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, outs[0][1]) for _, y in outs)
+    m.set_stream(0)
+
+
+@pytest.mark.parametrize("on_device", [False, True])
+def test_new_factors_change_the_form(on_device):
+    """Updates that keep, add and drop non-identity factors."""
+    rng = np.random.default_rng(5)
+    d, n = 3, 2
+    table, top = tables(d, 5, False)
+    patterns = [[(0,), (1,)], [(1,), (1, 2)], [(0,), (1,)], [(0, 1, 2), (2,)], [(), (0,)]]
+    ops = factors(rng, d, n, top, patterns[0])
+    m = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, 2,
+                                              grid.build_vA(d, n, 2, top, ops))
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+    y0 = np.zeros(m.output_size())
+    for active in patterns:
+        ops = factors(rng, d, n, top, active)
+        vA = grid.build_vA(d, n, 2, top, ops)
+        if on_device:
+            m.update_operators([torch.from_numpy(np.ascontiguousarray(o.T)).cuda()
+                                for o in ops])
+        else:
+            m.update_stored_coefficients(vA)
+        got, want = both(m, x, 1.0, 0.0, y0)
+        assert close(got, want, np.float64), active
+        fresh = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, 2, vA)
+        fresh.set_tuning(waves_per_row=4)
+        y = torch.zeros_like(x)
+        fresh.apply(1.0, x, 0.0, y)
+        assert close(got, y.cpu().numpy(), np.float64), active
+
+
+def test_forms_the_split_does_not_cover():
+    """Cells missing from a level, factors that are not finite and repeated
+    cells stay with the pair kernels."""
+    rng = np.random.default_rng(9)
+    table, top = tables(2, 5, False)
+    ops = factors(rng, 2, 2, top, [(0, 1)])
+    y0 = np.zeros(len(table) * 4)
+    for cells in (table[:-1], np.concatenate([table, table[:1]])):
+        vA = grid.build_vA(2, 2, 1, top, ops)
+        m = asgard_amd.KronmultMatrix.sparse_grid(2, 2, cells, top, 1, vA)
+        x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+        got, want = both(m, x, 1.0, 0.0, np.zeros(m.output_size()))
+        assert close(got, want, np.float64)
+    bad = grid.build_vA(2, 2, 1, top, factors(rng, 2, 2, top, [(0,)]))
+    bad[3] = np.inf
+    m = asgard_amd.KronmultMatrix.sparse_grid(2, 2, table, top, 1, bad)
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+    got, want = both(m, x, 1.0, 0.0, y0)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+
+
+def test_autotuned_small_and_large_agree():
+    rng = np.random.default_rng(13)
+    d, n, level = 6, 2, 5
+    table, top = tables(d, level, False)
+    active = [(0, 3), (1, 4), (2, 5)]
+    vA = grid.build_vA(d, n, 3, top, factors(rng, d, n, top, active))
+    m = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, 3, vA)
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+    m.autotune(x, torch.zeros_like(x))
+    y = torch.zeros_like(x)
+    m.apply(1.0, x, 0.0, y)
+    m.set_tuning(waves_per_row=4)
+    ref = torch.zeros_like(x)
+    m.apply(1.0, x, 0.0, ref)
+    assert close(y.cpu().numpy(), ref.cpu().numpy(), np.float64)
