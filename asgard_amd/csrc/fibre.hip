@@ -38,6 +38,7 @@
 #include <array>
 #include <map>
 #include <numeric>
+#include <type_traits>
 
 namespace akm
 {
@@ -70,7 +71,8 @@ struct fl_slot_rec
 };
 static_assert(sizeof(fl_slot_rec) == 7 * sizeof(int4), "slot records are seven int4");
 
-template<typename P>
+//! P: values of the factors, work vectors and sums; X: of the input and y.
+template<typename P, typename X = P>
 struct fl_args
 {
   const int4 *slots;
@@ -78,13 +80,14 @@ struct fl_args
   const P *tab;
   int n, N, nslot;
   int64_t stride;
-  const P *x;
+  const X *x;
   P *work;
-  P *y;
-  const P *xg;
+  X *y;
+  const X *xg;
   const double *pc;
   double jdt;
   P alpha, beta, gamma;
+  double between; // X != P: y = xg + between * sum
   int identities;
 };
 
@@ -112,8 +115,8 @@ __device__ __forceinline__ int fl_digit(int e, unsigned magic, int n)
 
 //! c[r] += the first U of a piece's connections: column `s` of each block
 //! times entry e of the connected cell.  All loads precede their uses.
-template<typename P, int NT, int U>
-__device__ __forceinline__ void fl_connections(const P *__restrict__ in, const P *__restrict__ tab,
+template<typename P, typename X, int NT, int U>
+__device__ __forceinline__ void fl_connections(const X *__restrict__ in, const P *__restrict__ tab,
                                                int N, int len, const int4 *ent, P (&c)[NT])
 {
   P av[U][NT], xv[U];
@@ -122,7 +125,7 @@ __device__ __forceinline__ void fl_connections(const P *__restrict__ in, const P
   {
     const int cell = (u % 2 == 0) ? ent[u / 2].x : ent[u / 2].z;
     const int block = (u % 2 == 0) ? ent[u / 2].y : ent[u / 2].w;
-    xv[u] = in[int64_t(cell) * N];
+    xv[u] = static_cast<P>(in[int64_t(cell) * N]);
     fl_column<P, NT>(tab + int64_t(block) * (NT * NT), av[u]);
   }
 #pragma unroll
@@ -136,9 +139,16 @@ __device__ __forceinline__ void fl_connections(const P *__restrict__ in, const P
 }
 
 //! A finished sum of entry pos of a vector: into its work vector, or into y.
-template<typename P>
-__device__ __forceinline__ void fl_store(fl_args<P> const &a, int vec, int64_t pos, P sum)
+template<typename P, typename X>
+__device__ __forceinline__ void fl_store(fl_args<P, X> const &a, int vec, int64_t pos, P sum)
 {
+  if constexpr (!std::is_same_v<P, X>)
+  {
+    if (a.identities > 0)
+      sum += static_cast<P>(a.identities) * static_cast<P>(a.x[pos]);
+    a.y[pos] = fma(a.between, static_cast<X>(sum), a.xg[pos]);
+    return;
+  }
   if (vec >= 0)
   {
     a.work[int64_t(vec) * a.stride + pos] = sum;
@@ -159,8 +169,8 @@ __device__ __forceinline__ void fl_store(fl_args<P> const &a, int vec, int64_t p
 //! One stage: a workgroup's slots, then each cell's slot partials added in
 //! slot order.  A slot whose pieces act in several dimensions takes a round
 //! per dimension.  LDS: NT values per thread.
-template<typename P, int NT>
-__global__ void __launch_bounds__(1024) fl_stage(fl_args<P> a, int group0)
+template<typename P, int NT, typename X = P>
+__global__ void __launch_bounds__(1024) fl_stage(fl_args<P, X> a, int group0)
 {
   extern __shared__ __align__(16) unsigned char fl_smem[];
   P *ex = reinterpret_cast<P *>(fl_smem);
@@ -192,7 +202,9 @@ __global__ void __launch_bounds__(1024) fl_stage(fl_args<P> a, int group0)
     {
       const int len = ph.w & 0xffff;
       open = (ph.w >> 16) == 0;
-      const P *in = ((ph.x == 0) ? a.x : a.work + int64_t(ph.x - 1) * a.stride) + e;
+      const X *in = a.x + e;
+      if constexpr (std::is_same_v<P, X>)
+        in = ((ph.x == 0) ? a.x : a.work + int64_t(ph.x - 1) * a.stride) + e;
       const int4 cur[fl_piece / 2] = {ent[0], ent[1], ent[2], ent[3]};
       have = more > 0;
       if (have)
@@ -205,9 +217,9 @@ __global__ void __launch_bounds__(1024) fl_stage(fl_args<P> a, int group0)
         more--;
       }
       if (__any(len > fl_piece / 2))
-        fl_connections<P, NT, fl_piece>(in, a.tab + s * NT, N, len, cur, c);
+        fl_connections<P, X, NT, fl_piece>(in, a.tab + s * NT, N, len, cur, c);
       else
-        fl_connections<P, NT, fl_piece / 2>(in, a.tab + s * NT, N, len, cur, c);
+        fl_connections<P, X, NT, fl_piece / 2>(in, a.tab + s * NT, N, len, cur, c);
     }
     // lane e holds shares of the rows of its fibre: row r's entry is e with
     // its digit s replaced by r
@@ -788,33 +800,63 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
   return AKM_SUCCESS;
 }
 
+//! Rebuilds the factor tables when vA changed since they were built.
 template<typename P>
-int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, P *y, P gamma,
-                const P *xg, const double *pc, double jdt)
+static int fibre_tables(akm_matrix_s &m, fibre_plan &plan)
 {
+  if (plan.tab_valid && plan.stamp == m.vA_stamp)
+    return AKM_SUCCESS;
   const int nn = m.n * m.n;
-  P *tab = reinterpret_cast<P *>(plan.tab.data());
-  if (!plan.tab_valid || plan.stamp != m.vA_stamp)
-  {
-    const int64_t count = int64_t(plan.nconn + 2 * plan.M) * nn * plan.ntab + nn;
-    const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
-    fl_tables<P><<<static_cast<unsigned>(blocks), 256, 0, m.stream>>>(
-        reinterpret_cast<const P *>(m.vA.data()), plan.tab_ptr.data(), plan.tab_src.data(),
-        plan.c1_diag.data(), plan.ntab, plan.nconn, plan.M, m.n, m.d, m.T, tab);
-    AKM_TRY(check_launch("fibre tables"));
-    plan.stamp = m.vA_stamp;
-    plan.tab_valid = true;
-  }
-  fl_args<P> a{};
+  const int64_t count = int64_t(plan.nconn + 2 * plan.M) * nn * plan.ntab + nn;
+  const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
+  fl_tables<P><<<static_cast<unsigned>(blocks), 256, 0, m.stream>>>(
+      reinterpret_cast<const P *>(m.vA.data()), plan.tab_ptr.data(), plan.tab_src.data(),
+      plan.c1_diag.data(), plan.ntab, plan.nconn, plan.M, m.n, m.d, m.T,
+      reinterpret_cast<P *>(plan.tab.data()));
+  plan.stamp = m.vA_stamp;
+  plan.tab_valid = true;
+  return check_launch("fibre tables");
+}
+
+//! The plan's part of the kernel arguments.
+template<typename P, typename X>
+static fl_args<P, X> fibre_args(akm_matrix_s const &m, fibre_plan const &plan)
+{
+  fl_args<P, X> a{};
   a.slots = plan.slots.data();
   a.pieces = plan.pieces.data();
-  a.tab = tab;
+  a.tab = reinterpret_cast<const P *>(plan.tab.data());
   a.n = m.n;
   a.N = static_cast<int>(m.N);
   a.nslot = plan.nslot;
   a.stride = plan.stride;
-  a.x = x;
   a.work = reinterpret_cast<P *>(plan.work.data());
+  a.identities = plan.identities;
+  return a;
+}
+
+template<typename P, typename X>
+static int launch_stage(akm_matrix_s const &m, fibre_plan const &plan,
+                        fibre_plan::stage const &st, fl_args<P, X> const &a)
+{
+  const dim3 grid(static_cast<unsigned>(st.groups)), tpb(static_cast<unsigned>(plan.tpb));
+  const size_t lds = sizeof(P) * plan.tpb * m.n;
+  if (m.n == 2)
+    fl_stage<P, 2, X><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+  else if (m.n == 3)
+    fl_stage<P, 3, X><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+  else
+    fl_stage<P, 4, X><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+  return check_launch("fibre stage");
+}
+
+template<typename P>
+int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, P *y, P gamma,
+                const P *xg, const double *pc, double jdt)
+{
+  AKM_TRY(fibre_tables<P>(m, plan));
+  fl_args<P> a = fibre_args<P, P>(m, plan);
+  a.x = x;
   a.y = y;
   a.xg = xg;
   a.pc = pc;
@@ -822,22 +864,31 @@ int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, 
   a.alpha = alpha;
   a.beta = beta;
   a.gamma = gamma;
-  a.identities = plan.identities;
-  const size_t lds = sizeof(P) * plan.tpb * m.n;
   for (auto const &st : plan.stages)
   {
-    const dim3 grid(static_cast<unsigned>(st.groups)), tpb(static_cast<unsigned>(plan.tpb));
-    if (!plan.slots_of_lanes)
-      fl_stage_any<P><<<grid, tpb, 0, m.stream>>>(a, st.first_group);
-    else if (m.n == 2)
-      fl_stage<P, 2><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
-    else if (m.n == 3)
-      fl_stage<P, 3><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
-    else
-      fl_stage<P, 4><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+    if (plan.slots_of_lanes)
+    {
+      AKM_TRY(launch_stage(m, plan, st, a));
+      continue;
+    }
+    fl_stage_any<P><<<static_cast<unsigned>(st.groups), plan.tpb, 0, m.stream>>>(a,
+                                                                                st.first_group);
     AKM_TRY(check_launch("fibre stage"));
   }
   return AKM_SUCCESS;
+}
+
+bool fibre_apply_between(akm_matrix_s &m, fibre_plan &plan, const double *v, double c, double *w)
+{
+  if (!plan.built || !plan.slots_of_lanes || plan.stages.size() != 1 || plan.vectors != 0 ||
+      fibre_tables<float>(m, plan) != AKM_SUCCESS)
+    return false;
+  fl_args<float, double> a = fibre_args<float, double>(m, plan);
+  a.x = v;
+  a.y = w;
+  a.xg = v;
+  a.between = c;
+  return launch_stage(m, plan, plan.stages[0], a) == AKM_SUCCESS;
 }
 
 template int fibre_apply<double>(akm_matrix_s &, fibre_plan &, double, const double *, double,

@@ -93,4 +93,8 @@ int64_t fibre_lanes(akm_matrix_s const &m, std::vector<gk_lists> const &lists,
 template<typename P>
 int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, P *y, P gamma,
                 const P *xg, const double *pc, double jdt);
+
+//! w = v + c * fp64(A fp32(v)) of an FP32 operator on FP64 vectors, in one
+//! launch; false when the plan has several stages.
+bool fibre_apply_between(akm_matrix_s &m, fibre_plan &plan, const double *v, double c, double *w);
 } // namespace akm

@@ -1343,6 +1343,17 @@ int global_apply(akm_matrix_s &m, double alpha, const void *x, double beta, void
                                    jacobi, jdt);
 }
 
+bool apply_f32_between(akm_matrix_s &m, const double *v, double c, double *w)
+{
+  if (m.prec != AKM_F32 || !m.gk || (m.mode != mode_global && (!m.factored || m.pair_kernels)))
+    return false;
+  akm_global_s &g = *m.gk;
+  if (g.slab || g.lanes != 8 || g.active_cells == 0)
+    return false;
+  std::lock_guard<std::mutex> lock(m.factored_mtx);
+  return fibre_apply_between(m, g.fl, v, c, w);
+}
+
 int global_update(akm_matrix_s &m, const void *vA)
 {
   AKM_HIP(hipMemcpyAsync(m.vA.data(), vA, m.num_vA * m.esize, hipMemcpyHostToDevice, m.stream));

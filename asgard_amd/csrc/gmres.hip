@@ -3,14 +3,25 @@
 //
 // akm_gmres_euler is the algorithm of solver::simple_gmres
 // (src/solver.cpp:156-298) with every vector and Hessenberg operation on the
-// GPU.  Per inner iteration: one fused apply (kronmult + identity), the
-// classical Gram-Schmidt dot products V^T w, the update w -= V h (which first
-// reduces the dot partials to h) fused with the partial sums of |w|^2, and
-// one kernel that finishes the norm and scales w while its first workgroup
-// rotates the new Hessenberg column and the right-hand side (reference BLAS
-// rot/rotg semantics) and writes the residual estimate.
-// Reductions use fixed block partitions and orders, so results repeat
-// bit for bit.  The host reads one scalar per iteration to test convergence.
+// GPU.  An inner iteration is the fused apply (kronmult + identity) and two
+// kernels: the classical Gram-Schmidt dot products V^T w, and the update
+// w -= V h with the partial sums of |w|^2.  What only needs those sums (the
+// norm, the rotation of the Hessenberg column and of the right-hand side with
+// reference BLAS rot/rotg semantics, the residual estimate) is done by an
+// extra workgroup of the next step's dot products, beside them, and stored
+// straight to pinned host memory.  A Krylov vector stays as the update leaves
+// it, with its 1/norm kept aside: the operator is linear, so the factor goes
+// into the next step's coefficients and no pass scales vectors (except for
+// preconditioned directions, which may be nonlinear).  Reductions use fixed
+// partitions and orders, so results repeat bit for bit.  The host reads one
+// scalar per iteration to test convergence.
+//
+// What bounds a step at 64,768 unknowns: the latency of its three dependent
+// launches, 8.5 (apply) + 4.8 + 6.2 us.  One kernel each for the dots, the
+// reduction and update, the Givens step with the scaling, and a copy of the
+// state to the host took 8.4 + 10.6 + 4.8 + 2.7 us beside the apply; letting
+// the update's last workgroup finish the step took 14.2 us for the update
+// (the tail of device-scope accesses is serial).
 //
 // akm_gmres_euler_mixed is an FP64 iterative refinement around flexible
 // GMRES cycles: the residual b - (I - dt*A)x, the Krylov basis, the
@@ -24,6 +35,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <functional>
 #include <limits>
 #include <mutex>
@@ -32,14 +44,19 @@
 namespace akm
 {
 constexpr int gm_threads = 256;
-constexpr int gm_cols = 8; // Krylov columns per dot-product block
-// the Givens kernel stages 3 * restart values in LDS (64 KB)
+constexpr int gm_cols = 4; // Krylov columns per dot-product block
+// the update's parts: columns are split over gm_split threads per row
+constexpr int gm_split = 4;
+constexpr int gm_tile = 128; // rows of an update block at a time
+constexpr int gm_upd_threads = gm_split * gm_tile;
+constexpr int gm_lanes = 8; // lanes that add one column's dot partials
+// finishing a step stages 3 * restart values in LDS (64 KB)
 constexpr int gm_max_restart = 2000;
 // host copies of the step state: Arnoldi steps in flight at once (the step
 // waited for plus the speculative ones) stay below this
-constexpr int gm_slots = 4;
-// speculative steps enqueued past the one waited for (two measured no faster
-// than one at d=4: the step is bound by the GPU's kernel chain, not the host)
+constexpr int gm_slots = 8;
+// speculative steps enqueued past the one waited for: one step on the GPU
+// (about 15 us at d=4) covers the host's poll and its three launches
 constexpr int gm_ahead = 1;
 
 template<typename P>
@@ -47,9 +64,26 @@ struct gm_state
 {
   P nrm;       // norm of the last orthogonalised vector
   P inner_res; // residual estimate |s_j g_j|
-  P inv_nrm;   // 1 / nrm (0 if nrm == 0)
-  P pad;
+  P pad[2];
 };
+
+//! What the host reads of a step, in pinned memory: the value and the value
+//! xor the step's number, so that the two stores need no order between them.
+struct gm_host_state
+{
+  uint64_t value, check;
+  uint64_t pad[6];
+};
+
+//! A step's scalar to the host (nothing when there is no slot).
+__device__ __forceinline__ void gm_publish(gm_host_state *hs, double value, uint64_t seq)
+{
+  if (hs == nullptr)
+    return;
+  const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(value));
+  __hip_atomic_store(&hs->value, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&hs->check, bits ^ seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 template<typename P>
 __device__ __forceinline__ P block_sum(P v, P *sh)
@@ -68,113 +102,6 @@ __device__ __forceinline__ P block_sum(P v, P *sh)
     r += sh[w];
   __syncthreads();
   return r;
-}
-
-//! Fixed-order sum over one wavefront (the shuffle tree of block_sum).
-template<typename P>
-__device__ __forceinline__ P wave_sum(P v)
-{
-#pragma unroll
-  for (int off = wave_size / 2; off > 0; off >>= 1)
-    v += __shfl_xor(v, off, wave_size);
-  return v;
-}
-
-//! partial[k*nblk + bx] = sum over rows of block bx of V_k[i] * w[i],
-//! for k in [k0, k0 + gm_cols) intersect [0, ncols).
-template<typename P>
-__global__ void __launch_bounds__(gm_threads)
-gm_dots(int64_t n, int64_t rows_per_block, const P *V, int64_t ldv, const P *w, int ncols,
-        P *partial)
-{
-  __shared__ P sh[gm_threads];
-  const int64_t r0 = blockIdx.x * rows_per_block;
-  const int64_t r1 = min(n, r0 + rows_per_block);
-  const int k0 = blockIdx.y * gm_cols;
-  P acc[gm_cols];
-#pragma unroll
-  for (int c = 0; c < gm_cols; c++)
-    acc[c] = 0;
-  for (int64_t i = r0 + threadIdx.x; i < r1; i += gm_threads)
-  {
-    const P wi = w[i];
-#pragma unroll
-    for (int c = 0; c < gm_cols; c++)
-      if (k0 + c < ncols)
-        acc[c] = fma(V[(k0 + c) * ldv + i], wi, acc[c]);
-  }
-#pragma unroll
-  for (int c = 0; c < gm_cols; c++)
-  {
-    P s = block_sum(acc[c], sh);
-    if (threadIdx.x == 0 && k0 + c < ncols)
-      partial[int64_t(k0 + c) * gridDim.x + blockIdx.x] = s;
-  }
-}
-
-//! w -= V[:, 0:ncols] h and sq_partial[bx] = sum of w^2 over the block's
-//! rows, with h formed first by every block from the dot partials:
-//! h[k] = sum_b partial[k*nblk + b] (one wavefront per column, lanes striding
-//! over the blocks, then the shuffle tree; the same order in every block).
-//! Block 0 stores h.
-template<typename P>
-__global__ void __launch_bounds__(gm_threads)
-gm_reduce_update(int64_t n, int64_t rows_per_block, const P *V, int64_t ldv, P *w, int ncols,
-                 const P *partial, P *h, P *sq_partial)
-{
-  __shared__ P sh[gm_threads];
-  extern __shared__ unsigned char hs_raw[];
-  P *hs = reinterpret_cast<P *>(hs_raw);
-  const int nblk = gridDim.x;
-  const int wave = threadIdx.x / wave_size, lane = threadIdx.x % wave_size;
-  for (int k = wave; k < ncols; k += gm_threads / wave_size)
-  {
-    P v = 0;
-    for (int b = lane; b < nblk; b += wave_size)
-      v += partial[int64_t(k) * nblk + b];
-    v = wave_sum(v);
-    if (lane == 0)
-    {
-      hs[k] = v;
-      if (blockIdx.x == 0)
-        h[k] = v;
-    }
-  }
-  __syncthreads();
-  const int64_t r0 = blockIdx.x * rows_per_block;
-  const int64_t r1 = min(n, r0 + rows_per_block);
-  P sq = 0;
-  for (int64_t i = r0 + threadIdx.x; i < r1; i += gm_threads)
-  {
-    P s = 0;
-    for (int k = 0; k < ncols; k++)
-      s = fma(V[k * ldv + i], hs[k], s);
-    const P v = w[i] - s;
-    w[i] = v;
-    sq = fma(v, v, sq);
-  }
-  sq = block_sum(sq, sh);
-  if (threadIdx.x == 0)
-    sq_partial[blockIdx.x] = sq;
-}
-
-//! sq_partial[bx] = sum of x^2 over the block's rows (x is only read).
-template<typename P>
-__global__ void __launch_bounds__(gm_threads)
-gm_sumsq(int64_t n, int64_t rows_per_block, const P *x, P *sq_partial)
-{
-  __shared__ P sh[gm_threads];
-  const int64_t r0 = blockIdx.x * rows_per_block;
-  const int64_t r1 = min(n, r0 + rows_per_block);
-  P sq = 0;
-  for (int64_t i = r0 + threadIdx.x; i < r1; i += gm_threads)
-  {
-    const P v = x[i];
-    sq = fma(v, v, sq);
-  }
-  sq = block_sum(sq, sh);
-  if (threadIdx.x == 0)
-    sq_partial[blockIdx.x] = sq;
 }
 
 template<typename P>
@@ -207,48 +134,62 @@ __device__ __forceinline__ void dev_rotg(P &a, P b, P &c, P &s)
   a = r;
 }
 
-//! Finishes the norm from the block partials.  With j < 0 this starts a
-//! restart cycle (g[0] = |r|); otherwise it processes Hessenberg column j:
-//! stores h, applies the previous rotations, computes the new one, the
-//! residual estimate and rotates g.  With rotate_always == 0, g is rotated
-//! only while the estimate is above tol, as simple_gmres does
-//! (src/solver.cpp:261-267).
+//! What finishing a step reads and writes: the step's |w|^2 partials and
+//! Hessenberg column h, the rotations, the right-hand side, and the state.
 template<typename P>
-__global__ void __launch_bounds__(64)
-gm_givens(int nblk, const P *sq_partial, const P *h, int j, P *H, P *cs, P *sn, P *g, P tol,
-          int rotate_always, gm_state<P> *st)
+struct gm_arrays
 {
-  // column j, then the previous rotations, staged in LDS so that the serial
-  // part below runs on registers and LDS (dynamic LDS: 3j + 1 values)
-  __shared__ P sh[64];
-  extern __shared__ unsigned char gv_raw[];
-  P *lc = reinterpret_cast<P *>(gv_raw);
-  P *lcs = lc + (j + 1);
-  P *lsn = lcs + j;
-  for (int k = threadIdx.x; k <= j; k += 64)
-    lc[k] = h[k];
-  for (int k = threadIdx.x; k < j; k += 64)
+  P *h, *H, *cs, *sn, *g; // column, packed columns, rotations, right-hand side
+  P *inv;                 // 1/norm of every stored Krylov vector; null: all unit
+  P *sqp;                 // |w|^2 partials
+  gm_state<P> *st;
+};
+
+//! The step an extra workgroup finishes: column j (-1: the start of a cycle,
+//! where the norm is that of the residual), or nothing (count 0).
+template<typename P>
+struct gm_pending
+{
+  int j, count; // count: |w|^2 partials
+  P tol;
+  int rotate_always;
+  gm_host_state *hs;
+  uint64_t seq;
+};
+
+//! Finishes a step in one workgroup (see the file comment).  With j < 0:
+//! g_0 = |r|.  Otherwise the old rotations down column j, the new one, the
+//! residual estimate and the rotation of g, which with rotate_always == 0
+//! happens only while the estimate is above tol, as simple_gmres does
+//! (src/solver.cpp:261-267).  `lds`: 3 (j + 1) values.
+template<typename P>
+__device__ __forceinline__ void gm_finish_step(gm_arrays<P> const &a, gm_pending<P> const &p,
+                                               P *lds, P *sh)
+{
+  const int j = p.j, t = threadIdx.x;
+  P *lc = lds, *lcs = lds + (j + 1), *lsn = lcs + (j + 1);
+  for (int k = t; k <= j; k += blockDim.x)
+    lc[k] = a.h[k];
+  for (int k = t; k < j; k += blockDim.x)
   {
-    lcs[k] = cs[k];
-    lsn[k] = sn[k];
+    lcs[k] = a.cs[k];
+    lsn[k] = a.sn[k];
   }
+  const P gj = (j >= 0) ? a.g[j] : P{0};
   P s = 0;
-  for (int b = threadIdx.x; b < nblk; b += 64)
-    s += sq_partial[b];
+#pragma unroll 4
+  for (int b = t; b < p.count; b += blockDim.x)
+    s += a.sqp[b];
   s = block_sum(s, sh); // its barriers also order the LDS writes above
-  if (threadIdx.x == 0)
+  const P nrm = sqrt(s);
+  if (t == 0)
   {
-    const P nrm = sqrt(s);
-    st->nrm = nrm;
-    st->inv_nrm = (nrm > P{0}) ? P{1} / nrm : P{0};
+    P res = nrm;
     if (j < 0)
-    {
-      g[0] = nrm;
-      st->inner_res = nrm;
-    }
+      a.g[0] = nrm;
     else
     {
-      // apply the old rotations down the column, the running entry in a register
+      // down the column, the running entry in a register
       P x = lc[0];
       for (int k = 0; k < j; k++)
       {
@@ -260,118 +201,235 @@ gm_givens(int nblk, const P *sq_partial, const P *h, int j, P *H, P *cs, P *sn, 
       P c, sv;
       dev_rotg(x, nrm, c, sv);
       lc[j] = x;
-      cs[j] = c;
-      sn[j] = sv;
-      const P res = fabs(sv * g[j]);
-      st->inner_res = res;
-      if (rotate_always != 0 || res > tol)
+      a.cs[j] = c;
+      a.sn[j] = sv;
+      res = fabs(sv * gj);
+      if (p.rotate_always != 0 || res > p.tol)
       {
-        g[j + 1] = 0;
-        dev_rot(g[j], g[j + 1], c, sv);
+        P u = gj, v = 0;
+        dev_rot(u, v, c, sv);
+        a.g[j] = u;
+        a.g[j + 1] = v;
       }
     }
+    gm_publish(p.hs, static_cast<double>(res), p.seq);
+    a.st->nrm = nrm;
+    a.st->inner_res = res;
+    if (a.inv != nullptr)
+      a.inv[j + 1] = (nrm > P{0}) ? P{1} / nrm : P{0};
   }
-  if (j < 0)
-    return;
   __syncthreads();
-  P *col = H + (j * (j + 1)) / 2; // packed upper triangle, column j
-  for (int k = threadIdx.x; k <= j; k += 64)
-    col[k] = lc[k];
+  for (int k = t; k <= j; k += blockDim.x)
+    a.H[(j * (j + 1)) / 2 + k] = lc[k]; // packed upper triangle, column j
 }
 
-//! gm_givens for column j >= 0 and gm_scale in one launch: every block
-//! finishes the norm from the partials (the first wavefront, in gm_givens'
-//! order) and scales its rows of w; block 0 also rotates the Hessenberg
-//! column and the right-hand side and writes the state (dynamic LDS:
-//! 3j + 1 values).
+//! gm_finish_step alone (the host waits for it before the next step is
+//! enqueued).  Dynamic LDS: 3 (j + 1) values.
+template<typename P>
+__global__ void __launch_bounds__(gm_threads) gm_finish(gm_arrays<P> a, gm_pending<P> p)
+{
+  __shared__ P sh[gm_threads / wave_size];
+  extern __shared__ unsigned char gf_raw[];
+  gm_finish_step(a, p, reinterpret_cast<P *>(gf_raw), sh);
+}
+
+//! sqp[bx] = sum of x^2 over the block's rows (x is only read).
 template<typename P>
 __global__ void __launch_bounds__(gm_threads)
-gm_givens_scale(int64_t n, P *w, int nblk, const P *sq_partial, const P *h, int j, P *H, P *cs,
-                P *sn, P *g, P tol, int rotate_always, gm_state<P> *st)
+gm_sumsq(int64_t n, int64_t rows_per_block, const P *x, P *sqp)
 {
-  __shared__ P s_nrm;
-  extern __shared__ unsigned char gs_raw[];
-  if (threadIdx.x < wave_size)
+  __shared__ P sh[gm_threads / wave_size];
+  const int64_t r0 = blockIdx.x * rows_per_block;
+  const int64_t r1 = min(n, r0 + rows_per_block);
+  P sq = 0;
+#pragma unroll 4
+  for (int64_t i = r0 + threadIdx.x; i < r1; i += gm_threads)
+  {
+    const P v = x[i];
+    sq = fma(v, v, sq);
+  }
+  sq = block_sum(sq, sh);
+  if (threadIdx.x == 0)
+    sqp[blockIdx.x] = sq;
+}
+
+//! partial[k*ndot + bx] = sum over rows of block bx of V_k[i] * w[i],
+//! for k in [k0, k0 + gm_cols) intersect [0, ncols).  The wavefront reduces
+//! its gm_cols sums together: each exchange halves the columns a lane holds.
+//! Workgroup (ndot, 0) finishes the step before instead (pend.count > 0;
+//! dynamic LDS: 3 (pend.j + 1) values).
+template<typename P>
+__global__ void __launch_bounds__(gm_threads)
+gm_dots(int64_t n, int64_t rows_per_block, const P *V, int64_t ldv, const P *w, int ncols,
+        int ndot, P *partial, gm_arrays<P> arr, gm_pending<P> pend)
+{
+  static_assert(gm_cols == 4, "the exchange below halves four columns twice");
+  __shared__ P sh[gm_threads / wave_size][gm_cols];
+  extern __shared__ unsigned char gd_raw[];
+  if (static_cast<int>(blockIdx.x) == ndot)
+  {
+    if (blockIdx.y == 0)
+      gm_finish_step(arr, pend, reinterpret_cast<P *>(gd_raw), &sh[0][0]);
+    return;
+  }
+  const int64_t r0 = blockIdx.x * rows_per_block;
+  const int64_t r1 = min(n, r0 + rows_per_block);
+  const int k0 = blockIdx.y * gm_cols;
+  P acc[gm_cols];
+  const P *col[gm_cols];
+#pragma unroll
+  for (int c = 0; c < gm_cols; c++)
+  {
+    acc[c] = 0;
+    // columns past the last repeat it; their sums are dropped
+    col[c] = V + int64_t(min(k0 + c, ncols - 1)) * ldv;
+  }
+#pragma unroll 4
+  for (int64_t i = r0 + threadIdx.x; i < r1; i += gm_threads)
+  {
+    const P wi = w[i];
+#pragma unroll
+    for (int c = 0; c < gm_cols; c++)
+      acc[c] = fma(col[c][i], wi, acc[c]);
+  }
+  const int lane = threadIdx.x % wave_size;
+  const bool up = (lane & 32) != 0, odd = (lane & 16) != 0;
+  // lanes below 32 keep columns 0 and 1, the others 2 and 3; then one each
+  const P a0 = (up ? acc[2] : acc[0]) + __shfl_xor(up ? acc[0] : acc[2], 32, wave_size);
+  const P a1 = (up ? acc[3] : acc[1]) + __shfl_xor(up ? acc[1] : acc[3], 32, wave_size);
+  P v = (odd ? a1 : a0) + __shfl_xor(odd ? a0 : a1, 16, wave_size);
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1)
+    v += __shfl_xor(v, off, wave_size);
+  if ((lane & 15) == 0)
+    sh[threadIdx.x / wave_size][(up ? 2 : 0) + (odd ? 1 : 0)] = v;
+  __syncthreads();
+  if (threadIdx.x < gm_cols && k0 + static_cast<int>(threadIdx.x) < ncols)
   {
     P s = 0;
-    for (int b = threadIdx.x; b < nblk; b += wave_size)
-      s += sq_partial[b];
-    s = wave_sum(s);
-    if (threadIdx.x == 0)
-      s_nrm = sqrt(s);
+#pragma unroll
+    for (int w2 = 0; w2 < gm_threads / wave_size; w2++)
+      s += sh[w2][threadIdx.x];
+    partial[int64_t(k0 + threadIdx.x) * ndot + blockIdx.x] = s;
   }
-  P *lc = reinterpret_cast<P *>(gs_raw);
-  P *lcs = lc + (j + 1);
-  P *lsn = lcs + j;
-  if (blockIdx.x == 0)
+}
+
+//! Arnoldi step j after the dots (ndot partials per column): h, then
+//! w <- w / |v_j| - V h with the |w|^2 partials; columns split over gm_split
+//! threads per row.  Block 0 stores h.  Dynamic LDS: j + 1 values.
+template<typename P>
+__global__ void __launch_bounds__(gm_upd_threads)
+gm_update(int64_t n, int64_t rows_per_block, const P *V, int64_t ldv, P *w, int j,
+          const P *dotp, int ndot, gm_arrays<P> a)
+{
+  __shared__ P red[gm_split][gm_tile];
+  __shared__ P sh[gm_upd_threads / wave_size];
+  extern __shared__ unsigned char up_raw[];
+  P *cf = reinterpret_cast<P *>(up_raw); // h_k / |stored v_k|
+  const int t = threadIdx.x, ncols = j + 1;
+  const P invj = (a.inv != nullptr) ? a.inv[j] : P{1};
+  // gm_lanes lanes add one column's partials, the same order in every block
+  for (int k = t / gm_lanes; k < ncols; k += gm_upd_threads / gm_lanes)
   {
-    for (int k = threadIdx.x; k <= j; k += gm_threads)
-      lc[k] = h[k];
-    for (int k = threadIdx.x; k < j; k += gm_threads)
+    const P ik = (a.inv != nullptr) ? a.inv[k] : P{1};
+    P v = 0;
+#pragma unroll 8
+    for (int b = t % gm_lanes; b < ndot; b += gm_lanes)
+      v += dotp[int64_t(k) * ndot + b];
+#pragma unroll
+    for (int off = gm_lanes / 2; off > 0; off >>= 1)
+      v += __shfl_xor(v, off, wave_size);
+    if (t % gm_lanes == 0)
     {
-      lcs[k] = cs[k];
-      lsn[k] = sn[k];
+      const P h = v * ik * invj;
+      cf[k] = h * ik;
+      if (blockIdx.x == 0)
+        a.h[k] = h;
     }
   }
   __syncthreads();
-  const P nrm = s_nrm;
-  const P inv = (nrm > P{0}) ? P{1} / nrm : P{0};
-  if (blockIdx.x == 0)
+  const int part = t / gm_tile, lane = t % gm_tile;
+  const int64_t r0 = blockIdx.x * rows_per_block;
+  const int64_t r1 = min(n, r0 + rows_per_block);
+  P sq = 0;
+  for (int64_t base = r0; base < r1; base += gm_tile)
   {
-    if (threadIdx.x == 0)
+    const int64_t i = base + lane;
+    P s = 0;
+    if (i < r1)
     {
-      st->nrm = nrm;
-      st->inv_nrm = inv;
-      P x = lc[0];
-      for (int k = 0; k < j; k++)
-      {
-        P y = lc[k + 1];
-        dev_rot(x, y, lcs[k], lsn[k]);
-        lc[k] = x;
-        x = y;
-      }
-      P c, sv;
-      dev_rotg(x, nrm, c, sv);
-      lc[j] = x;
-      cs[j] = c;
-      sn[j] = sv;
-      const P res = fabs(sv * g[j]);
-      st->inner_res = res;
-      if (rotate_always != 0 || res > tol)
-      {
-        g[j + 1] = 0;
-        dev_rot(g[j], g[j + 1], c, sv);
-      }
+#pragma unroll 8
+      for (int k = part; k < ncols; k += gm_split)
+        s = fma(V[int64_t(k) * ldv + i], cf[k], s);
+    }
+    red[part][lane] = s;
+    __syncthreads();
+    if (part == 0 && i < r1)
+    {
+      P sum = red[0][lane];
+#pragma unroll
+      for (int q = 1; q < gm_split; q++)
+        sum += red[q][lane];
+      const P v = fma(w[i], invj, -sum);
+      w[i] = v;
+      sq = fma(v, v, sq);
     }
     __syncthreads();
-    P *col = H + (j * (j + 1)) / 2; // packed upper triangle, column j
-    for (int k = threadIdx.x; k <= j; k += gm_threads)
-      col[k] = lc[k];
   }
-  if (inv == P{0})
-    return;
-  for (int64_t i = blockIdx.x * int64_t(gm_threads) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * gm_threads)
-    w[i] *= inv;
+  sq = block_sum(sq, sh);
+  if (t == 0)
+    a.sqp[blockIdx.x] = sq;
 }
 
+//! w /= |w| (the norm of the state), for vectors a nonlinear map reads.
 template<typename P>
 __global__ void __launch_bounds__(gm_threads) gm_scale(int64_t n, P *w, const gm_state<P> *st)
 {
-  const P inv = st->inv_nrm;
-  if (inv == P{0})
+  const P nrm = st->nrm;
+  if (!(nrm > P{0}))
     return;
+  const P inv = P{1} / nrm;
   for (int64_t i = blockIdx.x * int64_t(gm_threads) + threadIdx.x; i < n;
        i += int64_t(gridDim.x) * gm_threads)
     w[i] *= inv;
 }
 
-//! Packed upper-triangular back-solve H y = g (tpsv 'U','N','N'), in g.
-//! One workgroup; g (and H when it fits, `h_in_lds`) staged in LDS; column
-//! by column, the updates of one column spread over the threads (the same
-//! operations in the same order per entry as a serial solve).
+//! Packed upper-triangular back-solve H y = g (tpsv 'U','N','N') in g, then
+//! y_k / |stored v_k|.  One wavefront with an entry per lane for m <= 64
+//! (no barriers: 11 us became 4 at m = 35); else one workgroup, g (and H when
+//! it fits, `h_in_lds`) in LDS, the updates of one column over the threads.
+//! The same operations in the same order per entry as a serial solve.
 template<typename P>
-__global__ void __launch_bounds__(256) gm_backsolve(int m, const P *H, P *g, int h_in_lds)
+__global__ void __launch_bounds__(64) gm_backsolve_wave(int m, const P *H, P *g, const P *inv)
+{
+  __shared__ P lh[64 * 65 / 2];
+  const int lane = threadIdx.x;
+#pragma unroll 8
+  for (int i = lane; i < m * (m + 1) / 2; i += 64)
+    lh[i] = H[i];
+  P v = (lane < m) ? g[lane] : P{0};
+  __syncthreads();
+  const P own = (lane < m) ? lh[lane + (lane * (lane + 1)) / 2] : P{0};
+  for (int j = m - 1; j >= 0; j--)
+  {
+    const P hij = (lane < j) ? lh[lane + (j * (j + 1)) / 2] : P{0};
+    // every lane divides by its own diagonal, lane j's quotient counts.  A
+    // zero diagonal only follows an exact breakdown (residual already zero);
+    // that column then takes no part in the solution
+    const P q = (own != P{0}) ? v / own : P{0};
+    const P gj = __shfl(q, j, wave_size);
+    if (lane < j)
+      v -= gj * hij;
+    else if (lane == j)
+      v = gj;
+  }
+  if (lane < m)
+    g[lane] = (inv != nullptr) ? v * inv[lane] : v;
+}
+
+template<typename P>
+__global__ void __launch_bounds__(256)
+gm_backsolve(int m, const P *H, P *g, int h_in_lds, const P *inv)
 {
   extern __shared__ unsigned char bs_raw[];
   P *lg = reinterpret_cast<P *>(bs_raw);
@@ -389,8 +447,6 @@ __global__ void __launch_bounds__(256) gm_backsolve(int m, const P *H, P *g, int
     if (tid == 0)
     {
       const P hjj = Hs[j + (j * (j + 1)) / 2];
-      // a zero diagonal only follows an exact breakdown (residual already
-      // zero); that column then takes no part in the solution
       lg[j] = (hjj != P{0}) ? lg[j] / hjj : P{0};
     }
     __syncthreads();
@@ -400,26 +456,44 @@ __global__ void __launch_bounds__(256) gm_backsolve(int m, const P *H, P *g, int
     __syncthreads();
   }
   for (int i = tid; i < m; i += 256)
-    g[i] = lg[i];
+    g[i] = (inv != nullptr) ? lg[i] * inv[i] : lg[i];
 }
 
-//! x += V[:, 0:m] y
+//! x += V[:, 0:m] y, the columns split over gm_split threads per row.
 template<typename P>
-__global__ void __launch_bounds__(gm_threads)
-gm_xupdate(int64_t n, const P *V, int64_t ldv, int m, const P *y, P *x)
+__global__ void __launch_bounds__(gm_upd_threads)
+gm_xupdate(int64_t n, int64_t rows_per_block, const P *V, int64_t ldv, int m, const P *y, P *x)
 {
+  __shared__ P red[gm_split][gm_tile];
   extern __shared__ unsigned char ys_raw[];
   P *ys = reinterpret_cast<P *>(ys_raw);
-  for (int k = threadIdx.x; k < m; k += gm_threads)
+  for (int k = threadIdx.x; k < m; k += gm_upd_threads)
     ys[k] = y[k];
   __syncthreads();
-  for (int64_t i = blockIdx.x * int64_t(gm_threads) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * gm_threads)
+  const int part = threadIdx.x / gm_tile, lane = threadIdx.x % gm_tile;
+  const int64_t r0 = blockIdx.x * rows_per_block;
+  const int64_t r1 = min(n, r0 + rows_per_block);
+  for (int64_t base = r0; base < r1; base += gm_tile)
   {
+    const int64_t i = base + lane;
     P s = 0;
-    for (int k = 0; k < m; k++)
-      s = fma(V[k * ldv + i], ys[k], s);
-    x[i] += s;
+    if (i < r1)
+    {
+#pragma unroll 8
+      for (int k = part; k < m; k += gm_split)
+        s = fma(V[int64_t(k) * ldv + i], ys[k], s);
+    }
+    red[part][lane] = s;
+    __syncthreads();
+    if (part == 0 && i < r1)
+    {
+      P sum = red[0][lane];
+#pragma unroll
+      for (int q = 1; q < gm_split; q++)
+        sum += red[q][lane];
+      x[i] += sum;
+    }
+    __syncthreads();
   }
 }
 
@@ -523,15 +597,12 @@ struct akm_gmres_workspace
   // flexible / mixed-precision solver only
   akm::dev_buffer<double> Z, xprev;
   akm::dev_buffer<float> v32, y32;
-  void *host_state = nullptr; // pinned, gm_slots slots
-  hipEvent_t state_ready[akm::gm_slots] = {};
+  akm::gm_host_state *host_state = nullptr; // pinned, gm_slots slots
+  uint64_t seq = 0;                         // step numbers given out so far
   ~akm_gmres_workspace()
   {
     if (host_state != nullptr)
       (void)hipHostFree(host_state);
-    for (auto &e : state_ready)
-      if (e != nullptr)
-        (void)hipEventDestroy(e);
   }
 };
 
@@ -539,12 +610,13 @@ static void delete_workspace(akm_gmres_workspace *w) { delete w; }
 
 namespace akm
 {
-//! Rows of a vector handled by one reduction block: at least 256 (one row per
-//! thread), otherwise enough blocks to cover the chip (about 1024) and no
-//! more, so the per-column partial sums stay short.
-static int64_t rows_per_block_for(int64_t n)
+//! Rows of a dot-product (and norm) block: four per thread, more past 512
+//! blocks, so the per-column partial sums stay short.
+static int64_t dot_rows(int64_t n) { return std::max<int64_t>(1024, (n + 511) / 512); }
+//! Rows of an update block: one tile, more past 1024 blocks.
+static int64_t update_rows(int64_t n)
 {
-  return std::max<int64_t>(256, (n + 1023) / 1024);
+  return std::max<int64_t>(1, (n + 1024 * gm_tile - 1) / (1024 * gm_tile)) * gm_tile;
 }
 
 //! Arnoldi steps are enqueued one ahead of the host's convergence check when
@@ -575,27 +647,35 @@ static int timed_on_stream(hipStream_t s, F &&f, double &ms)
 }
 
 //! Memory of one solve: the Krylov basis V (n x (restart + 1)), the small
-//! work array (h, packed H, cs, sn, g, dot and norm partials:
-//! gm_work_values of them), the device step state, gm_slots host copies of
-//! it, and gm_slots events marking those copies (or null: the host then
-//! waits for the whole stream).  Every value is written by a kernel before
-//! any kernel or the host reads it, so none needs clearing between solves.
+//! work array (h, packed H, cs, sn, g, 1/norms, dot and norm partials:
+//! gm_work_values of them), the device step state, and gm_slots pinned host
+//! slots with the number of steps published to them, or one plain host state
+//! (the host then waits for the whole stream).  Every value on the device is
+//! written by a kernel before any kernel or the host reads it, so none needs
+//! clearing between solves.
 struct gm_memory
 {
   void *V = nullptr;
   void *work = nullptr;
   void *state = nullptr;
+  gm_host_state *slots = nullptr;
+  uint64_t *seq = nullptr;
   void *host_state = nullptr;
-  hipEvent_t *ready = nullptr;
 };
 
 //! Values in the small work array of a solve.
 static int64_t gm_work_values(int64_t n, int restart)
 {
-  const int64_t rpb = rows_per_block_for(n);
+  // sized for 256-row partials of every column, more than those in use
+  // (dot_rows, update_rows) and the 1/norms take
+  const int64_t rpb = std::max<int64_t>(256, (n + 1023) / 1024);
   const int64_t nblk = (n + rpb - 1) / rpb;
-  return 4 * int64_t(restart + 2) + int64_t(restart) * (restart + 1) / 2 + 2 +
-         int64_t(restart + 1) * nblk + nblk + 16;
+  const int64_t columns = int64_t(restart) * (restart + 1) / 2;
+  const int64_t ndot = (n + dot_rows(n) - 1) / dot_rows(n);
+  const int64_t nupd = (n + update_rows(n) - 1) / update_rows(n);
+  return std::max(4 * int64_t(restart + 2) + columns + 2 + int64_t(restart + 1) * nblk + nblk + 16,
+                  5 * int64_t(restart + 2) + columns + 2 + int64_t(restart + 1) * ndot +
+                      std::max(nupd, ndot));
 }
 
 //! The memory of a solve in a matrix's workspace.
@@ -605,8 +685,8 @@ static gm_memory memory_of(akm_gmres_workspace &ws)
   mem.V = ws.V.data();
   mem.work = ws.work.data();
   mem.state = ws.state.data();
-  mem.host_state = ws.host_state;
-  mem.ready = ws.state_ready;
+  mem.slots = ws.host_state;
+  mem.seq = &ws.seq;
   return mem;
 }
 
@@ -620,12 +700,16 @@ struct gm_cycle
   P *V = nullptr;
   P *Z = nullptr; // preconditioned directions (flexible GMRES), else null
   int64_t ldv = 0;
-  int64_t rpb = 0;
-  int nblk = 0, sblocks = 0;
-  P *h = nullptr, *H = nullptr, *cs = nullptr, *sn = nullptr, *g = nullptr;
+  int64_t drows = 0, urows = 0;
+  int ndot = 0, nupd = 0, sblocks = 0;
+  P *h = nullptr, *H = nullptr, *cs = nullptr, *sn = nullptr, *g = nullptr, *inv = nullptr;
   P *dotp = nullptr, *sqp = nullptr;
   gm_state<P> *st = nullptr, *hst = nullptr;
-  hipEvent_t *ready = nullptr;
+  gm_host_state *slots = nullptr;
+  uint64_t *seq = nullptr;
+  uint64_t start_seq = 0; // number of the cycle's start, step j is start + 1 + j
+  int finished = -2;      // last step finished by a launch (-1: the start)
+  bool lazy = true; // Krylov vectors stored beside their 1/norm
   int rotate_always = 0;
 
   gm_cycle(gm_memory const &mem, int64_t n_, hipStream_t s_, int restart_, P *Z_,
@@ -634,78 +718,129 @@ struct gm_cycle
   {
     V = static_cast<P *>(mem.V);
     ldv = n;
-    rpb = rows_per_block_for(n);
-    nblk = static_cast<int>((n + rpb - 1) / rpb);
+    drows = dot_rows(n);
+    ndot = static_cast<int>((n + drows - 1) / drows);
+    urows = update_rows(n);
+    nupd = static_cast<int>((n + urows - 1) / urows);
     sblocks = static_cast<int>(std::min<int64_t>((n + gm_threads - 1) / gm_threads, 2048));
-    // small work arrays: h, H (packed), cs, sn, g, dot partials, sq partials
+    // small work arrays: h, H (packed), cs, sn, g, 1/norms, dot and norm partials
     h = static_cast<P *>(mem.work);
     H = h + (restart + 1);
     cs = H + int64_t(restart) * (restart + 1) / 2 + 1;
     sn = cs + (restart + 1);
     g = sn + (restart + 1);
-    dotp = g + (restart + 2);
-    sqp = dotp + int64_t(restart + 1) * nblk;
+    inv = g + (restart + 2);
+    dotp = inv + (restart + 2);
+    sqp = dotp + int64_t(restart + 1) * ndot;
     st = static_cast<gm_state<P> *>(mem.state);
     hst = static_cast<gm_state<P> *>(mem.host_state);
-    ready = mem.ready;
+    slots = mem.slots;
+    seq = mem.seq;
   }
 
-  int sync_state()
+  gm_arrays<P> arrays() const
   {
-    AKM_HIP(hipMemcpyAsync(hst, st, sizeof(gm_state<P>), hipMemcpyDeviceToHost, s));
-    AKM_HIP(hipStreamSynchronize(s));
+    return gm_arrays<P>{h, H, cs, sn, g, lazy ? inv : nullptr, sqp, st};
+  }
+
+  //! Step j (-1: the start) as the kernel that finishes it sees it.
+  gm_pending<P> pending(int j, P tol) const
+  {
+    const uint64_t number = start_seq + 1 + j;
+    return gm_pending<P>{j,   (j < 0) ? ndot : nupd, tol, rotate_always,
+                         (slots != nullptr) ? slots + number % gm_slots : nullptr, number};
+  }
+
+  //! Finishes step j in a launch of its own.
+  int finish_step(int j, P tol)
+  {
+    gm_finish<P><<<1, gm_threads, 3 * sizeof(P) * (j + 1), s>>>(arrays(), pending(j, tol));
+    finished = j;
+    return check_launch("gmres step");
+  }
+
+  //! Waits until step j (-1: the start) is finished; res = its estimate.
+  //! Polls the pinned slot the kernel writes; a stream that has run dry
+  //! without writing it has failed.
+  int wait_step(int j, P &res)
+  {
+    if (slots == nullptr)
+    {
+      AKM_HIP(hipMemcpyAsync(hst, st, sizeof(gm_state<P>), hipMemcpyDeviceToHost, s));
+      AKM_HIP(hipStreamSynchronize(s));
+      res = hst->inner_res;
+      return AKM_SUCCESS;
+    }
+    const uint64_t number = start_seq + 1 + j;
+    const gm_host_state *slot = slots + number % gm_slots;
+    uint64_t value = 0;
+    auto arrived = [&]() {
+      value = __atomic_load_n(&slot->value, __ATOMIC_ACQUIRE);
+      return (value ^ __atomic_load_n(&slot->check, __ATOMIC_ACQUIRE)) == number;
+    };
+    for (unsigned spin = 1; !arrived(); spin++)
+    {
+      if (spin % 4096 != 0)
+      {
+        __builtin_ia32_pause();
+        continue;
+      }
+      const hipError_t e = hipStreamQuery(s);
+      (void)hipGetLastError();
+      if (e != hipErrorNotReady && (e != hipSuccess || !arrived()))
+        return set_error(AKM_ERR_HIP, "gmres: step state not written: %s",
+                         hipGetErrorString(e));
+    }
+    double v;
+    std::memcpy(&v, &value, sizeof(v));
+    res = static_cast<P>(v);
     return AKM_SUCCESS;
+  }
+
+  //! A new cycle: |x|^2 partials of x; the steps' numbers follow the start's.
+  int sumsq(const P *x)
+  {
+    if (seq != nullptr)
+    {
+      // past every number the cycle before may still publish
+      start_seq = *seq + 1;
+      *seq = start_seq + restart + 1;
+    }
+    finished = -2;
+    gm_sumsq<P><<<ndot, gm_threads, 0, s>>>(n, drows, x, sqp);
+    return check_launch("gmres norm");
   }
 
   //! |x| of a vector that is only read.
   int norm(const P *x, P &out)
   {
-    gm_sumsq<P><<<nblk, gm_threads, 0, s>>>(n, rpb, x, sqp);
-    gm_givens<P><<<1, 64, 0, s>>>(nblk, sqp, h, -1, H, cs, sn, g, P{0}, rotate_always, st);
-    AKM_TRY(check_launch("gmres norm"));
-    AKM_TRY(sync_state());
-    out = hst->nrm;
-    return AKM_SUCCESS;
+    AKM_TRY(sumsq(x));
+    AKM_TRY(finish_step(-1, P{0}));
+    return wait_step(-1, out);
   }
 
-  //! V_0 holds a residual r: g_0 = |r|, V_0 = r / |r|; beta = |r|.
-  int start(P tol, P &beta)
+  //! V_0 holds a residual r: g_0 = |r| and 1/|r| beside it, finished by the
+  //! first step's dot products (or finish_start).
+  int start_async()
   {
-    gm_sumsq<P><<<nblk, gm_threads, 0, s>>>(n, rpb, V, sqp);
-    gm_givens<P><<<1, 64, 0, s>>>(nblk, sqp, h, -1, H, cs, sn, g, tol, rotate_always, st);
+    AKM_TRY(sumsq(V));
+    if (lazy)
+      return AKM_SUCCESS;
+    AKM_TRY(finish_step(-1, P{0}));
     gm_scale<P><<<sblocks, gm_threads, 0, s>>>(n, V, st);
-    AKM_TRY(check_launch("gmres restart"));
-    AKM_TRY(sync_state());
-    beta = hst->inner_res;
-    return AKM_SUCCESS;
+    return check_launch("gmres restart");
   }
-
-  //! start() without the host's wait: the state goes to the last host slot,
-  //! which run_steps reads (with beta_pending) after enqueueing its first
-  //! steps, so the GPU runs on through the round trip.  Needs events.
-  int start_async(P tol)
+  //! start_async, then beta = |r|.
+  int start(P &beta)
   {
-    static_assert(gm_ahead + 1 < gm_slots, "the first steps in flight reach the start's slot");
-    gm_sumsq<P><<<nblk, gm_threads, 0, s>>>(n, rpb, V, sqp);
-    gm_givens<P><<<1, 64, 0, s>>>(nblk, sqp, h, -1, H, cs, sn, g, tol, rotate_always, st);
-    gm_scale<P><<<sblocks, gm_threads, 0, s>>>(n, V, st);
-    AKM_TRY(check_launch("gmres restart"));
-    AKM_HIP(hipMemcpyAsync(hst + (gm_slots - 1), st, sizeof(gm_state<P>),
-                           hipMemcpyDeviceToHost, s));
-    AKM_HIP(hipEventRecord(ready[gm_slots - 1], s));
-    return AKM_SUCCESS;
+    AKM_TRY(start_async());
+    if (finished < -1)
+      AKM_TRY(finish_step(-1, P{0}));
+    return wait_step(-1, beta);
   }
 
-  //! Arnoldi step j: z_j = pre(v_j) (flexible) or v_j, w = op(z_j), CGS
-  //! against V_0..V_j, Givens; est = new residual estimate.
-  int step(int j, std::function<int(const P *, P *)> const &op,
-           std::function<int(const P *, P *)> const *pre, P tol, P &est)
-  {
-    AKM_TRY(launch_step(j, op, pre, tol));
-    return wait_step(j, est);
-  }
-
-  //! Enqueues Arnoldi step j and the copy of its state into host slot j % 2.
+  //! Enqueues Arnoldi step j: z_j = pre(v_j) (flexible) or v_j, w = op(z_j),
+  //! CGS against V_0..V_j, and beside it what is left of the step before.
   int launch_step(int j, std::function<int(const P *, P *)> const &op,
                   std::function<int(const P *, P *)> const *pre, P tol)
   {
@@ -720,62 +855,55 @@ struct gm_cycle
     }
     AKM_TRY(op(zj, w));
     const int ncols = j + 1;
-    dim3 grid(nblk, (ncols + gm_cols - 1) / gm_cols);
-    gm_dots<P><<<grid, gm_threads, 0, s>>>(n, rpb, V, ldv, w, ncols, dotp);
-    gm_reduce_update<P><<<nblk, gm_threads, sizeof(P) * ncols, s>>>(n, rpb, V, ldv, w, ncols,
-                                                                      dotp, h, sqp);
-    gm_givens_scale<P><<<sblocks, gm_threads, sizeof(P) * (3 * j + 1), s>>>(
-        n, w, nblk, sqp, h, j, H, cs, sn, g, tol, rotate_always, st);
-    AKM_TRY(check_launch("gmres inner iteration"));
-    AKM_HIP(hipMemcpyAsync(hst + (j % gm_slots), st, sizeof(gm_state<P>),
-                           hipMemcpyDeviceToHost, s));
-    if (ready != nullptr)
-      AKM_HIP(hipEventRecord(ready[j % gm_slots], s));
-    return AKM_SUCCESS;
+    const int extra = (finished < j - 1) ? 1 : 0;
+    const dim3 grid(ndot + extra, (ncols + gm_cols - 1) / gm_cols);
+    gm_dots<P><<<grid, gm_threads, extra * 3 * sizeof(P) * j, s>>>(
+        n, drows, V, ldv, w, ncols, ndot, dotp, arrays(), pending(j - 1, tol));
+    finished = std::max(finished, j - 1);
+    gm_update<P><<<nupd, gm_upd_threads, sizeof(P) * ncols, s>>>(n, urows, V, ldv, w, j, dotp,
+                                                                 ndot, arrays());
+    if (!lazy)
+    {
+      AKM_TRY(finish_step(j, tol));
+      gm_scale<P><<<sblocks, gm_threads, 0, s>>>(n, w, st);
+    }
+    return check_launch("gmres inner iteration");
   }
 
   //! Arnoldi steps 0, 1, ... until the estimate reaches `stop` or `limit`
-  //! steps ran; count = the steps taken.  With `speculate`, steps j + 1 ..
-  //! j + gm_ahead are enqueued before step j's estimate is read, which keeps
-  //! the GPU busy through the host's round trips.  When step j ends the
-  //! cycle the speculative steps' columns, Hessenberg columns, rotations and
+  //! steps ran; count = the steps taken.  With `speculate`, step j + 1 is
+  //! enqueued before step j's estimate is read (it finishes step j), which
+  //! keeps the GPU busy through the host's round trips.  When step j ends the
+  //! cycle the speculative step's columns, Hessenberg columns, rotations and
   //! g entries are never used (the update reads columns and g entries below
-  //! count only), and the stream runs them before any later work.
+  //! count only), and the stream runs them before any later work.  With
+  //! `beta_pending` the first steps also go out before the start's norm is
+  //! known; when that norm already meets `stop` they are never used (count 0).
   int run_steps(int limit, std::function<int(const P *, P *)> const &op,
                 std::function<int(const P *, P *)> const *pre, P tol, P stop, P &est,
                 int &count, bool speculate, bool beta_pending = false)
   {
-    static_assert(gm_ahead + 1 <= gm_slots, "steps in flight exceed the state slots");
+    // the start and the steps in flight each have a host slot of their own
+    static_assert(gm_ahead + 2 <= gm_slots, "steps in flight exceed the state slots");
+    // without slots the host copies the device state: one step at a time
+    const int depth = (speculate && slots != nullptr) ? gm_ahead + 1 : 1;
     count = 0;
     int launched = 0;
-    const int depth = speculate ? gm_ahead + 1 : 1;
     if (beta_pending)
     {
-      // the first steps go out before the start's residual norm is known;
-      // when that norm already meets `stop` they are never used (count 0)
       while (launched < depth && launched < limit)
         AKM_TRY(launch_step(launched++, op, pre, tol));
-      AKM_HIP(hipEventSynchronize(ready[gm_slots - 1]));
-      est = hst[gm_slots - 1].inner_res;
+      AKM_TRY(wait_step(-1, est));
     }
     while (est > stop && count < limit)
     {
       while (launched < count + depth && launched < limit)
         AKM_TRY(launch_step(launched++, op, pre, tol));
+      if (finished < count)
+        AKM_TRY(finish_step(count, tol));
       AKM_TRY(wait_step(count, est));
       ++count;
     }
-    return AKM_SUCCESS;
-  }
-
-  //! Waits for step j's state; est = its residual estimate.
-  int wait_step(int j, P &est)
-  {
-    if (ready != nullptr)
-      AKM_HIP(hipEventSynchronize(ready[j % gm_slots]));
-    else
-      AKM_HIP(hipStreamSynchronize(s));
-    est = hst[j % gm_slots].inner_res;
     return AKM_SUCCESS;
   }
 
@@ -784,10 +912,18 @@ struct gm_cycle
   {
     if (m <= 0)
       return AKM_SUCCESS;
-    const size_t hbytes = sizeof(P) * (size_t(m) * (m + 1) / 2);
-    const int h_in_lds = (hbytes + sizeof(P) * m <= 48 * 1024) ? 1 : 0;
-    gm_backsolve<P><<<1, 256, sizeof(P) * m + (h_in_lds ? hbytes : 0), s>>>(m, H, g, h_in_lds);
-    gm_xupdate<P><<<sblocks, gm_threads, sizeof(P) * m, s>>>(n, flexible ? Z : V, ldv, m, g, x);
+    const P *norms = (lazy && !flexible) ? inv : nullptr;
+    if (m <= wave_size)
+      gm_backsolve_wave<P><<<1, wave_size, 0, s>>>(m, H, g, norms);
+    else
+    {
+      const size_t hbytes = sizeof(P) * (size_t(m) * (m + 1) / 2);
+      const int h_in_lds = (hbytes + sizeof(P) * m <= 48 * 1024) ? 1 : 0;
+      gm_backsolve<P><<<1, 256, sizeof(P) * m + (h_in_lds ? hbytes : 0), s>>>(m, H, g, h_in_lds,
+                                                                             norms);
+    }
+    gm_xupdate<P><<<nupd, gm_upd_threads, sizeof(P) * m, s>>>(n, urows, flexible ? Z : V, ldv, m,
+                                                              g, x);
     return check_launch("gmres update");
   }
 };
@@ -808,13 +944,13 @@ static int gmres_outer(gm_cycle<P> &cyc, R &&residual,
   {
     AKM_TRY(residual(outer, speculate));
     ++total;
-    // with events the host reads the start's norm only once the first
+    // with host slots the host reads the start's norm only once the first
     // steps are enqueued
-    const bool pending = cyc.ready != nullptr;
+    const bool pending = cyc.slots != nullptr;
     if (pending)
-      AKM_TRY(cyc.start_async(tol));
+      AKM_TRY(cyc.start_async());
     else
-      AKM_TRY(cyc.start(tol, inner_res));
+      AKM_TRY(cyc.start(inner_res));
     int inner = 0;
     AKM_TRY(cyc.run_steps(restart, op, nullptr, tol, tol, inner_res, inner, speculate, pending));
     total += inner;
@@ -831,8 +967,8 @@ static int gmres_outer(gm_cycle<P> &cyc, R &&residual,
 }
 
 //! The solve of akm_gmres_euler on device vectors in the memory `mem`.
-//! Without events in `mem` the host waits for the whole stream after every
-//! step, and no step is enqueued ahead.
+//! Without host slots in `mem` the host waits for the whole stream after
+//! every step, and no step is enqueued ahead.
 template<typename P>
 static int gmres_typed(akm_matrix_s &m, gm_memory const &mem, P dt, P *x, const P *b,
                        int restart, int max_outer, P tol, double *err, int *iterations)
@@ -852,11 +988,11 @@ static int gmres_typed(akm_matrix_s &m, gm_memory const &mem, P dt, P *x, const 
   const std::function<int(const P *, P *)> op = [&](const P *v, P *w) -> int {
     return apply_op(-dt, v, P{0}, w, P{1}, v);
   };
-  // r = b - (I - dt A) x into V_0; the first one is timed (when events are
-  // at hand) to decide whether steps are enqueued ahead
+  // r = b - (I - dt A) x into V_0; the first one is timed (when steps may be
+  // in flight) to decide whether steps are enqueued ahead
   auto residual = [&](int outer, bool &speculate) -> int {
     AKM_HIP(hipMemcpyAsync(V, b, sizeof(P) * n, hipMemcpyDeviceToDevice, s));
-    if (outer == 0 && mem.ready != nullptr)
+    if (outer == 0 && mem.slots != nullptr)
     {
       // the first solve on the handle times its first apply (a host wait);
       // later solves reuse that time
@@ -886,6 +1022,8 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
   auto &ws = *m64.gmres;
   double *Z = (pre != nullptr) ? ws.Z.data() : nullptr;
   gm_cycle<double> cyc(memory_of(ws), n, s, restart, Z, 1);
+  // a preconditioner may be nonlinear: it reads unit vectors
+  cyc.lazy = pre == nullptr;
   double *V = cyc.V;
   const int sblocks = cyc.sblocks;
 
@@ -895,6 +1033,8 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
   };
   std::function<int(const double *, double *)> op32 = [&](const double *v, double *w) -> int {
     ++stats.applies_f32;
+    if (apply_f32_between(*m32, v, -dt, w))
+      return check_launch("gmres fp32 apply");
     gm_to_f32<<<sblocks, gm_threads, 0, s>>>(n, v, ws.v32.data());
     AKM_TRY(check_launch("gmres fp32 cast"));
     AKM_TRY(apply_device(*m32, 1.0, ws.v32.data(), 0.0, ws.y32.data(), 0.0, nullptr));
@@ -911,7 +1051,7 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     AKM_HIP(hipMemcpyAsync(V, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     ++stats.applies_f64;
     AKM_TRY(apply_device(m64, dt, x, 1.0, V, -1.0, x));
-    return cyc.start(0.0, beta);
+    return cyc.start(beta);
   };
 
   double bnorm = 0;
@@ -940,7 +1080,7 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     AKM_TRY(timed_on_stream(s, [&]() { return op32(x, V); }, first_ms));
     gm_rsub<double><<<sblocks, gm_threads, 0, s>>>(n, b, V);
     AKM_TRY(check_launch("gmres residual"));
-    AKM_TRY(cyc.start(0.0, beta));
+    AKM_TRY(cyc.start(beta));
   }
   else
   {
@@ -948,7 +1088,7 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     ++stats.applies_f64;
     AKM_TRY(timed_on_stream(s, [&]() { return apply_device(m64, dt, x, 1.0, V, -1.0, x); },
                             first_ms));
-    AKM_TRY(cyc.start(0.0, beta));
+    AKM_TRY(cyc.start(beta));
   }
   // speculative steps pay off when a step's operator is cheap next to the
   // host round trip; the preconditioner (if any) runs in every step too
@@ -1013,11 +1153,13 @@ static int size_workspace(akm_gmres_workspace &ws, int64_t n, int restart, size_
   AKM_TRY(ws.state.allocate(sizeof(gm_state<double>)));
   AKM_TRY(ws.xb.allocate(2 * n * int64_t(esize)));
   if (ws.host_state == nullptr)
-    AKM_HIP(hipHostMalloc(&ws.host_state, gm_slots * sizeof(gm_state<double>),
-                          hipHostMallocDefault));
-  for (auto &e : ws.state_ready)
-    if (e == nullptr)
-      AKM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  {
+    // coherent: a running kernel's stores are seen by the polling host
+    AKM_HIP(hipHostMalloc(reinterpret_cast<void **>(&ws.host_state),
+                          gm_slots * sizeof(gm_host_state), hipHostMallocCoherent));
+    for (int i = 0; i < gm_slots; i++)
+      ws.host_state[i] = gm_host_state{};
+  }
   // buffers of the flexible / mixed solver are sized on first use
   ws.Z.reset();
   ws.xprev.reset();
@@ -1201,7 +1343,7 @@ constexpr int noalloc_max_devices = 64;
 struct noalloc_slot
 {
   void *dev = nullptr;
-  alignas(64) unsigned char host[gm_slots * sizeof(gm_state<double>)];
+  alignas(64) unsigned char host[sizeof(gm_state<double>)];
 };
 static noalloc_slot noalloc_slots[noalloc_max_devices];
 static std::mutex noalloc_mtx;
@@ -1217,7 +1359,7 @@ static int64_t noalloc_bytes(int64_t n, int restart, size_t esize)
 }
 
 //! The solve's memory carved from the current GPU's scratch array, resolving
-//! its address on the first call on that GPU.  No events: the host waits for
+//! its address on the first call on that GPU.  No host slots: the host waits for
 //! the whole stream after every step and no step is enqueued ahead.
 static int noalloc_memory(int64_t n, int restart, size_t esize, gm_memory &mem)
 {
@@ -1245,7 +1387,6 @@ static int noalloc_memory(int64_t n, int restart, size_t esize, gm_memory &mem)
   mem.work = base + vbytes;
   mem.state = base + vbytes + wbytes;
   mem.host_state = slot.host;
-  mem.ready = nullptr;
   return AKM_SUCCESS;
 }
 } // namespace akm

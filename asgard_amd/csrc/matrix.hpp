@@ -108,6 +108,10 @@ int waves_per_row(akm_matrix_s const &m);
 //! `jacobi` is set.
 int global_apply(akm_matrix_s &m, double alpha, const void *x, double beta, void *y,
                  double gamma, const void *xg, bool jacobi, double jdt);
+//! w = v + c * fp64(A fp32(v)) of an FP32 operator in one launch on FP64
+//! vectors, when its form has one (a fibre walk of one stage); false, with
+//! nothing enqueued, otherwise.
+bool apply_f32_between(akm_matrix_s &m, const double *v, double c, double *w);
 //! Global operator: new factor values (same vA layout), Jacobi diagonal rebuilt.
 int global_update(akm_matrix_s &m, const void *vA);
 //! Global operator: Jacobi diagonal rebuilt on the device from the stored
