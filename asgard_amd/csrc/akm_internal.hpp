@@ -124,6 +124,7 @@ struct batch_system;
 //! systems with the same (D, n); `grid` persistent workgroups.
 int launch_rows_batch(int D, int n, int waves, const kron_args<double> *args,
                       const batch_system *sys, const int2 *work, int nwork, int grid,
-                      const int *jcol, const int *active, int phase, hipStream_t stream);
+                      const int *jcol, int joff, int limit, const int *active, int phase,
+                      hipStream_t stream);
 
 } // namespace akm

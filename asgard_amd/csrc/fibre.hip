@@ -166,20 +166,18 @@ __device__ __forceinline__ void fl_store(fl_args<P, X> const &a, int vec, int64_
   a.y[pos] = out;
 }
 
-//! One stage: a workgroup's slots, then each cell's slot partials added in
-//! slot order.  A slot whose pieces act in several dimensions takes a round
-//! per dimension.  LDS: NT values per thread.
-template<typename P, int NT, typename X = P>
-__global__ void __launch_bounds__(1024) fl_stage(fl_args<P, X> a, int group0)
+//! One workgroup's slots, then each cell's slot partials added in slot order.
+//! A slot whose pieces act in several dimensions takes a round per dimension.
+//! LDS: NT values per thread.
+template<typename P, int NT, typename X>
+__device__ __forceinline__ void fl_group(fl_args<P, X> const &a, int64_t group, P *ex)
 {
-  extern __shared__ __align__(16) unsigned char fl_smem[];
-  P *ex = reinterpret_cast<P *>(fl_smem);
   const int tpb = blockDim.x, t = threadIdx.x, N = a.N;
   const int slot = t / N;
   const int e = t - slot * N;
   const bool mine = slot < a.nslot;
   // idle lanes read slot 0's record and store nothing
-  const int4 *rec = a.slots + (int64_t(group0 + blockIdx.x) * a.nslot + (mine ? slot : 0)) * 7;
+  const int4 *rec = a.slots + (group * a.nslot + (mine ? slot : 0)) * 7;
   const int4 head = rec[0], tail = rec[1];
   int4 ph = rec[2];
   int4 ent[fl_piece / 2] = {rec[3], rec[4], rec[5], rec[6]};
@@ -216,10 +214,19 @@ __global__ void __launch_bounds__(1024) fl_stage(fl_args<P, X> a, int group0)
         next += 5;
         more--;
       }
-      if (__any(len > fl_piece / 2))
-        fl_connections<P, X, NT, fl_piece>(in, a.tab + s * NT, N, len, cur, c);
+      const P *tab = a.tab + s * NT;
+      if (NT == 4)
+      {
+        // eight blocks' columns of four values do not fit the registers
+        fl_connections<P, X, NT, fl_piece / 2>(in, tab, N, len, cur, c);
+        if (__any(len > fl_piece / 2))
+          fl_connections<P, X, NT, fl_piece / 2>(in, tab, N, len - fl_piece / 2,
+                                                 cur + fl_piece / 4, c);
+      }
+      else if (__any(len > fl_piece / 2))
+        fl_connections<P, X, NT, fl_piece>(in, tab, N, len, cur, c);
       else
-        fl_connections<P, X, NT, fl_piece / 2>(in, a.tab + s * NT, N, len, cur, c);
+        fl_connections<P, X, NT, fl_piece / 2>(in, tab, N, len, cur, c);
     }
     // lane e holds shares of the rows of its fibre: row r's entry is e with
     // its digit s replaced by r
@@ -256,6 +263,57 @@ __global__ void __launch_bounds__(1024) fl_stage(fl_args<P, X> a, int group0)
       sum += ex[r * tpb + t + i * N];
   }
   fl_store(a, head.z, int64_t(head.x) * N + e, sum);
+}
+
+//! One stage: a workgroup per group of slots from group0 on.
+template<typename P, int NT, int TPB, typename X>
+__global__ void __launch_bounds__(TPB) fl_stage(fl_args<P, X> a, int group0)
+{
+  extern __shared__ __align__(16) unsigned char fl_smem[];
+  fl_group<P, NT, X>(a, group0 + blockIdx.x, reinterpret_cast<P *>(fl_smem));
+}
+
+//! The single stage of every system of a batch: workgroup b takes group
+//! items[b].y of system items[b].x.  Phase 0 forms the residual of every active
+//! system, V[0] = b - (I - dt A) x (V[0] holds b on entry); phase 1 applies
+//! the implicit operator to Krylov column j = *jcol + joff < limit, V[j+1] =
+//! (I - dt A) V[j].
+//! Workgroups of 1024 threads serve tensors of 65 entries on, which in a
+//! batch have n = 3.
+template<int TPB>
+__global__ void __launch_bounds__(TPB)
+    fl_batch(const fibre_system *__restrict__ fs, const int2 *__restrict__ items,
+             const int *jcol, int joff, int limit, const int *active, int phase)
+{
+  extern __shared__ __align__(16) unsigned char fl_smem[];
+  double *ex = reinterpret_cast<double *>(fl_smem);
+  const int2 item = items[blockIdx.x];
+  // the same in every lane: the system's record is read by scalar loads
+  const int s = __builtin_amdgcn_readfirstlane(item.x);
+  const int j = *jcol + joff;
+  const fibre_system f = fs[s];
+  if (active[s] == 0 || (phase != 0 && j >= limit))
+    return;
+  fl_args<double> a{};
+  a.slots = f.slots;
+  a.pieces = f.pieces;
+  a.tab = f.tab;
+  a.N = f.N;
+  a.nslot = f.nslot;
+  a.identities = f.identities;
+  a.x = (phase == 0) ? f.X : f.V + int64_t(j) * f.size;
+  a.y = (phase == 0) ? f.V : f.V + int64_t(j + 1) * f.size;
+  a.xg = a.x;
+  a.alpha = (phase == 0) ? f.dt : -f.dt;
+  a.beta = (phase == 0) ? 1.0 : 0.0;
+  a.gamma = (phase == 0) ? -1.0 : 1.0;
+  const int64_t group = __builtin_amdgcn_readfirstlane(item.y);
+  if (TPB == 1024 || f.n == 3)
+    fl_group<double, 3, double>(a, group, ex);
+  else if (f.n == 2)
+    fl_group<double, 2, double>(a, group, ex);
+  else
+    fl_group<double, 4, double>(a, group, ex);
 }
 
 //! One stage for n > 4 or N > 1024: a workgroup per job, its threads over the
@@ -802,14 +860,14 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
 
 //! Rebuilds the factor tables when vA changed since they were built.
 template<typename P>
-static int fibre_tables(akm_matrix_s &m, fibre_plan &plan)
+static int fibre_tables(akm_matrix_s const &m, fibre_plan &plan, hipStream_t stream)
 {
   if (plan.tab_valid && plan.stamp == m.vA_stamp)
     return AKM_SUCCESS;
   const int nn = m.n * m.n;
   const int64_t count = int64_t(plan.nconn + 2 * plan.M) * nn * plan.ntab + nn;
   const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
-  fl_tables<P><<<static_cast<unsigned>(blocks), 256, 0, m.stream>>>(
+  fl_tables<P><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(
       reinterpret_cast<const P *>(m.vA.data()), plan.tab_ptr.data(), plan.tab_src.data(),
       plan.c1_diag.data(), plan.ntab, plan.nconn, plan.M, m.n, m.d, m.T,
       reinterpret_cast<P *>(plan.tab.data()));
@@ -841,20 +899,25 @@ static int launch_stage(akm_matrix_s const &m, fibre_plan const &plan,
 {
   const dim3 grid(static_cast<unsigned>(st.groups)), tpb(static_cast<unsigned>(plan.tpb));
   const size_t lds = sizeof(P) * plan.tpb * m.n;
+  auto go = [&](auto small, auto large) {
+    if (plan.tpb == 256)
+      small<<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+    else
+      large<<<grid, tpb, lds, m.stream>>>(a, st.first_group);
+    return check_launch("fibre stage");
+  };
   if (m.n == 2)
-    fl_stage<P, 2, X><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
-  else if (m.n == 3)
-    fl_stage<P, 3, X><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
-  else
-    fl_stage<P, 4, X><<<grid, tpb, lds, m.stream>>>(a, st.first_group);
-  return check_launch("fibre stage");
+    return go(fl_stage<P, 2, 256, X>, fl_stage<P, 2, 1024, X>);
+  if (m.n == 3)
+    return go(fl_stage<P, 3, 256, X>, fl_stage<P, 3, 1024, X>);
+  return go(fl_stage<P, 4, 256, X>, fl_stage<P, 4, 1024, X>);
 }
 
 template<typename P>
 int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, P *y, P gamma,
                 const P *xg, const double *pc, double jdt)
 {
-  AKM_TRY(fibre_tables<P>(m, plan));
+  AKM_TRY(fibre_tables<P>(m, plan, m.stream));
   fl_args<P> a = fibre_args<P, P>(m, plan);
   a.x = x;
   a.y = y;
@@ -878,10 +941,36 @@ int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, 
   return AKM_SUCCESS;
 }
 
+int fibre_refresh(akm_matrix_s const &m, fibre_plan &plan, hipStream_t stream)
+{
+  return fibre_tables<double>(m, plan, stream);
+}
+
+fibre_system fibre_batch_system(akm_matrix_s const &m, fibre_plan const &plan, double *V,
+                                double *X, int64_t size, double dt)
+{
+  const fl_args<double> a = fibre_args<double, double>(m, plan);
+  return fibre_system{a.slots, a.pieces, a.tab, V, X, size, dt, a.n, a.N, a.nslot, a.identities};
+}
+
+int launch_fibre_batch(int tpb, int groups, const fibre_system *fs, const int2 *items,
+                       const int *jcol, int joff, int limit, const int *active, int phase,
+                       hipStream_t stream)
+{
+  if (groups <= 0)
+    return AKM_SUCCESS;
+  const size_t lds = sizeof(double) * tpb * 4;
+  if (tpb == 256)
+    fl_batch<256><<<groups, 256, lds, stream>>>(fs, items, jcol, joff, limit, active, phase);
+  else
+    fl_batch<1024><<<groups, 1024, lds, stream>>>(fs, items, jcol, joff, limit, active, phase);
+  return check_launch("batched fibre walk");
+}
+
 bool fibre_apply_between(akm_matrix_s &m, fibre_plan &plan, const double *v, double c, double *w)
 {
   if (!plan.built || !plan.slots_of_lanes || plan.stages.size() != 1 || plan.vectors != 0 ||
-      fibre_tables<float>(m, plan) != AKM_SUCCESS)
+      fibre_tables<float>(m, plan, m.stream) != AKM_SUCCESS)
     return false;
   fl_args<float, double> a = fibre_args<float, double>(m, plan);
   a.x = v;

@@ -84,6 +84,29 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
                      std::vector<std::vector<int>> const &term_act,
                      std::vector<int> const &c1_diag, fibre_plan &plan);
 
+//! A single-stage FP64 plan and its system's vectors (Krylov basis, solution,
+//! size, time step) as the batch kernel reads them.
+struct fibre_system
+{
+  const int4 *slots, *pieces;
+  const double *tab;
+  double *V, *X;
+  int64_t size;
+  double dt;
+  int n, N, nslot, identities;
+};
+fibre_system fibre_batch_system(akm_matrix_s const &m, fibre_plan const &plan, double *V,
+                                double *X, int64_t size, double dt);
+//! Rebuilds an FP64 plan's factor tables on `stream` when vA changed.
+int fibre_refresh(akm_matrix_s const &m, fibre_plan &plan, hipStream_t stream);
+//! One workgroup of tpb threads per (system, group) of `items`.
+int launch_fibre_batch(int tpb, int groups, const fibre_system *fs, const int2 *items,
+                       const int *jcol, int joff, int limit, const int *active, int phase,
+                       hipStream_t stream);
+//! The plan of a sparse-grid FP64 matrix for a batch: true when its factored
+//! form runs in one stage.
+bool factored_batch_plan(akm_matrix_s const &m, fibre_plan &plan, int &rc);
+
 //! (lane, connection) steps of one apply of the plan, without building it.
 int64_t fibre_lanes(akm_matrix_s const &m, std::vector<gk_lists> const &lists,
                     std::vector<std::vector<int>> const &term_act);

@@ -1427,6 +1427,19 @@ static int need_fibre_plan(akm_matrix_s &m)
                           g.c1_diag_h, g.fl);
 }
 
+bool factored_batch_plan(akm_matrix_s const &m, fibre_plan &plan, int &rc)
+{
+  rc = AKM_SUCCESS;
+  // (the batch kernel's forms: n = 3 alone past 64 entries a cell)
+  if (!m.factored || !m.gk || m.prec != AKM_F64 || m.gk->max_stages > 1 || m.n < 2 || m.n > 4 ||
+      m.N > (m.n == 3 ? 1024 : 64))
+    return false;
+  akm_global_s const &g = *m.gk;
+  rc = build_fibre_plan(m, g.active_cells, g.cells, g.elem_host.data(), g.lists, g.term_act,
+                        g.c1_diag_h, plan);
+  return rc == AKM_SUCCESS;
+}
+
 int64_t global_flops(akm_matrix_s const &m) { return m.gk ? m.gk->flops : 0; }
 
 int global_layout(akm_matrix_s const &m)
@@ -2497,6 +2510,7 @@ int factored_refresh(akm_matrix_s &m, const void *values)
   }
   if (!finite)
   {
+    m.form_stamp += m.factored ? 1 : 0;
     m.factored = false;
     return AKM_SUCCESS;
   }
@@ -2507,6 +2521,7 @@ int factored_refresh(akm_matrix_s &m, const void *values)
     covered = mask[i] <= m.factored_mask[i];
   if (covered)
   {
+    m.form_stamp += m.factored ? 0 : 1;
     m.factored = true;
     return AKM_SUCCESS;
   }
@@ -2521,6 +2536,7 @@ int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem, std::vect
   m.gk.reset();
   m.factored = false;
   m.factored_mask = mask;
+  m.form_stamp++;
   int widest = 0;
   for (int t = 0; t < m.T; t++)
     widest = std::max(widest, static_cast<int>(std::count(mask.begin() + t * m.d,

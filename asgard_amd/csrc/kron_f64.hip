@@ -37,9 +37,11 @@ namespace akm
 {
 int launch_rows_batch(int D, int n, int waves, const kron_args<double> *args,
                       const batch_system *sys, const int2 *work, int nwork, int grid,
-                      const int *jcol, const int *active, int phase, hipStream_t stream)
+                      const int *jcol, int joff, int limit, const int *active, int phase,
+                      hipStream_t stream)
 {
-  return launch_rows_batch_impl(D, n, waves, args, sys, work, nwork, grid, jcol, active, phase,
+  return launch_rows_batch_impl(D, n, waves, args, sys, work, nwork, grid, jcol, joff, limit,
+                                active, phase,
                                 stream);
 }
 } // namespace akm

@@ -580,7 +580,7 @@ bool launch_with_lds(K kern, size_t lds)
 //! sparse-grid operators with the same (d, n): workgroup b takes items b,
 //! b + gridDim.x, ...  Phase 0 forms the residual of every active system,
 //! V_s[0] = b_s - (I - dt_s A_s) x_s (V_s[0] holds b_s on entry); phase 1
-//! applies the implicit operator to the current Krylov column j = *jcol,
+//! applies the implicit operator to Krylov column j = *jcol + joff < limit,
 //! V_s[j+1] = (I - dt_s A_s) V_s[j].
 // Two wavefronts per SIMD: the persistent loop would otherwise take ~300
 // VGPRs at d=5 n=3 (one wavefront per SIMD); the few spills this costs
@@ -588,7 +588,7 @@ bool launch_with_lds(K kern, size_t lds)
 template<int D, int n, int g, int W>
 __global__ void __launch_bounds__(W *wave_size) __attribute__((amdgpu_waves_per_eu(2)))
 kron_rows_batch(const kron_args<double> *args, const batch_system *sys, const int2 *work,
-                int nwork, const int *jcol, const int *active, int phase)
+                int nwork, const int *jcol, int joff, int limit, const int *active, int phase)
 {
   constexpr int N = ipow<n, D>::value;
   constexpr int CPW = wave_size / ipow<n, g>::value;
@@ -615,9 +615,12 @@ kron_rows_batch(const kron_args<double> *args, const batch_system *sys, const in
     }
     else
     {
-      const double *xj = v.V + int64_t(*jcol) * v.n;
+      const int j = *jcol + joff;
+      if (j >= limit)
+        return; // the same in every workgroup
+      const double *xj = v.V + int64_t(j) * v.n;
       a.x = xj;
-      a.y = v.V + int64_t(*jcol + 1) * v.n;
+      a.y = v.V + int64_t(j + 1) * v.n;
       a.xg = xj;
       a.alpha = -v.dt;
       a.beta = 0.0;
@@ -1092,7 +1095,8 @@ int launch_kronmult_impl(int D, int n, int mode, kron_args<P> const &a, int num_
 
 template<int D, int n, int W>
 bool launch_rows_batch_w(const kron_args<double> *args, const batch_system *sys, const int2 *work,
-                         int nwork, int grid, const int *jcol, const int *active, int phase,
+                         int nwork, int grid, const int *jcol, int joff, int limit,
+                         const int *active, int phase,
                          hipStream_t stream)
 {
   constexpr int g = lead_dims<double>(D, n);
@@ -1106,7 +1110,8 @@ bool launch_rows_batch_w(const kron_args<double> *args, const batch_system *sys,
     auto kern = kron_rows_batch<D, n, g, W>;
     if (!launch_with_lds(kern, lds))
       return false;
-    kern<<<grid, W * wave_size, lds, stream>>>(args, sys, work, nwork, jcol, active, phase);
+    kern<<<grid, W * wave_size, lds, stream>>>(args, sys, work, nwork, jcol, joff, limit, active,
+                                               phase);
     return true;
   }
 }
@@ -1114,20 +1119,29 @@ bool launch_rows_batch_w(const kron_args<double> *args, const batch_system *sys,
 template<int D, int n>
 bool launch_rows_batch_dn(int waves, const kron_args<double> *args, const batch_system *sys,
                           const int2 *work, int nwork, int grid, const int *jcol,
-                          const int *active, int phase, hipStream_t stream)
+                          int joff, int limit, const int *active, int phase, hipStream_t stream)
 {
   switch (waves)
   {
-  case 1: return launch_rows_batch_w<D, n, 1>(args, sys, work, nwork, grid, jcol, active, phase, stream);
-  case 2: return launch_rows_batch_w<D, n, 2>(args, sys, work, nwork, grid, jcol, active, phase, stream);
-  case 8: return launch_rows_batch_w<D, n, 8>(args, sys, work, nwork, grid, jcol, active, phase, stream);
-  default: return launch_rows_batch_w<D, n, 4>(args, sys, work, nwork, grid, jcol, active, phase, stream);
+  case 1:
+    return launch_rows_batch_w<D, n, 1>(args, sys, work, nwork, grid, jcol, joff, limit, active,
+                                        phase, stream);
+  case 2:
+    return launch_rows_batch_w<D, n, 2>(args, sys, work, nwork, grid, jcol, joff, limit, active,
+                                        phase, stream);
+  case 8:
+    return launch_rows_batch_w<D, n, 8>(args, sys, work, nwork, grid, jcol, joff, limit, active,
+                                        phase, stream);
+  default:
+    return launch_rows_batch_w<D, n, 4>(args, sys, work, nwork, grid, jcol, joff, limit, active,
+                                        phase, stream);
   }
 }
 
 inline int launch_rows_batch_impl(int D, int n, int waves, const kron_args<double> *args,
                                   const batch_system *sys, const int2 *work, int nwork, int grid,
-                                  const int *jcol, const int *active, int phase,
+                                  const int *jcol, int joff, int limit, const int *active,
+                                  int phase,
                                   hipStream_t stream)
 {
   if (nwork == 0)
@@ -1135,8 +1149,8 @@ inline int launch_rows_batch_impl(int D, int n, int waves, const kron_args<doubl
   bool done = false;
 #define AKM_BCASE(DD, NN)                                                                          \
   if (!done && D == DD && n == NN)                                                                 \
-    done = launch_rows_batch_dn<DD, NN>(waves, args, sys, work, nwork, grid, jcol, active, phase,  \
-                                        stream);
+    done = launch_rows_batch_dn<DD, NN>(waves, args, sys, work, nwork, grid, jcol, joff, limit,    \
+                                        active, phase, stream);
   AKM_BCASE(1, 2) AKM_BCASE(1, 3) AKM_BCASE(1, 4)
   AKM_BCASE(2, 2) AKM_BCASE(2, 3) AKM_BCASE(2, 4)
   AKM_BCASE(3, 2) AKM_BCASE(3, 3) AKM_BCASE(3, 4)

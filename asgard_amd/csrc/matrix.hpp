@@ -74,6 +74,8 @@ struct akm_matrix_s
   // sparse-grid handles: the operator runs one dimension at a time (gk)
   // instead of pair by pair, because its factors allow it
   bool factored = false;
+  // advanced when the form or the products it was built for change
+  uint64_t form_stamp = 0;
   bool pair_kernels = false;        // the caller asked for the pair kernels
   // held while a factored apply is enqueued: its launches share work vectors,
   // so two threads' applies follow each other on the stream

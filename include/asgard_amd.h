@@ -425,9 +425,11 @@ akm_status akm_gmres_euler_mixed(akm_matrix mat, akm_matrix mat32, akm_precond p
  * simple_gmres_euler each).  A batch of independent implicit steps
  * (I - dt_s A_s) x_s = b_s over FP64 sparse-grid matrices of any sizes and
  * (d, n) (n in 2..4; d <= 6 with n = 2, d <= 5 with n = 3, d <= 3 with
- * n = 4): restarted GMRES(restart) in lockstep, every operator apply one
- * persistent launch per (d, n) group over a (system, row) work list, every
- * restart cycle three hipGraphs (start, Arnoldi iteration, update).  The
+ * n = 4): restarted GMRES(restart) in lockstep; operators that run one
+ * dimension at a time (akm_create_sparse_grid, one non-identity factor per
+ * term) are applied together, the others by one persistent launch per (d, n)
+ * group over a (system, row) work list; every restart cycle is three
+ * hipGraphs (start, eight Arnoldi iterations, update).  The
  * matrices must outlive the batch and keep their coefficients. */
 typedef struct akm_batch_s *akm_batch;
 
@@ -438,7 +440,8 @@ akm_status akm_batch_create(int count, const akm_matrix *mats, const double *dts
                             akm_batch *batch);
 
 /* restart used, number of (d, n) groups and each group's wavefronts per row
- * (group_waves has num_groups entries; groups ordered by (d, n)). */
+ * (group_waves has num_groups entries; groups ordered by (d, n); 1 when all
+ * its systems run one dimension at a time). */
 akm_status akm_batch_info(akm_batch batch, int *restart, int *num_groups, int *group_waves);
 
 /* Solves every system to |b_s - (I - dt_s A_s) x_s| <= tol*|b_s| (true FP64

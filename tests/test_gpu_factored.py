@@ -187,3 +187,39 @@ def test_autotuned_small_and_large_agree():
     ref = torch.zeros_like(x)
     m.apply(1.0, x, 0.0, ref)
     assert close(y.cpu().numpy(), ref.cpu().numpy(), np.float64)
+
+
+def test_batch_mixes_both_ways_of_applying():
+    """Systems along fibres (workgroups of 256, 512 and 1024 threads) and pair
+    by pair in one batch, across a restart and after new factors."""
+    rng = np.random.default_rng(17)
+    shapes = [(2, 2, 5, True, [(0,), (1,)]), (4, 3, 3, True, [(0,), (3,)]),
+              (5, 3, 2, False, [(4,), (0,)]), (3, 4, 3, False, [(1,)]),
+              (3, 2, 4, True, [(0, 2), (1,)]), (2, 3, 4, False, [(0, 1)])]
+    mats, problems = [], []
+    for d, n, level, refine, active in shapes:
+        table, top = tables(d, level, refine)
+        ops = [0.05 * o if not np.array_equal(o, np.eye(len(o))) else o
+               for o in factors(rng, d, n, top, active)]
+        vA = grid.build_vA(d, n, len(active), top, ops)
+        mats.append(asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, len(active), vA))
+        problems.append((d, n, table, top, len(active), vA))
+    dt = 0.05
+    batch = asgard_amd.BatchSolver(mats, [dt] * len(mats), restart=6)
+    bs = [torch.from_numpy(rng.uniform(-1, 1, m.output_size())).cuda() for m in mats]
+    for step in range(2):
+        xs = [torch.zeros_like(b) for b in bs]
+        res, its, conv = batch.solve(xs, bs, tol=1e-11)
+        assert conv.all() and (res <= 1e-11).all(), res
+        for p, x, b in zip(problems, xs, bs):
+            m = asgard_amd.KronmultMatrix.sparse_grid(*p)
+            m.set_tuning(waves_per_row=4)
+            r = b - m.apply_euler(dt, 1.0, x, 0.0, torch.zeros_like(x))
+            assert float(torch.linalg.norm(r) / torch.linalg.norm(b)) < 2e-11
+        # the first system's second term becomes an identity term and its
+        # first a product in both dimensions (pair by pair on these cells)
+        d, n, table, top, T, _ = problems[0]
+        ops = factors(rng, d, n, top, [(0, 1), ()])
+        vA = grid.build_vA(d, n, T, top, [0.1 * o if i < 2 else o for i, o in enumerate(ops)])
+        mats[0].update_stored_coefficients(vA)
+        problems[0] = (d, n, table, top, T, vA)
