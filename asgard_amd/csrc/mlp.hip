@@ -14,8 +14,11 @@
 //
 // Parameters live as one flat FP32 array
 //   [ W1 (H x K1) | b1 (H) | W2 (H x H) | b2 (H) | W3 (N3 x H) | b3 (N3) ]
-// with every W row-major (output x input).  Training (forward, backward,
-// Adam) runs in FP32 on an LDS-tiled GEMM kernel with fused epilogues; the
+// with every W row-major (output x input).  Training runs in FP32 on the
+// matrix cores (v_mfma_f32_16x16x4_f32: FP32 products and sums): one kernel
+// takes 16 samples through the whole forward and backward chain with their
+// activations in LDS, a second forms every weight and bias gradient, a third
+// adds its row parts; the
 // preconditioner itself runs on BF16 copies of W1..W3 with the MFMA
 // v_mfma_f32_16x16x16_bf16 (FP32 accumulation), one wavefront per 16 cells,
 // activations in LDS.
@@ -30,173 +33,352 @@
 
 namespace akm
 {
-constexpr int mm_tile = 64;    // GEMM output tile (rows and columns)
-constexpr int mm_k = 16;       // GEMM k step
-constexpr int mm_threads = 256;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-enum mm_epilogue
+constexpr int mc_rows = 16;    // samples per workgroup of the chain kernel
+constexpr int mc_waves = 16;   // its wavefronts, which share the output columns
+constexpr int mc_threads = mc_waves * 64;
+constexpr int wg_tile = 32;    // weight-gradient tile (outputs x inputs)
+constexpr int wg_threads = 256; // its four wavefronts split the rows
+constexpr int wg_max_parts = 16;
+
+//! Barrier that orders LDS accesses only: a full one would also wait for the
+//! activations' stores to memory, which no wavefront of the kernel reads.
+__device__ __forceinline__ void mlp_lds_barrier()
 {
-  ep_store = 0,     // C = A B
-  ep_bias = 1,      // C = A B + bias[col]
-  ep_bias_relu = 2, // C = max(A B + bias[col], 0)
-  ep_mask = 3       // C = (A B) * (mask[row, col] > 0)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+//! 16 samples x 16 outputs from j0 on: in (16 x K, LDS, rows ldi apart) times
+//! W^T (outputs x inputs, BACK = false) or times W (BACK = true: inputs x
+//! outputs).  Operands of v_mfma_f32_16x16x4_f32: lane l holds
+//! A[l % 16][l / 16] and B[l / 16][l % 16], and gets D[4 (l / 16) + i][l % 16].
+//! The sum over k may run in any order, so lane group g takes k = 16 b + 4 g
+//! + i in step i: four consecutive inputs, one 16-byte read.  The four steps
+//! have a sum each, added at the end: shorter chains of rounded sums, and no
+//! step waits for the one before.
+template<bool BACK>
+__device__ __forceinline__ f32x4 mlp_tile(const float *in, int ldi, int K, const float *W,
+                                          int ldw, int j0)
+{
+  constexpr int U = 4; // blocks of 16 inputs read ahead
+  f32x4 acc[4] = {};
+  const int lane = threadIdx.x % 64, row = lane % 16, g = lane / 16;
+  const float *arow = in + row * ldi + 4 * g;
+  const float *w = BACK ? W + int64_t(4 * g) * ldw + j0 + row
+                        : W + int64_t(j0 + row) * ldw + 4 * g;
+  // all reads of U blocks in flight; those past K repeat the last block's
+  auto read = [&](int k0, f32x4 (&b)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+    {
+      const int k = min(k0 + 16 * u, K - 16);
+      if constexpr (BACK)
+      {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          b[u][i] = w[int64_t(k + i) * ldw];
+      }
+      else
+        b[u] = *reinterpret_cast<const f32x4 *>(w + k);
+    }
+  };
+  f32x4 cur[U], next[U];
+  read(0, cur);
+  for (int k0 = 0; k0 < K; k0 += 16 * U)
+  {
+    read(k0 + 16 * U, next);
+    // the scheduler would move each read to its use
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k0 + 16 * u < K)
+      {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(arow + k0 + 16 * u);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], cur[u][i], acc[i], 0, 0, 0);
+      }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      cur[u] = next[u];
+  }
+  return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
+
+//! One layer for the workgroup's 16 samples: put(sample, output, values of
+//! this and the next three samples) for every output of J (a multiple of 16).
+//! Wavefronts take every mc_waves-th tile of 16 outputs.
+template<bool BACK, typename Put>
+__device__ __forceinline__ void mlp_layer(const float *in, int ldi, int K, const float *W,
+                                          int ldw, int J, Put &&put)
+{
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+#pragma nounroll
+  for (int j0 = 16 * wave; j0 < J; j0 += 16 * mc_waves)
+    put(4 * (lane / 16), j0 + lane % 16, mlp_tile<BACK>(in, ldi, K, W, ldw, j0));
+}
+
+//! Shapes, parameters and buffers of a training pass.
+struct mlp_pass
+{
+  int64_t rows;
+  int N, N3, K1, H;
+  const float *W1, *b1, *W2, *b2, *W3, *b3;
+  const float *X, *T;
+  float *H1, *H2, *O, *dO, *dH2, *dH1;
+  float scale;     // of the output gradient
+  double *partial; // per workgroup: sum of (O - T)^2
 };
 
-//! C[m, c] = sum_k A(m, k) B(k, c) with A(m, k) = A[m*sam + k*sak] and
-//! B(k, c) = B[k*sbk + c*sbn], then the epilogue.  64 x 64 tile per block,
-//! 4 x 4 outputs per thread, k in steps of 16 through LDS.
-template<int EP>
-__global__ void __launch_bounds__(mm_threads)
-mlp_gemm(int M, int N, int K, const float *A, int64_t sam, int64_t sak, const float *B,
-         int64_t sbk, int64_t sbn, float *C, int64_t ldc, const float *bias, const float *mask,
-         int64_t ldm, int kchunk, int64_t zstride)
+//! 16 samples through the layers (H1, H2, O to memory), and with BACK back
+//! again: dO = scale (O - T) on the first N of N3 outputs, dH2, dH1.
+//! What bounds it: the weights' way from L2, which every workgroup reads whole;
+//! with the products taken out the 256 x 256 layer takes as long (10 us), with
+//! the reads taken out half as long, and its matrix-core time is 3.6 us.
+//! 1024 samples of 80 -> 256 -> 256 -> 64 take 30 us (64 workgroups),
+//! 32768 take 260 us; with 8 wavefronts of two tiles each 33 and 311 us.
+//! Separate tiled products took 12-34 us for each of the layers (64 x 64
+//! tiles leave most of the chip idle).
+//! LDS: 16 x (K1 + 2 H + N3 + 16) floats, rows 4 floats apart beyond their
+//! length so that 16-byte reads of 16 rows spread over the banks.
+template<bool BACK>
+__global__ void __launch_bounds__(mc_threads) mlp_chain(mlp_pass p)
 {
-  __shared__ float As[mm_k][mm_tile + 4];
-  __shared__ float Bs[mm_k][mm_tile + 4];
-  const int t = threadIdx.x;
-  const int m0 = blockIdx.y * mm_tile, c0 = blockIdx.x * mm_tile;
-  const int tm = (t / 16) * 4, tc = (t % 16) * 4;
-  // split K: block z sums k in [z*kchunk, min(K, (z+1)*kchunk)) into its own
-  // output slice C + z*zstride
-  const int kb = blockIdx.z * kchunk;
-  const int ke = min(K, kb + kchunk);
-  C += blockIdx.z * zstride;
-  float acc[4][4] = {};
-  for (int k0 = kb; k0 < ke; k0 += mm_k)
+  extern __shared__ __align__(16) float mc_lds[];
+  __shared__ double sh[mc_waves];
+  const int ldx = p.K1 + 4, ldh = p.H + 4, ldo = p.N3 + 4;
+  float *Xs = mc_lds, *A1 = Xs + mc_rows * ldx, *A2 = A1 + mc_rows * ldh,
+        *Os = A2 + mc_rows * ldh;
+  const int64_t r0 = int64_t(blockIdx.x) * mc_rows;
+  const int live = static_cast<int>(min(int64_t(mc_rows), p.rows - r0));
+  for (int e = threadIdx.x; e < mc_rows * p.K1; e += mc_threads)
   {
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-    {
-      const int e = t + mm_threads * q; // 0 .. 1023
-      const int mm = e % mm_tile, kk = e / mm_tile;
-      const int gm = m0 + mm, gk = k0 + kk;
-      As[kk][mm] = (gm < M && gk < ke) ? A[gm * sam + gk * sak] : 0.0f;
-      const int gc = c0 + mm;
-      Bs[kk][mm] = (gc < N && gk < ke) ? B[gk * sbk + gc * sbn] : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < mm_k; kk++)
-    {
-      float a[4], b[4];
+    const int r = e / p.K1, i = e - r * p.K1;
+    Xs[r * ldx + i] = (r < live) ? p.X[(r0 + r) * p.K1 + i] : 0.0f;
+  }
+  mlp_lds_barrier();
+  double sq = 0;
+  auto hidden = [&](const float *in, int K, const float *W, const float *bias, float *keep,
+                    float *out) {
+    mlp_layer<false>(in, K + 4, K, W, K, p.H, [&](int r, int j, f32x4 v) {
+      const float b = bias[j];
 #pragma unroll
       for (int i = 0; i < 4; i++)
       {
-        a[i] = As[kk][tm + i];
-        b[i] = Bs[kk][tc + i];
+        const float x = fmaxf(v[i] + b, 0.0f);
+        keep[(r + i) * ldh + j] = x;
+        if (r + i < live)
+          out[(r0 + r + i) * p.H + j] = x;
       }
+    });
+    mlp_lds_barrier();
+  };
+  hidden(Xs, p.K1, p.W1, p.b1, A1, p.H1);
+  hidden(A1, p.H, p.W2, p.b2, A2, p.H2);
+  mlp_layer<false>(A2, ldh, p.H, p.W3, p.H, p.N3, [&](int r, int j, f32x4 v) {
+    const float b = p.b3[j];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+    {
+      float x = v[i] + b;
+      if constexpr (BACK)
+      {
+        float grad = 0.0f;
+        if (r + i < live && j < p.N)
+        {
+          const float diff = x - p.T[(r0 + r + i) * p.N3 + j];
+          sq += double(diff) * double(diff);
+          grad = p.scale * diff;
+        }
+        Os[(r + i) * ldo + j] = grad;
+        x = grad;
+      }
+      if (r + i < live)
+        (BACK ? p.dO : p.O)[(r0 + r + i) * p.N3 + j] = x;
+    }
+  });
+  if constexpr (BACK)
+  {
+    mlp_lds_barrier();
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      sq += __shfl_xor(sq, off);
+    if (threadIdx.x % 64 == 0)
+      sh[threadIdx.x / 64] = sq;
+    // the masks are the activations, which their gradients replace in LDS
+    auto back = [&](const float *in, int K, const float *W, float *mask, float *out) {
+      mlp_layer<true>(in, K + 4, K, W, p.H, p.H, [&](int r, int j, f32x4 v) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+        {
+          const float x = (mask[(r + i) * ldh + j] > 0.0f) ? v[i] : 0.0f;
+          mask[(r + i) * ldh + j] = x;
+          if (r + i < live)
+            out[(r0 + r + i) * p.H + j] = x;
+        }
+      });
+      mlp_lds_barrier();
+    };
+    back(Os, p.N3, p.W3, A2, p.dH2);
+    back(A2, p.H, p.W2, A1, p.dH1);
+    if (threadIdx.x == 0)
+    {
+      double t = 0;
+      for (int w = 0; w < mc_waves; w++)
+        t += sh[w];
+      p.partial[blockIdx.x] = t;
+    }
+  }
+}
+
+//! One weight gradient dW = G^T Y (G: rows x M, Y: rows x C, dW: M x C) and
+//! its bias gradient (the column sums of G), as a range of tiles.
+struct wg_layer
+{
+  const float *G, *Y;
+  int M, C;
+  int64_t oW, ob; // offsets in the flat gradient
+  int tile0;      // first tile of the layer
+};
+struct wg_args
+{
+  wg_layer layer[3];
+  int64_t rows, chunk; // rows per part
+  int64_t stride;      // values of one part
+  float *out;          // part z of the gradient at out + z * stride
+};
+
+//! A 32 x 32 tile of one layer's gradient over the rows of part blockIdx.y.
+//! The four wavefronts take every fourth 16 rows and their sums meet in LDS
+//! in wavefront order.
+__global__ void __launch_bounds__(wg_threads) mlp_weight_grad(wg_args a)
+{
+  __shared__ float red[4][wg_tile][wg_tile + 1];
+  __shared__ float bred[4][wg_tile];
+  const int tile = blockIdx.x;
+  const int li = (tile >= a.layer[2].tile0) ? 2 : (tile >= a.layer[1].tile0 ? 1 : 0);
+  const wg_layer L = a.layer[li];
+  const int ctiles = (L.C + wg_tile - 1) / wg_tile;
+  const int m0 = (tile - L.tile0) / ctiles * wg_tile, c0 = (tile - L.tile0) % ctiles * wg_tile;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, col = lane % 16, g = lane / 16;
+  const int64_t b0 = blockIdx.y * a.chunk, b1 = min(a.rows, b0 + a.chunk);
+  f32x4 acc[2][2] = {};
+  float bias[2] = {0.0f, 0.0f};
+  // outputs and inputs past the layer's read its first ones and are dropped
+  int mi[2], ci[2];
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+  {
+    mi[t] = (m0 + 16 * t < L.M) ? m0 + 16 * t + col : col;
+    ci[t] = (c0 + 16 * t < L.C) ? c0 + 16 * t + col : col;
+  }
+  // two blocks of 16 rows a round, all reads in flight
+  constexpr int U = 2;
+  for (int64_t b = b0 + 16 * wave; b < b1; b += 64 * U)
+  {
+    float gv[U][2][4], yv[U][2][4];
+#pragma unroll
+    for (int u = 0; u < U; u++)
 #pragma unroll
       for (int i = 0; i < 4; i++)
+      {
+        const int64_t r = b + 64 * u + 4 * g + i;
+        const int64_t rr = (r < b1) ? r : b0;
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
+        for (int t = 0; t < 2; t++)
+        {
+          gv[u][t][i] = L.G[rr * L.M + mi[t]];
+          yv[u][t][i] = L.Y[rr * L.C + ci[t]];
+        }
+      }
+    __builtin_amdgcn_sched_barrier(0); // the reads stay ahead of the products
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+      {
+        const bool live = b + 64 * u + 4 * g + i < b1;
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+        {
+          gv[u][t][i] = live ? gv[u][t][i] : 0.0f;
+          yv[u][t][i] = live ? yv[u][t][i] : 0.0f;
+          bias[t] += gv[u][t][i];
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int v = 0; v < 2; v++)
+            acc[t][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[u][t][i], yv[u][v][i], acc[t][v],
+                                                             0, 0, 0);
+      }
   }
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int t = 0; t < 2; t++)
   {
-    const int gm = m0 + tm + i;
-    if (gm >= M)
-      continue;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-    {
-      const int gc = c0 + tc + j;
-      if (gc >= N)
-        continue;
-      float v = acc[i][j];
-      if constexpr (EP == ep_bias || EP == ep_bias_relu)
-        v += bias[gc];
-      if constexpr (EP == ep_bias_relu)
-        v = fmaxf(v, 0.0f);
-      if constexpr (EP == ep_mask)
-        v = (mask[gm * ldm + gc] > 0.0f) ? v : 0.0f;
-      C[gm * ldc + gc] = v;
-    }
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        red[wave][16 * t + 4 * g + i][16 * u + col] = acc[t][u][i];
+    bias[t] += __shfl_xor(bias[t], 16);
+    bias[t] += __shfl_xor(bias[t], 32);
+    if (g == 0)
+      bred[wave][16 * t + col] = bias[t];
+  }
+  __syncthreads();
+  float *out = a.out + blockIdx.y * a.stride;
+  for (int e = threadIdx.x; e < wg_tile * wg_tile; e += wg_threads)
+  {
+    const int m = e / wg_tile, c = e % wg_tile;
+    if (m0 + m < L.M && c0 + c < L.C)
+      out[L.oW + int64_t(m0 + m) * L.C + c0 + c] =
+          (red[0][m][c] + red[1][m][c]) + (red[2][m][c] + red[3][m][c]);
+  }
+  if (c0 == 0 && threadIdx.x < wg_tile && m0 + static_cast<int>(threadIdx.x) < L.M)
+  {
+    const int m = threadIdx.x;
+    out[L.ob + m0 + m] = (bred[0][m] + bred[1][m]) + (bred[2][m] + bred[3][m]);
   }
 }
 
-//! dO = scale * (O - T) on the first N of N3 columns (0 on the padding);
-//! partial[block] = sum of (O - T)^2 over the block's entries.
+//! grad[e] = sum over z < parts of part[z*count + e] in order (parts = 1: grad
+//! is already complete); the last block adds the `losses` partial losses into
+//! loss[0] (accumulated if `accumulate`), in a fixed order, and stores it to
+//! the host as well.
 __global__ void __launch_bounds__(256)
-mlp_out_grad(int64_t rows, int N, int N3, const float *O, const float *T, float scale, float *dO,
-             double *partial)
+mlp_sum_parts(int64_t count, int parts, const float *part, float *grad, int losses,
+              const double *partial, double *loss, int accumulate, double *host_loss)
 {
   __shared__ double sh[256];
-  double sq = 0;
-  const int64_t total = rows * N3;
-  for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < total; e += 256ll * gridDim.x)
+  if (blockIdx.x + 1 == gridDim.x)
   {
-    const int col = static_cast<int>(e % N3);
-    float g = 0.0f;
-    if (col < N)
+    double s = 0;
+    for (int i = threadIdx.x; i < losses; i += 256)
+      s += partial[i];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1)
     {
-      const float diff = O[e] - T[e];
-      sq += double(diff) * double(diff);
-      g = scale * diff;
+      if (threadIdx.x < k)
+        sh[threadIdx.x] += sh[threadIdx.x + k];
+      __syncthreads();
     }
-    dO[e] = g;
-  }
-  sh[threadIdx.x] = sq;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1)
-  {
-    if (threadIdx.x < s)
-      sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    partial[blockIdx.x] = sh[0];
-}
-
-//! out[0] (+)= sum of partial[0 .. count) (one block, fixed order).
-__global__ void __launch_bounds__(256) mlp_sum(int count, const double *partial, double *out,
-                                               int accumulate)
-{
-  __shared__ double sh[256];
-  double s = 0;
-  for (int i = threadIdx.x; i < count; i += 256)
-    s += partial[i];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1)
-  {
-    if (threadIdx.x < k)
-      sh[threadIdx.x] += sh[threadIdx.x + k];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    out[0] = accumulate ? out[0] + sh[0] : sh[0];
-}
-
-//! partial[z*cols + c] = sum over rows r in chunk z of X[r*ld + c]
-//! (block (x, z): 256 columns of chunk z).
-__global__ void __launch_bounds__(256)
-mlp_colsum_part(int64_t rows, int cols, const float *X, int64_t ld, int64_t chunk,
-                float *partial)
-{
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= cols)
+    if (threadIdx.x == 0)
+    {
+      const double total = accumulate ? loss[0] + sh[0] : sh[0];
+      loss[0] = total;
+      __hip_atomic_store(host_loss, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     return;
-  const int64_t r0 = blockIdx.z * chunk;
-  const int64_t r1 = min(rows, r0 + chunk);
-  float s = 0.0f;
-  for (int64_t r = r0; r < r1; r++)
-    s += X[r * ld + c];
-  partial[int64_t(blockIdx.z) * cols + c] = s;
-}
-
-//! out[e] = sum over z < parts of partial[z*count + e] (fixed order).
-__global__ void __launch_bounds__(256)
-mlp_sum_parts(int64_t count, int parts, const float *partial, float *out)
-{
-  for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < count; e += 256ll * gridDim.x)
+  }
+  for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < count; e += 256ll * (gridDim.x - 1))
   {
-    float s = 0.0f;
-    for (int z = 0; z < parts; z++)
-      s += partial[z * count + e];
-    out[e] = s;
+    float s = part[e];
+    for (int z = 1; z < parts; z++)
+      s += part[z * count + e];
+    grad[e] = s;
   }
 }
 
@@ -285,7 +467,6 @@ mlp_to_bf16(int64_t count, const float *src, unsigned short *dst)
 }
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int mlp_cells_per_wave = 16;
 
@@ -426,13 +607,23 @@ struct akm_mlp_s final : akm_precond_s
   int64_t adam_t = 0;
   // batch buffers (sized for `batch` rows)
   int batch = 0;
-  dev_buffer<float> Xb, Tb, H1, H2, O, dO, dH2, dH1;
-  dev_buffer<float> scratch; // split-K partial products
-  static constexpr int split_parts = 16;
+  dev_buffer<float> Xb, Tb, H1, H2, dO, dH2, dH1;
+  dev_buffer<float> parts; // row parts of the gradient
   dev_buffer<double> partial, loss;
+  double *host_loss = nullptr; // pinned copy of loss[0]
   hipStream_t stream = nullptr;
 
+  ~akm_mlp_s() override
+  {
+    if (host_loss != nullptr)
+      (void)hipHostFree(host_loss);
+  }
+
   int64_t size() const override { return cells * N; }
+
+  static int chain_groups(int B) { return (B + mc_rows - 1) / mc_rows; }
+  //! Row parts of the weight gradients: 128 rows each, at most wg_max_parts.
+  static int row_parts(int B) { return std::clamp(B / 128, 1, wg_max_parts); }
 
   int ensure_batch(int B)
   {
@@ -443,92 +634,84 @@ struct akm_mlp_s final : akm_precond_s
     AKM_TRY(Tb.allocate(int64_t(B) * N3));
     AKM_TRY(H1.allocate(int64_t(B) * H));
     AKM_TRY(H2.allocate(int64_t(B) * H));
-    AKM_TRY(O.allocate(int64_t(B) * N3));
     AKM_TRY(dO.allocate(int64_t(B) * N3));
     AKM_TRY(dH2.allocate(int64_t(B) * H));
     AKM_TRY(dH1.allocate(int64_t(B) * H));
-    AKM_TRY(partial.allocate(4096));
+    AKM_TRY(partial.allocate(chain_groups(B)));
     AKM_TRY(loss.allocate(2));
-    const int64_t widest = std::max<int64_t>({int64_t(H) * K1, int64_t(H) * H, int64_t(N3) * H});
-    AKM_TRY(scratch.allocate(split_parts * widest));
+    if (host_loss == nullptr)
+      AKM_HIP(hipHostMalloc(reinterpret_cast<void **>(&host_loss), sizeof(double),
+                            hipHostMallocDefault));
+    AKM_TRY(parts.allocate(row_parts(B) * num_params));
     return AKM_SUCCESS;
   }
 
-  template<int EP>
-  int gemm(hipStream_t s, int M, int Nc, int K, const float *A, int64_t sam, int64_t sak,
-           const float *B, int64_t sbk, int64_t sbn, float *C, int64_t ldc,
-           const float *bias = nullptr, const float *mask = nullptr, int64_t ldm = 0)
-  {
-    dim3 grid((Nc + mm_tile - 1) / mm_tile, (M + mm_tile - 1) / mm_tile, 1);
-    mlp_gemm<EP><<<grid, mm_threads, 0, s>>>(M, Nc, K, A, sam, sak, B, sbk, sbn, C, ldc, bias,
-                                              mask, ldm, K, 0);
-    return check_launch("mlp gemm");
-  }
-
-  //! C (M x Nc, ldc = Nc) = A B for a long K (the batch): K is split over
-  //! blocks into partial products that are then summed in a fixed order.
-  int gemm_long_k(hipStream_t s, int M, int Nc, int K, const float *A, int64_t sam, int64_t sak,
-                  const float *B, int64_t sbk, int64_t sbn, float *C)
-  {
-    const int parts = std::max(1, std::min(split_parts, (K + 127) / 128));
-    const int kchunk = (K + parts - 1) / parts;
-    const int64_t zstride = int64_t(M) * Nc;
-    dim3 grid((Nc + mm_tile - 1) / mm_tile, (M + mm_tile - 1) / mm_tile, parts);
-    mlp_gemm<ep_store><<<grid, mm_threads, 0, s>>>(M, Nc, K, A, sam, sak, B, sbk, sbn,
-                                                    scratch.data(), Nc, nullptr, nullptr, 0,
-                                                    kchunk, zstride);
-    mlp_sum_parts<<<grid_for(zstride), 256, 0, s>>>(zstride, parts, scratch.data(), C);
-    return check_launch("mlp gemm (split k)");
-  }
-
-  //! out[c] = sum over the B rows of X[r*ld + c].
-  int colsum(hipStream_t s, int64_t rows, int cols, const float *X, int64_t ld, float *out)
-  {
-    const int parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(split_parts, (rows + 63) / 64)));
-    const int64_t chunk = (rows + parts - 1) / parts;
-    mlp_colsum_part<<<dim3((cols + 255) / 256, 1, parts), 256, 0, s>>>(rows, cols, X, ld, chunk,
-                                                                      scratch.data());
-    mlp_sum_parts<<<grid_for(cols), 256, 0, s>>>(cols, parts, scratch.data(), out);
-    return check_launch("mlp column sums");
-  }
-
-  //! FP32 forward of B rows of Xb into H1, H2, O.
-  int forward(hipStream_t s, int B, const float *X)
+  //! The chain kernel on B rows of X (and T with BACK; O without).
+  template<bool BACK>
+  int chain(hipStream_t s, int B, const float *X, const float *T, float *O)
   {
     const float *p = params.data();
-    AKM_TRY(gemm<ep_bias_relu>(s, B, H, K1, X, K1, 1, p + oW1, 1, K1, H1.data(), H, p + ob1));
-    AKM_TRY(gemm<ep_bias_relu>(s, B, H, H, H1.data(), H, 1, p + oW2, 1, H, H2.data(), H,
-                               p + ob2));
-    AKM_TRY(gemm<ep_bias>(s, B, N3, H, H2.data(), H, 1, p + oW3, 1, H, O.data(), N3, p + ob3));
-    return AKM_SUCCESS;
+    mlp_pass a{};
+    a.rows = B;
+    a.N = N;
+    a.N3 = N3;
+    a.K1 = K1;
+    a.H = H;
+    a.W1 = p + oW1;
+    a.b1 = p + ob1;
+    a.W2 = p + oW2;
+    a.b2 = p + ob2;
+    a.W3 = p + oW3;
+    a.b3 = p + ob3;
+    a.X = X;
+    a.T = T;
+    a.H1 = H1.data();
+    a.H2 = H2.data();
+    a.O = O;
+    a.dO = dO.data();
+    a.dH2 = dH2.data();
+    a.dH1 = dH1.data();
+    a.scale = 2.0f / (float(B) * float(N));
+    a.partial = partial.data();
+    const size_t lds = sizeof(float) * mc_rows * size_t(K1 + 2 * H + N3 + 16);
+    if (lds > 64 * 1024)
+      AKM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mlp_chain<BACK>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  static_cast<int>(lds)));
+    mlp_chain<BACK><<<chain_groups(B), mc_threads, lds, s>>>(a);
+    return check_launch("mlp layers");
   }
 
-  //! Loss (mean squared error over B rows and N outputs) into loss[slot]
-  //! (accumulated if `accumulate`) and the gradient of every parameter into
-  //! grad, for the rows of X / T (forward must have run on X).
-  int backward(hipStream_t s, int B, const float *X, const float *T, int accumulate)
+  //! FP32 forward of B rows of X into O (B x N3).
+  int forward(hipStream_t s, int B, const float *X, float *O)
   {
-    const float *p = params.data();
-    float *g = grad.data();
-    const float scale = 2.0f / (float(B) * float(N));
-    const int blocks = std::min(4096, grid_for(int64_t(B) * N3));
-    mlp_out_grad<<<blocks, 256, 0, s>>>(B, N, N3, O.data(), T, scale, dO.data(), partial.data());
-    mlp_sum<<<1, 256, 0, s>>>(blocks, partial.data(), loss.data(), accumulate);
-    AKM_TRY(check_launch("mlp loss"));
-    // layer 3
-    AKM_TRY(gemm_long_k(s, N3, H, B, dO.data(), 1, N3, H2.data(), H, 1, g + oW3));
-    AKM_TRY(colsum(s, B, N3, dO.data(), N3, g + ob3));
-    AKM_TRY(gemm<ep_mask>(s, B, H, N3, dO.data(), N3, 1, p + oW3, H, 1, dH2.data(), H, nullptr,
-                          H2.data(), H));
-    // layer 2
-    AKM_TRY(gemm_long_k(s, H, H, B, dH2.data(), 1, H, H1.data(), H, 1, g + oW2));
-    AKM_TRY(colsum(s, B, H, dH2.data(), H, g + ob2));
-    AKM_TRY(gemm<ep_mask>(s, B, H, H, dH2.data(), H, 1, p + oW2, H, 1, dH1.data(), H, nullptr,
-                          H1.data(), H));
-    // layer 1
-    AKM_TRY(gemm_long_k(s, H, K1, B, dH1.data(), 1, H, X, K1, 1, g + oW1));
-    AKM_TRY(colsum(s, B, H, dH1.data(), H, g + ob1));
-    return check_launch("mlp backward");
+    return chain<false>(s, B, X, nullptr, O);
+  }
+
+  //! Forward and backward of B rows: loss (squared error over B rows and N
+  //! outputs) into loss[0] (accumulated if `accumulate`) and the gradient of
+  //! every parameter into `out`.
+  int gradients(hipStream_t s, int B, const float *X, const float *T, int accumulate, float *out)
+  {
+    AKM_TRY(chain<true>(s, B, X, T, nullptr));
+    const int np = row_parts(B);
+    wg_args a{};
+    auto tiles = [](int M, int C) {
+      return ((M + wg_tile - 1) / wg_tile) * ((C + wg_tile - 1) / wg_tile);
+    };
+    a.layer[0] = wg_layer{dH2.data(), H1.data(), H, H, oW2, ob2, 0};
+    a.layer[1] = wg_layer{dH1.data(), X, H, K1, oW1, ob1, tiles(H, H)};
+    a.layer[2] = wg_layer{dO.data(), H2.data(), N3, H, oW3, ob3, tiles(H, H) + tiles(H, K1)};
+    a.rows = B;
+    a.chunk = ((B + np - 1) / np + 15) / 16 * 16;
+    a.stride = num_params;
+    a.out = (np == 1) ? out : parts.data();
+    mlp_weight_grad<<<dim3(a.layer[2].tile0 + tiles(N3, H), np), wg_threads, 0, s>>>(a);
+    AKM_TRY(check_launch("mlp weight gradients"));
+    const int blocks = (np == 1) ? 0 : grid_for(num_params);
+    mlp_sum_parts<<<blocks + 1, 256, 0, s>>>(num_params, np, parts.data(), out, chain_groups(B),
+                                             partial.data(), loss.data(), accumulate, host_loss);
+    return check_launch("mlp gradients");
   }
 
   int adam(hipStream_t s, const float *g, float lr)
@@ -708,9 +891,7 @@ akm_status akm_mlp_forward(akm_precond p, const float *X, int64_t rows, float *O
   if (rows < 1 || rows > (1 << 24))
     return set_error(AKM_ERR_INVALID, "mlp: rows %lld out of range", static_cast<long long>(rows));
   AKM_TRY(m->ensure_batch(static_cast<int>(rows)));
-  AKM_TRY(m->forward(m->stream, static_cast<int>(rows), X));
-  AKM_HIP(hipMemcpyAsync(O, m->O.data(), sizeof(float) * rows * m->N3, hipMemcpyDeviceToDevice,
-                         m->stream));
+  AKM_TRY(m->forward(m->stream, static_cast<int>(rows), X, O));
   AKM_HIP(hipStreamSynchronize(m->stream));
   return AKM_SUCCESS;
 }
@@ -725,16 +906,10 @@ akm_status akm_mlp_gradients(akm_precond p, const float *X, const float *T, int6
     return set_error(AKM_ERR_INVALID, "mlp: rows %lld out of range", static_cast<long long>(rows));
   const int B = static_cast<int>(rows);
   AKM_TRY(m->ensure_batch(B));
-  AKM_TRY(m->forward(m->stream, B, X));
-  AKM_TRY(m->backward(m->stream, B, X, T, 0));
-  if (grad != nullptr)
-    AKM_HIP(hipMemcpyAsync(grad, m->grad.data(), sizeof(float) * m->num_params,
-                           hipMemcpyDeviceToDevice, m->stream));
-  double l = 0;
-  AKM_HIP(hipMemcpyAsync(&l, m->loss.data(), sizeof(double), hipMemcpyDeviceToHost, m->stream));
+  AKM_TRY(m->gradients(m->stream, B, X, T, 0, grad != nullptr ? grad : m->grad.data()));
   AKM_HIP(hipStreamSynchronize(m->stream));
   if (loss)
-    *loss = l / (double(B) * m->N);
+    *loss = *m->host_loss / (double(B) * m->N);
   return AKM_SUCCESS;
 }
 
@@ -786,8 +961,7 @@ akm_status akm_mlp_train(akm_precond p, const double *residuals, const double *c
       mlp_gather<<<B, 256, 0, s>>>(B, perm_d.data(), bi * B, m->K1, m->N3, X.data(), T.data(),
                                     m->Xb.data(), m->Tb.data());
       AKM_TRY(check_launch("mlp gather"));
-      AKM_TRY(m->forward(s, B, m->Xb.data()));
-      AKM_TRY(m->backward(s, B, m->Xb.data(), m->Tb.data(), bi > 0));
+      AKM_TRY(m->gradients(s, B, m->Xb.data(), m->Tb.data(), bi > 0, m->grad.data()));
       AKM_TRY(m->adam(s, m->grad.data(), static_cast<float>(lr)));
     }
     // the host copy of perm is reshuffled next epoch: wait for the upload
