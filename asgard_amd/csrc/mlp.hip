@@ -18,10 +18,9 @@
 // matrix cores (v_mfma_f32_16x16x4_f32: FP32 products and sums): one kernel
 // takes 16 samples through the whole forward and backward chain with their
 // activations in LDS, a second forms every weight and bias gradient, a third
-// adds its row parts; the
-// preconditioner itself runs on BF16 copies of W1..W3 with the MFMA
-// v_mfma_f32_16x16x16_bf16 (FP32 accumulation), one wavefront per 16 cells,
-// activations in LDS.
+// adds its row parts.  The preconditioner itself runs on BF16 copies of W1..W3
+// with v_mfma_f32_16x16x32_bf16 (FP32 accumulation), eight wavefronts per 16 to
+// 64 cells, activations in LDS.
 #include "precond.hpp"
 
 #include <algorithm>
@@ -459,127 +458,197 @@ __device__ __forceinline__ unsigned short to_bf16(float f)
   return static_cast<unsigned short>(u >> 16);
 }
 
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+//! BF16 copy of W (J x K, J a multiple of 16) in the order the matrix cores
+//! take it: tiles of 16 outputs x 32 inputs (the last one filled with zeros),
+//! and in a tile 8 inputs for each lane, so that a wavefront reads 1 KB in
+//! one piece.  KB tiles along the inputs, J16 along the outputs; outputs past
+//! J are zero.
 __global__ void __launch_bounds__(256)
-mlp_to_bf16(int64_t count, const float *src, unsigned short *dst)
+mlp_pack_bf16(int J, int K, int J16, int KB, const float *src, unsigned short *dst)
 {
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < count; i += 256ll * gridDim.x)
-    dst[i] = to_bf16(src[i]);
-}
-
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-
-constexpr int mlp_cells_per_wave = 16;
-
-//! One dense layer of the 16 cells of a wavefront on the matrix cores:
-//! out[m][j] = act(sum_k in[m][k] W[j][k] + b[j]) for j < J (J, K multiples
-//! of 16), in/out BF16 rows in LDS.  v_mfma_f32_16x16x16_bf16 operands:
-//! lane l holds A[l%16][4(l/16) .. +3] and B[4(l/16) .. +3][l%16], and gets
-//! D[4(l/16) + i][l%16], i = 0..3.
-__device__ __forceinline__ void mfma_layer(const unsigned short *in, int ldi, int K,
-                                           const unsigned short *W, const float *bias, int J,
-                                           unsigned short *out, int ldo)
-{
-  const int lane = threadIdx.x;
-  const int row = lane % 16, quad = lane / 16;
-  for (int j0 = 0; j0 < J; j0 += 16)
+  const int count = J16 * KB * 512;
+  for (int e = blockIdx.x * 256 + threadIdx.x; e < count; e += 256 * gridDim.x)
   {
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const unsigned short *wrow = W + int64_t(j0 + row) * K + 4 * quad;
-    const unsigned short *arow = in + row * ldi + 4 * quad;
-    for (int k0 = 0; k0 < K; k0 += 16)
-    {
-      const bf16x4 a = *reinterpret_cast<const bf16x4 *>(arow + k0);
-      const bf16x4 b = *reinterpret_cast<const bf16x4 *>(wrow + k0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-    }
-    const float bj = bias[j0 + row];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-      out[(4 * quad + i) * ldo + j0 + row] = to_bf16(fmaxf(acc[i] + bj, 0.0f));
+    const int tile = e / 512, lane = e / 8 % 64;
+    const int j = tile / KB * 16 + lane % 16, k = tile % KB * 32 + lane / 16 * 8 + e % 8;
+    dst[e] = (j < J && k < K) ? to_bf16(src[int64_t(j) * K + k]) : 0;
   }
 }
 
-//! z = v + s * o(x) per cell (see the file comment); one wavefront per 16
-//! cells.  LDS: X [16][K1+4], H1 [16][H+4], H2 [16][H+4] (BF16), s [16].
-__global__ void __launch_bounds__(64)
-mlp_apply_bf16(int64_t cells, int N, int d, int K1, int H, int N3, const double *v, double *z,
-               const float *feat, const unsigned short *W1, const float *b1,
+constexpr int ma_waves = 8; // wavefronts of a workgroup, which share the outputs
+
+//! T tiles of 16 outputs (from tile jt on) x R tiles of 16 cells on the matrix
+//! cores: W packed (see mlp_pack_bf16), in BF16 rows of KB * 32 inputs in LDS.
+//! v_mfma_f32_16x16x32_bf16 with the outputs as rows: lane l gives
+//! W[l % 16][8 (l / 16) .. +7] and in[8 (l / 16) .. +7][l % 16] and gets
+//! outputs 4 (l / 16) .. +3 of cell l % 16.
+template<int T, int R>
+__device__ __forceinline__ void mfma_tiles(const unsigned short *in, int ldi, int KB,
+                                           const unsigned short *W, int jt, f32x4 (&acc)[T][R])
+{
+  constexpr int U = 2; // input tiles read ahead
+  const int lane = threadIdx.x % 64;
+  const unsigned short *arow = in + lane % 16 * ldi + lane / 16 * 8;
+  const unsigned short *w = W + int64_t(jt) * KB * 512 + lane * 8;
+#pragma unroll
+  for (int t = 0; t < T; t++)
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      acc[t][r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto read = [&](int kb, bf16x8 (&b)[U][T]) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int t = 0; t < T; t++)
+        b[u][t] = *reinterpret_cast<const bf16x8 *>(w + (t * KB + min(kb + u, KB - 1)) * 512);
+  };
+  bf16x8 cur[U][T], next[U][T];
+  read(0, cur);
+  for (int kb = 0; kb < KB; kb += U)
+  {
+    read(kb + U, next);
+    // the scheduler would move each read to its use
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (kb + u < KB)
+      {
+        bf16x8 a[R];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          a[r] = *reinterpret_cast<const bf16x8 *>(arow + 16 * r * ldi + (kb + u) * 32);
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+          for (int r = 0; r < R; r++)
+            acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[u][t], a[r], acc[t][r], 0, 0, 0);
+      }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int t = 0; t < T; t++)
+        cur[u][t] = next[u][t];
+  }
+}
+
+//! A hidden layer (ReLU) of the workgroup's 16 R cells: 2 JT tiles of outputs,
+//! J of them real; the others come out as zero.
+template<int R>
+__device__ __forceinline__ void mfma_layer(const unsigned short *in, int ldi, int KB,
+                                           const unsigned short *W, const float *bias, int J,
+                                           int JT, unsigned short *out, int ldo)
+{
+  const int lane = threadIdx.x % 64;
+  for (int p = threadIdx.x / 64; p < JT; p += ma_waves)
+  {
+    f32x4 acc[2][R];
+    f32x4 b[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+      {
+        const int j = 32 * p + 16 * t + lane / 16 * 4 + i;
+        b[t][i] = (j < J) ? bias[j] : 0.0f;
+      }
+    mfma_tiles<2, R>(in, ldi, KB, W, 2 * p, acc);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int r = 0; r < R; r++)
+      {
+        f32x4 x;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          x[i] = fmaxf(acc[t][r][i] + b[t][i], 0.0f);
+        *reinterpret_cast<bf16x4 *>(out + (16 * r + lane % 16) * ldo + 32 * p + 16 * t +
+                                    lane / 16 * 4) = __builtin_convertvector(x, bf16x4);
+      }
+  }
+}
+
+//! z = v + s * o(x) per cell (see the file comment) for 16 R cells a
+//! workgroup, eight wavefronts sharing the outputs of each layer.
+//! What bounds it: latency, from layer to layer, of the weights' way from L2
+//! (208 KB a workgroup, in 1 KB pieces); at 16172 cells of 64 values, 256
+//! wide, matrix-core time is 1.4 us and memory time 4 us of its 16.  One
+//! wavefront per 16 cells, reading the weights row by row in 8-byte pieces
+//! with nothing in flight beside the product, took 71 us.
+//! LDS: rows of lda (inputs, then the second layer) and ldh (first layer)
+//! BF16 values, 16 bytes longer than their contents so that 16 rows spread
+//! over the banks; the norms.
+template<int R>
+__global__ void __launch_bounds__(64 * ma_waves, 4)
+mlp_apply_bf16(int64_t cells, int N, int d, int H, int N3, int KB1, int KBH, const double *v,
+               double *z, const float *feat, const unsigned short *W1, const float *b1,
                const unsigned short *W2, const float *b2, const unsigned short *W3,
                const float *b3)
 {
-  extern __shared__ unsigned char lds_raw[];
-  const int ldx = K1 + 4, ldh = H + 4;
+  constexpr int C = 16 * R, TPC = 64 * ma_waves / C; // cells; threads per cell
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int lda = 32 * max(KB1, KBH) + 8, ldh = 32 * KBH + 8;
   float *snorm = reinterpret_cast<float *>(lds_raw);
-  unsigned short *Xs = reinterpret_cast<unsigned short *>(lds_raw + 64);
-  unsigned short *H1s = Xs + mlp_cells_per_wave * ldx;
-  unsigned short *H2s = H1s + mlp_cells_per_wave * ldh;
-  const int lane = threadIdx.x;
-  const int64_t c0 = int64_t(blockIdx.x) * mlp_cells_per_wave;
-
-  // cell norms: 4 lanes per cell
+  unsigned short *A = reinterpret_cast<unsigned short *>(lds_raw + sizeof(float) * C);
+  unsigned short *H1s = A + C * lda;
+  const int64_t c0 = int64_t(blockIdx.x) * C;
   {
-    const int m = lane / 4, sub = lane % 4;
+    const int m = threadIdx.x / TPC, sub = threadIdx.x % TPC;
     const int64_t c = c0 + m;
+    const double *vc = v + c * N;
     double sq = 0;
     if (c < cells)
-      for (int i = sub; i < N; i += 4)
-      {
-        const double vi = v[c * N + i];
-        sq = fma(vi, vi, sq);
-      }
-    sq += __shfl_xor(sq, 1);
-    sq += __shfl_xor(sq, 2);
-    if (sub == 0)
-      snorm[m] = static_cast<float>(sqrt(sq));
-  }
-  __syncthreads();
-  // inputs
-  for (int e = lane; e < mlp_cells_per_wave * K1; e += 64)
-  {
-    const int m = e / K1, i = e % K1;
-    const int64_t c = c0 + m;
-    float x = 0.0f;
-    if (c < cells)
-    {
-      if (i < N)
-      {
-        const float s = snorm[m];
-        x = (s > 0.0f) ? static_cast<float>(v[c * N + i] / double(s)) : 0.0f;
-      }
-      else if (i < N + d)
-        x = feat[c * d + (i - N)];
-    }
-    Xs[m * ldx + i] = to_bf16(x);
-  }
-  __syncthreads();
-  mfma_layer(Xs, ldx, K1, W1, b1, H, H1s, ldh);
-  __syncthreads();
-  mfma_layer(H1s, ldh, H, W2, b2, H, H2s, ldh);
-  __syncthreads();
-  // output layer, linear, straight to z
-  const int row = lane % 16, quad = lane / 16;
-  for (int j0 = 0; j0 < N3; j0 += 16)
-  {
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const unsigned short *wrow = W3 + int64_t(j0 + row) * H + 4 * quad;
-    const unsigned short *arow = H2s + row * ldh + 4 * quad;
-    for (int k0 = 0; k0 < H; k0 += 16)
-    {
-      const bf16x4 a = *reinterpret_cast<const bf16x4 *>(arow + k0);
-      const bf16x4 b = *reinterpret_cast<const bf16x4 *>(wrow + k0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-    }
-    const int j = j0 + row;
-    if (j >= N)
-      continue;
-    const float bj = b3[j];
+      for (int i = sub; i < N; i += TPC)
+        sq = fma(vc[i], vc[i], sq);
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int off = 1; off < TPC; off <<= 1)
+      sq += __shfl_xor(sq, off);
+    const float s = static_cast<float>(sqrt(sq));
+    if (sub == 0)
+      snorm[m] = s;
+    for (int i = sub; i < 32 * KB1; i += TPC)
     {
-      const int m = 4 * quad + i;
-      const int64_t c = c0 + m;
+      float x = 0.0f;
       if (c < cells)
-        z[c * N + j] = v[c * N + j] + double(snorm[m]) * double(acc[i] + bj);
+      {
+        if (i < N)
+          x = (s > 0.0f) ? static_cast<float>(vc[i] / double(s)) : 0.0f;
+        else if (i < N + d)
+          x = feat[c * d + (i - N)];
+      }
+      A[m * lda + i] = to_bf16(x);
+    }
+  }
+  mlp_lds_barrier();
+  mfma_layer<R>(A, lda, KB1, W1, b1, H, KBH, H1s, ldh);
+  mlp_lds_barrier();
+  mfma_layer<R>(H1s, ldh, KBH, W2, b2, H, KBH, A, lda);
+  mlp_lds_barrier();
+  // output layer, linear, straight to z
+  constexpr int RO = (R > 1) ? 2 : 1;
+  const int lane = threadIdx.x % 64;
+  for (int u = threadIdx.x / 64; u < N3 / 16 * (R / RO); u += ma_waves)
+  {
+    const int jt = u / (R / RO), r0 = u % (R / RO) * RO;
+    f32x4 acc[1][RO];
+    mfma_tiles<1, RO>(A + 16 * r0 * lda, lda, KBH, W3, jt, acc);
+#pragma unroll
+    for (int r = 0; r < RO; r++)
+    {
+      const int m = 16 * (r0 + r) + lane % 16;
+      const int64_t c = c0 + m;
+      if (c >= cells)
+        continue;
+      const double s = snorm[m];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+      {
+        const int j = 16 * jt + lane / 16 * 4 + i;
+        if (j < N)
+          z[c * N + j] = v[c * N + j] + s * double(acc[0][r][i] + b3[j]);
+      }
     }
   }
 }
@@ -602,7 +671,7 @@ struct akm_mlp_s final : akm_precond_s
   int max_level = 0;
   int64_t oW1 = 0, ob1 = 0, oW2 = 0, ob2 = 0, oW3 = 0, ob3 = 0, num_params = 0;
   dev_buffer<float> params, grad, adam_m, adam_v, feat;
-  dev_buffer<unsigned short> wbf; // W1 | W2 | W3 in BF16
+  dev_buffer<unsigned short> wbf; // W1 | W2 | W3 in BF16 tiles
   bool bf16_current = false;
   int64_t adam_t = 0;
   // batch buffers (sized for `batch` rows)
@@ -732,31 +801,56 @@ struct akm_mlp_s final : akm_precond_s
       return AKM_SUCCESS;
     const float *p = params.data();
     unsigned short *w = wbf.data();
-    const int64_t n1 = int64_t(H) * K1, n2 = int64_t(H) * H, n3 = int64_t(N3) * H;
-    mlp_to_bf16<<<grid_for(n1), 256, 0, s>>>(n1, p + oW1, w);
-    mlp_to_bf16<<<grid_for(n2), 256, 0, s>>>(n2, p + oW2, w + n1);
-    mlp_to_bf16<<<grid_for(n3), 256, 0, s>>>(n3, p + oW3, w + n1 + n2);
+    const int kb1 = kb(K1), kbh = kb(H);
+    mlp_pack_bf16<<<grid_for(packed(2 * kbh, kb1)), 256, 0, s>>>(H, K1, 2 * kbh, kb1, p + oW1, w);
+    w += packed(2 * kbh, kb1);
+    mlp_pack_bf16<<<grid_for(packed(2 * kbh, kbh)), 256, 0, s>>>(H, H, 2 * kbh, kbh, p + oW2, w);
+    w += packed(2 * kbh, kbh);
+    mlp_pack_bf16<<<grid_for(packed(N3 / 16, kbh)), 256, 0, s>>>(N3, H, N3 / 16, kbh, p + oW3, w);
     AKM_TRY(check_launch("mlp bf16 weights"));
     bf16_current = true;
     return AKM_SUCCESS;
   }
 
-  size_t apply_lds_bytes() const
+  //! Tiles of 32 inputs, and values of a packed layer.
+  static int kb(int K) { return (K + 31) / 32; }
+  static int64_t packed(int J16, int KB) { return int64_t(J16) * KB * 512; }
+  int64_t packed_weights() const
   {
-    return 64 + sizeof(unsigned short) * mlp_cells_per_wave * size_t((K1 + 4) + 2 * (H + 4));
+    return packed(2 * kb(H), kb(K1)) + packed(2 * kb(H), kb(H)) + packed(N3 / 16, kb(H));
+  }
+
+  template<int R>
+  int apply_cells(const double *v, double *z, hipStream_t s)
+  {
+    const int kb1 = kb(K1), kbh = kb(H);
+    const size_t lds = 16 * R * (sizeof(float) + sizeof(unsigned short) *
+                                                     size_t(32 * (std::max(kb1, kbh) + kbh) + 16));
+    if (lds > 64 * 1024)
+      AKM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mlp_apply_bf16<R>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  static_cast<int>(lds)));
+    const unsigned short *w1 = wbf.data(), *w2 = w1 + packed(2 * kbh, kb1),
+                         *w3 = w2 + packed(2 * kbh, kbh);
+    const float *p = params.data();
+    mlp_apply_bf16<R><<<static_cast<unsigned>((cells + 16 * R - 1) / (16 * R)), 64 * ma_waves, lds,
+                        s>>>(cells, N, d, H, N3, kb1, kbh, v, z, feat.data(), w1, p + ob1, w2,
+                             p + ob2, w3, p + ob3);
+    return check_launch("mlp preconditioner");
   }
 
   int apply(const double *v, double *z, hipStream_t s) override
   {
     AKM_TRY(refresh_bf16(s));
-    const int64_t blocks = (cells + mlp_cells_per_wave - 1) / mlp_cells_per_wave;
-    const unsigned short *w = wbf.data();
-    const int64_t n1 = int64_t(H) * K1, n2 = int64_t(H) * H;
-    const float *p = params.data();
-    mlp_apply_bf16<<<static_cast<unsigned>(blocks), 64, apply_lds_bytes(), s>>>(
-        cells, N, d, K1, H, N3, v, z, feat.data(), w, p + ob1, w + n1, p + ob2, w + n1 + n2,
-        p + ob3);
-    return check_launch("mlp preconditioner");
+    // Cells a workgroup: as many as share one reading of the weights while
+    // the chip stays full.  16 / 32 / 64 cells took, 256 wide, 64 values:
+    // 7.9 / 8.4 / 9.5 us for 4 K cells, 12.4 / 11.6 / 11.1 for 8 K,
+    // 23.2 / 16.2 / 15.3 for 16 K and 56 / 41 / 35 for 47 K.
+    if (cells <= 16 * 256)
+      return apply_cells<1>(v, z, s);
+    if (cells <= 32 * 512)
+      return apply_cells<2>(v, z, s);
+    return apply_cells<4>(v, z, s);
   }
 };
 
@@ -815,7 +909,7 @@ akm_status akm_mlp_create(int d, int n, int64_t num_cells, const int *table, int
   AKM_TRY(m->adam_m.upload(zeros.data(), m->num_params));
   AKM_TRY(m->adam_v.upload(zeros.data(), m->num_params));
   AKM_TRY(m->grad.upload(zeros.data(), m->num_params));
-  AKM_TRY(m->wbf.allocate(H * K1 + H * H + N3 * H));
+  AKM_TRY(m->wbf.allocate(m->packed_weights()));
   // features: (level + (position + 1/2) / cells of the level) / (max_level + 1)
   std::vector<float> f(num_cells * d);
   for (int64_t c = 0; c < num_cells; c++)

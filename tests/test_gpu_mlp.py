@@ -142,6 +142,31 @@ def test_bf16_apply_matches_oracle(d, n, L, hidden):
     assert np.abs(err).max() < 0.05 * np.abs(corr).max()
 
 
+@pytest.mark.parametrize("d,n,L,hidden", [
+    (1, 1, 1, 16),   # two cells, half a tile of inputs, one wavefront's outputs
+    (2, 3, 5, 48),   # odd values a cell, hidden width between tiles of 32
+    (3, 3, 9, 80),   # 32 cells a workgroup, a remainder
+    (1, 3, 15, 32),  # 64 cells a workgroup
+    (1, 4, 14, 512), # the widest layers, the last of the 32-cell sizes
+    (3, 4, 5, 272)])
+def test_bf16_apply_at_tile_edges(d, n, L, hidden):
+    """Against the oracle as above, where the tiles of cells, inputs and
+    outputs end: tolerance of BF16 weights and activations in three layers
+    (2^-9 relative each, a factor of 8 for their random sum)."""
+    rng = np.random.default_rng(40 + d)
+    table, pre, lay = make(d, n, L, hidden)
+    p = random_params(lay, rng, scale=0.15)
+    pre.set_params(p)
+    cells = table.shape[0]
+    v = rng.standard_normal(cells * lay.N)
+    z = torch.empty(v.size, dtype=torch.float64, device="cuda")
+    pre.apply(dev(v), z)
+    ref = omlp.precondition(lay, p.astype(np.float64), v, omlp.features(table, L))
+    err = host(z) - ref
+    assert np.linalg.norm(err) < 8 * 3 * 2.0 ** -9 * np.linalg.norm(ref - v)
+    assert np.abs(err).reshape(cells, -1).max(axis=1).max() < 0.1 * np.abs(ref - v).max()
+
+
 def test_training_on_solver_pairs_lowers_the_loss():
     d, n, L, dt = 2, 2, 5, 0.02
     table, _ = grid.element_table([L] * d)
