@@ -498,12 +498,22 @@ struct gs_group
 };
 
 //! One pass: a chain's stage.  mode 0: x -> sum (one-stage chain); 1: x ->
-//! intermediate; 2: intermediate -> sum.
+//! intermediate; 2: intermediate -> sum; 3: the same stage of two chains at
+//! once (the last of one, the first of the next), intermediate -> sum and x
+//! -> intermediate.
 struct gs_pass
 {
   int tab;  // factor table index within the group
   int j;    // slab dimension index (0 or 1)
   int fill, mode;
+};
+
+//! A split item's pass and its lanes.
+struct gs_lane_pass
+{
+  gs_pass ps;
+  int slot0, nslot; // in gs_args::slots
+  int rec0;         // their records in gs_args::recs
 };
 
 //! One workgroup's work: a chunk of a bundle with its group's data, so that
@@ -512,7 +522,7 @@ struct gs_item
 {
   int cell0, ncell; // the bundle's cells in gs_args::cells
   int C;            // other-index combinations per chunk
-  int cb, nq;       // the group's first compact factor table in gs_ctab, nq blocks each
+  int cb, tstride;  // the group's first compact factor table in gs_ctab, values per table
   int resident;     // 1: every factor table and both lists staged once
   int list0;        // first int of the bundle's list images
   int llen[2];      // per slab dimension: image length
@@ -524,8 +534,10 @@ struct gs_item
   int slot;         // work-buffer slot of the group's sum
   // a split item (one chain of a large slab): its chain of the bundle's nch
   // and the bundle's first partial in the partial buffer (-1: not split);
-  // cell c's partial of chain k is partial part + c * nch + k (N values)
+  // cell c's partial of chain k is partial part + c * nch + k (N values);
+  // its passes
   int part, nch, chain;
+  gs_lane_pass pass[2];
 };
 
 struct gs_args
@@ -541,7 +553,13 @@ struct gs_args
   // its factor block's element offset in the compact table << 16)
   const int *lists;
   const int *offs; // tensor offsets of the other-index combinations
+  const int *slots; // split items' lanes: record | entry << 16 (-1: none)
+  const int *recs;
 };
+
+//! Values of one compact factor table of nq n x n blocks, filled up to
+//! whole 16 bytes of either precision.
+__host__ __device__ inline int gs_table_values(int nq, int nn) { return (nq * nn + 3) / 4 * 4; }
 
 //! LDS bytes of one work item: x (and the intermediate when nd = 2), ntab
 //! factor tables of nq blocks, then the int lists (nlist_ints).
@@ -550,8 +568,16 @@ __host__ __device__ inline int64_t gs_lds_bytes(int esize, int nd, int n, int nc
 {
   const int64_t ds = (nd == 1) ? n : int64_t(n) * n;
   const int64_t bd = int64_t(ncell) * (ds * C + gs_pad);
-  const int64_t vals = bd * nd + int64_t(ntab) * nq * n * n;
+  const int64_t vals = bd * nd + int64_t(ntab) * gs_table_values(nq, n * n);
   return int64_t(16) * npass + (vals * esize + 15) / 16 * 16 + 4 * nlist_ints;
+}
+
+//! The same of a split item: x, the intermediate, one factor table.
+__host__ __device__ inline int64_t gs_split_lds(int esize, int nd, int n, int ncell, int C, int nq)
+{
+  const int64_t ds = (nd == 1) ? n : int64_t(n) * n;
+  const int64_t bd = int64_t(ncell) * (ds * C + gs_pad);
+  return (bd * nd * esize + 15) / 16 * 16 + int64_t(gs_table_values(nq, n * n)) * esize;
 }
 
 //! dst[i] = src[i], i < count, by a workgroup of TPB threads with
@@ -647,13 +673,47 @@ __device__ __forceinline__ int gs_at(int si, int ob, int vs)
     return ob + si * vs;
 }
 
+//! Where value w of block q sits in a compact factor table of nq blocks:
+//! FP64 blocks of an even value count in planes of pairs, others in one
+//! piece.
+template<typename P>
+__host__ __device__ inline int gs_table_at(int q, int w, int nq, int nn)
+{
+  return (sizeof(P) == 8 && nn % 2 == 0) ? (w / 2 * nq + q) * 2 + w % 2 : q * nn + w;
+}
+
+//! A block of DS values at xb, its values (pairs, when pair-major) vs apart.
+template<typename P, int DS>
+__device__ __forceinline__ void gs_x_load(const P *xb, int vs, P (&xv)[DS])
+{
+  if constexpr (gs_pair_major<P, DS>)
+  {
+#pragma unroll
+    for (int q = 0; q < DS / 2; q++)
+    {
+      const double2 t = *reinterpret_cast<const double2 *>(xb + q * vs);
+      xv[2 * q] = t.x;
+      xv[2 * q + 1] = t.y;
+    }
+  }
+  else
+  {
+#pragma unroll
+    for (int k = 0; k < DS; k++)
+      xv[k] = xb[k * vs];
+  }
+}
+
 //! The factor block and the x block of one list entry: the block starts at
 //! in + ob + the entry's cell offset, its values (pairs, when pair-major)
-//! vs apart.  Factor blocks of an even value count are read in 16-byte
-//! pairs (FP64 tables start 16-byte aligned, blocks n*n values apart).
+//! vs apart.  FP64 factor blocks of an even value count are read in 16-byte
+//! pairs, each pair of the block in a plane of its own (gs_table_at), planes
+//! `plane` values apart: lanes on neighbouring blocks then read neighbouring
+//! words, where blocks in one piece (32 bytes for n = 2) left half the LDS
+//! banks unused by each read (the operator above: 111 -> 103 us).
 template<typename P, int NT, int ND>
-__device__ __forceinline__ void gs_block_load(const P *tab, const P *in, unsigned e, int ob,
-                                              int vs, P (&av)[NT * NT],
+__device__ __forceinline__ void gs_block_load(const P *tab, int plane, const P *in, unsigned e,
+                                              int ob, int vs, P (&av)[NT * NT],
                                               P (&xv)[(ND == 1) ? NT : NT * NT])
 {
   constexpr int ds = (ND == 1) ? NT : NT * NT;
@@ -664,7 +724,7 @@ __device__ __forceinline__ void gs_block_load(const P *tab, const P *in, unsigne
 #pragma unroll
     for (int q = 0; q < NT * NT / 2; q++)
     {
-      const double2 t = reinterpret_cast<const double2 *>(A)[q];
+      const double2 t = *reinterpret_cast<const double2 *>(A + q * plane);
       av[2 * q] = t.x;
       av[2 * q + 1] = t.y;
     }
@@ -675,22 +735,7 @@ __device__ __forceinline__ void gs_block_load(const P *tab, const P *in, unsigne
     for (int k = 0; k < NT * NT; k++)
       av[k] = A[k];
   }
-  if constexpr (gs_pair_major<P, ds>)
-  {
-#pragma unroll
-    for (int q = 0; q < ds / 2; q++)
-    {
-      const double2 t = *reinterpret_cast<const double2 *>(xb + q * vs);
-      xv[2 * q] = t.x;
-      xv[2 * q + 1] = t.y;
-    }
-  }
-  else
-  {
-#pragma unroll
-    for (int k = 0; k < ds; k++)
-      xv[k] = xb[k * vs];
-  }
+  gs_x_load<P, ds>(xb, vs, xv);
 }
 
 //! One pass along slab dimension J for one block (cell c >= 0, block base
@@ -703,43 +748,57 @@ __device__ __forceinline__ void gs_block_load(const P *tab, const P *in, unsigne
 //! is the first connection of an upper fill and the last of a lower one.
 //! The loop is software-pipelined: the blocks of the next connection and
 //! the list entry after it are read while this connection's products run.
-template<typename P, int NT, int ND, int J>
-__device__ __forceinline__ void gs_pass_block(const P *in, const P *tab, const int *st,
-                                              const int *dg, const unsigned *ent, int c, int ob,
-                                              int vs, int fill, P *v)
+//! Two inputs of one pass (M = 2, in1 beside in) share the list entries and
+//! factor blocks.
+template<typename P, int NT, int ND, int J, int M>
+__device__ __forceinline__ void gs_pass_block(const P *in, const P *in1, const P *tab, int plane,
+                                              const int *st, const int *dg, const unsigned *ent,
+                                              int c, int ob, int vs, int fill, P *v, P *v1)
 {
   constexpr int ds = (ND == 1) ? NT : NT * NT;
   const int d0 = dg[c];
   const int lo = (fill == gk_upper) ? d0 + 1 : st[c];
   const int hi = (fill == gk_lower) ? d0 : st[c + 1];
-  P av[NT * NT], xv[ds];
+  P av[NT * NT], xv[M][ds];
+  auto load = [&](unsigned e, P(&a)[NT * NT], P(&b)[M][ds]) {
+    gs_block_load<P, NT, ND>(tab, plane, in, e, ob, vs, a, b[0]);
+    if constexpr (M == 2)
+      gs_x_load<P, ds>(in1 + (e & 0xffffu) + ob, vs, b[1]);
+  };
+  auto apply = [&](auto cols) {
+    gs_block_fma<P, NT, ND, J, cols.value>(av, xv[0], v);
+    if constexpr (M == 2)
+      gs_block_fma<P, NT, ND, J, cols.value>(av, xv[1], v1);
+  };
   if (fill == gk_upper)
   {
-    gs_block_load<P, NT, ND>(tab, in, ent[d0], ob, vs, av, xv);
-    gs_block_fma<P, NT, ND, J, gs_from_diag>(av, xv, v);
+    load(ent[d0], av, xv);
+    apply(std::integral_constant<int, gs_from_diag>{});
   }
   if (lo < hi)
   {
-    gs_block_load<P, NT, ND>(tab, in, ent[lo], ob, vs, av, xv);
+    load(ent[lo], av, xv);
     unsigned en = ent[(lo + 1 < hi) ? lo + 1 : d0];
     for (int p = lo; p < hi; p++)
     {
-      P an[NT * NT], xn[ds];
-      gs_block_load<P, NT, ND>(tab, in, en, ob, vs, an, xn);
+      P an[NT * NT], xn[M][ds];
+      load(en, an, xn);
       en = ent[(p + 2 < hi) ? p + 2 : d0];
-      gs_block_fma<P, NT, ND, J, gs_all>(av, xv, v);
+      apply(std::integral_constant<int, gs_all>{});
 #pragma unroll
       for (int k = 0; k < NT * NT; k++)
         av[k] = an[k];
 #pragma unroll
-      for (int k = 0; k < ds; k++)
-        xv[k] = xn[k];
+      for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int k = 0; k < ds; k++)
+          xv[m][k] = xn[m][k];
     }
   }
   if (fill == gk_lower)
   {
-    gs_block_load<P, NT, ND>(tab, in, ent[d0], ob, vs, av, xv);
-    gs_block_fma<P, NT, ND, J, gs_before_diag>(av, xv, v);
+    load(ent[d0], av, xv);
+    apply(std::integral_constant<int, gs_before_diag>{});
   }
 }
 
@@ -753,7 +812,7 @@ __device__ __forceinline__ void gs_pass_block(const P *in, const P *tab, const i
 template<typename P, int NT, int ND, int TPB>
 __global__ void __launch_bounds__(TPB)
     gk_slab(gs_args a, const P *__restrict__ ctab, const gs_item *__restrict__ items,
-            const P *__restrict__ x, P *work, P *part)
+            const P *__restrict__ x, P *work)
 {
   extern __shared__ __align__(16) unsigned char gs_smem[];
   constexpr int nn = NT * NT;
@@ -764,15 +823,15 @@ __global__ void __launch_bounds__(TPB)
   // neighbouring cells fall on different LDS banks
   const int D = ds * C + gs_pad;
   const int BD = b.ncell * D;
-  const int nq = b.nq;
   const int ntab_lds = b.resident ? b.ntab : 1;
+  const int plane = b.tstride / ((nn + 1) / 2);
   gs_pass *pass = reinterpret_cast<gs_pass *>(gs_smem);
   P *X = reinterpret_cast<P *>(gs_smem + 16 * b.npass);
   P *Z = X + BD; // used when ND = 2
   P *tab = X + int64_t(BD) * ND;
   int *lists = reinterpret_cast<int *>(
       gs_smem + 16 * b.npass +
-      ((int64_t(BD) * ND + int64_t(ntab_lds) * nq * nn) * int64_t(sizeof(P)) + 15) / 16 * 16);
+      ((int64_t(BD) * ND + int64_t(ntab_lds) * b.tstride) * int64_t(sizeof(P)) + 15) / 16 * 16);
   gs_copy<TPB>(reinterpret_cast<int *>(pass), reinterpret_cast<const int *>(a.passes + b.pass0),
                4 * b.npass);
 
@@ -802,7 +861,7 @@ __global__ void __launch_bounds__(TPB)
   for (int si = 0; si < ds; si++)
     xv[si] = active ? x[gidx(si)] : P{0};
   if (b.resident)
-    gs_copy<TPB>(tab, ctab + b.cb, b.ntab * nq * nn);
+    gs_copy<TPB>(tab, ctab + b.cb, b.ntab * b.tstride);
   if (mine)
   {
 #pragma unroll
@@ -815,6 +874,10 @@ __global__ void __launch_bounds__(TPB)
 #pragma unroll
   for (int si = 0; si < ds; si++)
     acc[si] = 0;
+  P next[ds];
+#pragma unroll
+  for (int si = 0; si < ds; si++)
+    next[si] = 0;
   int cur_tab = -1, cur_j = -1;
   for (int pi = 0; pi < b.npass; pi++)
   {
@@ -827,26 +890,38 @@ __global__ void __launch_bounds__(TPB)
         gs_copy<TPB>(lists, a.lists + b.list0 + (ps.j == 0 ? 0 : b.llen[0]),
                      ps.j == 0 ? b.llen[0] : b.llen[1]);
       if (ps.tab != cur_tab)
-        gs_copy<TPB>(tab, ctab + b.cb + int64_t(ps.tab) * nq * nn, nq * nn);
+        gs_copy<TPB>(tab, ctab + b.cb + int64_t(ps.tab) * b.tstride, b.tstride);
       cur_tab = ps.tab;
       cur_j = ps.j;
     }
     __syncthreads();
     if (mine)
     {
-      const P *tb = b.resident ? tab + int64_t(ps.tab) * nq * nn : tab;
+      const P *tb = b.resident ? tab + int64_t(ps.tab) * b.tstride : tab;
       const int *st = (b.resident && ps.j == 1) ? lists + b.llen[0] : lists;
       const int *dg = st + b.ncell + 1;
       const unsigned *ent = reinterpret_cast<const unsigned *>(dg + b.ncell);
-      const P *in = (ps.mode == 2) ? Z : X;
-      P v[ds];
+      const P *in = (ps.mode >= 2) ? Z : X;
+      P v[ds], w[ds];
 #pragma unroll
       for (int si = 0; si < ds; si++)
-        v[si] = 0;
-      if (ND == 1 || ps.j == 0)
-        gs_pass_block<P, NT, ND, 0>(in, tb, st, dg, ent, c, ob, vs, ps.fill, v);
+        v[si] = w[si] = 0;
+      if constexpr (ND == 2)
+      {
+        if (ps.mode == 3)
+        {
+          if (ps.j == 0)
+            gs_pass_block<P, NT, ND, 0, 2>(in, X, tb, plane, st, dg, ent, c, ob, vs, ps.fill, v, w);
+          else
+            gs_pass_block<P, NT, ND, 1, 2>(in, X, tb, plane, st, dg, ent, c, ob, vs, ps.fill, v, w);
+        }
+        else if (ps.j == 1)
+          gs_pass_block<P, NT, ND, 1, 1>(in, in, tb, plane, st, dg, ent, c, ob, vs, ps.fill, v, w);
+        else
+          gs_pass_block<P, NT, ND, 0, 1>(in, in, tb, plane, st, dg, ent, c, ob, vs, ps.fill, v, w);
+      }
       else
-        gs_pass_block<P, NT, ND, 1>(in, tb, st, dg, ent, c, ob, vs, ps.fill, v);
+        gs_pass_block<P, NT, ND, 0, 1>(in, in, tb, plane, st, dg, ent, c, ob, vs, ps.fill, v, w);
 #pragma unroll
       for (int si = 0; si < ds; si++)
       {
@@ -854,6 +929,17 @@ __global__ void __launch_bounds__(TPB)
           Z[c * D + gs_at<P, ds>(si, ob, vs)] = v[si];
         else
           acc[si] += v[si];
+        next[si] = w[si];
+      }
+    }
+    if (ND == 2 && ps.mode == 3)
+    {
+      __syncthreads(); // the intermediate is read before it is replaced
+      if (mine)
+      {
+#pragma unroll
+        for (int si = 0; si < ds; si++)
+          Z[c * D + gs_at<P, ds>(si, ob, vs)] = next[si];
       }
     }
     // the next pass may overwrite what this one read, or read what it wrote
@@ -861,13 +947,235 @@ __global__ void __launch_bounds__(TPB)
   }
   if (active)
   {
-    // the cell in the group's slot, or this chain's partial of the cell
-    // (split items); entries at their offsets within the cell
-    P *out = (b.part < 0) ? work + int64_t(b.slot) * a.stride + int64_t(gc) * a.N
-                          : part + (int64_t(b.part) + int64_t(c) * b.nch + b.chain) * a.N;
+    P *out = work + int64_t(b.slot) * a.stride;
 #pragma unroll
     for (int si = 0; si < ds; si++)
-      out[gidx(si) - int64_t(gc) * a.N] = acc[si];
+      out[gidx(si)] = acc[si];
+  }
+}
+
+typedef int gs_int4 __attribute__((ext_vector_type(4)));
+
+constexpr int gs_rec_steps = 8;                // connections per lane of a split item
+constexpr int gs_rec_ints = 4 + gs_rec_steps;  // a lane record
+//! 16-byte pieces of a factor table a thread reads ahead: 80 KB for 1024
+//! threads, less where the blocks take the registers.
+constexpr int gs_table_ahead(int n) { return n == 2 ? 5 : (n == 3 ? 2 : 1); }
+
+//! First int of a lane record: its cell, the log2 of the lanes that share the
+//! block, whether it is the first of them, and its connections.  The second
+//! is the diagonal's list entry; from the fourth on the entries,
+//! filled up by repeating one.
+__host__ __device__ constexpr int gs_rec_meta(int c, int lg, bool first, int count)
+{
+  return c | lg << 10 | (first ? 1 : 0) << 13 | count << 16;
+}
+
+//! One split item (one chain of a large slab, one chunk) per workgroup: the
+//! chain's one or two passes, its partial of every cell written out.  Blocks
+//! in LDS as in gk_slab.
+//! What bounded a thread per block here was waiting: for the longest list
+//! (the level 0 and 1 cells are connected to their whole fibre, 128
+//! connections at level 7, 10 on average), and for one read of memory after
+//! another.  So a block with more than gs_rec_steps connections is shared by
+//! 2, 4 ... 64 neighbouring lanes, whose sums meet by shuffles; every lane
+//! reads its connections in one piece, a record ahead; and the factor table
+//! of the second pass is read while the first one runs.  The 1248 items of
+//! the d=6 n=2 level-7 FP64 Vlasov operator: 66 -> 48 us (LDS busy a third of
+//! it; what is left is the way from one read of memory to the next at an
+//! item's start, and two rounds of lanes where a pass has more than threads).
+template<typename P, int NT, int ND, int TPB>
+__global__ void __launch_bounds__(TPB, NT == 2 ? 4 : 1)
+    gk_slab_chain(gs_args a, const P *__restrict__ ctab, const gs_item *__restrict__ items,
+                  const P *__restrict__ x, P *part)
+{
+  extern __shared__ __align__(16) unsigned char gs_smem[];
+  constexpr int ds = (ND == 1) ? NT : NT * NT;
+  // the next connection's blocks are read ahead where registers allow
+  constexpr bool ahead_blocks = (NT * NT + ds) * sizeof(P) <= 144 / (TPB / 512 > 1 ? 2 : 1);
+  const gs_item b = items[blockIdx.x];
+  const int C = b.C;
+  const int D = ds * C + gs_pad;
+  const int BD = b.ncell * D;
+  P *X = reinterpret_cast<P *>(gs_smem);
+  P *Z = X + BD; // used when ND = 2
+  P *tab = reinterpret_cast<P *>(gs_smem + (int64_t(BD) * ND * sizeof(P) + 15) / 16 * 16);
+  const int plane = b.tstride / ((NT * NT + 1) / 2);
+  const int vs = gs_pair_major<P, ds> ? 2 * C : (gs_value_major<P> ? C : 1);
+  auto base = [&](int o) {
+    return gs_pair_major<P, ds> ? 2 * o : (gs_value_major<P> ? o : ds * o);
+  };
+  auto digit = [&](int si) { // entry si of a block, in its cell's tensor
+    return (ND == 1) ? si * b.str[0] : si / NT * b.str[0] + si % NT * b.str[1];
+  };
+  // factor table of pass p, first pieces into registers
+  const int pieces = b.tstride * int(sizeof(P)) / 16;
+  constexpr int TA = gs_table_ahead(NT);
+  gs_int4 ahead[TA];
+  // a pass by value: an index into b would put b into scratch memory
+  auto stage = [&](int p) { return p == 0 ? b.pass[0] : b.pass[1]; };
+  auto table = [&](int p) {
+    return reinterpret_cast<const gs_int4 *>(ctab + b.cb + int64_t(stage(p).ps.tab) * b.tstride);
+  };
+  auto read_table = [&](int p) {
+    const gs_int4 *src = table(p); // past its end the last piece again
+#pragma unroll
+    for (int u = 0; u < TA; u++)
+      ahead[u] = src[min(int(threadIdx.x) + u * TPB, pieces - 1)];
+  };
+  auto store_table = [&](int p) {
+#pragma unroll
+    for (int u = 0; u < TA; u++)
+    {
+      const int k = threadIdx.x + u * TPB;
+      if (k < pieces)
+        reinterpret_cast<gs_int4 *>(tab)[k] = ahead[u];
+    }
+    for (int k = threadIdx.x + TA * TPB; k < pieces; k += TPB)
+      reinterpret_cast<gs_int4 *>(tab)[k] = table(p)[k];
+  };
+  // lane i of pass p: record and entry
+  struct lane_rec
+  {
+    int o, off;
+    gs_int4 head, e0, e1;
+  };
+  auto read_lane = [&](int p, int i) {
+    lane_rec r;
+    const gs_lane_pass q = stage(p);
+    const int h = (i < q.nslot) ? a.slots[q.slot0 + i] : -1;
+    r.o = h < 0 ? -1 : h >> 16;
+    if (h >= 0)
+    {
+      const gs_int4 *rec =
+          reinterpret_cast<const gs_int4 *>(a.recs + q.rec0 + (h & 0xffff) * gs_rec_ints);
+      r.head = rec[0];
+      r.e0 = rec[1];
+      r.e1 = rec[2];
+      r.off = a.offs[b.off + r.o];
+    }
+    return r;
+  };
+  read_table(0);
+  lane_rec lane = read_lane(0, threadIdx.x);
+  {
+    const int c = threadIdx.x / C, o = threadIdx.x - c * C;
+    const int gc = (c < b.ncell) ? a.cells[b.cell0 + c] : -1;
+    const bool active = gc >= 0 && gc < a.active_cells;
+    const int64_t gbase = active ? int64_t(gc) * a.N + a.offs[b.off + o] : 0;
+    P xv[ds];
+#pragma unroll
+    for (int si = 0; si < ds; si++)
+      xv[si] = active ? x[gbase + digit(si)] : P{0};
+    store_table(0);
+    if (c < b.ncell)
+    {
+#pragma unroll
+      for (int si = 0; si < ds; si++)
+        X[c * D + gs_at<P, ds>(si, base(o), vs)] = xv[si];
+    }
+  }
+  __syncthreads();
+  for (int p = 0; p < b.npass; p++)
+  {
+    const gs_pass ps = stage(p).ps;
+    const int nslot = stage(p).nslot;
+    const P *in = (ps.mode == 2) ? Z : X;
+    if (p + 1 < b.npass)
+      read_table(p + 1);
+    // whole wavefronts: nslot is a multiple of 64, the most shared first
+    for (int i = threadIdx.x; i < nslot; i += TPB)
+    {
+      const lane_rec r = lane;
+      lane = read_lane(p, i + TPB);
+      const int meta = (r.o < 0) ? 0 : r.head.x;
+      const int c = meta & 1023, lg = meta >> 10 & 7, count = meta >> 16;
+      const bool first = (meta >> 13 & 1) != 0;
+      P v[ds];
+#pragma unroll
+      for (int si = 0; si < ds; si++)
+        v[si] = 0;
+      if (r.o >= 0)
+      {
+        const int ob = base(r.o);
+        auto fma_j = [&](auto cols, const P(&av)[NT * NT], const P(&xv)[ds]) {
+          if (ND == 1 || ps.j == 0)
+            gs_block_fma<P, NT, ND, 0, cols.value>(av, xv, v);
+          else
+            gs_block_fma<P, NT, ND, 1, cols.value>(av, xv, v);
+        };
+        P av[NT * NT], xv[ds];
+        if (first && ps.fill == gk_upper)
+        {
+          gs_block_load<P, NT, ND>(tab, plane, in, r.head.y, ob, vs, av, xv);
+          fma_j(std::integral_constant<int, gs_from_diag>{}, av, xv);
+        }
+        const unsigned e[gs_rec_steps + 1] = {
+            unsigned(r.e0.x), unsigned(r.e0.y), unsigned(r.e0.z), unsigned(r.e0.w), unsigned(r.e1.x),
+            unsigned(r.e1.y), unsigned(r.e1.z), unsigned(r.e1.w), unsigned(r.e1.w)};
+        if constexpr (ahead_blocks)
+          gs_block_load<P, NT, ND>(tab, plane, in, e[0], ob, vs, av, xv);
+#pragma unroll
+        for (int s = 0; s < gs_rec_steps; s++)
+        {
+          if (s >= count)
+            break;
+          if constexpr (ahead_blocks)
+          {
+            P an[NT * NT], xn[ds];
+            gs_block_load<P, NT, ND>(tab, plane, in, e[s + 1], ob, vs, an, xn);
+            fma_j(std::integral_constant<int, gs_all>{}, av, xv);
+#pragma unroll
+            for (int k = 0; k < NT * NT; k++)
+              av[k] = an[k];
+#pragma unroll
+            for (int k = 0; k < ds; k++)
+              xv[k] = xn[k];
+          }
+          else
+          {
+            gs_block_load<P, NT, ND>(tab, plane, in, e[s], ob, vs, av, xv);
+            fma_j(std::integral_constant<int, gs_all>{}, av, xv);
+          }
+        }
+        if (first && ps.fill == gk_lower)
+        {
+          gs_block_load<P, NT, ND>(tab, plane, in, r.head.y, ob, vs, av, xv);
+          fma_j(std::integral_constant<int, gs_before_diag>{}, av, xv);
+        }
+      }
+      const int most = __builtin_amdgcn_readfirstlane(lg);
+      for (int k = 0; k < most; k++)
+#pragma unroll
+        for (int si = 0; si < ds; si++)
+        {
+          const P w = __shfl_xor(v[si], 1 << k);
+          v[si] += (k < lg) ? w : P{0};
+        }
+      if (!first)
+        continue;
+      if (ps.mode == 1)
+      {
+#pragma unroll
+        for (int si = 0; si < ds; si++)
+          Z[c * D + gs_at<P, ds>(si, base(r.o), vs)] = v[si];
+      }
+      else
+      {
+        P *out = part + (int64_t(b.part) + int64_t(c) * b.nch + b.chain) * a.N + r.off;
+#pragma unroll
+        for (int si = 0; si < ds; si++)
+          out[digit(si)] = v[si];
+      }
+    }
+    if (p + 1 < b.npass)
+    {
+      // the next pass reads what this one wrote, with its own table
+      lane = read_lane(p + 1, threadIdx.x);
+      __syncthreads();
+      store_table(p + 1);
+      __syncthreads();
+    }
   }
 }
 
@@ -1011,7 +1319,8 @@ struct akm_global_s
   // run through the cell-layout stages
   bool slab = false; // chosen by global_autotune or akm_set_tuning
   int ngroups = 0;
-  akm::dev_buffer<int> gs_passes, gs_tabs, gs_items, gs_cells, gs_lists, gs_offs, gs_qmap;
+  akm::dev_buffer<int> gs_passes, gs_tabs, gs_items, gs_cells, gs_lists, gs_offs, gs_qmap,
+      gs_slots, gs_recs;
   // compact factor tables (per level bound, every group table), built from
   // vA by gs_tables at the first slab apply after vA changed (the matrix's
   // vA_stamp differs from gs_ctab_stamp); gs_lv: qmap starts then table
@@ -1026,6 +1335,7 @@ struct akm_global_s
   {
     int tpb;     // 256 or 1024 threads
     int nd;      // slab dimensions of its groups
+    bool split;  // one chain of a large slab per item
     bool side;   // on the side stream (split or 1024-thread items)
     int64_t lds; // dynamic LDS bytes (largest item of the launch)
     int first, count; // its items
@@ -1097,11 +1407,12 @@ static gk_args global_args(akm_matrix_s const &m)
   return a;
 }
 
-//! Launches one slab work-item class: `count` items from `items`.
+//! Launches one slab work-item class: `count` items from `items`, split ones
+//! into the partials, the others into the work buffer.
 template<typename P, int TPB>
-static int gs_launch_class(hipStream_t stream, int n, int nd, gs_args const &ga, const P *ctab,
-                           const gs_item *items, int count, int64_t lds, const P *x, P *work,
-                           P *part)
+static int gs_launch_class(hipStream_t stream, int n, int nd, bool split, gs_args const &ga,
+                           const P *ctab, const gs_item *items, int count, int64_t lds,
+                           const P *x, P *out)
 {
   auto go = [&](auto kern) -> int {
     if (lds > 64 * 1024 &&
@@ -1113,23 +1424,23 @@ static int gs_launch_class(hipStream_t stream, int n, int nd, gs_args const &ga,
       return set_error(AKM_ERR_HIP, "global kron slab: %lld bytes of LDS refused",
                        static_cast<long long>(lds));
     }
-    kern<<<count, TPB, static_cast<size_t>(lds), stream>>>(ga, ctab, items, x, work, part);
+    kern<<<count, TPB, static_cast<size_t>(lds), stream>>>(ga, ctab, items, x, out);
     return check_launch("global kron slab");
   };
   switch (n * 4 + nd)
   {
   case 2 * 4 + 1:
-    return go(gk_slab<P, 2, 1, TPB>);
+    return split ? go(gk_slab_chain<P, 2, 1, TPB>) : go(gk_slab<P, 2, 1, TPB>);
   case 2 * 4 + 2:
-    return go(gk_slab<P, 2, 2, TPB>);
+    return split ? go(gk_slab_chain<P, 2, 2, TPB>) : go(gk_slab<P, 2, 2, TPB>);
   case 3 * 4 + 1:
-    return go(gk_slab<P, 3, 1, TPB>);
+    return split ? go(gk_slab_chain<P, 3, 1, TPB>) : go(gk_slab<P, 3, 1, TPB>);
   case 3 * 4 + 2:
-    return go(gk_slab<P, 3, 2, TPB>);
+    return split ? go(gk_slab_chain<P, 3, 2, TPB>) : go(gk_slab<P, 3, 2, TPB>);
   case 4 * 4 + 1:
-    return go(gk_slab<P, 4, 1, TPB>);
+    return split ? go(gk_slab_chain<P, 4, 1, TPB>) : go(gk_slab<P, 4, 1, TPB>);
   case 4 * 4 + 2:
-    return go(gk_slab<P, 4, 2, TPB>);
+    return split ? go(gk_slab_chain<P, 4, 2, TPB>) : go(gk_slab<P, 4, 2, TPB>);
   default:
     return set_error(AKM_ERR_UNSUPPORTED, "global kron slab: n = %d", n);
   }
@@ -1152,11 +1463,19 @@ __global__ void __launch_bounds__(gk_threads)
     while (Lp + 1 < levels && i >= lv[levels + 1 + Lp + 1])
       Lp++;
     const int64_t rem = i - lv[levels + 1 + Lp];
-    const int64_t per = int64_t(lv[Lp + 1] - lv[Lp]) * nn;
+    const int nq = lv[Lp + 1] - lv[Lp];
+    const int64_t per = gs_table_values(nq, nn);
     const int t = static_cast<int>(rem / per);
-    const int64_t r2 = rem - t * per;
-    const int64_t qc = r2 / nn;
-    const int w = static_cast<int>(r2 - qc * nn);
+    const int r2 = static_cast<int>(rem - t * per);
+    if (r2 >= nq * nn)
+    {
+      ctab[i] = P{0};
+      continue;
+    }
+    // block qc, value w (gs_table_at)
+    const bool planes = sizeof(P) == 8 && nn % 2 == 0;
+    const int qc = planes ? r2 / 2 % nq : r2 / nn;
+    const int w = planes ? r2 / 2 / nq * 2 + r2 % 2 : r2 - qc * nn;
     const int q = qmap[lv[Lp] + qc];
     ctab[i] = vA[int64_t(q) * cstride + int64_t(tabs[2 * t]) * tstride +
                  int64_t(tabs[2 * t + 1]) * nn + w];
@@ -1179,6 +1498,8 @@ static int gs_apply(akm_matrix_s &m, const P *vA, const P *x, P *work)
   ga.cells = g.gs_cells.data();
   ga.lists = g.gs_lists.data();
   ga.offs = g.gs_offs.data();
+  ga.slots = g.gs_slots.data();
+  ga.recs = g.gs_recs.data();
   // the compact factor tables, rebuilt when vA changed since they were built
   const P *ctab = reinterpret_cast<const P *>(g.gs_ctab.data());
   if (!g.gs_ctab_valid || g.gs_ctab_stamp != m.vA_stamp)
@@ -1208,29 +1529,30 @@ static int gs_apply(akm_matrix_s &m, const P *vA, const P *x, P *work)
   const int bound = fork ? g.gs_side_items - std::min(g.gs_moved, g.gs_side_items)
                          : g.gs_side_items;
   P *part = reinterpret_cast<P *>(g.gs_part.data());
-  auto run = [&](hipStream_t s, int tpb, int nd, int first, int count) -> int {
+  auto run = [&](hipStream_t s, auto const &l, int first, int count) -> int {
     if (count <= 0)
       return AKM_SUCCESS;
     const gs_item *items = reinterpret_cast<const gs_item *>(g.gs_items.data()) + first;
     const int64_t lds = *std::max_element(g.gs_item_lds.begin() + first,
                                           g.gs_item_lds.begin() + first + count);
-    if (tpb == 1024)
-      return gs_launch_class<P, 1024>(s, m.n, nd, ga, ctab, items, count, lds, x, work, part);
-    if (tpb == 512)
-      return gs_launch_class<P, 512>(s, m.n, nd, ga, ctab, items, count, lds, x, work, part);
-    return gs_launch_class<P, 256>(s, m.n, nd, ga, ctab, items, count, lds, x, work, part);
+    P *out = l.split ? part : work;
+    if (l.tpb == 1024)
+      return gs_launch_class<P, 1024>(s, m.n, l.nd, l.split, ga, ctab, items, count, lds, x, out);
+    if (l.tpb == 512)
+      return gs_launch_class<P, 512>(s, m.n, l.nd, l.split, ga, ctab, items, count, lds, x, out);
+    return gs_launch_class<P, 256>(s, m.n, l.nd, l.split, ga, ctab, items, count, lds, x, out);
   };
   for (auto const &l : g.gs_launches)
     if (l.side)
-      AKM_TRY(run(side, l.tpb, l.nd, l.first, std::min(l.first + l.count, bound) - l.first));
+      AKM_TRY(run(side, l, l.first, std::min(l.first + l.count, bound) - l.first));
   for (auto const &l : g.gs_launches)
     if (!l.side)
-      AKM_TRY(run(m.stream, l.tpb, l.nd, l.first, l.count));
+      AKM_TRY(run(m.stream, l, l.first, l.count));
   for (auto const &l : g.gs_launches)
     if (l.side)
     {
       const int f = std::max(l.first, bound);
-      AKM_TRY(run(m.stream, l.tpb, l.nd, f, l.first + l.count - f));
+      AKM_TRY(run(m.stream, l, f, l.first + l.count - f));
     }
   if (fork)
   {
@@ -1646,6 +1968,69 @@ struct gs_plan_bundle
   int C = 1, Lp = 0, tpb = 256;
 };
 
+//! Where the lanes of a split bundle's pass are: slots, records.
+struct gs_lane_range
+{
+  int slot0 = -1, nslot = 0, rec0 = 0;
+};
+
+//! The lanes of a pass over a split bundle's cells with the `fill` part of
+//! their lists: every block shared by as many lanes (a power of two, at most
+//! 64) as its list has lots of gs_rec_steps connections, lane k taking every
+//! lanes-th from the k-th on; the most shared first, so that a block's lanes
+//! stay in one wavefront; filled up with -1 to whole wavefronts.  entry(p) is
+//! the packed LDS offsets of list position p; false when something does not
+//! fit.
+template<typename Entry>
+static bool gs_lanes(std::vector<int> const &cells, gk_lists const &ls, int fill, int C,
+                     Entry &&entry, std::vector<int> &slots, std::vector<int> &recs)
+{
+  std::vector<int> by_lg[7];
+  auto range = [&](int gc) {
+    return std::make_pair(fill == gk_upper ? ls.diag[gc] + 1 : ls.ptr[gc],
+                          fill == gk_lower ? ls.diag[gc] : ls.ptr[gc + 1]);
+  };
+  for (size_t c = 0; c < cells.size(); c++)
+  {
+    auto const [lo, hi] = range(cells[c]);
+    int lg = 0;
+    while (lg < 6 && (gs_rec_steps << lg) < static_cast<int>(hi - lo))
+      lg++;
+    if ((gs_rec_steps << lg) < static_cast<int>(hi - lo))
+      return false; // more than 512 connections: its table does not fit LDS either
+    by_lg[lg].push_back(static_cast<int>(c));
+  }
+  int nrec = 0;
+  for (int lg = 6; lg >= 0; lg--)
+    for (int c : by_lg[lg])
+    {
+      auto const [lo, hi] = range(cells[c]);
+      const int lanes = 1 << lg;
+      unsigned diag = 0;
+      if (!entry(ls.diag[cells[c]], diag))
+        return false;
+      for (int sub = 0; sub < lanes; sub++)
+      {
+        const int count = std::max<int>(0, static_cast<int>(hi - lo) - sub + lanes - 1) / lanes;
+        recs.insert(recs.end(), {gs_rec_meta(c, lg, sub == 0, count), static_cast<int>(diag), 0, 0});
+        unsigned e = diag;
+        for (int k = 0; k < gs_rec_steps; k++)
+        {
+          if (k < count && !entry(lo + sub + k * lanes, e))
+            return false;
+          recs.push_back(static_cast<int>(e));
+        }
+      }
+      for (int o = 0; o < C; o++)
+        for (int sub = 0; sub < lanes; sub++)
+          slots.push_back((nrec + sub) | o << 16);
+      nrec += lanes;
+    }
+  while (slots.size() % wave_size != 0)
+    slots.push_back(-1);
+  return nrec <= 0x10000;
+}
+
 //! Builds the slab layout: groups of the terms with one or two non-identity
 //! dimensions (act[t] after the flux swap), their slabs, bundles, lists and
 //! work items.  A group whose largest slab does not fit one workgroup at
@@ -1699,7 +2084,7 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     term_group[t] = static_cast<int>(gi);
   }
 
-  std::vector<int> bundles, groups, passes, tabs, items, cells, lists_img, offs;
+  std::vector<int> bundles, groups, passes, tabs, items, cells, lists_img, offs, slots, recs;
   struct item_rec
   {
     int bundle, h, tpb, nd;
@@ -1708,6 +2093,8 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     int chain = -1;          // >= 0: this chain of the group only (a split item)
     int Lp = 0;              // level bound of its bundle
     int pass_off = 0, pass_cnt = 0; // its passes within the group's
+    gs_pass pass[2] = {};
+    gs_lane_range lanes[2]; // its passes' lanes
   };
   std::vector<item_rec> irec;
   std::vector<int> loc(g.cells, -1);
@@ -1790,9 +2177,35 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
         open_vals += full;
         continue;
       }
-      // a slab whose chains run split (long lists) takes the widest chunks
-      const bool wide = lp >= gs_split_level && group_chains > 1;
-      const int64_t cap = (msz * ds <= gs_cap_small && !wide) ? gs_cap_small : gs_cap_large;
+      if (lp >= gs_split_level && group_chains > 1)
+      {
+        // its chains run split: chunks for 512 threads that let two
+        // workgroups share a CU, else for 1024
+        const int nq = qm0[lp + 1] - qm0[lp];
+        gs_plan_bundle one;
+        one.cells = sc;
+        one.Lp = lp;
+        for (int tpb : {512, 1024})
+        {
+          one.tpb = tpb;
+          one.C = call;
+          auto fits = [&] {
+            return msz * one.C <= tpb &&
+                   gs_split_lds(esize, nd, n, static_cast<int>(msz), one.C, nq) <=
+                       (tpb == 512 ? gs_lds_max / 2 : gs_lds_max);
+          };
+          while (one.C > 1 && !fits())
+            one.C /= n;
+          ok = fits();
+          if (ok)
+            break;
+        }
+        if (!ok)
+          break;
+        plan.push_back(one);
+        continue;
+      }
+      const int64_t cap = (msz * ds <= gs_cap_small) ? gs_cap_small : gs_cap_large;
       if (msz * ds > cap)
       {
         ok = false;
@@ -1804,10 +2217,6 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       one.tpb = (cap == gs_cap_small) ? blocks_small : 1024;
       one.C = call;
       while (msz * ds * one.C > cap)
-        one.C /= n;
-      // x and the intermediate of a wide chunk within 64 KB, which leaves LDS
-      // for the factor table and the lists
-      while (wide && one.C > 1 && msz * ds * one.C * esize * nd > 64 * 1024)
         one.C /= n;
       plan.push_back(one);
     }
@@ -1826,11 +2235,34 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     const int ntab = static_cast<int>(gterms.size()) * nd;
     int npass = 0;
     std::vector<std::pair<int, int>> gchains; // (first pass, passes) per chain
+    std::vector<gs_pass> gpass;               // their passes
+    std::vector<int> own;                     // the group's chains
+    auto pass_of = [&](int c, int st) {
+      const int ti = static_cast<int>(std::find(gterms.begin(), gterms.end(), ch_term[c]) -
+                                      gterms.begin());
+      const int j = (ch_dim[c * gk_max_dims + st] == S[0]) ? 0 : 1;
+      return gs_pass{ti * nd + j, j, ch_fill[c * gk_max_dims + st],
+                     (ch_nst[c] == 1) ? 0 : (st == 0 ? 1 : 2)};
+    };
+    auto add_pass = [](std::vector<int> &to, gs_pass const &ps) {
+      to.insert(to.end(), {ps.tab, ps.j, ps.fill, ps.mode});
+    };
+    // the first stage of chain c is the last of chain c2 of the same term:
+    // they run at once and share the lists and factor blocks (d=6 n=2 Vlasov
+    // at level 5 33.5 -> 31 us, level 6 43 -> 39 us, level 7 the same)
+    auto merged = [&](int c, int c2) {
+      return nd == 2 && ch_term[c] == ch_term[c2] && ch_nst[c] == 2 && ch_nst[c2] == 2 &&
+             ch_dim[c * gk_max_dims] == ch_dim[c2 * gk_max_dims + 1] &&
+             ch_fill[c * gk_max_dims] == ch_fill[c2 * gk_max_dims + 1];
+    };
     for (size_t c = 0; c < ch_term.size(); c++)
       if (term_group[ch_term[c]] == static_cast<int>(gi))
       {
+        own.push_back(static_cast<int>(c));
         gchains.emplace_back(npass, ch_nst[c]);
         npass += ch_nst[c];
+        for (int st = 0; st < ch_nst[c]; st++)
+          gpass.push_back(pass_of(static_cast<int>(c), st));
       }
 
     // each bundle's cells by their longest list, longest first: a wavefront
@@ -1850,7 +2282,7 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
 
     // lists, LDS sizes and items of the plan (checked before anything is kept)
     const int group_index = ngroups;
-    std::vector<int> b_rec, p_cells, p_lists;
+    std::vector<int> b_rec, p_cells, p_lists, p_slots, p_recs;
     std::vector<item_rec> p_items;
     const int bundle_base = static_cast<int>(bundles.size() / (sizeof(gs_bundle) / sizeof(int)));
     for (size_t bi = 0; bi < plan.size() && ok; bi++)
@@ -1866,8 +2298,35 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       rec.list0 = static_cast<int>(lists_img.size() + p_lists.size());
       for (int c = 0; c < ncell; c++)
         loc[pb.cells[c]] = c;
+      // element offset of the connected cell in x / the intermediate,
+      // element offset of its factor block in the table; false outside the
+      // slab (cannot happen) or past 16-bit offsets
+      auto entry = [&](gk_lists const &ls, int64_t p, unsigned &e) {
+        const int64_t xo = int64_t(loc[ls.cell[p]]) * (ds * pb.C + gs_pad);
+        const int64_t ao = int64_t(qc_of[pb.Lp][ls.q[p]]) * ((esize == 8 && nn % 2 == 0) ? 2 : nn);
+        e = static_cast<unsigned>(xo) | (static_cast<unsigned>(ao) << 16);
+        return xo >= 0 && ao >= 0 && xo <= 0xffff && ao <= 0xffff;
+      };
+      // a slab with long connection lists (level bound >= gs_split_level) runs
+      // one workgroup per chain: its passes are the longest.  The lanes of its
+      // passes, by (slab dimension, fill)
+      const bool split = pb.Lp >= gs_split_level && gchains.size() > 1;
+      gs_lane_range lanes_of[2][3];
+      for (size_t pi = 0; split && ok && pi < gpass.size(); pi++)
+      {
+        auto &where = lanes_of[gpass[pi].j][gpass[pi].fill];
+        if (where.slot0 >= 0)
+          continue;
+        gk_lists const &ls = lists[S[gpass[pi].j]];
+        const size_t s0 = p_slots.size();
+        where.slot0 = static_cast<int>(slots.size() + s0);
+        where.rec0 = static_cast<int>(recs.size() + p_recs.size());
+        ok = gs_lanes(pb.cells, ls, gpass[pi].fill, pb.C,
+                      [&](int64_t p, unsigned &e) { return entry(ls, p, e); }, p_slots, p_recs);
+        where.nslot = static_cast<int>(p_slots.size() - s0);
+      }
       int nent_max = 0, nent_sum = 0;
-      for (int j = 0; j < nd && ok; j++)
+      for (int j = 0; j < nd && ok && !split; j++)
       {
         // image: ncell + 1 starts, ncell diagonal positions, the entries
         gk_lists const &ls = lists[S[j]];
@@ -1881,17 +2340,13 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
           p_lists[img + ncell + 1 + c] = cnt + ls.diag[gc] - ls.ptr[gc];
           for (int p = ls.ptr[gc]; p < ls.ptr[gc + 1]; p++)
           {
-            // element offset of the connected cell in x / the intermediate,
-            // element offset of its factor block in the table
-            const int64_t xo = int64_t(loc[ls.cell[p]]) * (ds * pb.C + gs_pad);
-            const int64_t ao = int64_t(qc_of[pb.Lp][ls.q[p]]) * nn;
-            if (xo < 0 || ao < 0 || xo > 0xffff || ao > 0xffff)
+            unsigned e;
+            if (!entry(ls, p, e))
             {
-              ok = false; // outside the slab (cannot happen) or past 16-bit offsets
+              ok = false;
               break;
             }
-            p_lists.push_back(static_cast<int>(static_cast<unsigned>(xo) |
-                                               (static_cast<unsigned>(ao) << 16)));
+            p_lists.push_back(static_cast<int>(e));
             cnt++;
           }
         }
@@ -1912,6 +2367,8 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       rec.resident = (lds <= gs_lds_resident) ? 1 : 0;
       if (!rec.resident)
         lds = gs_lds_bytes(esize, nd, n, ncell, pb.C, nq, 1, 2 * ncell + 1 + nent_max, npass);
+      if (split)
+        lds = gs_split_lds(esize, nd, n, ncell, pb.C, nq);
       if (lds > gs_lds_max)
       {
         ok = false;
@@ -1920,9 +2377,6 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       const int *rp = reinterpret_cast<const int *>(&rec);
       b_rec.insert(b_rec.end(), rp, rp + sizeof(gs_bundle) / sizeof(int));
       p_cells.insert(p_cells.end(), pb.cells.begin(), pb.cells.end());
-      // a slab with long connection lists (level bound >= gs_split_level) runs
-      // one workgroup per chain: its passes are the longest
-      const bool split = pb.Lp >= gs_split_level && gchains.size() > 1;
       for (int h = 0; h < call / pb.C; h++)
       {
         if (!split)
@@ -1933,14 +2387,17 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
         }
         for (size_t k = 0; k < gchains.size(); k++)
         {
-          item_rec r{bundle_base + static_cast<int>(bi), h, pb.tpb, nd,
-                     gs_lds_bytes(esize, nd, n, ncell, pb.C, nq, 1, 2 * ncell + 1 + nent_max,
-                                  gchains[k].second),
-                     0};
+          item_rec r{bundle_base + static_cast<int>(bi), h, pb.tpb, nd, lds, 0};
           r.chain = static_cast<int>(k);
           r.Lp = pb.Lp;
           r.pass_off = gchains[k].first;
           r.pass_cnt = gchains[k].second;
+          for (int st = 0; st < r.pass_cnt; st++)
+          {
+            auto const &ps = gpass[r.pass_off + st];
+            r.pass[st] = ps;
+            r.lanes[st] = lanes_of[ps.j][ps.fill];
+          }
           p_items.push_back(r);
         }
       }
@@ -1981,22 +2438,21 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       for (int j = 0; j < nd; j++)
         tabs.insert(tabs.end(), {t, S[j]});
     grec.pass0 = static_cast<int>(passes.size() / 4);
-    for (size_t c = 0; c < ch_term.size(); c++)
+    for (size_t c = 0; c < own.size(); c++)
     {
-      const int t = ch_term[c];
-      if (term_group[t] != static_cast<int>(gi))
-        continue;
-      const int ti = static_cast<int>(std::find(gterms.begin(), gterms.end(), t) -
-                                      gterms.begin());
-      const int ns = ch_nst[c];
-      for (int st = 0; st < ns; st++)
+      if (c + 1 < own.size() && merged(own[c], own[c + 1]))
       {
-        const int k = ch_dim[c * gk_max_dims + st];
-        const int j = (k == S[0]) ? 0 : 1;
-        const gs_pass ps{ti * nd + j, j, ch_fill[c * gk_max_dims + st],
-                         (ns == 1) ? 0 : (st == 0 ? 1 : 2)};
-        passes.insert(passes.end(), {ps.tab, ps.j, ps.fill, ps.mode});
+        // F then L and U then F: U, both F at once, L
+        gs_pass f = pass_of(own[c], 0);
+        f.mode = 3;
+        add_pass(passes, pass_of(own[c + 1], 0));
+        add_pass(passes, f);
+        add_pass(passes, pass_of(own[c], 1));
+        c++;
+        continue;
       }
+      for (int st = 0; st < ch_nst[own[c]]; st++)
+        add_pass(passes, pass_of(own[c], st));
     }
     grec.npass = static_cast<int>(passes.size() / 4) - grec.pass0;
     grec.slot = 2 * g.nslots + group_index;
@@ -2005,6 +2461,8 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     bundles.insert(bundles.end(), b_rec.begin(), b_rec.end());
     cells.insert(cells.end(), p_cells.begin(), p_cells.end());
     lists_img.insert(lists_img.end(), p_lists.begin(), p_lists.end());
+    slots.insert(slots.end(), p_slots.begin(), p_slots.end());
+    recs.insert(recs.end(), p_recs.begin(), p_recs.end());
     irec.insert(irec.end(), p_items.begin(), p_items.end());
     gslot[gi] = group_index;
     ngroups++;
@@ -2023,11 +2481,11 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
   // largest slabs among them), about half the work on the Vlasov operator;
   // they come first, and gs_apply may run the last gs_moved of them on the
   // main stream
-  auto on_side = [](item_rec const &r) { return r.tpb == 1024; };
+  auto on_side = [](item_rec const &r) { return r.chain >= 0 || r.tpb == 1024; };
   auto cls = [&](item_rec const &r) {
     const int side = on_side(r) ? 0 : 1;
     const int size = (r.tpb == 1024) ? 0 : (r.tpb == 512 ? 1 : 2);
-    return (side * 3 + size) * 2 + (r.nd - 1);
+    return ((side * 3 + size) * 2 + (r.nd - 1)) * 2 + (r.chain >= 0 ? 0 : 1);
   };
   // within a launch the largest items first (the longest-running workgroups
   // start early)
@@ -2058,7 +2516,7 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
   const int64_t ntab_all = static_cast<int64_t>(tabs.size() / 2);
   std::vector<int64_t> cbase(L + 2, 0);
   for (int Lp = 0; Lp <= L; Lp++)
-    cbase[Lp + 1] = cbase[Lp] + ntab_all * (qm0[Lp + 1] - qm0[Lp]) * nn;
+    cbase[Lp + 1] = cbase[Lp] + ntab_all * gs_table_values(qm0[Lp + 1] - qm0[Lp], nn);
   if (cbase[L + 1] > (int64_t(1) << 31) - 1)
     return set_error(AKM_ERR_UNSUPPORTED, "global kron: slab factor tables too large");
   const gs_bundle *hb = reinterpret_cast<const gs_bundle *>(bundles.data());
@@ -2071,8 +2529,8 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     it.cell0 = bb.cell0;
     it.ncell = bb.ncell;
     it.C = bb.C;
-    it.nq = qm0[bb.Lp + 1] - qm0[bb.Lp];
-    it.cb = static_cast<int>(cbase[bb.Lp] + int64_t(gg.tab0) * it.nq * nn);
+    it.tstride = gs_table_values(qm0[bb.Lp + 1] - qm0[bb.Lp], nn);
+    it.cb = static_cast<int>(cbase[bb.Lp] + int64_t(gg.tab0) * it.tstride);
     it.resident = irec[i].resident;
     it.list0 = bb.list0;
     it.llen[0] = bb.llen[0];
@@ -2084,17 +2542,22 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     it.tab0 = gg.tab0;
     it.ntab = gg.ntab;
     const bool split = irec[i].chain >= 0;
-    it.pass0 = gg.pass0 + (split ? irec[i].pass_off : 0);
+    it.pass0 = gg.pass0;
     it.npass = split ? irec[i].pass_cnt : gg.npass;
     // a split item writes its chain's partials, which gk_sum adds
     it.slot = gg.slot;
     it.part = split ? part0[irec[i].bundle] : -1;
     it.nch = split ? nch_of[irec[i].bundle] : 0;
     it.chain = split ? irec[i].chain : 0;
+    for (int st = 0; split && st < irec[i].pass_cnt; st++)
+    {
+      it.pass[st] = gs_lane_pass{irec[i].pass[st], irec[i].lanes[st].slot0,
+                                 irec[i].lanes[st].nslot, irec[i].lanes[st].rec0};
+    }
     const int *ip = reinterpret_cast<const int *>(&it);
     items.insert(items.end(), ip, ip + sizeof(gs_item) / sizeof(int));
     if (g.gs_launches.empty() || cls(irec[i - 1]) != cls(irec[i]))
-      g.gs_launches.push_back({irec[i].tpb, irec[i].nd, on_side(irec[i]), 0,
+      g.gs_launches.push_back({irec[i].tpb, irec[i].nd, split, on_side(irec[i]), 0,
                                static_cast<int>(i), 0});
     auto &l = g.gs_launches.back();
     l.lds = std::max(l.lds, irec[i].lds);
@@ -2145,6 +2608,11 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     AKM_TRY(g.gs_cells.upload(cells.data(), int64_t(cells.size())));
     AKM_TRY(g.gs_lists.upload(lists_img.data(), int64_t(lists_img.size())));
     AKM_TRY(g.gs_offs.upload(offs.data(), int64_t(offs.size())));
+    if (!slots.empty())
+    {
+      AKM_TRY(g.gs_slots.upload(slots.data(), int64_t(slots.size())));
+      AKM_TRY(g.gs_recs.upload(recs.data(), int64_t(recs.size())));
+    }
     AKM_TRY(g.gs_qmap.upload(qmap.data(), int64_t(qmap.size())));
     std::vector<int> lv(qm0.begin(), qm0.end());
     for (int64_t v : cbase)

@@ -291,6 +291,31 @@ def test_slab_layout_parity(spec):
     assert rel(host(y32), ref) < TOL32
 
 
+@pytest.mark.parametrize("d,n,L,act", [
+    (1, 2, 7, [{0}]),             # a 128-connection list, 16 lanes a block
+    (1, 3, 6, [{0}, {0}]),        # blocks of an odd count of values
+    (2, 2, 5, [{0, 1}]),          # the first level that runs split, one term
+    (2, 2, 6, [{1}, {0, 1}]),     # 512 threads, one and two dimensions
+    (2, 3, 6, [{0, 1}]),          # FP64 of 9 values: 1024 threads
+    (2, 4, 5, [{0, 1}, {0, 1}]),  # 16 values a block
+    (3, 3, 5, [{0, 2}, {1}]),     # several chunks of a slab
+    (4, 2, 5, [{0, 3}, {1, 2}, {0, 3}])])
+def test_slab_layout_shared_lists(d, n, L, act):
+    """Slabs whose long connection lists several lanes share, against the
+    oracle; the parity bars of this file."""
+    c = grid_case(d, n, L, len(act), seed=57, identity=identity_for(d, act))
+    ref = gk.apply(d, n, c["table"], L, len(act), c["vA"], 0.75, c["x"], 2.0, c["y"],
+                   active=c["active"])
+    for dtype, tol in ((np.float64, TOL64), (np.float32, TOL32)):
+        m = global_matrix(c, active=True) if dtype == np.float64 else global_matrix(
+            c, np.float32, active=True)
+        m.set_tuning(waves_per_row=6)
+        assert m.slab_info()[0] == len({frozenset(a) for a in act})
+        y = dev(c["y"].astype(dtype))
+        m.apply(0.75, dev(c["x"].astype(dtype)), 2.0, y)
+        assert rel(host(y), ref) < tol
+
+
 def test_slab_layout_flux_direction_and_solve():
     from tests import global_dense
     from tests.kron_cases import grid_case_ops
