@@ -60,7 +60,10 @@ template<bool BACK>
 __device__ __forceinline__ f32x4 mlp_tile(const float *in, int ldi, int K, const float *W,
                                           int ldw, int j0)
 {
-  constexpr int U = 4; // blocks of 16 inputs read ahead
+  // blocks of 16 inputs read ahead: with two a row's 128-byte lines are read
+  // whole; three and four are slower (35 us, as below), as more rows' lines
+  // contend for the same sets of the first-level cache
+  constexpr int U = 2;
   f32x4 acc[4] = {};
   const int lane = threadIdx.x % 64, row = lane % 16, g = lane / 16;
   const float *arow = in + row * ldi + 4 * g;
@@ -135,8 +138,8 @@ struct mlp_pass
 //! What bounds it: the weights' way from L2, which every workgroup reads whole;
 //! with the products taken out the 256 x 256 layer takes as long (10 us), with
 //! the reads taken out half as long, and its matrix-core time is 3.6 us.
-//! 1024 samples of 80 -> 256 -> 256 -> 64 take 30 us (64 workgroups),
-//! 32768 take 260 us; with 8 wavefronts of two tiles each 33 and 311 us.
+//! 1024 samples of 80 -> 256 -> 256 -> 64 take 32 us (64 workgroups),
+//! 32768 take 235 us; with 8 wavefronts of two tiles each 37 and 311 us.
 //! Separate tiled products took 12-34 us for each of the layers (64 x 64
 //! tiles leave most of the chip idle).
 //! LDS: 16 x (K1 + 2 H + N3 + 16) floats, rows 4 floats apart beyond their
