@@ -2180,7 +2180,9 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       if (lp >= gs_split_level && group_chains > 1)
       {
         // its chains run split: chunks for 512 threads that let two
-        // workgroups share a CU, else for 1024
+        // workgroups share a CU, else for 1024 (d=6 n=2 Vlasov, levels 5 / 6 /
+        // 7: 31 / 39 / 92 us; 256 threads first 30 / 45 / 101, 1024 only
+        // 32 / 60 / 89)
         const int nq = qm0[lp + 1] - qm0[lp];
         gs_plan_bundle one;
         one.cells = sc;
