@@ -917,7 +917,6 @@ template<typename P>
 int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, P *y, P gamma,
                 const P *xg, const double *pc, double jdt)
 {
-  AKM_TRY(fibre_tables<P>(m, plan, m.stream));
   fl_args<P> a = fibre_args<P, P>(m, plan);
   a.x = x;
   a.y = y;
@@ -943,7 +942,8 @@ int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, 
 
 int fibre_refresh(akm_matrix_s const &m, fibre_plan &plan, hipStream_t stream)
 {
-  return fibre_tables<double>(m, plan, stream);
+  return (m.prec == AKM_F64) ? fibre_tables<double>(m, plan, stream)
+                             : fibre_tables<float>(m, plan, stream);
 }
 
 fibre_system fibre_batch_system(akm_matrix_s const &m, fibre_plan const &plan, double *V,
@@ -969,8 +969,7 @@ int launch_fibre_batch(int tpb, int groups, const fibre_system *fs, const int2 *
 
 bool fibre_apply_between(akm_matrix_s &m, fibre_plan &plan, const double *v, double c, double *w)
 {
-  if (!plan.built || !plan.slots_of_lanes || plan.stages.size() != 1 || plan.vectors != 0 ||
-      fibre_tables<float>(m, plan, m.stream) != AKM_SUCCESS)
+  if (!plan.built || !plan.slots_of_lanes || plan.stages.size() != 1 || plan.vectors != 0)
     return false;
   fl_args<float, double> a = fibre_args<float, double>(m, plan);
   a.x = v;

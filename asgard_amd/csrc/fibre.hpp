@@ -67,8 +67,7 @@ struct fibre_plan
   dev_buffer<int4> slots, pieces;
   dev_buffer<unsigned char> work, tab;
   // factor tables: table i sums the (term, dimension) pairs
-  // tab_src[tab_ptr[i] .. tab_ptr[i+1]); rebuilt when the matrix's vA_stamp
-  // differs from `stamp`
+  // tab_src[tab_ptr[i] .. tab_ptr[i+1]) of the vA the matrix had at `stamp`
   dev_buffer<int> tab_ptr, tab_src, c1_diag;
   int ntab = 0, nconn = 0, M = 0;
   int64_t stride = 0; // work vector size
@@ -97,7 +96,7 @@ struct fibre_system
 };
 fibre_system fibre_batch_system(akm_matrix_s const &m, fibre_plan const &plan, double *V,
                                 double *X, int64_t size, double dt);
-//! Rebuilds an FP64 plan's factor tables on `stream` when vA changed.
+//! Rebuilds the plan's factor tables on `stream` when vA changed.
 int fibre_refresh(akm_matrix_s const &m, fibre_plan &plan, hipStream_t stream);
 //! One workgroup of tpb threads per (system, group) of `items`.
 int launch_fibre_batch(int tpb, int groups, const fibre_system *fs, const int2 *items,

@@ -1322,14 +1322,11 @@ struct akm_global_s
   akm::dev_buffer<int> gs_passes, gs_tabs, gs_items, gs_cells, gs_lists, gs_offs, gs_qmap,
       gs_slots, gs_recs;
   // compact factor tables (per level bound, every group table), built from
-  // vA by gs_tables at the first slab apply after vA changed (the matrix's
-  // vA_stamp differs from gs_ctab_stamp); gs_lv: qmap starts then table
-  // starts per level bound (gs_levels + 1 each)
+  // vA by gs_tables with the layout and by every call that rewrites vA;
+  // gs_lv: qmap starts then table starts per level bound (gs_levels + 1 each)
   akm::dev_buffer<unsigned char> gs_ctab;
   akm::dev_buffer<int> gs_lv;
   int64_t gs_ctab_count = 0;
-  uint64_t gs_ctab_stamp = 0;
-  bool gs_ctab_valid = false;
   int gs_levels = 0;
   struct gs_launch
   {
@@ -1482,9 +1479,37 @@ __global__ void __launch_bounds__(gk_threads)
   }
 }
 
+//! The compact factor tables of the slab layout, from vA.
+template<typename P>
+static int gs_refresh(akm_matrix_s const &m, akm_global_s &g)
+{
+  const int nn = m.n * m.n;
+  const int64_t tstride = int64_t(m.d) * nn;
+  gs_tables<P><<<gk_blocks(g.gs_ctab_count), gk_threads, 0, m.stream>>>(
+      reinterpret_cast<const P *>(m.vA.data()), g.gs_tabs.data(),
+      static_cast<int>(g.gs_tabs.size() / 2), g.gs_qmap.data(), g.gs_lv.data(), g.gs_levels, nn,
+      tstride, tstride * m.T, g.gs_ctab_count, reinterpret_cast<P *>(g.gs_ctab.data()));
+  return check_launch("global kron slab tables");
+}
+
+static int gs_refresh(akm_matrix_s const &m, akm_global_s &g)
+{
+  return (m.prec == AKM_F64) ? gs_refresh<double>(m, g) : gs_refresh<float>(m, g);
+}
+
+int global_tables(akm_matrix_s &m)
+{
+  akm_global_s &g = *m.gk;
+  if (g.fl.built)
+    AKM_TRY(fibre_refresh(m, g.fl, m.stream));
+  if (g.ngroups > 0)
+    AKM_TRY(gs_refresh(m, g));
+  return AKM_SUCCESS;
+}
+
 //! Every slab group's sum into its work-buffer slot.
 template<typename P>
-static int gs_apply(akm_matrix_s &m, const P *vA, const P *x, P *work)
+static int gs_apply(akm_matrix_s &m, const P *x, P *work)
 {
   akm_global_s &g = *m.gk;
   gs_args ga{};
@@ -1500,20 +1525,7 @@ static int gs_apply(akm_matrix_s &m, const P *vA, const P *x, P *work)
   ga.offs = g.gs_offs.data();
   ga.slots = g.gs_slots.data();
   ga.recs = g.gs_recs.data();
-  // the compact factor tables, rebuilt when vA changed since they were built
   const P *ctab = reinterpret_cast<const P *>(g.gs_ctab.data());
-  if (!g.gs_ctab_valid || g.gs_ctab_stamp != m.vA_stamp)
-  {
-    const int nn = m.n * m.n;
-    const int64_t tstride = int64_t(m.d) * nn;
-    gs_tables<P><<<gk_blocks(g.gs_ctab_count), gk_threads, 0, m.stream>>>(
-        vA, g.gs_tabs.data(), static_cast<int>(g.gs_tabs.size() / 2), g.gs_qmap.data(),
-        g.gs_lv.data(), g.gs_levels, nn, tstride, tstride * m.T, g.gs_ctab_count,
-        reinterpret_cast<P *>(g.gs_ctab.data()));
-    AKM_TRY(check_launch("global kron slab tables"));
-    g.gs_ctab_stamp = m.vA_stamp;
-    g.gs_ctab_valid = true;
-  }
   // the side launches come first and run on the side stream; gk_sum
   // follows the join
   // with every side item moved there is nothing to fork
@@ -1635,7 +1647,7 @@ static int global_apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y
     AKM_TRY(check_launch("global kron stage"));
   }
   if (slab)
-    AKM_TRY(gs_apply<P>(m, vA, x, work));
+    AKM_TRY(gs_apply<P>(m, x, work));
   const int *src = slab ? g.src_slab.data() : g.src_chain.data();
   const int nsrc = slab ? g.nsrc_slab : g.nsrc_chain;
   gs_split_view<P> sv{};
@@ -1680,6 +1692,7 @@ int global_update(akm_matrix_s &m, const void *vA)
 {
   AKM_HIP(hipMemcpyAsync(m.vA.data(), vA, m.num_vA * m.esize, hipMemcpyHostToDevice, m.stream));
   AKM_TRY(global_device_jacobi(m));
+  AKM_TRY(global_tables(m));
   AKM_HIP(hipStreamSynchronize(m.stream));
   return AKM_SUCCESS;
 }
@@ -1738,15 +1751,18 @@ int global_device_jacobi(akm_matrix_s &m)
   return check_launch("global kron Jacobi diagonal");
 }
 
-//! Builds the fibre-walk plan on first use.
+//! Builds the fibre-walk plan and its tables on first use.
 static int need_fibre_plan(akm_matrix_s &m)
 {
   akm_global_s &g = *m.gk;
   if (g.fl.built)
     return AKM_SUCCESS;
   g.fl = fibre_plan();
-  return build_fibre_plan(m, g.active_cells, g.cells, g.elem_host.data(), g.lists, g.term_act,
-                          g.c1_diag_h, g.fl);
+  AKM_TRY(build_fibre_plan(m, g.active_cells, g.cells, g.elem_host.data(), g.lists, g.term_act,
+                           g.c1_diag_h, g.fl));
+  AKM_TRY(fibre_refresh(m, g.fl, m.stream));
+  AKM_HIP(hipStreamSynchronize(m.stream)); // another stream may be captured next
+  return AKM_SUCCESS;
 }
 
 bool factored_batch_plan(akm_matrix_s const &m, fibre_plan &plan, int &rc)
@@ -2622,7 +2638,6 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     AKM_TRY(g.gs_lv.upload(lv.data(), int64_t(lv.size())));
     AKM_TRY(g.gs_ctab.allocate(cbase[L + 1] * esize));
     g.gs_ctab_count = cbase[L + 1];
-    g.gs_ctab_valid = false;
     g.gs_levels = L + 1;
   }
 
@@ -2665,7 +2680,7 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
   return AKM_SUCCESS;
 }
 
-//! Builds the slab layout on first use.  Chains outside its groups run in the
+//! Builds the slab layout and its tables on first use.  Chains outside its groups run in the
 //! chain layouts, which a pair handle does not have.
 static int need_slabs(akm_matrix_s &m, akm_global_s &g)
 {
@@ -2673,12 +2688,15 @@ static int need_slabs(akm_matrix_s &m, akm_global_s &g)
     return AKM_SUCCESS;
   g.slabs_built = true;
   AKM_TRY(build_slabs(m, g));
-  if (!g.pair)
-    return AKM_SUCCESS;
-  if (g.max_stages > 0 && g.stage_count_rest[0] > 0)
+  if (g.pair && g.max_stages > 0 && g.stage_count_rest[0] > 0)
     g.ngroups = 0;
-  return (g.ngroups > 0) ? g.work.allocate(int64_t(g.ngroups) * g.cells * m.N * int64_t(m.esize))
-                         : AKM_SUCCESS;
+  if (g.ngroups == 0)
+    return AKM_SUCCESS;
+  if (g.pair)
+    AKM_TRY(g.work.allocate(int64_t(g.ngroups) * g.cells * m.N * int64_t(m.esize)));
+  AKM_TRY(gs_refresh(m, g));
+  AKM_HIP(hipStreamSynchronize(m.stream)); // another stream may be captured next
+  return AKM_SUCCESS;
 }
 
 //! Builds the padded cell set, the fibres, the chains and the work buffers
@@ -2993,7 +3011,7 @@ int factored_refresh(akm_matrix_s &m, const void *values)
   {
     m.form_stamp += m.factored ? 0 : 1;
     m.factored = true;
-    return AKM_SUCCESS;
+    return global_tables(m);
   }
   if (mask == m.factored_mask)
     return AKM_SUCCESS; // no factored form for these factors

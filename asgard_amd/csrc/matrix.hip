@@ -198,6 +198,18 @@ void use_stream(akm_matrix_s &m, hipStream_t stream)
   (void)hipGetLastError(); // a destroyed old stream has no work left
 }
 
+//! True while work enqueued on the stream is recorded into a graph (the null
+//! stream cannot be captured).
+static bool capturing(hipStream_t stream)
+{
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (stream == nullptr)
+    return false;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess)
+    (void)hipGetLastError();
+  return status != hipStreamCaptureStatusNone;
+}
+
 int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void *y,
                  double gamma, const void *xg)
 {
@@ -205,7 +217,10 @@ int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void
     return set_error(AKM_ERR_INVALID, "identity term needs a square operator");
   if (m.mode == mode_global)
     return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
-  if (m.factored && !m.pair_kernels)
+  // A captured apply is replayed whenever its owner likes, beside other applies
+  // and after new factors of another form: it takes the pair kernels, which
+  // read nothing but x and the stored factors, at addresses that stay.
+  if (m.factored && !m.pair_kernels && !capturing(m.stream))
   {
     std::lock_guard<std::mutex> lock(m.factored_mtx);
     return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
@@ -287,8 +302,6 @@ akm_status akm_set_stream(akm_matrix mat, void *stream)
   if (mat == nullptr)
     return set_error(AKM_ERR_INVALID, "null matrix");
   use_stream(*mat, static_cast<hipStream_t>(stream));
-  // tables derived from vA are rebuilt on the new stream
-  mat->vA_stamp++;
   return AKM_SUCCESS;
 }
 

@@ -25,8 +25,8 @@ struct akm_matrix_s
   akm::dev_buffer<int> indx, iA;
   akm::dev_buffer<unsigned char> vA;
   int64_t num_vA = 0;
-  // advanced by every call that rewrites vA, so tables derived from it know
-  // when to rebuild
+  // advanced by every call that rewrites vA, so that a batch knows when to
+  // rebuild the tables of its plans
   uint64_t vA_stamp = 0;
   // the first implicit solve's timed operator apply (ms; -1 before it),
   // which decides whether GMRES steps are enqueued ahead
@@ -119,6 +119,10 @@ int global_update(akm_matrix_s &m, const void *vA);
 //! Global operator: Jacobi diagonal rebuilt on the device from the stored
 //! factor blocks (after they were written on the device).
 int global_device_jacobi(akm_matrix_s &m);
+//! Rebuilds the factor tables of every plan the handle has from the stored
+//! factors, in place.  An apply never does: it may be captured into a graph,
+//! or be the first after one was.
+int global_tables(akm_matrix_s &m);
 //! Sparse-grid handle: builds the factored form of its operator (`elem`: cell
 //! 1D indices, vA: host factor blocks) when the factors allow one that is
 //! faster than the pair kernels.

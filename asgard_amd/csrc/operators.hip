@@ -119,7 +119,10 @@ static int update_operators_typed(akm_matrix_s &m, const void *const *ops_dev, i
     AKM_TRY(check_launch("operator update (LDS tables)"));
   }
   if (m.mode == mode_global)
+  {
     AKM_TRY(global_device_jacobi(m));
+    AKM_TRY(global_tables(m));
+  }
   return AKM_SUCCESS;
 }
 

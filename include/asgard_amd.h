@@ -112,7 +112,10 @@ akm_status akm_create_sparse(int d, int n, int rows, int cols, int num_terms,
  * non-identity factors couple.  akm_update_coefficients and
  * akm_update_operators look at the new factors and choose again; a shape
  * given to akm_set_tuning or akm_set_kernel_family selects the pair-by-pair
- * kernels, akm_set_tuning(mat, 0, -1, 0) the automatic choice. */
+ * kernels, akm_set_tuning(mat, 0, -1, 0) the automatic choice.  An apply
+ * captured into a graph always records the pair-by-pair kernels: they use no
+ * work vectors and read the stored factors in place, so a replay applies the
+ * operator of its time, whatever the form of the factors it was updated to. */
 akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *table,
                                   int max_level, int num_terms, const void *vA,
                                   int64_t num_vA, akm_prec prec, akm_matrix *mat);
