@@ -103,16 +103,17 @@ __device__ __forceinline__ double bt_block_sum(double v, double *sh)
   return r;
 }
 
-//! Start of a cycle: active = !converged, m = 0; column counter = 0.
-__global__ void bt_begin(int nsys, bt_state *st, int *active, int *jcol)
+//! Start of a cycle: active = open = !converged, m = 0; column counter = 0.
+__global__ void bt_begin(int nsys, bt_state *st, int *active, int *open, int *jcol)
 {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s == 0)
     *jcol = 0;
   if (s < nsys)
   {
-    active[s] = st[s].converged ? 0 : 1;
-    st[s].open = active[s];
+    const int on = st[s].converged ? 0 : 1;
+    active[s] = open[s] = on;
+    st[s].open = on;
     st[s].m = 0;
     st[s].finished = -2;
   }
@@ -235,9 +236,11 @@ __device__ __forceinline__ void bt_rotg(double &a, double b, double &c, double &
 //! One workgroup finishes step j of system s (j < 0: the cycle's start, with
 //! the convergence test on the true residual): |w|, Hessenberg column j, old
 //! rotations, the new one, the estimate; m = j + 1; a system whose estimate is
-//! below tolerance leaves the cycle.
-__device__ __forceinline__ void bt_finish_step(bt_sys const &q, bt_state *st, int *active, int s,
-                                               int j)
+//! below tolerance leaves the cycle: open = 0.  `active` is only read: row
+//! workgroups of the same launch read it too, and the update after them takes
+//! it over from `open`.
+__device__ __forceinline__ void bt_finish_step(bt_sys const &q, bt_state *st, const int *active,
+                                               int *open, int s, int j)
 {
   __shared__ double sh[bt_threads / wave_size];
   __shared__ double lc[bt_max_restart], lcs[bt_max_restart], lsn[bt_max_restart];
@@ -270,7 +273,7 @@ __device__ __forceinline__ void bt_finish_step(bt_sys const &q, bt_state *st, in
       {
         state.converged = 1;
         state.open = 0;
-        active[s] = 0;
+        open[s] = 0;
       }
     }
     else
@@ -298,7 +301,7 @@ __device__ __forceinline__ void bt_finish_step(bt_sys const &q, bt_state *st, in
       if (state.res <= state.tol)
       {
         state.open = 0;
-        active[s] = 0;
+        open[s] = 0;
       }
     }
   }
@@ -308,20 +311,24 @@ __device__ __forceinline__ void bt_finish_step(bt_sys const &q, bt_state *st, in
 }
 
 //! Finishes the start of the cycle (advance = 0), or the last step of a chunk
-//! of `advance` iterations and advances the column counter.
+//! of `advance` iterations.
 __global__ void __launch_bounds__(bt_threads)
-bt_finish(const bt_sys *sys, bt_state *st, int *active, const int *jcol, int advance, int limit)
+bt_finish(const bt_sys *sys, bt_state *st, int *active, int *open, const int *jcol, int advance,
+          int limit)
 {
   const int s = blockIdx.x;
-  bt_finish_step(sys[s], st, active, s,
+  bt_finish_step(sys[s], st, active, open, s,
                  (advance == 0) ? -1 : min(*jcol + advance, limit) - 1);
+  __syncthreads(); // every thread has read the flag
+  if (threadIdx.x == 0)
+    active[s] = open[s];
 }
 
 //! partial dots of V_s[k], k <= j, with w = V_s[j+1]; the workgroups past the
 //! row blocks finish step j - 1 of their system.  The reduction is gm_dots'.
 __global__ void __launch_bounds__(bt_threads)
-bt_dots(const int *dot_sys, int total, const bt_sys *sys, bt_state *st, int *active,
-        const int *jcol, int joff, int limit)
+bt_dots(const int *dot_sys, int total, const bt_sys *sys, bt_state *st, const int *active,
+        int *open, const int *jcol, int joff, int limit)
 {
   static_assert(bt_cols == 4, "the exchange below halves four columns twice");
   __shared__ double sh[bt_threads / wave_size][bt_cols];
@@ -332,14 +339,14 @@ bt_dots(const int *dot_sys, int total, const bt_sys *sys, bt_state *st, int *act
   {
     const int s = blockIdx.x - total;
     if (blockIdx.y == 0)
-      bt_finish_step(sys[s], st, active, s, j - 1);
+      bt_finish_step(sys[s], st, active, open, s, j - 1);
     return;
   }
   const int s = dot_sys[blockIdx.x];
   const int ncols = j + 1;
   const int k0 = blockIdx.y * bt_cols;
-  // a system that leaves in this launch may or may not be skipped here; the
-  // update skips it either way
+  // a system that leaves in this launch is still taken here; the update
+  // skips it
   if (k0 >= ncols || !active[s])
     return;
   const bt_sys q = sys[s];
@@ -383,20 +390,26 @@ bt_dots(const int *dot_sys, int total, const bt_sys *sys, bt_state *st, int *act
   }
 }
 
-//! h_s, then w <- w / |v_j| - V_s[0..j] h_s and the partials of |w|^2.
+//! h_s, then w <- w / |v_j| - V_s[0..j] h_s and the partials of |w|^2 for the
+//! systems still open; a system's first workgroup takes its flag over.
 __global__ void __launch_bounds__(bt_upd_threads)
-bt_update(const int *upd_sys, const bt_sys *sys, const int *active, const int *jcol, int joff,
-          int limit)
+bt_update(const int *upd_sys, const bt_sys *sys, int *active, const int *open, const int *jcol,
+          int joff, int limit)
 {
   __shared__ double red[bt_split][bt_tile];
   __shared__ double sh[bt_upd_threads / wave_size];
   __shared__ double cf[bt_max_restart]; // h_k / |stored v_k|
   const int s = upd_sys[blockIdx.x];
   const int j = *jcol + joff;
-  if (j >= limit || !active[s])
+  if (j >= limit)
     return;
   const bt_sys q = sys[s];
   const int t = threadIdx.x, ncols = j + 1, lb = blockIdx.x - q.upd0;
+  const int on = open[s]; // not written in this launch
+  if (lb == 0 && t == 0)
+    active[s] = on;
+  if (on == 0)
+    return;
   const double invj = q.inv[j];
   for (int k = t / bt_lanes; k < ncols; k += bt_upd_threads / bt_lanes)
   {
@@ -570,7 +583,7 @@ struct akm_batch_s
   std::vector<batch_system> host_vsys;
   dev_buffer<bt_sys> sys;
   dev_buffer<bt_state> state;
-  dev_buffer<int> active, jcol, dot_sys, upd_sys;
+  dev_buffer<int> active, open_dev, jcol, dot_sys, upd_sys;
   dev_buffer<double> V, X, B, small;
   bt_state *host_state = nullptr; // pinned
   std::vector<int> dot0;          // first dot-product block per system, and the total
@@ -615,14 +628,14 @@ struct akm_batch_s
   int enqueue_start()
   {
     bt_begin<<<(nsys + 255) / 256, 256, 0, stream>>>(nsys, state.data(), active.data(),
-                                                   jcol.data());
+                                                     open_dev.data(), jcol.data());
     bt_copy_rhs<<<dot_blocks, bt_threads, 0, stream>>>(dot_sys.data(), sys.data(),
                                                        active.data());
     AKM_TRY(check_launch("batch start"));
     AKM_TRY(apply_all(0, 0));
     bt_sumsq<<<dot_blocks, bt_threads, 0, stream>>>(dot_sys.data(), sys.data(), active.data());
     bt_finish<<<nsys, bt_threads, 0, stream>>>(sys.data(), state.data(), active.data(),
-                                               jcol.data(), 0, restart);
+                                               open_dev.data(), jcol.data(), 0, restart);
     return check_launch("batch residual");
   }
 
@@ -633,14 +646,14 @@ struct akm_batch_s
       AKM_TRY(apply_all(1, i));
       const dim3 dgrid(dot_blocks + nsys, (restart + bt_cols - 1) / bt_cols);
       bt_dots<<<dgrid, bt_threads, 0, stream>>>(dot_sys.data(), dot_blocks, sys.data(),
-                                               state.data(), active.data(), jcol.data(), i,
-                                               restart);
+                                               state.data(), active.data(), open_dev.data(),
+                                               jcol.data(), i, restart);
       bt_update<<<upd_blocks, bt_upd_threads, 0, stream>>>(upd_sys.data(), sys.data(),
-                                                           active.data(), jcol.data(), i,
-                                                           restart);
+                                                           active.data(), open_dev.data(),
+                                                           jcol.data(), i, restart);
     }
     bt_finish<<<nsys, bt_threads, 0, stream>>>(sys.data(), state.data(), active.data(),
-                                               jcol.data(), bt_chunk, restart);
+                                               open_dev.data(), jcol.data(), bt_chunk, restart);
     bt_advance<<<1, 64, 0, stream>>>(jcol.data(), bt_chunk);
     return check_launch("batch iterations");
   }
@@ -952,6 +965,7 @@ akm_status akm_batch_create(int count, const akm_matrix *mats, const double *dts
   AKM_TRY(b->state.upload(st0.data(), count));
   std::vector<int> ones(count, 1);
   AKM_TRY(b->active.upload(ones.data(), count));
+  AKM_TRY(b->open_dev.upload(ones.data(), count));
   int zero = 0;
   AKM_TRY(b->jcol.upload(&zero, 1));
   AKM_HIP(hipHostMalloc(reinterpret_cast<void **>(&b->host_state), sizeof(bt_state) * count,

@@ -98,3 +98,22 @@ def test_batch_rejects_unsupported_systems():
     m6 = asgard_amd.KronmultMatrix.sparse_grid(6, 3, t6, 1, 1, v6)
     with pytest.raises(asgard_amd.AkmError):
         asgard_amd.BatchSolver([m6], [0.1])
+
+
+def test_systems_leave_the_cycle_one_by_one():
+    """Systems that converge at different steps of one cycle: each result is
+    bit for bit the one it has alone."""
+    specs = [(2, 2, 4, 1e-4), (2, 2, 5, 2e-2), (3, 2, 4, 1e-3), (2, 3, 4, 5e-3), (3, 2, 3, 5e-2)]
+    mats = [make_system(d, n, L, seed=20 + i) for i, (d, n, L, _) in enumerate(specs)]
+    dts = [s[3] for s in specs]
+    rng = np.random.default_rng(6)
+    bs = [dev(rng.uniform(-1, 1, m.output_size())) for m in mats]
+    xs = [torch.zeros_like(b) for b in bs]
+    batch = asgard_amd.BatchSolver(mats, dts, restart=40)
+    _, its, conv = batch.solve(xs, bs, tol=1e-9)
+    assert conv.all() and len(set(its.tolist())) > 2, its
+    for m, dt, x, b, it in zip(mats, dts, xs, bs, its):
+        alone = torch.zeros_like(b)
+        _, own, _ = asgard_amd.BatchSolver([m], [dt], restart=40).solve([alone], [b], tol=1e-9)
+        assert own[0] == it
+        assert torch.equal(alone, x)
