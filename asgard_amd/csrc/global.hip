@@ -1588,14 +1588,18 @@ static int global_apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y
                                                                   jdt);
     return check_launch("global kron scale");
   }
-  if (!g.slab && g.lanes == 8)
+  // the walk's last stage writes y while other workgroups still read x: a
+  // global handle's apply in place takes the chain layout, which forms y in a
+  // pass of its own that reads x at its own positions only
+  const bool in_place = !g.pair && x < y + dofs && y < x + dofs;
+  if (!g.slab && g.lanes == 8 && !in_place)
     return fibre_apply<P>(m, g.fl, alpha, x, beta, y, gamma, xg, pc, jdt);
   const gk_args a = global_args(m);
   const P *vA = reinterpret_cast<const P *>(m.vA.data());
   P *work = reinterpret_cast<P *>(g.work.data());
   // the slab layout runs the chains outside its groups in the cell layout
   const bool slab = g.slab;
-  const int lanes = slab ? (m.N <= wave_size ? 0 : 1) : g.lanes;
+  const int lanes = (slab || g.lanes == 8) ? (m.N <= wave_size ? 0 : 1) : g.lanes;
   for (int st = 0; st < g.max_stages; st++)
   {
     const int nl = slab ? g.stage_count_rest[st] : g.stage_count[st];

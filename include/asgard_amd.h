@@ -187,7 +187,8 @@ akm_status akm_update_operators(akm_matrix mat, const void *const *ops, int64_t 
 
 /* kronmult_matrix<P>::apply<resource>(alpha, x, beta, y)
  * (src/asgard_kronmult_matrix.hpp:340-478): y = alpha*A*x + beta*y.
- * With no terms: y = beta*y.  beta == 0 never reads y. */
+ * With no terms: y = beta*y.  beta == 0 never reads y.  y may be x on a global
+ * handle; elsewhere the two must not overlap. */
 akm_status akm_apply(akm_matrix mat, double alpha, const void *x, double beta, void *y,
                      int on_device);
 

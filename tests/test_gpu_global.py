@@ -73,7 +73,7 @@ def _case_and_refs(spec):
     return _ORACLE[key]
 
 
-# lane per DOF, 8 lanes per DOF, wavefront per cell (3: grouped first stage;
+# lane per DOF, the fibre walk, wavefront per cell (3: grouped first stage;
 # 4, 5: 2, 3 with XCD-contiguous workgroups), 6: slabs (terms with one or two
 # non-identity dimensions per workgroup in LDS, the rest as layout 2)
 LAYOUTS = (1, 8, 2, 3, 4, 5, 6)
@@ -389,3 +389,29 @@ def test_slab_layout_vlasov_d6_full_size():
     if layout32 == 6:
         assert torch.equal(z1, z2)
     assert rel(host(z2).astype(np.float64), host(y1)) < 1e-5
+
+
+IN_PLACE = [dict(d=2, n=2, L=7, T=2), dict(d=3, n=2, L=5, T=2, refine=0.3),
+            dict(d=2, n=5, L=4, T=1), dict(d=4, n=3, L=4, T=1)]
+
+
+@pytest.mark.parametrize("spec,layout", [
+    (s, l) for s in IN_PLACE for l in LAYOUTS + (0,)
+    if s["n"] ** s["d"] <= 64 or l not in (2, 3, 4, 5)],  # the cell layouts' limit
+    ids=lambda v: "-".join(f"{k}{w}" for k, w in v.items()) if isinstance(v, dict) else str(v))
+def test_apply_in_place(spec, layout):
+    """y and x the same vector: every layout forms y after its last read of
+    other cells' x."""
+    c = _case_and_refs(spec)[0]
+    m = global_matrix(c, active=False)
+    m.set_tuning(waves_per_row=layout)
+    x = dev(c["x"])
+    want = x.clone()
+    m.apply(0.75, x, 0.5, want)
+    got = x.clone()
+    m.apply(0.75, got, 0.5, got)
+    assert rel(host(got), host(want)) < TOL64
+    m.apply_euler(0.01, 1.5, x, 0.0, want)
+    got = x.clone()
+    m.apply_euler(0.01, 1.5, got, 0.0, got)
+    assert rel(host(got), host(want)) < TOL64
