@@ -506,12 +506,25 @@ __global__ void __launch_bounds__(gm_threads) gm_rsub(int64_t n, const P *b, P *
     r[i] = b[i] - r[i];
 }
 
-//! y = fp32(x)
-__global__ void __launch_bounds__(gm_threads) gm_to_f32(int64_t n, const double *x, float *y)
+//! y = fp32(scale * x)
+__global__ void __launch_bounds__(gm_threads)
+gm_to_f32(int64_t n, const double *x, double scale, float *y)
 {
   for (int64_t i = blockIdx.x * int64_t(gm_threads) + threadIdx.x; i < n;
        i += int64_t(gridDim.x) * gm_threads)
-    y[i] = static_cast<float>(x[i]);
+    y[i] = static_cast<float>(scale * x[i]);
+}
+
+//! Residual norms between which a residual goes into FP32 as it is: entries
+//! and products a factor of 1e26 away from its norm still have all their bits.
+constexpr double gm_f32_least = 1e-12, gm_f32_most = 1e12;
+
+//! The power of two that brings a norm near one; 1 when it needs none.
+static double f32_scale(double norm)
+{
+  if ((norm >= gm_f32_least && norm <= gm_f32_most) || !std::isfinite(norm) || norm == 0.0)
+    return 1.0;
+  return std::ldexp(1.0, -std::clamp(std::ilogb(norm), -1000, 1000));
 }
 
 //! w = v + c * y, y in FP32 (the identity part of I - dt*A stays FP64).
@@ -1031,14 +1044,18 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     ++stats.applies_f64;
     return apply_device(m64, -dt, v, 0.0, w, 1.0, v);
   };
+  double beta = 0; // |r| of the current cycle
   std::function<int(const double *, double *)> op32 = [&](const double *v, double *w) -> int {
     ++stats.applies_f32;
-    if (apply_f32_between(*m32, v, -dt, w))
+    // V_0 is the residual itself, at the scale of b; the other vectors of the
+    // cycle have the norms of their steps
+    const double scale = (cyc.lazy && v == V) ? f32_scale(beta) : 1.0;
+    if (scale == 1.0 && apply_f32_between(*m32, v, -dt, w))
       return check_launch("gmres fp32 apply");
-    gm_to_f32<<<sblocks, gm_threads, 0, s>>>(n, v, ws.v32.data());
+    gm_to_f32<<<sblocks, gm_threads, 0, s>>>(n, v, scale, ws.v32.data());
     AKM_TRY(check_launch("gmres fp32 cast"));
     AKM_TRY(apply_device(*m32, 1.0, ws.v32.data(), 0.0, ws.y32.data(), 0.0, nullptr));
-    gm_axpy_f32<<<sblocks, gm_threads, 0, s>>>(n, v, -dt, ws.y32.data(), w);
+    gm_axpy_f32<<<sblocks, gm_threads, 0, s>>>(n, v, -dt / scale, ws.y32.data(), w);
     return check_launch("gmres fp32 axpy");
   };
   std::function<int(const double *, double *)> precond = [&](const double *v,
@@ -1046,12 +1063,12 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     ++stats.precond_applies;
     return pre->apply(v, z, s);
   };
-  // r = b - (I - dt A) x in FP64 into V_0, normalised; beta = |r|
-  auto true_residual = [&](double &beta) -> int {
+  // r = b - (I - dt A) x in FP64 into V_0; norm = |r|
+  auto true_residual = [&](double &norm) -> int {
     AKM_HIP(hipMemcpyAsync(V, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     ++stats.applies_f64;
     AKM_TRY(apply_device(m64, dt, x, 1.0, V, -1.0, x));
-    return cyc.start(beta);
+    return cyc.start(norm);
   };
 
   double bnorm = 0;
@@ -1071,7 +1088,6 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
   // ~FP32 epsilon, so it stops at inner_rel of its starting residual
   const double cycle_rel = (m32 != nullptr) ? inner_rel : 0.0;
 
-  double beta = 0;
   double first_ms = 0;
   if (m32 != nullptr)
   {

@@ -186,3 +186,27 @@ def test_learned_preconditioner_gain():
     assert np.abs(host(x2) - u0).max() < 1e-7
     assert info["loss_after"] < info["loss_before"]
     assert s2.iterations <= s1.iterations
+
+
+@pytest.mark.parametrize("layout", [None, "pair"])
+@pytest.mark.parametrize("scale", [1e-100, 1e-30, 1e-14, 1e14, 1e60])
+def test_fp32_cycles_do_not_depend_on_the_scale(scale, layout):
+    """The cycles of a scaled right-hand side are those of the unscaled one:
+    as many steps, no fallback, the scaled solution (both residuals are at
+    most 1e-10, the operator's condition here is below 10)."""
+    d, n, L, dt = 3, 2, 5, 1e-3
+    table, vA, T = operator_case(d, n, L)
+    m64 = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, L, T, vA)
+    m32 = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, L, T, vA.astype(np.float32),
+                                                dtype=np.float32)
+    if layout == "pair":
+        m32.set_tuning(waves_per_row=4)
+    b = dev(np.random.default_rng(8).uniform(-1, 1, m64.output_size()))
+    out = []
+    for f in (1.0, scale):
+        x = torch.zeros_like(b)
+        st = asgard_amd.gmres_euler_mixed(dt, m64, x, f * b, mat32=m32, restart=40, tol=1e-10)
+        assert st.converged == 1 and st.fallback == 0, (f, st.as_dict())
+        out.append((st.iterations, st.cycles, x / f))
+    assert out[0][:2] == out[1][:2]
+    assert float(torch.linalg.norm(out[1][2] - out[0][2]) / torch.linalg.norm(out[0][2])) < 2e-9
