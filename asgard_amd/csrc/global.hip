@@ -36,7 +36,6 @@
 #include "matrix.hpp"
 
 #include <algorithm>
-#include <cmath>
 #include <map>
 #include <memory>
 #include <vector>
@@ -2933,46 +2932,7 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
   return global_set_layout(m, layout);
 }
 
-//! Which of the T*d factors of vA are not exactly the identity (0 off the
-//! diagonal blocks, the unit matrix on them); false when a value is not
-//! finite.
-template<typename P>
-static bool active_factors(const P *vA, int T, int d, int n,
-                           std::vector<int> const &c1_pntr, std::vector<int> const &c1_diag,
-                           std::vector<int> &mask)
-{
-  const int nn = n * n, pairs = T * d;
-  mask.assign(pairs, 0);
-  bool finite = true;
-  for (size_t r = 0; r + 1 < c1_pntr.size(); r++)
-    for (int64_t q = c1_pntr[r]; q < c1_pntr[r + 1]; q++)
-      for (int td = 0; td < pairs; td++)
-      {
-        const P *b = vA + (q * pairs + td) * nn;
-        for (int i = 0; i < nn; i++)
-        {
-          const P want = (q == c1_diag[r] && i % (n + 1) == 0) ? P{1} : P{0};
-          if (b[i] != want)
-            mask[td] = 1;
-          finite = finite && std::isfinite(b[i]);
-        }
-      }
-  return finite;
-}
-
-//! active_factors of host values of the matrix's precision.
-static int active_factors_of(akm_matrix_s const &m, const void *vA, std::vector<int> &mask,
-                             bool &finite)
-{
-  std::vector<int> p1, i1, dg;
-  AKM_TRY(build_connect_1d(m.max_level, true, p1, i1, dg));
-  finite = (m.prec == AKM_F64)
-               ? active_factors(static_cast<const double *>(vA), m.T, m.d, m.n, p1, dg, mask)
-               : active_factors(static_cast<const float *>(vA), m.T, m.d, m.n, p1, dg, mask);
-  return AKM_SUCCESS;
-}
-
-int factored_build(akm_matrix_s &m, std::vector<int> const &elem, const void *vA)
+int factored_build(akm_matrix_s &m, std::vector<int> const &elem)
 {
   m.gk.reset();
   m.factored = false;
@@ -2980,26 +2940,20 @@ int factored_build(akm_matrix_s &m, std::vector<int> const &elem, const void *vA
     return AKM_SUCCESS;
   std::vector<int> mask;
   bool finite = false;
-  AKM_TRY(active_factors_of(m, vA, mask, finite));
+  AKM_TRY(stored_factors(m, mask, finite));
   return finite ? factored_build_mask(m, elem, mask) : AKM_SUCCESS;
 }
 
-int factored_refresh(akm_matrix_s &m, const void *values)
+int factored_refresh(akm_matrix_s &m)
 {
   if (m.T == 0 || m.rows == 0)
     return AKM_SUCCESS;
+  // the tables of the present plans, wanted or not: one wait for both
+  if (m.gk)
+    AKM_TRY(global_tables(m));
   std::vector<int> mask;
   bool finite = false;
-  if (values != nullptr)
-    AKM_TRY(active_factors_of(m, values, mask, finite));
-  else
-  {
-    std::vector<unsigned char> host(m.num_vA * m.esize);
-    AKM_HIP(hipMemcpyAsync(host.data(), m.vA.data(), host.size(), hipMemcpyDeviceToHost,
-                           m.stream));
-    AKM_HIP(hipStreamSynchronize(m.stream));
-    AKM_TRY(active_factors_of(m, host.data(), mask, finite));
-  }
+  AKM_TRY(stored_factors(m, mask, finite));
   if (!finite)
   {
     m.form_stamp += m.factored ? 1 : 0;
@@ -3015,7 +2969,7 @@ int factored_refresh(akm_matrix_s &m, const void *values)
   {
     m.form_stamp += m.factored ? 0 : 1;
     m.factored = true;
-    return global_tables(m);
+    return AKM_SUCCESS;
   }
   if (mask == m.factored_mask)
     return AKM_SUCCESS; // no factored form for these factors

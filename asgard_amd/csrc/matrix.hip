@@ -469,7 +469,7 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
   AKM_TRY(build_schedule(*m));
   m->elem_host = std::move(elem);
   if (T > 0)
-    AKM_TRY(factored_build(*m, m->elem_host, vA));
+    AKM_TRY(factored_build(*m, m->elem_host));
   *mat = m.release();
   return AKM_SUCCESS;
 }
@@ -536,7 +536,7 @@ akm_status akm_update_coefficients(akm_matrix mat, const void *values)
     if (mat->vAk.data() != nullptr)
       AKM_TRY(upload_vAk(*mat, values));
     if (mat->mode == mode_grid)
-      AKM_TRY(factored_refresh(*mat, values));
+      AKM_TRY(factored_refresh(*mat));
   }
   AKM_HIP(hipStreamSynchronize(mat->stream));
   return AKM_SUCCESS;

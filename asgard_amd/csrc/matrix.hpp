@@ -63,6 +63,9 @@ struct akm_matrix_s
   // operator update on the device: connect_1d (rows, then columns) in vA
   // order, and the device copy of the caller's operator pointers
   akm::dev_buffer<int> op_conn;
+  // the last scan of the stored factors: its number, and its findings
+  int op_scan = 0;
+  akm::dev_buffer<int> op_flags;
   akm::dev_buffer<const void *> op_ptrs;
   // IMEX step vectors (four of output_size), on the implicit handle
   akm::dev_buffer<double> imex_ws;
@@ -123,13 +126,16 @@ int global_device_jacobi(akm_matrix_s &m);
 //! factors, in place.  An apply never does: it may be captured into a graph,
 //! or be the first after one was.
 int global_tables(akm_matrix_s &m);
+//! Which of a sparse-grid handle's T x d stored factors are not exactly the
+//! identity, and whether all their values are finite: scanned on the device.
+int stored_factors(akm_matrix_s &m, std::vector<int> &mask, bool &finite);
 //! Sparse-grid handle: builds the factored form of its operator (`elem`: cell
-//! 1D indices, vA: host factor blocks) when the factors allow one that is
-//! faster than the pair kernels.
-int factored_build(akm_matrix_s &m, std::vector<int> const &elem, const void *vA);
-//! After new factor values (host values, or null: the values are on the
-//! device): keeps the factored form when it still holds, else builds it anew.
-int factored_refresh(akm_matrix_s &m, const void *values);
+//! 1D indices) when the stored factors allow one that is faster than the pair
+//! kernels.
+int factored_build(akm_matrix_s &m, std::vector<int> const &elem);
+//! After new factor values: keeps the factored form when it still holds, else
+//! builds it anew.
+int factored_refresh(akm_matrix_s &m);
 //! The same as factored_build for known non-identity factors (mask, T x d, all values finite).
 int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem,
                         std::vector<int> const &mask);

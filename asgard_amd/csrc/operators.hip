@@ -14,6 +14,8 @@
 #include "grid.hpp"
 #include "matrix.hpp"
 
+#include <algorithm>
+#include <limits>
 #include <vector>
 
 namespace akm
@@ -126,6 +128,94 @@ static int update_operators_typed(akm_matrix_s &m, const void *const *ops_dev, i
   return AKM_SUCCESS;
 }
 
+//! connect_1d on the device as (row, column) per connection, in vA order.
+static int need_connections(akm_matrix_s &m)
+{
+  if (m.op_conn.size() > 0)
+    return AKM_SUCCESS;
+  std::vector<int> p1, i1, dg;
+  AKM_TRY(build_connect_1d(m.max_level, true, p1, i1, dg));
+  const int64_t nconn = static_cast<int64_t>(i1.size());
+  if (nconn * m.T * m.d * m.n * m.n != m.num_vA)
+    return set_error(AKM_ERR_INVALID, "operator update: stored blocks do not match connect_1d");
+  std::vector<int> rc(2 * nconn);
+  for (int r = 0; r + 1 < static_cast<int>(p1.size()); r++)
+    for (int j = p1[r]; j < p1[r + 1]; j++)
+    {
+      rc[j] = r;
+      rc[nconn + j] = i1[j];
+    }
+  return m.op_conn.upload(rc.data(), 2 * nconn, m.stream);
+}
+
+//! flags[t*d + k] = scan for a factor that is not exactly the identity (0 off
+//! the diagonal blocks, the unit matrix on them), flags[T*d] = scan when any
+//! value is not finite; the others keep a lower number.  A row of workgroups
+//! per factor.
+template<typename P>
+__global__ void __launch_bounds__(op_threads)
+    scan_factors(const P *vA, const int *conn_row, const int *conn_col, int64_t nconn, int pairs,
+                 int n, int scan, int *flags)
+{
+  const int nn = n * n;
+  for (int td = blockIdx.y; td < pairs; td += gridDim.y)
+  {
+    int other = 0, infinite = 0;
+    for (int64_t i = blockIdx.x * int64_t(op_threads) + threadIdx.x; i < nconn * nn;
+         i += int64_t(gridDim.x) * op_threads)
+    {
+      const int64_t q = i / nn;
+      const int w = static_cast<int>(i - q * nn);
+      const P v = vA[(q * pairs + td) * nn + w];
+      const P unit = (conn_row[q] == conn_col[q] && w % (n + 1) == 0) ? P(1) : P(0);
+      other |= (v != unit);
+      infinite |= !isfinite(v);
+    }
+    other = __syncthreads_or(other);
+    infinite = __syncthreads_or(infinite);
+    if (threadIdx.x == 0 && other != 0)
+      atomicMax(flags + td, scan);
+    if (threadIdx.x == 0 && infinite != 0)
+      atomicMax(flags + pairs, scan);
+  }
+}
+
+int stored_factors(akm_matrix_s &m, std::vector<int> &mask, bool &finite)
+{
+  AKM_TRY(need_connections(m));
+  const int64_t nconn = m.op_conn.size() / 2;
+  const int pairs = m.T * m.d;
+  if (m.op_flags.size() == 0 || m.op_scan == std::numeric_limits<int>::max())
+  {
+    const std::vector<int> none(pairs + 1, 0);
+    AKM_TRY(m.op_flags.upload(none.data(), pairs + 1, m.stream));
+    m.op_scan = 0;
+  }
+  const int scan = ++m.op_scan;
+  // four values a thread, so that the 2.7 MB of a d = 6 level-7 operator of
+  // six terms are read by 360 workgroups
+  const dim3 grid(op_blocks((nconn * m.n * m.n + 3) / 4), std::min(pairs, 65535));
+  const int *row = m.op_conn.data(), *col = row + nconn;
+  if (m.prec == AKM_F64)
+    scan_factors<double><<<grid, op_threads, 0, m.stream>>>(
+        reinterpret_cast<const double *>(m.vA.data()), row, col, nconn, pairs, m.n, scan,
+        m.op_flags.data());
+  else
+    scan_factors<float><<<grid, op_threads, 0, m.stream>>>(
+        reinterpret_cast<const float *>(m.vA.data()), row, col, nconn, pairs, m.n, scan,
+        m.op_flags.data());
+  AKM_TRY(check_launch("factor scan"));
+  mask.resize(pairs + 1);
+  AKM_HIP(hipMemcpyAsync(mask.data(), m.op_flags.data(), sizeof(int) * (pairs + 1),
+                         hipMemcpyDeviceToHost, m.stream));
+  AKM_HIP(hipStreamSynchronize(m.stream));
+  for (int &f : mask)
+    f = (f == scan) ? 1 : 0;
+  finite = mask.back() == 0;
+  mask.pop_back();
+  return AKM_SUCCESS;
+}
+
 } // namespace akm
 
 using namespace akm;
@@ -155,23 +245,8 @@ akm_status akm_update_operators(akm_matrix mat, const void *const *ops, int64_t 
   if (lda < need)
     return set_error(AKM_ERR_INVALID, "operator update: lda %lld below the operator size %lld",
                      static_cast<long long>(lda), static_cast<long long>(need));
-  if (mat->mode != mode_dense && mat->op_conn.size() == 0)
-  {
-    // connect_1d as (row, column) per connection, in vA order
-    std::vector<int> p1, i1, dg;
-    AKM_TRY(build_connect_1d(mat->max_level, true, p1, i1, dg));
-    const int64_t nconn = static_cast<int64_t>(i1.size());
-    if (nconn * mat->T * mat->d * mat->n * mat->n != mat->num_vA)
-      return set_error(AKM_ERR_INVALID, "operator update: stored blocks do not match connect_1d");
-    std::vector<int> rc(2 * nconn);
-    for (int r = 0; r + 1 < static_cast<int>(p1.size()); r++)
-      for (int j = p1[r]; j < p1[r + 1]; j++)
-      {
-        rc[j] = r;
-        rc[nconn + j] = i1[j];
-      }
-    AKM_TRY(mat->op_conn.upload(rc.data(), 2 * nconn, mat->stream));
-  }
+  if (mat->mode != mode_dense)
+    AKM_TRY(need_connections(*mat));
   std::vector<const void *> ptrs(ops, ops + nops);
   AKM_TRY(mat->op_ptrs.upload(ptrs.data(), nops, mat->stream));
   if (mat->prec == AKM_F64)
@@ -179,7 +254,7 @@ akm_status akm_update_operators(akm_matrix mat, const void *const *ops, int64_t 
   else
     AKM_TRY(update_operators_typed<float>(*mat, mat->op_ptrs.data(), lda));
   if (mat->mode == mode_grid)
-    AKM_TRY(factored_refresh(*mat, nullptr));
+    AKM_TRY(factored_refresh(*mat));
   AKM_HIP(hipStreamSynchronize(mat->stream));
   return AKM_SUCCESS;
 }
