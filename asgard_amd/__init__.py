@@ -49,7 +49,8 @@ EXPORTS = (
     "akm_global_jacobi", "akm_create_dense", "akm_update_coefficients",
     "akm_update_operators", "akm_imex_step", "akm_dg_term",
     "akm_apply", "akm_apply_euler", "akm_matrix_info", "akm_set_tuning",
-    "akm_autotune", "akm_set_kernel_family", "akm_time_apply", "akm_destroy", "akm_gmres_euler",
+    "akm_autotune", "akm_apply_form", "akm_set_kernel_family", "akm_time_apply", "akm_destroy",
+    "akm_gmres_euler",
     "akm_gmres_euler_noalloc", "akm_gmres_dense",
     "akm_gmres_euler_mixed", "akm_mlp_create", "akm_mlp_info", "akm_mlp_set_stream",
     "akm_mlp_get_params", "akm_mlp_set_params", "akm_mlp_forward", "akm_mlp_gradients",
@@ -149,6 +150,7 @@ def load_library(path: str = LIB_PATH):
     L.akm_set_tuning.argtypes = [_vp, _i, _i, _i]
     L.akm_time_apply.argtypes = [_vp, _d, _vp, _d, _vp, _i, ctypes.POINTER(_d)]
     L.akm_autotune.argtypes = [_vp, _vp, _vp, ctypes.POINTER(_i), ctypes.POINTER(_i)]
+    L.akm_apply_form.argtypes = [_vp, ctypes.POINTER(_i), ctypes.POINTER(_i)]
     L.akm_set_kernel_family.argtypes = [_vp, _i]
     L.akm_destroy.argtypes = [_vp]
     L.akm_gmres_euler.argtypes = [_vp, _d, _vp, _vp, _i, _i, _d, _i, ctypes.POINTER(_d),
@@ -450,6 +452,15 @@ class KronmultMatrix:
         w, l = _i(), _i()
         _check(load_library().akm_autotune(self._h, px, py, ctypes.byref(w), ctypes.byref(l)))
         return w.value, l.value
+
+    def apply_form(self):
+        """(layout, stages) of an apply now: layout 0 = pair by pair, else the
+        layout of the products taken one dimension at a time (8 fibre walk,
+        6 slabs), stages = the most of them that follow each other."""
+        layout, stages = _i(), _i()
+        _check(load_library().akm_apply_form(self._h, ctypes.byref(layout),
+                                             ctypes.byref(stages)))
+        return layout.value, stages.value
 
     def time_apply(self, alpha, x, beta, y, iterations):
         px, dx = _vec_ptr(x, self.dtype)

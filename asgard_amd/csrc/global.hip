@@ -1682,7 +1682,7 @@ int global_apply(akm_matrix_s &m, double alpha, const void *x, double beta, void
 
 bool apply_f32_between(akm_matrix_s &m, const double *v, double c, double *w)
 {
-  if (m.prec != AKM_F32 || !m.gk || (m.mode != mode_global && (!m.factored || m.pair_kernels)))
+  if (m.prec != AKM_F32 || !m.gk || (m.mode != mode_global && (!m.factored || m.pair_kernels || m.pair_tuned)))
     return false;
   akm_global_s &g = *m.gk;
   if (g.slab || g.lanes != 8 || g.active_cells == 0)
@@ -1772,7 +1772,7 @@ bool factored_batch_plan(akm_matrix_s const &m, fibre_plan &plan, int &rc)
 {
   rc = AKM_SUCCESS;
   // (the batch kernel's forms: n = 3 alone past 64 entries a cell)
-  if (!m.factored || !m.gk || m.prec != AKM_F64 || m.gk->max_stages > 1 || m.n < 2 || m.n > 4 ||
+  if (!m.factored || m.pair_kernels || !m.gk || m.prec != AKM_F64 || m.gk->max_stages > 1 || m.n < 2 || m.n > 4 ||
       m.N > (m.n == 3 ? 1024 : 64))
     return false;
   akm_global_s const &g = *m.gk;
@@ -1793,6 +1793,8 @@ int global_layout(akm_matrix_s const &m)
     return (m.gk->first_grouped ? 3 : 2) + (m.gk->xcd_order ? 2 : 0);
   return m.gk->lanes;
 }
+
+int global_stages(akm_matrix_s const &m) { return m.gk ? m.gk->max_stages : 0; }
 
 int global_set_layout(akm_matrix_s &m, int layout)
 {
@@ -2983,6 +2985,7 @@ int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem, std::vect
   m.factored = false;
   m.factored_mask = mask;
   m.form_stamp++;
+  m.pair_tuned = false; // it was timed against another form, or none
   int widest = 0;
   for (int t = 0; t < m.T; t++)
     widest = std::max(widest, static_cast<int>(std::count(mask.begin() + t * m.d,

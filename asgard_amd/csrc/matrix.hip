@@ -220,7 +220,7 @@ int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void
   // A captured apply is replayed whenever its owner likes, beside other applies
   // and after new factors of another form: it takes the pair kernels, which
   // read nothing but x and the stored factors, at addresses that stay.
-  if (m.factored && !m.pair_kernels && !capturing(m.stream))
+  if (m.factored && !m.pair_kernels && !m.pair_tuned && !capturing(m.stream))
   {
     std::lock_guard<std::mutex> lock(m.factored_mtx);
     return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
@@ -232,6 +232,16 @@ int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void
   return apply_typed<float>(m, static_cast<float>(alpha), static_cast<const float *>(x),
                             static_cast<float>(beta), static_cast<float *>(y),
                             static_cast<float>(gamma), static_cast<const float *>(xg));
+}
+
+//! The caller's choice between the pair kernels and the automatic one, which
+//! batches follow as well.
+static void ask_pair_kernels(akm_matrix_s &m, bool pair)
+{
+  if (m.pair_kernels != pair && m.factored)
+    m.form_stamp++;
+  m.pair_kernels = pair;
+  m.pair_tuned = false;
 }
 
 static int check_common(int d, int n, int rows, int cols, int T, akm_prec prec,
@@ -605,7 +615,7 @@ akm_status akm_set_tuning(akm_matrix mat, int waves_per_row, int lds_cap_bytes,
   mat->lds_cap = (lds_cap_bytes < 0) ? -1 : lds_cap_bytes;
   mat->force_generic = force_generic;
   // a shape of the pair kernels was asked for, or everything automatic
-  mat->pair_kernels = waves_per_row != 0 || lds_cap_bytes >= 0 || force_generic != 0;
+  ask_pair_kernels(*mat, waves_per_row != 0 || lds_cap_bytes >= 0 || force_generic != 0);
   return AKM_SUCCESS;
 }
 
@@ -659,6 +669,7 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
   if (mat->factored)
     key.insert(key.end(), mat->factored_mask.begin(), mat->factored_mask.end());
   choice best{0, -1, 0, -1};
+  ask_pair_kernels(*mat, false); // tuning takes the place of a request
   bool cached = false;
   {
     std::lock_guard<std::mutex> lock(mtx);
@@ -673,12 +684,11 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
   {
     best.factored = -1;
     double factored_ms = 1e300;
-    mat->pair_kernels = false;
     if (mat->factored)
     {
       AKM_TRY(global_autotune(*mat, x, y, factored_ms));
       best.factored = factored_shape(*mat);
-      mat->pair_kernels = true;
+      mat->pair_tuned = true; // while the pair kernels are timed
     }
     // the pair kernels are not timed when even twice the best rate they have
     // reached (67 TFLOP/s FP64, 98 FP32) would be slower than that
@@ -694,9 +704,9 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
       const int iters = std::max(1, std::min(50, int(2.0 / std::max(probe, 1e-3))));
       if (best.factored >= 0)
       {
-        mat->pair_kernels = false;
+        mat->pair_tuned = false;
         AKM_TRY(akm_time_apply(mat, 1.0, x, 0.0, y, iters, &factored_ms));
-        mat->pair_kernels = true;
+        mat->pair_tuned = true;
       }
       // (against a factored form the pair kernels have to win clearly: short
       // applies are timed at the rate the host launches them)
@@ -742,7 +752,7 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
     mat->waves = 0;
     mat->lds_cap = -1;
     mat->family = 0;
-    mat->pair_kernels = false;
+    mat->pair_tuned = false;
     if (waves_per_row)
       *waves_per_row = 1;
     if (lds_tables)
@@ -752,11 +762,24 @@ akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_r
   mat->waves = best.waves;
   mat->lds_cap = best.lds;
   mat->family = best.family;
-  mat->pair_kernels = true;
+  mat->pair_tuned = true; // until new factors change the form
   if (waves_per_row)
     *waves_per_row = best.waves;
   if (lds_tables)
     *lds_tables = (best.family == 1) ? 2 : (best.lds != 0 && mat->vAk.data() != nullptr) ? 1 : 0;
+  return AKM_SUCCESS;
+}
+
+akm_status akm_apply_form(akm_matrix mat, int *layout, int *stages)
+{
+  if (mat == nullptr)
+    return set_error(AKM_ERR_INVALID, "null matrix");
+  const bool form = mat->mode == mode_global ||
+                    (mat->factored && !mat->pair_kernels && !mat->pair_tuned);
+  if (layout)
+    *layout = form ? global_layout(*mat) : 0;
+  if (stages)
+    *stages = form ? global_stages(*mat) : 1;
   return AKM_SUCCESS;
 }
 
@@ -773,7 +796,7 @@ akm_status akm_set_kernel_family(akm_matrix mat, int family)
                      "kernel family 1 needs an FP64 sparse-grid matrix with d = 3, n = 3, "
                      "1 to 8 terms and max_level <= 10");
   mat->family = family;
-  mat->pair_kernels = true;
+  ask_pair_kernels(*mat, true);
   return AKM_SUCCESS;
 }
 

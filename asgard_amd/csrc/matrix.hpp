@@ -80,6 +80,7 @@ struct akm_matrix_s
   // advanced when the form or the products it was built for change
   uint64_t form_stamp = 0;
   bool pair_kernels = false;        // the caller asked for the pair kernels
+  bool pair_tuned = false;          // akm_autotune found them faster than the form
   // held while a factored apply is enqueued: its launches share work vectors,
   // so two threads' applies follow each other on the stream
   std::mutex factored_mtx;
@@ -144,6 +145,8 @@ int64_t global_flops(akm_matrix_s const &m);
 //! Global operator: row layout in use, as akm_set_tuning takes it (1, 8, 2,
 //! 3, 4, 5 or 6).
 int global_layout(akm_matrix_s const &m);
+//! Dependent products of its longest chain.
+int global_stages(akm_matrix_s const &m);
 //! Global operator: times the layouts on the operator and keeps the fastest;
 //! best_ms = its time per apply.
 int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms);

@@ -110,9 +110,10 @@ akm_status akm_create_sparse(int d, int n, int rows, int cols, int num_terms,
  * levels closed under lowering a level (any factors).  The products left out
  * are exact zeros; a non-finite entry of x then reaches only the rows its
  * non-identity factors couple.  akm_update_coefficients and
- * akm_update_operators look at the new factors and choose again; a shape
- * given to akm_set_tuning or akm_set_kernel_family selects the pair-by-pair
- * kernels, akm_set_tuning(mat, 0, -1, 0) the automatic choice.  An apply
+ * akm_update_operators look at the new factors and choose again, also after
+ * akm_autotune; a shape given to akm_set_tuning or akm_set_kernel_family
+ * selects the pair-by-pair kernels, in batches too, and
+ * akm_set_tuning(mat, 0, -1, 0) the automatic choice.  An apply
  * captured into a graph always records the pair-by-pair kernels: they use no
  * work vectors and read the stored factors in place, so a replay applies the
  * operator of its time, whatever the form of the factors it was updated to. */
@@ -236,6 +237,12 @@ akm_status akm_set_tuning(akm_matrix mat, int waves_per_row, int lds_cap_bytes,
  * pointers are not NULL.  No counterpart in the reference (fixed launch shapes). */
 akm_status akm_autotune(akm_matrix mat, const void *x, void *y, int *waves_per_row,
                         int *lds_tables);
+
+/* How an apply runs now: *layout = 0 pair by pair, else the layout of the
+ * products taken one dimension at a time (8 fibre walk, 6 slabs, a global
+ * handle's as akm_set_tuning takes it), and *stages = the most such products
+ * that follow each other.  No counterpart in the reference. */
+akm_status akm_apply_form(akm_matrix mat, int *layout, int *stages);
 
 /* Kernel family of the apply: 0 = the register / LDS-table kernels, 1 = the
  * sum-factorised matrix-core kernels for FP64 sparse-grid matrices with

@@ -223,3 +223,50 @@ def test_batch_mixes_both_ways_of_applying():
         vA = grid.build_vA(d, n, T, top, [0.1 * o if i < 2 else o for i, o in enumerate(ops)])
         mats[0].update_stored_coefficients(vA)
         problems[0] = (d, n, table, top, T, vA)
+
+
+def test_tuned_handles_choose_again_with_new_factors():
+    """The pair kernels chosen by autotune hold until the form changes; a
+    shape asked for holds until it is taken back."""
+    rng = np.random.default_rng(19)
+    table, top = tables(2, 6, False)
+    cells = table[:-1]  # a cell missing: dense factors have no form here
+    vA = grid.build_vA(2, 2, 2, top, factors(rng, 2, 2, top, [(0, 1), (1,)]))
+    m = asgard_amd.KronmultMatrix.sparse_grid(2, 2, cells, top, 2, vA)
+    assert m.apply_form() == (0, 1)
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+    m.autotune(x, torch.zeros_like(x))
+    assert m.apply_form() == (0, 1)
+    m.update_stored_coefficients(
+        grid.build_vA(2, 2, 2, top, factors(rng, 2, 2, top, [(0,), (1,)])))
+    assert m.apply_form() == (8, 1)
+    y0 = np.zeros(m.output_size())
+    got, want = both(m, x, 1.0, 0.0, y0)
+    assert close(got, want, np.float64)
+    m.set_tuning(waves_per_row=2)
+    m.update_stored_coefficients(
+        grid.build_vA(2, 2, 2, top, factors(rng, 2, 2, top, [(1,), ()])))
+    assert m.apply_form() == (0, 1)
+    m.set_tuning()
+    assert m.apply_form() == (8, 1)
+
+
+def test_batch_follows_a_request_for_the_pair_kernels():
+    rng = np.random.default_rng(37)
+    table, top = tables(3, 4, True)
+    ops = [0.05 * o if not np.array_equal(o, np.eye(len(o))) else o
+           for o in factors(rng, 3, 2, top, [(0,), (2,)])]
+    m = asgard_amd.KronmultMatrix.sparse_grid(3, 2, table, top, 2,
+                                              grid.build_vA(3, 2, 2, top, ops))
+    b = torch.from_numpy(rng.uniform(-1, 1, m.output_size())).cuda()
+    batch = asgard_amd.BatchSolver([m], [0.05], restart=20)
+    out = []
+    for waves in (0, 4, 0):
+        m.set_tuning(waves_per_row=waves)
+        x = torch.zeros_like(b)
+        _, _, conv = batch.solve([x], [b], tol=1e-11)
+        assert conv.all()
+        out.append(x.cpu().numpy())
+    assert np.array_equal(out[0], out[2])  # the walk again
+    assert not np.array_equal(out[0], out[1])  # other sums
+    assert np.abs(out[0] - out[1]).max() < 1e-9 * np.abs(out[0]).max()
