@@ -95,7 +95,7 @@ struct fl_args
 template<typename P, int NT>
 __device__ __forceinline__ void fl_column(const P *A, P (&v)[NT])
 {
-  constexpr int W = (NT == 3) ? 1 : ((sizeof(P) == 4) ? NT : 2); // values per read
+  constexpr int W = (NT % 2 != 0) ? 1 : ((sizeof(P) == 4) ? NT : 2); // values per read
   typedef P vec __attribute__((ext_vector_type(W)));
 #pragma unroll
   for (int j = 0; j < NT; j += W)
@@ -316,34 +316,55 @@ __global__ void __launch_bounds__(TPB)
     fl_group<double, 4, double>(a, group, ex);
 }
 
-//! One stage for n > 4 or N > 1024: a workgroup per job, its threads over the
-//! cell's entries, row by row.
-template<typename P>
-__global__ void __launch_bounds__(256) fl_stage_any(fl_args<P> a, int group0)
+//! One stage for n > 4 or N > 1024: a workgroup per job and up to fl_any_width
+//! of the cell's entries, row by row.  Its threads form groups of that many,
+//! which take the pieces of the cell's list in turn (one group alone walked
+//! the 256 connections of a level-0 cell at d = 2, n = 5, level 7 for 136 us)
+//! and whose sums meet in LDS in group order.  NT: n where it is known, else 0.
+//! Measured (FP64, us per apply; one group / groups / pair kernels / best other
+//! global layout): d = 2 n = 5 level 7 136 / 12 / 23 / 51; d = 3 n = 5 level 6
+//! 109 / 30 / 175 / 59; d = 2 n = 6 level 6 80 / 20 / 1352 / 56; d = 4 n = 6
+//! level 3 132 / 16 / 3984 / 19.
+constexpr int fl_any_width = 256;
+template<typename P, int NT, int TPB>
+__global__ void __launch_bounds__(TPB) fl_stage_any(fl_args<P> a, int group0)
 {
+  __shared__ P part[TPB];
   const int4 *rec = a.slots + int64_t(group0 + blockIdx.x) * 7;
   const int4 head = rec[0], tail = rec[1];
-  const int n = a.n;
-  for (int e = threadIdx.x; e < a.N; e += blockDim.x)
+  const int n = (NT > 0) ? NT : a.n;
+  const int width = min(a.N, fl_any_width), groups = TPB / width;
+  const int g = threadIdx.x / width, lane = threadIdx.x - g * width;
+  const int e = blockIdx.y * fl_any_width + lane;
+  P sum = 0;
+  if (g < groups && e < a.N)
   {
-    P sum = 0;
-    for (int i = 0; i <= head.w; i++)
+    for (int i = g; i <= head.w; i += groups)
     {
       const int4 *p = (i == 0) ? rec + 2 : a.pieces + int64_t(tail.x + i - 1) * 5;
       const int4 ph = p[0];
       const int s = fl_digit(e, static_cast<unsigned>(ph.z), n);
       const P *in = ((ph.x == 0) ? a.x : a.work + int64_t(ph.x - 1) * a.stride) + e - s * ph.y;
       const int2 *ent = reinterpret_cast<const int2 *>(p + 1);
-      for (int u = 0; u < (ph.w & 0xffff); u++)
+      const int len = ph.w & 0xffff;
+#pragma unroll 4
+      for (int u = 0; u < len; u++)
       {
         const P *A = a.tab + int64_t(ent[u].y) * (int64_t(n) * n) + s;
         const P *xin = in + int64_t(ent[u].x) * a.N;
+#pragma unroll
         for (int j = 0; j < n; j++)
           sum = fma(A[j * n], xin[j * ph.y], sum);
       }
     }
-    fl_store(a, head.z, int64_t(head.x) * a.N + e, sum);
   }
+  part[threadIdx.x] = sum;
+  __syncthreads();
+  if (g != 0 || e >= a.N)
+    return;
+  for (int i = 1; i < min(groups, head.w + 1); i++)
+    sum += part[i * width + lane];
+  fl_store(a, head.z, int64_t(head.x) * a.N + e, sum);
 }
 
 //! Factor tables: block q of table i is the sum over its (term, dimension)
@@ -664,12 +685,12 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
   const int d = m.d, n = m.n, N = static_cast<int>(m.N);
   const program prog(m.T, term_act);
   // lanes share a workgroup's LDS by slot; wider tensors and larger blocks
-  // take one workgroup per cell.  Workgroups of 256 threads start sooner
+  // take one workgroup per cell and 256 entries.  Workgroups of 256 threads start sooner
   // (d = 2, n = 2, level 5: 3.2 us an apply against 3.6 with 512 and 5.0 with
   // 1024); from 65 entries on a cell's list needs the slots of 1024 (d = 4,
   // n = 3, level 5: 9.4 us against 10.9 with 256 or 512)
-  plan.slots_of_lanes = n >= 2 && n <= 4 && N <= 1024;
-  plan.tpb = !plan.slots_of_lanes ? 256 : (N <= 64 ? 256 : 1024);
+  plan.slots_of_lanes = n <= 4 && N <= 1024;
+  plan.tpb = N <= 64 ? 256 : 1024;
   plan.nslot = plan.slots_of_lanes ? plan.tpb / N : 1;
   plan.vectors = prog.vectors;
   plan.identities = prog.identities;
@@ -906,6 +927,8 @@ static int launch_stage(akm_matrix_s const &m, fibre_plan const &plan,
       large<<<grid, tpb, lds, m.stream>>>(a, st.first_group);
     return check_launch("fibre stage");
   };
+  if (m.n == 1)
+    return go(fl_stage<P, 1, 256, X>, fl_stage<P, 1, 256, X>); // one lane a slot
   if (m.n == 2)
     return go(fl_stage<P, 2, 256, X>, fl_stage<P, 2, 1024, X>);
   if (m.n == 3)
@@ -933,8 +956,18 @@ int fibre_apply(akm_matrix_s &m, fibre_plan &plan, P alpha, const P *x, P beta, 
       AKM_TRY(launch_stage(m, plan, st, a));
       continue;
     }
-    fl_stage_any<P><<<static_cast<unsigned>(st.groups), plan.tpb, 0, m.stream>>>(a,
-                                                                                st.first_group);
+    const dim3 grid(static_cast<unsigned>(st.groups),
+                    static_cast<unsigned>((a.N + fl_any_width - 1) / fl_any_width));
+    auto go = [&](auto small, auto large) {
+      if (plan.tpb == 256)
+        small<<<grid, 256, 0, m.stream>>>(a, st.first_group);
+      else
+        large<<<grid, 1024, 0, m.stream>>>(a, st.first_group);
+    };
+    if (a.n == 5)
+      go(fl_stage_any<P, 5, 256>, fl_stage_any<P, 5, 1024>);
+    else
+      go(fl_stage_any<P, 0, 256>, fl_stage_any<P, 0, 1024>);
     AKM_TRY(check_launch("fibre stage"));
   }
   return AKM_SUCCESS;

@@ -270,3 +270,43 @@ def test_batch_follows_a_request_for_the_pair_kernels():
     assert np.array_equal(out[0], out[2])  # the walk again
     assert not np.array_equal(out[0], out[1])  # other sums
     assert np.abs(out[0] - out[1]).max() < 1e-9 * np.abs(out[0]).max()
+
+
+WIDE = [
+    # (d, n, level, non-identity dimensions per term)
+    (1, 1, 9, [(0,)]),                  # one entry a cell, 512 connections
+    (2, 1, 6, [(0,), (0, 1)]),
+    (6, 1, 3, [(0, 3), (1, 4), ()]),
+    (2, 5, 6, [(0,), (1,)]),            # 25 entries: ten groups, a remainder
+    (3, 6, 3, [(0, 1, 2)]),             # 216 entries: one more than half
+    (1, 16, 4, [(0,)]),
+    (2, 16, 3, [(1,), (0, 1)]),         # 256 entries: the widest single chunk
+    (3, 7, 3, [(0,), (2,)]),            # 343: a second, ragged chunk
+    (4, 5, 2, [(3,), (0, 2)]),          # 625: three chunks
+    (6, 4, 1, [(0, 5)]),                # 4096: sixteen
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("case", WIDE, ids=str)
+def test_walk_of_single_entries_and_wide_blocks(case, dtype):
+    """The fibre walk (a global handle pinned to it) against pair kernels."""
+    d, n, level, active = case
+    rng = np.random.default_rng(41)
+    table, top = tables(d, level, False)
+    T = len(active)
+    ops = factors(rng, d, n, top, active)
+    vA = grid.build_vA(d, n, T, top, ops).astype(dtype)
+    pair = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, T, vA, dtype=dtype)
+    pair.set_tuning(waves_per_row=4)
+    walk = asgard_amd.KronmultMatrix.global_grid(d, n, table, top, T, vA, dtype=dtype,
+                                                 active=grid.identity_mask(ops, T, d))
+    walk.set_tuning(waves_per_row=8)
+    x = torch.from_numpy(rng.uniform(-1, 1, pair.input_size()).astype(dtype)).cuda()
+    y0 = rng.uniform(-1, 1, pair.output_size()).astype(dtype)
+    out = []
+    for m in (walk, pair):
+        y = torch.from_numpy(y0.copy()).cuda()
+        m.apply(-0.7, x, 0.4, y)
+        out.append(y.cpu().numpy().astype(np.float64))
+    assert close(out[0], out[1], dtype)
