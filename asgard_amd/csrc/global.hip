@@ -1829,8 +1829,17 @@ int global_set_layout(akm_matrix_s &m, int layout)
 //! bytes).
 constexpr int64_t fl_lanes_tuned = int64_t(1) << 26;
 //! The layout of a handle that is not tuned: the fibre walk up to this many
-//! (lane, connection) steps, then the slab layout.
-constexpr int64_t fl_lanes_default = int64_t(1) << 26;
+//! (lane, connection) steps, then the slab layout where it takes every chain.
+//! With two dimensions a term the slabs save the walk's way of the
+//! intermediate through memory; us per apply of walk / slabs on the d = 6
+//! n = 2 Vlasov operator: 6.0 M steps (level 5) FP64 37 / 43, FP32 29 / 39;
+//! 22 M (level 6) 87 / 44 and 70 / 45; 76 M (level 7) 254 / 100.  With one
+//! dimension a term neither is ahead throughout: d = 6 n = 2 7.4 M 29 / 23,
+//! 25 M 85 / 101; d = 4 n = 2 level 8 4.3 M 15 / 56; d = 5 n = 3 4.3 M 34 / 17.
+static int64_t fl_lanes_default(int stages)
+{
+  return (stages > 1) ? int64_t(1) << 23 : int64_t(1) << 26;
+}
 
 //! Up to this many steps the fibre walk is always the faster of the two.
 constexpr int64_t fl_lanes_small = int64_t(1) << 20;
@@ -1839,12 +1848,14 @@ constexpr int64_t fl_lanes_small = int64_t(1) << 20;
 //! operator of a pair handle has none.
 static int default_layout(akm_matrix_s const &m, akm_global_s const &g)
 {
-  if (g.fl_lanes <= fl_lanes_default)
+  if (g.fl_lanes <= fl_lanes_default(g.max_stages))
     return 8;
   if (g.ngroups > 0 && (g.max_stages == 0 || g.stage_count_rest[0] == 0))
     return 6;
+  if (g.fl_lanes <= fl_lanes_tuned)
+    return 8;
   if (g.pair)
-    return g.fl_lanes <= fl_lanes_tuned ? 8 : -1;
+    return -1;
   return (m.N <= wave_size) ? 2 : 1;
 }
 
@@ -2915,7 +2926,7 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
   }
   g->fl_lanes = fibre_lanes(m, lists, term_act);
   // a pair handle plans slabs when it is to use or to time them
-  if (!pair || g->fl_lanes > fl_lanes_default)
+  if (!pair || g->fl_lanes > fl_lanes_default(g->max_stages))
     AKM_TRY(need_slabs(m, *g));
   if (!pair && nslots + g->ngroups > 0)
     AKM_TRY(g->work.allocate((int64_t(2) * nslots + g->ngroups) * g->cells * m.N *
@@ -3012,8 +3023,8 @@ int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem, std::vect
     return AKM_SUCCESS;
   }
   // Estimated times: the pair kernels' fixed part and rate, the fibre walk's
-  // per launch and per step (the slab layout, taken only past the walk's
-  // range, is faster than that).
+  // per launch and per step (the slab layout is taken where it is faster
+  // than that).
   const double pair_us = 4.0 + double(m.flops()) / (m.prec == AKM_F64 ? 25e6 : 50e6);
   const double walk_us = 1.0 + 3.0 * std::max(g.max_stages, 1) + double(g.fl_lanes) / 0.6e6;
   m.factored = walk_us < pair_us;

@@ -310,3 +310,21 @@ def test_walk_of_single_entries_and_wide_blocks(case, dtype):
         m.apply(-0.7, x, 0.4, y)
         out.append(y.cpu().numpy().astype(np.float64))
     assert close(out[0], out[1], dtype)
+
+
+@pytest.mark.parametrize("level,active,form", [
+    (5, [(0, 3), (1, 4), (2, 5)], (8, 2)),
+    (6, [(0, 3), (1, 4), (2, 5)], (6, 2)),          # past 2^23 steps: slabs
+    (6, [(0, 3), (1, 4, 2), (5,)], (8, 3)),         # which take no third dimension
+    (6, [(k,) for k in range(6)], (8, 1))])
+def test_layout_of_untuned_handles(level, active, form):
+    """Both sides of the line between the walk and the slabs."""
+    rng = np.random.default_rng(43)
+    table, top = tables(6, level, False)
+    T = len(active)
+    vA = grid.build_vA(6, 2, T, top, factors(rng, 6, 2, top, active))
+    m = asgard_amd.KronmultMatrix.sparse_grid(6, 2, table, top, T, vA)
+    assert m.apply_form() == form
+    x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
+    got, want = both(m, x, 1.3, -0.4, rng.uniform(-1, 1, m.output_size()))
+    assert close(got, want, np.float64)
