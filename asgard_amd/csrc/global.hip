@@ -1870,11 +1870,12 @@ int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms)
   AKM_HIP(hipEventCreate(&e0));
   AKM_HIP(hipEventCreate(&e1));
   float best = -1;
-  int best_lanes = 1;
-  bool best_grouped = false;
+  // (the layout so far, should no candidate run)
+  int best_lanes = g.lanes;
+  bool best_grouped = g.first_grouped;
   int rc = AKM_SUCCESS;
-  bool best_xcd = false, best_slab = false;
-  int best_moved = 0;
+  bool best_xcd = g.xcd_order, best_slab = g.slab;
+  int best_moved = g.gs_moved;
   // layouts 1 and 8 (when its records stay small), then the cell layout with
   // and without the grouped first stage (shared input reads against fewer, longer wavefronts), each
   // cell layout with and without the XCD-contiguous workgroup order, then
@@ -1895,12 +1896,9 @@ int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms)
       continue;
     if (g.pair && lanes != 8 && !slab)
       continue;
-    if (slab && g.pair && g.fl_lanes > fl_lanes_small)
-    {
-      rc = need_slabs(m, g);
-      if (rc != AKM_SUCCESS)
-        break;
-    }
+    // (without room for the slabs the walk is left)
+    if (slab && g.pair && g.fl_lanes > fl_lanes_small && need_slabs(m, g) != AKM_SUCCESS)
+      (void)hipGetLastError();
     if (slab && g.ngroups == 0)
       continue;
     if (lanes == 8)
@@ -1947,7 +1945,7 @@ int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms)
   g.xcd_order = best_xcd;
   g.slab = best_slab;
   g.gs_moved = best_moved;
-  best_ms = best / 5;
+  best_ms = (best < 0) ? 1e300 : best / 5;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return rc;
@@ -1958,9 +1956,10 @@ int factored_shape(akm_matrix_s const &m) { return global_layout(m) + 16 * m.gk-
 int factored_set_shape(akm_matrix_s &m, int shape)
 {
   int layout = shape % 16;
-  if (layout == 6)
-    AKM_TRY(need_slabs(m, *m.gk));
-  // the number may come from another grid of the same size
+  if (layout == 6 && need_slabs(m, *m.gk) != AKM_SUCCESS)
+    (void)hipGetLastError();
+  // the number may come from another grid of the same size, or there is no
+  // room for the slabs
   if (layout == 6 && m.gk->ngroups == 0)
     layout = 8;
   AKM_TRY(global_set_layout(m, layout));
@@ -2703,16 +2702,22 @@ static int need_slabs(akm_matrix_s &m, akm_global_s &g)
   if (g.slabs_built)
     return AKM_SUCCESS;
   g.slabs_built = true;
-  AKM_TRY(build_slabs(m, g));
-  if (g.pair && g.max_stages > 0 && g.stage_count_rest[0] > 0)
-    g.ngroups = 0;
-  if (g.ngroups == 0)
+  auto build = [&]() -> int {
+    AKM_TRY(build_slabs(m, g));
+    if (g.pair && g.max_stages > 0 && g.stage_count_rest[0] > 0)
+      g.ngroups = 0;
+    if (g.ngroups == 0)
+      return AKM_SUCCESS;
+    if (g.pair)
+      AKM_TRY(g.work.allocate(int64_t(g.ngroups) * g.cells * m.N * int64_t(m.esize)));
+    AKM_TRY(gs_refresh(m, g));
+    AKM_HIP(hipStreamSynchronize(m.stream)); // another stream may be captured next
     return AKM_SUCCESS;
-  if (g.pair)
-    AKM_TRY(g.work.allocate(int64_t(g.ngroups) * g.cells * m.N * int64_t(m.esize)));
-  AKM_TRY(gs_refresh(m, g));
-  AKM_HIP(hipStreamSynchronize(m.stream)); // another stream may be captured next
-  return AKM_SUCCESS;
+  };
+  const int rc = build();
+  if (rc != AKM_SUCCESS)
+    g.ngroups = 0; // too large, or out of memory: what was made is not used
+  return rc;
 }
 
 //! Builds the padded cell set, the fibres, the chains and the work buffers
