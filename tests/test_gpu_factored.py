@@ -3,8 +3,9 @@ kernels of the same handle.
 
 A handle whose factors are mostly the identity (or whose grid allows the
 split of every product) applies its operator along fibres instead of pair by
-pair.  ``set_tuning`` with a shape selects the pair kernels, which are the
-general path here.  Bars: 1e-13 of the largest result in FP64 and 1e-5 in
+pair where that is estimated to be faster.  ``set_tuning`` with a shape selects
+the pair kernels, which are the general path here; ``apply_form`` tells which
+way an apply goes, and every test looks.  Bars: 1e-13 of the largest result in FP64 and 1e-5 in
 FP32, the kronmult parity bars.
 """
 import numpy as np
@@ -40,11 +41,14 @@ def tables(d, level, refine):
     return table, int(table[:, :d].max())
 
 
-def both(m, x, alpha, beta, y0):
-    """The result of the chosen path and of the pair kernels."""
+def both(m, x, alpha, beta, y0, form=None):
+    """The result of the chosen path (`form`, unless None) and of the pair
+    kernels."""
     out = []
     for waves in (0, 4):
         m.set_tuning(waves_per_row=waves)
+        assert waves == 0 or m.apply_form() == (0, 1)
+        assert waves or form is None or m.apply_form() == form
         y = torch.from_numpy(y0.copy()).cuda()
         m.apply(alpha, x, beta, y)
         out.append(y.cpu().numpy().astype(np.float64))
@@ -58,12 +62,12 @@ def close(a, b, dtype):
 
 CASES = [
     # (d, n, level, refine, non-identity dimensions per term)
-    (1, 2, 5, True, [(0,)]),
+    (1, 2, 7, True, [(0,)] * 24),                   # one table for all terms
     (2, 2, 6, False, [(0,), (1,), (1,)]),           # two terms share a table
     (2, 3, 5, True, [(1,), ()]),                    # an identity term, refined
-    (2, 4, 5, False, [(0, 1), (1,)]),               # n = 4, two stages
-    (3, 2, 6, False, [(0, 2), (0, 1, 2), ()]),
-    (3, 3, 5, False, [(0, 1, 2), (1, 2)]),
+    (3, 4, 5, False, [(0, 1), (1,)]),               # n = 4, two stages
+    (4, 2, 6, False, [(0, 2), (0, 1, 2), ()]),      # three stages
+    (4, 3, 5, False, [(0, 1, 2), (1, 2)]),
     (3, 4, 4, True, [(0,), (2,)]),
     (4, 2, 6, True, [(0,), (1,), (2,), (3,)]),
     (4, 3, 4, False, [(3,), (0,)]),                 # 81 lanes: 1024-thread groups
@@ -87,8 +91,9 @@ def test_matches_pair_kernels(case, dtype):
     m = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, T, vA, dtype=dtype)
     x = torch.from_numpy(rng.uniform(-1, 1, m.input_size()).astype(dtype)).cuda()
     y0 = rng.uniform(-1, 1, m.output_size()).astype(dtype)
+    form = (8, max(len(a) for a in active))
     for alpha, beta in ((1.0, 0.0), (-0.7, 0.4), (0.0, 2.0)):
-        got, want = both(m, x, alpha, beta, y0)
+        got, want = both(m, x, alpha, beta, y0, form)
         assert close(got, want, dtype), (alpha, beta)
     if dtype == np.float64:
         out = []
@@ -102,9 +107,10 @@ def test_matches_pair_kernels(case, dtype):
 
 def test_repeats_bit_for_bit_and_streams():
     rng = np.random.default_rng(3)
-    table, top = tables(3, 5, False)
-    vA = grid.build_vA(3, 2, 1, top, factors(rng, 3, 2, top, [(0, 1, 2)]))
-    m = asgard_amd.KronmultMatrix.sparse_grid(3, 2, table, top, 1, vA)
+    table, top = tables(4, 6, False)
+    vA = grid.build_vA(4, 2, 1, top, factors(rng, 4, 2, top, [(0, 1, 2)]))
+    m = asgard_amd.KronmultMatrix.sparse_grid(4, 2, table, top, 1, vA)
+    assert m.apply_form() == (8, 3)  # its stages share work vectors
     x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
     torch.cuda.synchronize()
     outs = []
@@ -124,17 +130,19 @@ def test_repeats_bit_for_bit_and_streams():
 
 @pytest.mark.parametrize("on_device", [False, True])
 def test_new_factors_change_the_form(on_device):
-    """Updates that keep, add and drop non-identity factors."""
+    """Updates that keep, add and drop non-identity factors; a form whose
+    factors cover the new ones stays (its stages too)."""
     rng = np.random.default_rng(5)
-    d, n = 3, 2
-    table, top = tables(d, 5, False)
-    patterns = [[(0,), (1,)], [(1,), (1, 2)], [(0,), (1,)], [(0, 1, 2), (2,)], [(), (0,)]]
-    ops = factors(rng, d, n, top, patterns[0])
+    d, n = 4, 2
+    table, top = tables(d, 6, False)
+    steps = [([(0,), (1,)], 1), ([(0,), (1, 2)], 2), ([(0,), (1,)], 2), ([(0,), ()], 2),
+             ([(3,), (0, 1, 2)], 3), ([(3,), (0, 2)], 3), ([(0, 1, 2), (2,)], 3), ([(), (3,)], 1)]
+    ops = factors(rng, d, n, top, steps[0][0])
     m = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, 2,
                                               grid.build_vA(d, n, 2, top, ops))
     x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
     y0 = np.zeros(m.output_size())
-    for active in patterns:
+    for active, stages in steps:
         ops = factors(rng, d, n, top, active)
         vA = grid.build_vA(d, n, 2, top, ops)
         if on_device:
@@ -142,7 +150,7 @@ def test_new_factors_change_the_form(on_device):
                                 for o in ops])
         else:
             m.update_stored_coefficients(vA)
-        got, want = both(m, x, 1.0, 0.0, y0)
+        got, want = both(m, x, 1.0, 0.0, y0, (8, stages))
         assert close(got, want, np.float64), active
         fresh = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, 2, vA)
         fresh.set_tuning(waves_per_row=4)
@@ -153,23 +161,42 @@ def test_new_factors_change_the_form(on_device):
 
 def test_forms_the_split_does_not_cover():
     """Cells missing from a level, factors that are not finite and repeated
-    cells stay with the pair kernels."""
+    cells stay with the pair kernels, on a grid whose operators have a form
+    otherwise."""
     rng = np.random.default_rng(9)
-    table, top = tables(2, 5, False)
-    ops = factors(rng, 2, 2, top, [(0, 1)])
-    y0 = np.zeros(len(table) * 4)
-    for cells in (table[:-1], np.concatenate([table, table[:1]])):
-        vA = grid.build_vA(2, 2, 1, top, ops)
-        m = asgard_amd.KronmultMatrix.sparse_grid(2, 2, cells, top, 1, vA)
+    d, n = 4, 2
+    table, top = tables(d, 6, False)
+
+    def make(cells, vA):
+        return asgard_amd.KronmultMatrix.sparse_grid(d, n, cells, top, 2, vA)
+
+    split = grid.build_vA(d, n, 2, top, factors(rng, d, n, top, [(0, 1), (2, 3)]))
+    plain = grid.build_vA(d, n, 2, top, factors(rng, d, n, top, [(0,), (2,)]))
+    assert make(table, split).apply_form() == (8, 2)
+    assert make(table, plain).apply_form() == (8, 1)
+    repeated = np.concatenate([table, table[:1]])
+    pair = (0, 1)
+    for cells, vA, form in ((table[:-1], split, pair), (repeated, split, pair),
+                            (table[:-1], plain, (8, 1)), (repeated, plain, pair)):
+        m = make(cells, vA)
         x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
-        got, want = both(m, x, 1.0, 0.0, np.zeros(m.output_size()))
+        got, want = both(m, x, 1.0, 0.0, np.zeros(m.output_size()), form)
         assert close(got, want, np.float64)
-    bad = grid.build_vA(2, 2, 1, top, factors(rng, 2, 2, top, [(0,)]))
+    bad = plain.copy()
     bad[3] = np.inf
-    m = asgard_amd.KronmultMatrix.sparse_grid(2, 2, table, top, 1, bad)
+    m = make(table, bad)
     x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
-    got, want = both(m, x, 1.0, 0.0, y0)
-    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    y0 = np.zeros(m.output_size())
+    got, want = both(m, x, 1.0, 0.0, y0, pair)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want)) and not np.isfinite(got).all()
+    m.update_stored_coefficients(plain)
+    got, want = both(m, x, 1.0, 0.0, y0, (8, 1))
+    assert close(got, want, np.float64)
+    m.update_stored_coefficients(bad)
+    assert m.apply_form() == pair
+    m.update_stored_coefficients(plain)
+    got, want = both(m, x, 1.0, 0.0, y0, (8, 1))
+    assert close(got, want, np.float64)
 
 
 def test_autotuned_small_and_large_agree():
@@ -180,7 +207,8 @@ def test_autotuned_small_and_large_agree():
     vA = grid.build_vA(d, n, 3, top, factors(rng, d, n, top, active))
     m = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, top, 3, vA)
     x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
-    m.autotune(x, torch.zeros_like(x))
+    assert m.autotune(x, torch.zeros_like(x))[1] == 3
+    assert m.apply_form() in ((8, 2), (6, 2))  # whichever was faster
     y = torch.zeros_like(x)
     m.apply(1.0, x, 0.0, y)
     m.set_tuning(waves_per_row=4)
@@ -190,8 +218,8 @@ def test_autotuned_small_and_large_agree():
 
 
 def test_batch_mixes_both_ways_of_applying():
-    """Systems along fibres (workgroups of 256, 512 and 1024 threads) and pair
-    by pair in one batch, across a restart and after new factors."""
+    """Systems along fibres (workgroups of 256 and 1024 threads) and pair by
+    pair in one batch, across a restart and after new factors."""
     rng = np.random.default_rng(17)
     shapes = [(2, 2, 5, True, [(0,), (1,)]), (4, 3, 3, True, [(0,), (3,)]),
               (5, 3, 2, False, [(4,), (0,)]), (3, 4, 3, False, [(1,)]),
@@ -302,6 +330,7 @@ def test_walk_of_single_entries_and_wide_blocks(case, dtype):
     walk = asgard_amd.KronmultMatrix.global_grid(d, n, table, top, T, vA, dtype=dtype,
                                                  active=grid.identity_mask(ops, T, d))
     walk.set_tuning(waves_per_row=8)
+    assert walk.apply_form() == (8, max(len(a) for a in active))
     x = torch.from_numpy(rng.uniform(-1, 1, pair.input_size()).astype(dtype)).cuda()
     y0 = rng.uniform(-1, 1, pair.output_size()).astype(dtype)
     out = []

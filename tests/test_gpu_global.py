@@ -212,6 +212,8 @@ def test_same_operator_as_pairwise_at_bench_size():
     # d=3 n=3 |l|_1 <= 6, 3 terms: the bench workload
     c = grid_case(3, 3, 6, 3, seed=0)
     pair = asgard_amd.KronmultMatrix.sparse_grid(3, 3, c["table"], 6, 3, c["vA"])
+    pair.set_tuning(waves_per_row=4)
+    assert pair.apply_form() == (0, 1)
     glob = global_matrix(c)
     x = dev(c["x"])
     y1 = dev(np.zeros_like(c["x"]))
@@ -349,6 +351,8 @@ def test_slab_layout_vlasov_d6_full_size():
     ops = dg.operators_vlasov(n, L)
     vA = oracle.build_vA(d, n, T, L, ops)
     pair = asgard_amd.KronmultMatrix.sparse_grid(d, n, table, L, T, vA)
+    pair.set_tuning(waves_per_row=4)
+    assert pair.apply_form() == (0, 1)
     # identity factors skipped, as the reference does for its mass terms
     act = grid.identity_mask(ops, T, d)
     glob = asgard_amd.KronmultMatrix.global_grid(d, n, table, L, T, vA, active=act)
