@@ -24,6 +24,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
 from collections import namedtuple
 
 import numpy as np
@@ -215,7 +216,7 @@ def _is_torch(t):
 def _vec_ptr(v, dtype):
     """(pointer, on_device) of a torch CUDA tensor or numpy array of `dtype`."""
     if _is_torch(v):
-        import torch
+        torch = sys.modules["torch"]  # an import statement costs 0.1 us a vector
         want = torch.float64 if dtype == np.float64 else torch.float32
         if v.dtype != want or not v.is_contiguous():
             raise AkmInvalid(AKM_ERR_INVALID, f"vector must be a contiguous {want} tensor")
@@ -422,7 +423,10 @@ class KronmultMatrix:
         py, dy = _vec_ptr(y, self.dtype)
         if dx != dy:
             raise AkmInvalid(AKM_ERR_INVALID, "x and y must both be host or both device")
-        _check(load_library().akm_apply(self._h, float(alpha), px, float(beta), py, dx))
+        # (a handle's library is loaded)
+        rc = _lib.akm_apply(self._h, float(alpha), px, float(beta), py, dx)
+        if rc != AKM_SUCCESS:
+            _check(rc)
         return y
 
     def apply_euler(self, dt, alpha, x, beta, y):
