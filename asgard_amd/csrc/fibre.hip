@@ -31,6 +31,7 @@
 // d = 2 n = 2 level 5 3.3 (3.9 / 6.5); d = 3 n = 3 level 6, every factor
 // dense, three stages 24 (23 / 60).
 #include "fibre.hpp"
+#include "grid.hpp"
 #include "kron_kernels.hpp"
 #include "matrix.hpp"
 
@@ -507,40 +508,6 @@ static void fill_range(gk_lists const &l, int cell, int fill, int &lo, int &hi)
   hi = (fill == gk_lower) ? l.diag[cell] + 1 : l.ptr[cell + 1];
 }
 } // namespace
-
-void order_by_dims(int d, int64_t cells, const int *elem, std::vector<int> const &dims, int M,
-                   std::vector<int> &order)
-{
-  order.resize(cells);
-  std::iota(order.begin(), order.end(), 0);
-  if (M > 16 * cells + 1024)
-  {
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-      for (int k : dims)
-      {
-        const int ea = elem[int64_t(a) * d + k], eb = elem[int64_t(b) * d + k];
-        if (ea != eb)
-          return ea < eb;
-      }
-      return false;
-    });
-    return;
-  }
-  // stable counting sorts, the least significant dimension first
-  std::vector<int> count(M + 1), next(cells);
-  for (size_t i = dims.size(); i-- > 0;)
-  {
-    const int k = dims[i];
-    std::fill(count.begin(), count.end(), 0);
-    for (int64_t c = 0; c < cells; c++)
-      count[elem[c * d + k] + 1]++;
-    for (int v = 0; v < M; v++)
-      count[v + 1] += count[v];
-    for (int c : order)
-      next[count[elem[int64_t(c) * d + k]]++] = c;
-    order.swap(next);
-  }
-}
 
 int build_fibre_lists(int d, int64_t cells, const int *elem, int k, int M,
                       std::vector<int> const &c1_pntr, std::vector<int> const &c1_indx,

@@ -31,11 +31,6 @@ struct gk_lists
   std::vector<int> ptr, cell, q, diag;
 };
 
-//! The cells 0 .. cells-1 ordered by their 1D indices in `dims` (the first
-//! the most significant), ties by cell id; 1D indices are below M.
-void order_by_dims(int d, int64_t cells, const int *elem, std::vector<int> const &dims, int M,
-                   std::vector<int> &order);
-
 //! Fibre lists along dimension k, and the cells fibre by fibre (fibres in
 //! the order of their other 1D indices).  `repeated` = the first cell equal
 //! to an earlier one, or -1.

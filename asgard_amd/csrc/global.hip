@@ -2783,7 +2783,14 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
     return set_error(AKM_ERR_UNSUPPORTED, "global kron: too many padded DOFs");
 
   // connect_1d (full hierarchy), the pattern of every 1D factor
-  AKM_TRY(build_connect_1d(m.max_level, true, g->c1_pntr_h, g->c1_indx_h, g->c1_diag_h));
+  if (pair)
+  {
+    g->c1_pntr_h = m.conn_pntr_host;
+    g->c1_indx_h = m.conn_indx_host;
+    g->c1_diag_h = m.conn_diag_host;
+  }
+  else
+    AKM_TRY(build_connect_1d(m.max_level, true, g->c1_pntr_h, g->c1_indx_h, g->c1_diag_h));
 
   // per dimension: the fibres (cells equal in every other 1D index) and for
   // every cell its connected cells of the fibre, 1D index ascending

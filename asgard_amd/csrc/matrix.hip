@@ -65,47 +65,20 @@ static int build_schedule(akm_matrix_s &m)
     order[r] = r;
   if (m.mode != mode_dense)
   {
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-      return (m.pntr[a + 1] - m.pntr[a]) > (m.pntr[b + 1] - m.pntr[b]);
-    });
+    int64_t longest = 0;
+    for (int r = 0; r < m.rows; r++)
+      longest = std::max(longest, m.pntr[r + 1] - m.pntr[r]);
+    int bits = 1;
+    while (longest >> bits != 0)
+      bits++;
+    std::vector<uint64_t> keys(m.rows);
+    for (int r = 0; r < m.rows; r++)
+      keys[r] = static_cast<uint64_t>(longest - (m.pntr[r + 1] - m.pntr[r]));
+    radix_order(keys, bits, order);
     AKM_TRY(m.pntr_dev.upload(m.pntr.data(), int64_t(m.pntr.size()), m.stream));
   }
   AKM_TRY(m.row_order.upload(order.data(), int64_t(order.size()), m.stream));
   return AKM_SUCCESS;
-}
-
-//! Re-lays the reference's vA ([connection][term][dim][n*n]) out as
-//! [dim][connection][term][nnp] for the LDS-table kernel: the blocks one
-//! row's 1D cell can touch in one dimension become one contiguous range.
-template<typename P>
-static void relayout_vA(akm_matrix_s const &m, const P *vA, std::vector<P> &out)
-{
-  const int d = m.d, T = m.T, nn = m.n * m.n, nnp = m.nnp;
-  out.assign(size_t(d) * m.nconn * T * nnp, P{0});
-  for (int64_t j = 0; j < m.nconn; j++)
-    for (int t = 0; t < T; t++)
-      for (int k = 0; k < d; k++)
-      {
-        const P *src = vA + ((j * T + t) * d + k) * nn;
-        P *dst = out.data() + ((int64_t(k) * m.nconn + j) * T + t) * nnp;
-        for (int q = 0; q < nn; q++)
-          dst[q] = src[q];
-      }
-}
-
-static int upload_vAk(akm_matrix_s &m, const void *vA)
-{
-  if (m.prec == AKM_F64)
-  {
-    std::vector<double> v;
-    relayout_vA(m, static_cast<const double *>(vA), v);
-    return m.vAk.upload(reinterpret_cast<const unsigned char *>(v.data()),
-                        int64_t(v.size() * sizeof(double)), m.stream);
-  }
-  std::vector<float> v;
-  relayout_vA(m, static_cast<const float *>(vA), v);
-  return m.vAk.upload(reinterpret_cast<const unsigned char *>(v.data()),
-                      int64_t(v.size() * sizeof(float)), m.stream);
 }
 
 //! LDS bytes the sparse-grid kernel may use: the whole 160 KB of a CU minus
@@ -412,8 +385,9 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
     return set_error(AKM_ERR_INVALID, "sparse-grid kronmult: level %d above max_level %d",
                      lmax, max_level);
   std::vector<int> offtab, p1, i1, dg;
-  AKM_TRY(build_offset_table(max_level, offtab));
-  AKM_TRY(build_connect_1d(max_level, true, p1, i1, dg));
+  if (max_level <= 12) // (build_offset_table refuses more)
+    AKM_TRY(build_connect_1d(max_level, true, p1, i1, dg));
+  AKM_TRY(build_offset_table(max_level, p1, i1, offtab));
   const int64_t nconn = static_cast<int64_t>(i1.size());
   const int64_t expect_vA = nconn * d * T * int64_t(n) * n;
   if (T > 0 && (vA == nullptr || num_vA != expect_vA))
@@ -429,7 +403,17 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
   // each row's columns in lexicographic order of their 1D indices: the
   // sum-factorised kernels close a group of columns when its prefix changes
   lexicographic_order(d, num_cells, elem.data(), lex);
-  AKM_TRY(device_sparse_pattern(d, num_cells, table, m->pntr, m->indx, lex.data()));
+  std::vector<uint64_t> pack; // 1D indices, 10 bits a dimension
+  if (max_level <= 10 && num_cells > 0)
+  {
+    pack.assign(num_cells, 0);
+    for (int64_t c = 0; c < num_cells; c++)
+      for (int k = 0; k < d; k++)
+        pack[c] |= static_cast<uint64_t>(elem[c * d + k]) << (10 * k);
+    AKM_TRY(device_sparse_pattern(d, pack, max_level, p1, i1, lex, m->pntr, m->indx));
+  }
+  else
+    AKM_TRY(device_sparse_pattern(d, num_cells, table, m->pntr, m->indx, lex.data()));
   m->nnz = m->pntr[num_cells];
   AKM_TRY(m->elem.upload(elem.data(), int64_t(elem.size())));
   AKM_TRY(m->off1d.upload(offtab.data(), int64_t(offtab.size())));
@@ -438,6 +422,8 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
   m->num_vA = num_vA;
   m->nconn = static_cast<int>(nconn);
   m->conn_pntr_host = p1;
+  m->conn_indx_host = i1;
+  m->conn_diag_host = dg;
   if (T > 0)
   {
     AKM_TRY(m->vA.upload(static_cast<const unsigned char *>(vA), num_vA * m->esize));
@@ -445,18 +431,11 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
     {
       // LDS-table kernel inputs: packed cell words, connect_1d row pointer,
       // factors re-laid out per dimension, largest per-row table
-      std::vector<unsigned long long> pack(num_cells);
-      for (int64_t c = 0; c < num_cells; c++)
-      {
-        unsigned long long w = 0;
-        for (int k = 0; k < d; k++)
-          w |= static_cast<unsigned long long>(elem[c * d + k]) << (10 * k);
-        pack[c] = w;
-      }
-      AKM_TRY(m->epack.upload(pack.data(), num_cells));
+      AKM_TRY(m->epack.upload(reinterpret_cast<const unsigned long long *>(pack.data()),
+                              num_cells));
       AKM_TRY(m->conn_pntr.upload(p1.data(), int64_t(p1.size())));
       m->nnp = (m->prec == AKM_F64) ? padded_block<double>(n) : padded_block<float>(n);
-      AKM_TRY(upload_vAk(*m, vA));
+      AKM_TRY(relayout_factors(*m));
       int64_t mx = 0, mx2 = 0;
       for (int64_t c = 0; c < num_cells; c++)
       {
@@ -544,7 +523,7 @@ akm_status akm_update_coefficients(akm_matrix mat, const void *values)
     AKM_HIP(hipMemcpyAsync(mat->vA.data(), values, mat->num_vA * mat->esize,
                            hipMemcpyHostToDevice, mat->stream));
     if (mat->vAk.data() != nullptr)
-      AKM_TRY(upload_vAk(*mat, values));
+      AKM_TRY(relayout_factors(*mat));
     if (mat->mode == mode_grid)
       AKM_TRY(factored_refresh(*mat));
   }

@@ -40,7 +40,7 @@ struct akm_matrix_s
   akm::dev_buffer<unsigned char> vAk;
   akm::dev_buffer<int> conn_pntr;
   akm::dev_buffer<unsigned long long> epack;
-  std::vector<int> conn_pntr_host;
+  std::vector<int> conn_pntr_host, conn_indx_host, conn_diag_host;
   int nconn = 0, nnp = 0;
   int64_t max_table_elems = 0;
   int64_t max_table_last4 = 0; // largest per-row table of the last four dimensions
@@ -127,6 +127,11 @@ int global_device_jacobi(akm_matrix_s &m);
 //! factors, in place.  An apply never does: it may be captured into a graph,
 //! or be the first after one was.
 int global_tables(akm_matrix_s &m);
+//! Fills vAk from vA: the factors re-laid from [connection][term][dim][n*n] to
+//! [dim][connection][term][nnp] for the LDS-table kernel, so that the blocks
+//! one row's 1D cell can touch in one dimension are one contiguous range.
+int relayout_factors(akm_matrix_s &m);
+
 //! Which of a sparse-grid handle's T x d stored factors are not exactly the
 //! identity, and whether all their values are finite: scanned on the device.
 int stored_factors(akm_matrix_s &m, std::vector<int> &mask, bool &finite);

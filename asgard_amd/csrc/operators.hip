@@ -93,6 +93,23 @@ __global__ void __launch_bounds__(op_threads)
   }
 }
 
+int relayout_factors(akm_matrix_s &m)
+{
+  const int64_t count = int64_t(m.d) * m.nconn * m.T * m.nnp;
+  AKM_TRY(m.vAk.allocate(count * int64_t(m.esize)));
+  auto go = [&](auto zero) {
+    using P = decltype(zero);
+    relayout_blocks<P><<<op_blocks(count), op_threads, 0, m.stream>>>(
+        reinterpret_cast<const P *>(m.vA.data()), m.nconn, m.T, m.d, m.n, m.nnp,
+        reinterpret_cast<P *>(m.vAk.data()));
+  };
+  if (m.prec == AKM_F64)
+    go(0.0);
+  else
+    go(0.0f);
+  return check_launch("LDS tables");
+}
+
 template<typename P>
 static int update_operators_typed(akm_matrix_s &m, const void *const *ops_dev, int64_t lda)
 {
@@ -115,11 +132,7 @@ static int update_operators_typed(akm_matrix_s &m, const void *const *ops_dev, i
       ops, lda, m.op_conn.data(), m.op_conn.data() + nconn, nconn, T, d, n, vA);
   AKM_TRY(check_launch("operator update (factor blocks)"));
   if (m.mode == mode_grid && m.vAk.data() != nullptr)
-  {
-    relayout_blocks<P><<<op_blocks(int64_t(d) * nconn * T * m.nnp), op_threads, 0, m.stream>>>(
-        vA, nconn, T, d, n, m.nnp, reinterpret_cast<P *>(m.vAk.data()));
-    AKM_TRY(check_launch("operator update (LDS tables)"));
-  }
+    AKM_TRY(relayout_factors(m));
   if (m.mode == mode_global)
   {
     AKM_TRY(global_device_jacobi(m));
@@ -133,8 +146,9 @@ static int need_connections(akm_matrix_s &m)
 {
   if (m.op_conn.size() > 0)
     return AKM_SUCCESS;
-  std::vector<int> p1, i1, dg;
-  AKM_TRY(build_connect_1d(m.max_level, true, p1, i1, dg));
+  std::vector<int> p1 = m.conn_pntr_host, i1 = m.conn_indx_host, dg;
+  if (i1.empty())
+    AKM_TRY(build_connect_1d(m.max_level, true, p1, i1, dg));
   const int64_t nconn = static_cast<int64_t>(i1.size());
   if (nconn * m.T * m.d * m.n * m.n != m.num_vA)
     return set_error(AKM_ERR_INVALID, "operator update: stored blocks do not match connect_1d");
