@@ -38,7 +38,7 @@
 #include <algorithm>
 #include <array>
 #include <map>
-#include <numeric>
+#include <memory>
 #include <type_traits>
 
 namespace akm
@@ -673,150 +673,217 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
   std::vector<int> stride(d, 1);
   for (int k = d - 2; k >= 0; k--)
     stride[k] = stride[k + 1] * n;
-  auto new_piece = [&](product const &p, int cell) {
-    fl_piece_rec r{};
-    r.in = p.in;
-    r.stride = stride[p.k];
-    r.magic = (r.stride == 1)
-                  ? 0
-                  : static_cast<unsigned>(((uint64_t(1) << 32) + r.stride - 1) / r.stride);
-    for (auto &en : r.entry)
-      en = make_int2(p.in == 0 && cell >= active_cells ? 0 : cell, zero_block);
-    return r;
+  std::vector<unsigned> magic(d);
+  for (int k = 0; k < d; k++)
+    magic[k] = (stride[k] == 1)
+                   ? 0
+                   : static_cast<unsigned>(((uint64_t(1) << 32) + stride[k] - 1) / stride[k]);
+
+  // A job is one cell of one output vector.  cut() deals its products'
+  // connections out in pieces: piece(product, list, from, to, connections,
+  // first of a slot) for every piece in order.
+  const int S = plan.nslot;
+  struct job
+  {
+    int out, cell;
+    int slots, more; // slots; pieces beyond the slots' first ones
+    int length;      // connections
+    int64_t slot0, piece0;
+  };
+  auto cut = [&](std::vector<int> const &prods, int c, auto &&piece) -> int64_t {
+    int64_t total = 0, whole = 0; // connections; slots with one piece each
+    for (int i : prods)
+    {
+      int lo, hi;
+      fill_range(lists[prog.prods[i].k], c, prog.prods[i].fill, lo, hi);
+      total += hi - lo;
+      whole += (hi - lo + fl_piece - 1) / fl_piece;
+    }
+    // slots of equal length when one-piece slots do not fit
+    const bool split = whole <= S;
+    const int64_t target = split ? fl_piece : (total + S - 1) / S;
+    int64_t room = 0;
+    for (int i : prods)
+    {
+      product const &p = prog.prods[i];
+      gk_lists const &l = lists[p.k];
+      int lo, hi;
+      fill_range(l, c, p.fill, lo, hi);
+      if (split)
+        room = 0; // pieces do not share slots
+      while (lo < hi)
+      {
+        const bool fresh = room == 0;
+        if (fresh)
+          room = target;
+        const int from = lo;
+        int len = 0;
+        if (p.in != 0 || active_cells == cells)
+        {
+          len = static_cast<int>(std::min<int64_t>({hi - lo, fl_piece, room}));
+          lo += len;
+        }
+        else
+          // cells the input does not hold are zero
+          for (; lo < hi && len < fl_piece && len < room; lo++)
+            len += (l.cell[lo] < active_cells) ? 1 : 0;
+        piece(p, l, from, lo, len, fresh);
+        room -= len;
+      }
+    }
+    return total;
   };
 
-  // slots, stage by stage
-  std::vector<fl_slot_rec> slots;
-  std::vector<fl_piece_rec> pieces;
-  fl_slot_rec empty{};
-  empty.cell = -1;
-  const int S = plan.nslot;
+  // stage by stage: every job's size, then the jobs of many slots first, then
+  // long ones (a wavefront's pieces are alike and the long jobs start early),
+  // which gives every record its place
   const int nstages = std::max(prog.stages, 1);
-  struct job_rec
-  {
-    int first, count, length; // its slots in `made`, its connections
-  };
+  std::vector<job> jobs; // in their order in the plan
+  std::vector<std::map<int, std::vector<int>>> outs(nstages); // output vector -> products
+  std::vector<size_t> stage_end(nstages);
+  int64_t nslots = 0, npieces = 0;
   for (int st = 0; st < nstages; st++)
   {
-    std::map<int, std::vector<int>> outs; // output vector -> its products
     for (size_t i = 0; i < prog.prods.size(); i++)
       if (prog.prods[i].stage == st)
-        outs[prog.prods[i].out].push_back(static_cast<int>(i));
+        outs[st][prog.prods[i].out].push_back(static_cast<int>(i));
     if (st + 1 == nstages)
-      outs[-1]; // y is always written
-    std::vector<fl_slot_rec> made;
-    std::vector<job_rec> jobs;
-    for (auto &ov : outs)
+      outs[st][-1]; // y is always written
+    std::vector<job> made;
+    int most = 0, longest = 0;
+    for (auto &ov : outs[st])
     {
       // products of one dimension together: a slot's rounds are few
       std::stable_sort(ov.second.begin(), ov.second.end(),
                        [&](int u, int v) { return prog.prods[u].k < prog.prods[v].k; });
       const int64_t ncell = (ov.first < 0) ? active_cells : cells;
-      for (int64_t c64 = 0; c64 < ncell; c64++)
+      for (int64_t c = 0; c < ncell; c++)
       {
-        const int c = static_cast<int>(c64);
-        int64_t total = 0;
-        int whole = 0; // slots with one piece each
-        for (int i : ov.second)
-        {
-          int lo, hi;
-          fill_range(lists[prog.prods[i].k], c, prog.prods[i].fill, lo, hi);
-          total += hi - lo;
-          whole += (hi - lo + fl_piece - 1) / fl_piece;
-        }
-        // slots of equal length when one-piece slots do not fit
-        const bool split = whole <= S;
-        const int64_t target = split ? fl_piece : (total + S - 1) / S;
-        const int first = static_cast<int>(made.size());
-        int64_t room = 0;
-        for (int i : ov.second)
-        {
-          product const &p = prog.prods[i];
-          gk_lists const &l = lists[p.k];
-          int lo, hi;
-          fill_range(l, c, p.fill, lo, hi);
-          if (split)
-            room = 0; // pieces do not share slots
-          while (lo < hi)
-          {
-            const bool fresh = room == 0;
-            if (fresh)
-              room = target;
-            fl_piece_rec pr = new_piece(p, c);
-            int len = 0;
-            for (; lo < hi && len < fl_piece && len < room; lo++)
-            {
-              // cells the input does not hold are zero
-              if (p.in == 0 && l.cell[lo] >= active_cells)
-                continue;
-              int q = l.q[lo];
-              if (lo == l.diag[c] && p.fill != gk_full)
-                q = plan.nconn + elem[c64 * d + p.k] + (p.fill == gk_lower ? plan.M : 0);
-              pr.entry[len++] = make_int2(l.cell[lo], static_cast<int>(p.table * blocks + q));
-            }
-            room -= len;
-            pr.len = len | (1 << 16);
-            if (fresh)
-            {
-              fl_slot_rec sr{};
-              sr.cell = c;
-              sr.group = static_cast<int>(made.size()) - first;
-              sr.vec = ov.first < 0 ? -1 : ov.first - 1;
-              sr.rounds = 1;
-              sr.p = pr;
-              made.push_back(sr);
-            }
-            else
-            {
-              fl_slot_rec &sr = made.back();
-              fl_piece_rec &before = (sr.more == 0) ? sr.p : pieces.back();
-              if (before.stride == pr.stride)
-                before.len &= 0xffff; // the same round goes on
-              else
-                sr.rounds++;
-              if (sr.more++ == 0)
-                sr.next = static_cast<int>(pieces.size());
-              pieces.push_back(pr);
-            }
-          }
-        }
-        if (static_cast<int>(made.size()) == first)
-        {
-          fl_slot_rec sr{};
-          sr.cell = c;
-          sr.vec = ov.first < 0 ? -1 : ov.first - 1;
-          sr.rounds = 1;
-          sr.p = new_piece(product{0, 0, 0, gk_full, 0, 0}, c);
-          sr.p.len = 1 << 16;
-          made.push_back(sr);
-        }
-        const int count = static_cast<int>(made.size()) - first;
-        for (int i = first; i < first + count; i++)
-          made[i].group |= count << 16;
-        jobs.push_back({first, count, static_cast<int>(std::min<int64_t>(total, 1 << 30))});
+        job jb{ov.first, static_cast<int>(c), 0, 0, 0, 0, 0};
+        const int64_t total =
+            cut(ov.second, jb.cell,
+                [&](product const &, gk_lists const &, int, int, int, bool fresh) {
+                  (fresh ? jb.slots : jb.more)++;
+                });
+        jb.slots = std::max(jb.slots, 1);
+        jb.length = static_cast<int>(std::min<int64_t>(total, 1 << 30));
+        most = std::max(most, jb.slots);
+        longest = std::max(longest, jb.length);
+        made.push_back(jb);
       }
     }
-    // jobs of many slots first, then long ones: a wavefront's pieces are
-    // alike and the long jobs start early
-    std::stable_sort(jobs.begin(), jobs.end(), [](job_rec const &u, job_rec const &v) {
-      return u.count != v.count ? u.count > v.count : u.length > v.length;
-    });
+    int bits = 1; // of a length
+    while (longest >> bits != 0)
+      bits++;
+    std::vector<uint64_t> keys(made.size());
+    for (size_t i = 0; i < made.size(); i++)
+      keys[i] = static_cast<uint64_t>(most - made[i].slots) << bits |
+                static_cast<uint64_t>(longest - made[i].length);
+    int all = bits + 1;
+    while (most >> (all - bits) != 0)
+      all++;
+    std::vector<int> order;
+    radix_order(keys, all, order);
     fibre_plan::stage rec;
-    rec.first_group = static_cast<int>(slots.size() / S);
-    for (auto const &j : jobs)
+    rec.first_group = static_cast<int>(nslots / S);
+    for (int i : order)
     {
-      while (slots.size() % S != 0 && S - static_cast<int>(slots.size() % S) < j.count)
-        slots.push_back(empty);
-      slots.insert(slots.end(), made.begin() + j.first, made.begin() + j.first + j.count);
+      job &jb = made[i];
+      if (nslots % S != 0 && S - nslots % S < jb.slots)
+        nslots += S - nslots % S;
+      jb.slot0 = nslots;
+      jb.piece0 = npieces;
+      nslots += jb.slots;
+      npieces += jb.more;
+      jobs.push_back(jb);
     }
-    while (slots.size() % S != 0)
-      slots.push_back(empty);
-    rec.groups = static_cast<int>(slots.size() / S) - rec.first_group;
+    nslots = (nslots + S - 1) / S * S;
+    rec.groups = static_cast<int>(nslots / S) - rec.first_group;
     plan.stages.push_back(rec);
+    stage_end[st] = jobs.size();
   }
-  if (slots.size() > (size_t(1) << 28) || pieces.size() > (size_t(1) << 28))
+  if (nslots > (int64_t(1) << 28) || npieces > (int64_t(1) << 28))
     return set_error(AKM_ERR_UNSUPPORTED, "fibre plan: too many slots");
-  for (size_t g = 0; g < slots.size(); g += S)
+
+  // the records, each written once where it stays
+  std::unique_ptr<fl_slot_rec[]> slots(new fl_slot_rec[nslots]);
+  std::unique_ptr<fl_piece_rec[]> pieces(new fl_piece_rec[npieces]);
+  auto write = [&](fl_piece_rec &r, product const &p, int cell, int len) {
+    r.in = p.in;
+    r.stride = stride[p.k];
+    r.magic = magic[p.k];
+    r.len = len | (1 << 16);
+    const int2 rest = make_int2(p.in == 0 && cell >= active_cells ? 0 : cell, zero_block);
+    for (int u = len; u < fl_piece; u++)
+      r.entry[u] = rest;
+  };
+  auto fill_job = [&](std::map<int, std::vector<int>> const &products, job const &jb) {
+    fl_slot_rec *sr = slots.get() + jb.slot0 - 1;
+    fl_piece_rec *more = pieces.get() + jb.piece0, *before = nullptr;
+    int rank = 0;
+    auto open_slot = [&] {
+      sr++;
+      sr->cell = jb.cell;
+      sr->group = rank++ | jb.slots << 16;
+      sr->vec = jb.out < 0 ? -1 : jb.out - 1;
+      sr->more = sr->next = 0;
+      sr->rounds = 1;
+      sr->pad[0] = sr->pad[1] = 0;
+    };
+    cut(products.at(jb.out), jb.cell,
+        [&](product const &p, gk_lists const &l, int from, int to, int len, bool fresh) {
+          if (fresh)
+            open_slot();
+          fl_piece_rec &r = fresh ? sr->p : *more;
+          write(r, p, jb.cell, len);
+          const bool all = p.in != 0 || active_cells == cells;
+          int u = 0;
+          for (int q = from; q < to; q++)
+          {
+            if (!all && l.cell[q] >= active_cells)
+              continue;
+            int b = l.q[q];
+            if (q == l.diag[jb.cell] && p.fill != gk_full)
+              b = plan.nconn + elem[int64_t(jb.cell) * d + p.k] +
+                  (p.fill == gk_lower ? plan.M : 0);
+            r.entry[u++] = make_int2(l.cell[q], static_cast<int>(p.table * blocks + b));
+          }
+          if (!fresh)
+          {
+            if (before->stride == r.stride)
+              before->len &= 0xffff; // the same round goes on
+            else
+              sr->rounds++;
+            if (sr->more++ == 0)
+              sr->next = static_cast<int>(more - pieces.get());
+            more++;
+          }
+          before = &r;
+        });
+    if (rank == 0)
+    {
+      open_slot();
+      write(sr->p, product{0, 0, 0, gk_full, 0, 0}, jb.cell, 0);
+    }
+  };
+  fl_slot_rec empty{};
+  empty.cell = -1;
+  int64_t done = 0; // slots written
+  size_t at = 0;
+  for (int st = 0; st < nstages; st++)
+  {
+    for (; at < stage_end[st]; at++)
+    {
+      for (; done < jobs[at].slot0; done++)
+        slots[done] = empty;
+      fill_job(outs[st], jobs[at]);
+      done = jobs[at].slot0 + jobs[at].slots;
+    }
+    const int64_t end = int64_t(plan.stages[st].first_group + plan.stages[st].groups) * S;
+    for (; done < end; done++)
+      slots[done] = empty;
+  }
+  for (int64_t g = 0; g < nslots; g += S)
   {
     int rounds = 1;
     for (int i = 0; i < S; i++)
@@ -832,13 +899,15 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
       src.insert(src.end(), {pr.first, pr.second});
     ptr.push_back(static_cast<int>(src.size() / 2));
   }
-  AKM_TRY(plan.slots.upload(reinterpret_cast<const int4 *>(slots.data()),
-                            int64_t(slots.size()) * 7, m.stream));
-  AKM_TRY(plan.pieces.upload(reinterpret_cast<const int4 *>(pieces.data()),
-                             int64_t(pieces.size()) * 5, m.stream));
-  AKM_TRY(plan.tab_ptr.upload(ptr.data(), int64_t(ptr.size()), m.stream));
-  AKM_TRY(plan.tab_src.upload(src.data(), int64_t(src.size()), m.stream));
-  AKM_TRY(plan.c1_diag.upload(c1_diag.data(), int64_t(c1_diag.size()), m.stream));
+  AKM_TRY(plan.slots.upload(reinterpret_cast<const int4 *>(slots.get()), nslots * 7, m.stream));
+  AKM_TRY(plan.pieces.upload(reinterpret_cast<const int4 *>(pieces.get()), npieces * 5, m.stream));
+  // one array: tab_ptr, tab_src, connect_1d's diagonal positions
+  std::vector<int> small = ptr;
+  plan.src0 = static_cast<int>(small.size());
+  small.insert(small.end(), src.begin(), src.end());
+  plan.diag0 = static_cast<int>(small.size());
+  small.insert(small.end(), c1_diag.begin(), c1_diag.end());
+  AKM_TRY(plan.tab_def.upload(small.data(), int64_t(small.size()), m.stream));
   AKM_TRY(plan.work.allocate(int64_t(plan.vectors) * plan.stride * int64_t(m.esize)));
   AKM_TRY(plan.tab.allocate((blocks * plan.ntab + 1) * n * n * int64_t(m.esize)));
   plan.tab_valid = false;
@@ -856,8 +925,8 @@ static int fibre_tables(akm_matrix_s const &m, fibre_plan &plan, hipStream_t str
   const int64_t count = int64_t(plan.nconn + 2 * plan.M) * nn * plan.ntab + nn;
   const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
   fl_tables<P><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(
-      reinterpret_cast<const P *>(m.vA.data()), plan.tab_ptr.data(), plan.tab_src.data(),
-      plan.c1_diag.data(), plan.ntab, plan.nconn, plan.M, m.n, m.d, m.T,
+      reinterpret_cast<const P *>(m.vA.data()), plan.tab_def.data(),
+      plan.tab_def.data() + plan.src0, plan.tab_def.data() + plan.diag0, plan.ntab, plan.nconn, plan.M, m.n, m.d, m.T,
       reinterpret_cast<P *>(plan.tab.data()));
   plan.stamp = m.vA_stamp;
   plan.tab_valid = true;

@@ -63,7 +63,10 @@ struct fibre_plan
   dev_buffer<unsigned char> work, tab;
   // factor tables: table i sums the (term, dimension) pairs
   // tab_src[tab_ptr[i] .. tab_ptr[i+1]) of the vA the matrix had at `stamp`
-  dev_buffer<int> tab_ptr, tab_src, c1_diag;
+  // (tab_def: tab_ptr, from src0 on tab_src, from diag0 on connect_1d's
+  // diagonal positions)
+  dev_buffer<int> tab_def;
+  int src0 = 0, diag0 = 0;
   int ntab = 0, nconn = 0, M = 0;
   int64_t stride = 0; // work vector size
   bool tab_valid = false;
