@@ -37,6 +37,7 @@
 
 #include <algorithm>
 #include <array>
+#include <deque>
 #include <map>
 #include <memory>
 #include <type_traits>
@@ -521,71 +522,73 @@ int build_fibre_lists(int d, int64_t cells, const int *elem, int k, int M,
   dims.push_back(k);
   order_by_dims(d, cells, elem, dims, M, order);
   repeated = -1;
-  // pass 0 counts every cell's connections, pass 1 writes them
-  std::vector<int> member(M, -1);
+  // fibre by fibre: every member's connections one after another, then each
+  // cell's piece to its place
+  struct link
+  {
+    int cell, q;
+  };
+  std::vector<int> member(M, -1), first(cells);
+  std::vector<link> found;
+  found.reserve(size_t(cells) * 4);
   out.ptr.assign(cells + 1, 0);
   out.diag.assign(cells, -1);
-  for (int pass = 0; pass < 2; pass++)
+  for (int64_t f0 = 0; f0 < cells;)
   {
-    for (int64_t f0 = 0; f0 < cells;)
+    const int *lead = elem + int64_t(order[f0]) * d;
+    int64_t f1 = f0;
+    for (; f1 < cells; f1++)
     {
-      const int *first = elem + int64_t(order[f0]) * d;
-      int64_t f1 = f0;
-      for (; f1 < cells; f1++)
-      {
-        const int *cell = elem + int64_t(order[f1]) * d;
-        bool same = true;
-        for (int j = 0; j < d && same; j++)
-          same = (j == k) || cell[j] == first[j];
-        if (!same)
-          break;
-        if (pass == 0 && member[cell[k]] >= 0 && (repeated < 0 || order[f1] < repeated))
-          repeated = order[f1];
-        member[cell[k]] = order[f1];
-      }
-      const int last = elem[int64_t(order[f1 - 1]) * d + k];
-      for (int64_t f = f0; f < f1; f++)
-      {
-        const int c = order[f], r = elem[int64_t(c) * d + k];
-        int cnt = 0;
-        const int base = out.ptr[c];
-        for (int q = c1_pntr[r]; q < c1_pntr[r + 1]; q++)
-        {
-          const int col = c1_indx[q];
-          if (col > last)
-            break;
-          if (member[col] < 0)
-            continue;
-          if (pass == 1)
-          {
-            if (q == c1_diag[r])
-              out.diag[c] = base + cnt;
-            out.cell[base + cnt] = member[col];
-            out.q[base + cnt] = q;
-          }
-          cnt++;
-        }
-        if (pass == 0)
-          out.ptr[c + 1] = cnt;
-      }
-      for (int64_t f = f0; f < f1; f++)
-        member[elem[int64_t(order[f]) * d + k]] = -1;
-      f0 = f1;
+      const int *cell = elem + int64_t(order[f1]) * d;
+      bool same = true;
+      for (int j = 0; j < d && same; j++)
+        same = (j == k) || cell[j] == lead[j];
+      if (!same)
+        break;
+      if (member[cell[k]] >= 0 && (repeated < 0 || order[f1] < repeated))
+        repeated = order[f1];
+      member[cell[k]] = order[f1];
     }
-    if (pass == 0)
+    const int last = elem[int64_t(order[f1 - 1]) * d + k];
+    for (int64_t f = f0; f < f1; f++)
     {
-      if (repeated >= 0)
-        return AKM_SUCCESS;
-      int64_t total = 0;
-      for (int64_t c = 0; c < cells; c++)
+      const int c = order[f], r = elem[int64_t(c) * d + k];
+      const size_t begin = found.size();
+      for (int q = c1_pntr[r]; q < c1_pntr[r + 1]; q++)
       {
-        total += out.ptr[c + 1];
-        if (total > (int64_t(1) << 31) - 1)
-          return set_error(AKM_ERR_UNSUPPORTED, "global kron: connection lists too large");
-        out.ptr[c + 1] = static_cast<int>(total);
+        const int col = c1_indx[q];
+        if (col > last)
+          break;
+        if (member[col] < 0)
+          continue;
+        if (q == c1_diag[r])
+          out.diag[c] = static_cast<int>(found.size() - begin);
+        found.push_back(link{member[col], q});
       }
-      out.cell.resize(total);
-      out.q.resize(total);
+      if (found.size() > (size_t(1) << 31) - 1)
+        return set_error(AKM_ERR_UNSUPPORTED, "global kron: connection lists too large");
+      first[c] = static_cast<int>(begin);
+      out.ptr[c + 1] = static_cast<int>(found.size() - begin);
+    }
+    for (int64_t f = f0; f < f1; f++)
+      member[elem[int64_t(order[f]) * d + k]] = -1;
+    f0 = f1;
+  }
+  if (repeated >= 0)
+    return AKM_SUCCESS;
+  for (int64_t c = 0; c < cells; c++)
+    out.ptr[c + 1] += out.ptr[c];
+  out.cell.resize(found.size());
+  out.q.resize(found.size());
+  for (int64_t c = 0; c < cells; c++)
+  {
+    const int base = out.ptr[c];
+    if (out.diag[c] >= 0)
+      out.diag[c] += base;
+    for (int i = 0; i < out.ptr[c + 1] - base; i++)
+    {
+      out.cell[base + i] = found[first[c] + i].cell;
+      out.q[base + i] = found[first[c] + i].q;
     }
   }
   for (int64_t c = 0; c < cells; c++)
@@ -683,19 +686,25 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
   // connections out in pieces: piece(product, list, from, to, connections,
   // first of a slot) for every piece in order.
   const int S = plan.nslot;
+  struct output
+  {
+    int vec; // as fl_slot_rec
+    std::vector<product> prods;
+  };
   struct job
   {
-    int out, cell;
+    const output *out;
+    int cell;
     int slots, more; // slots; pieces beyond the slots' first ones
     int length;      // connections
     int64_t slot0, piece0;
   };
-  auto cut = [&](std::vector<int> const &prods, int c, auto &&piece) -> int64_t {
+  auto cut = [&](output const &out, int c, auto &&piece) -> int64_t {
     int64_t total = 0, whole = 0; // connections; slots with one piece each
-    for (int i : prods)
+    for (product const &p : out.prods)
     {
       int lo, hi;
-      fill_range(lists[prog.prods[i].k], c, prog.prods[i].fill, lo, hi);
+      fill_range(lists[p.k], c, p.fill, lo, hi);
       total += hi - lo;
       whole += (hi - lo + fl_piece - 1) / fl_piece;
     }
@@ -703,9 +712,8 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
     const bool split = whole <= S;
     const int64_t target = split ? fl_piece : (total + S - 1) / S;
     int64_t room = 0;
-    for (int i : prods)
+    for (product const &p : out.prods)
     {
-      product const &p = prog.prods[i];
       gk_lists const &l = lists[p.k];
       int lo, hi;
       fill_range(l, c, p.fill, lo, hi);
@@ -739,38 +747,45 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
   // which gives every record its place
   const int nstages = std::max(prog.stages, 1);
   std::vector<job> jobs; // in their order in the plan
-  std::vector<std::map<int, std::vector<int>>> outs(nstages); // output vector -> products
+  std::deque<output> outs;
   std::vector<size_t> stage_end(nstages);
   int64_t nslots = 0, npieces = 0;
   for (int st = 0; st < nstages; st++)
   {
-    for (size_t i = 0; i < prog.prods.size(); i++)
-      if (prog.prods[i].stage == st)
-        outs[st][prog.prods[i].out].push_back(static_cast<int>(i));
+    std::map<int, std::vector<product>> by_out;
+    for (product const &p : prog.prods)
+      if (p.stage == st)
+        by_out[p.out].push_back(p);
     if (st + 1 == nstages)
-      outs[st][-1]; // y is always written
+      by_out[-1]; // y is always written
     std::vector<job> made;
-    int most = 0, longest = 0;
-    for (auto &ov : outs[st])
+    for (auto &ov : by_out)
     {
       // products of one dimension together: a slot's rounds are few
       std::stable_sort(ov.second.begin(), ov.second.end(),
-                       [&](int u, int v) { return prog.prods[u].k < prog.prods[v].k; });
+                       [](product const &u, product const &v) { return u.k < v.k; });
       const int64_t ncell = (ov.first < 0) ? active_cells : cells;
+      outs.push_back({ov.first < 0 ? -1 : ov.first - 1, std::move(ov.second)});
+      output const &out = outs.back();
+      made.reserve(made.size() + ncell);
       for (int64_t c = 0; c < ncell; c++)
       {
-        job jb{ov.first, static_cast<int>(c), 0, 0, 0, 0, 0};
+        job jb{&out, static_cast<int>(c), 0, 0, 0, 0, 0};
         const int64_t total =
-            cut(ov.second, jb.cell,
+            cut(out, jb.cell,
                 [&](product const &, gk_lists const &, int, int, int, bool fresh) {
                   (fresh ? jb.slots : jb.more)++;
                 });
         jb.slots = std::max(jb.slots, 1);
         jb.length = static_cast<int>(std::min<int64_t>(total, 1 << 30));
-        most = std::max(most, jb.slots);
-        longest = std::max(longest, jb.length);
         made.push_back(jb);
       }
+    }
+    int most = 0, longest = 0;
+    for (job const &jb : made)
+    {
+      most = std::max(most, jb.slots);
+      longest = std::max(longest, jb.length);
     }
     int bits = 1; // of a length
     while (longest >> bits != 0)
@@ -817,7 +832,7 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
     for (int u = len; u < fl_piece; u++)
       r.entry[u] = rest;
   };
-  auto fill_job = [&](std::map<int, std::vector<int>> const &products, job const &jb) {
+  auto fill_job = [&](job const &jb) {
     fl_slot_rec *sr = slots.get() + jb.slot0 - 1;
     fl_piece_rec *more = pieces.get() + jb.piece0, *before = nullptr;
     int rank = 0;
@@ -825,12 +840,12 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
       sr++;
       sr->cell = jb.cell;
       sr->group = rank++ | jb.slots << 16;
-      sr->vec = jb.out < 0 ? -1 : jb.out - 1;
+      sr->vec = jb.out->vec;
       sr->more = sr->next = 0;
       sr->rounds = 1;
       sr->pad[0] = sr->pad[1] = 0;
     };
-    cut(products.at(jb.out), jb.cell,
+    cut(*jb.out, jb.cell,
         [&](product const &p, gk_lists const &l, int from, int to, int len, bool fresh) {
           if (fresh)
             open_slot();
@@ -876,7 +891,7 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
     {
       for (; done < jobs[at].slot0; done++)
         slots[done] = empty;
-      fill_job(outs[st], jobs[at]);
+      fill_job(jobs[at]);
       done = jobs[at].slot0 + jobs[at].slots;
     }
     const int64_t end = int64_t(plan.stages[st].first_group + plan.stages[st].groups) * S;
@@ -888,8 +903,9 @@ int build_fibre_plan(akm_matrix_s const &m, int64_t active_cells, int64_t cells,
     int rounds = 1;
     for (int i = 0; i < S; i++)
       rounds = std::max(rounds, slots[g + i].rounds);
-    for (int i = 0; i < S; i++)
-      slots[g + i].rounds = rounds;
+    if (rounds > 1)
+      for (int i = 0; i < S; i++)
+        slots[g + i].rounds = rounds;
   }
 
   std::vector<int> ptr(1, 0), src;

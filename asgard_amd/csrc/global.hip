@@ -2115,7 +2115,9 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     term_group[t] = static_cast<int>(gi);
   }
 
-  std::vector<int> bundles, groups, passes, tabs, items, cells, lists_img, offs, slots, recs;
+  std::vector<gs_bundle> bundles;
+  std::vector<gs_group> groups;
+  std::vector<int> passes, tabs, items, cells, lists_img, offs, slots, recs;
   struct item_rec
   {
     int bundle, h, tpb, nd;
@@ -2128,11 +2130,19 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     gs_lane_range lanes[2]; // its passes' lanes
   };
   std::vector<item_rec> irec;
+  // a group's plan, its positions counted from its own first ones
+  struct group_plan
+  {
+    bool kept = false;
+    gs_group rec{};
+    std::vector<gs_bundle> bundles;
+    std::vector<int> cells, lists, slots, recs, offs, tabs, passes;
+    std::vector<item_rec> items;
+  };
+  std::vector<group_plan> plans(gdims.size());
   std::vector<int> loc(g.cells, -1);
-  std::vector<int> gslot(gdims.size(), -1);
-  int ngroups = 0;
-  for (size_t gi = 0; gi < gdims.size(); gi++)
-    for (int attempt = 0; attempt < 2; attempt++)
+  auto plan_group = [&](size_t gi, group_plan &gp) {
+    for (int attempt = 0; attempt < 2 && !gp.kept; attempt++)
   {
     // small bundles of gs_blocks_small_first blocks, else (second attempt,
     // when those do not fit) of gs_blocks_small; a failed attempt commits
@@ -2309,26 +2319,30 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
           len = std::max(len, lists[k].ptr[gc + 1] - lists[k].ptr[gc]);
         return len;
       };
-      std::stable_sort(pb.cells.begin(), pb.cells.end(),
-                       [&](int u, int v) { return longest(u) > longest(v); });
+      std::vector<std::pair<int, int>> by_length; // (-length, cell)
+      by_length.reserve(pb.cells.size());
+      for (int c : pb.cells)
+        by_length.emplace_back(-longest(c), c);
+      std::stable_sort(by_length.begin(), by_length.end(),
+                       [](auto const &u, auto const &v) { return u.first < v.first; });
+      for (size_t c = 0; c < pb.cells.size(); c++)
+        pb.cells[c] = by_length[c].second;
     }
 
     // lists, LDS sizes and items of the plan (checked before anything is kept)
-    const int group_index = ngroups;
-    std::vector<int> b_rec, p_cells, p_lists, p_slots, p_recs;
+    std::vector<gs_bundle> b_rec;
+    std::vector<int> p_cells, p_lists, p_slots, p_recs;
     std::vector<item_rec> p_items;
-    const int bundle_base = static_cast<int>(bundles.size() / (sizeof(gs_bundle) / sizeof(int)));
     for (size_t bi = 0; bi < plan.size() && ok; bi++)
     {
       gs_plan_bundle const &pb = plan[bi];
       const int ncell = static_cast<int>(pb.cells.size());
       gs_bundle rec{};
-      rec.group = group_index;
-      rec.cell0 = static_cast<int>(cells.size() + p_cells.size());
+      rec.cell0 = static_cast<int>(p_cells.size());
       rec.ncell = ncell;
       rec.C = pb.C;
       rec.Lp = pb.Lp;
-      rec.list0 = static_cast<int>(lists_img.size() + p_lists.size());
+      rec.list0 = static_cast<int>(p_lists.size());
       for (int c = 0; c < ncell; c++)
         loc[pb.cells[c]] = c;
       // element offset of the connected cell in x / the intermediate,
@@ -2352,8 +2366,8 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
           continue;
         gk_lists const &ls = lists[S[gpass[pi].j]];
         const size_t s0 = p_slots.size();
-        where.slot0 = static_cast<int>(slots.size() + s0);
-        where.rec0 = static_cast<int>(recs.size() + p_recs.size());
+        where.slot0 = static_cast<int>(s0);
+        where.rec0 = static_cast<int>(p_recs.size());
         ok = gs_lanes(pb.cells, ls, gpass[pi].fill, pb.C,
                       [&](int64_t p, unsigned &e) { return entry(ls, p, e); }, p_slots, p_recs);
         where.nslot = static_cast<int>(p_slots.size() - s0);
@@ -2407,20 +2421,18 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
         ok = false;
         break;
       }
-      const int *rp = reinterpret_cast<const int *>(&rec);
-      b_rec.insert(b_rec.end(), rp, rp + sizeof(gs_bundle) / sizeof(int));
+      b_rec.push_back(rec);
       p_cells.insert(p_cells.end(), pb.cells.begin(), pb.cells.end());
       for (int h = 0; h < call / pb.C; h++)
       {
         if (!split)
         {
-          p_items.push_back({bundle_base + static_cast<int>(bi), h, pb.tpb, nd, lds,
-                             rec.resident});
+          p_items.push_back({static_cast<int>(bi), h, pb.tpb, nd, lds, rec.resident});
           continue;
         }
         for (size_t k = 0; k < gchains.size(); k++)
         {
-          item_rec r{bundle_base + static_cast<int>(bi), h, pb.tpb, nd, lds, 0};
+          item_rec r{static_cast<int>(bi), h, pb.tpb, nd, lds, 0};
           r.chain = static_cast<int>(k);
           r.Lp = pb.Lp;
           r.pass_off = gchains[k].first;
@@ -2438,7 +2450,7 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     if (!ok)
       continue;
     // the group is kept
-    gs_group grec{};
+    gs_group &grec = gp.rec;
     grec.nd = nd;
     for (int j = 0; j < nd; j++)
     {
@@ -2449,7 +2461,6 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
       grec.str[j] = str;
     }
     grec.call = call;
-    grec.off0 = static_cast<int>(offs.size());
     for (int o = 0; o < call; o++)
     {
       // digits of o over the other dimensions, the last one fastest
@@ -2463,14 +2474,12 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
         }
         str *= n;
       }
-      offs.push_back(off);
+      gp.offs.push_back(off);
     }
-    grec.tab0 = static_cast<int>(tabs.size() / 2);
     grec.ntab = ntab;
     for (int t : gterms)
       for (int j = 0; j < nd; j++)
-        tabs.insert(tabs.end(), {t, S[j]});
-    grec.pass0 = static_cast<int>(passes.size() / 4);
+        gp.tabs.insert(gp.tabs.end(), {t, S[j]});
     for (size_t c = 0; c < own.size(); c++)
     {
       if (c + 1 < own.size() && merged(own[c], own[c + 1]))
@@ -2478,28 +2487,71 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
         // F then L and U then F: U, both F at once, L
         gs_pass f = pass_of(own[c], 0);
         f.mode = 3;
-        add_pass(passes, pass_of(own[c + 1], 0));
-        add_pass(passes, f);
-        add_pass(passes, pass_of(own[c], 1));
+        add_pass(gp.passes, pass_of(own[c + 1], 0));
+        add_pass(gp.passes, f);
+        add_pass(gp.passes, pass_of(own[c], 1));
         c++;
         continue;
       }
       for (int st = 0; st < ch_nst[own[c]]; st++)
-        add_pass(passes, pass_of(own[c], st));
+        add_pass(gp.passes, pass_of(own[c], st));
     }
-    grec.npass = static_cast<int>(passes.size() / 4) - grec.pass0;
-    grec.slot = 2 * g.nslots + group_index;
-    const int *gp = reinterpret_cast<const int *>(&grec);
-    groups.insert(groups.end(), gp, gp + sizeof(gs_group) / sizeof(int));
-    bundles.insert(bundles.end(), b_rec.begin(), b_rec.end());
-    cells.insert(cells.end(), p_cells.begin(), p_cells.end());
-    lists_img.insert(lists_img.end(), p_lists.begin(), p_lists.end());
-    slots.insert(slots.end(), p_slots.begin(), p_slots.end());
-    recs.insert(recs.end(), p_recs.begin(), p_recs.end());
-    irec.insert(irec.end(), p_items.begin(), p_items.end());
-    gslot[gi] = group_index;
-    ngroups++;
-    break;
+    grec.npass = static_cast<int>(gp.passes.size() / 4);
+    gp.bundles = std::move(b_rec);
+    gp.cells = std::move(p_cells);
+    gp.lists = std::move(p_lists);
+    gp.slots = std::move(p_slots);
+    gp.recs = std::move(p_recs);
+    gp.items = std::move(p_items);
+    gp.kept = true;
+  }
+  };
+  for (size_t gi = 0; gi < gdims.size(); gi++)
+    plan_group(gi, plans[gi]);
+  // the kept groups one after another
+  std::vector<int> gslot(gdims.size(), -1);
+  int ngroups = 0;
+  auto append = [](auto &to, auto const &from) { to.insert(to.end(), from.begin(), from.end()); };
+  for (size_t gi = 0; gi < gdims.size(); gi++)
+  {
+    group_plan &gp = plans[gi];
+    if (!gp.kept)
+      continue;
+    gp.rec.off0 = static_cast<int>(offs.size());
+    gp.rec.tab0 = static_cast<int>(tabs.size() / 2);
+    gp.rec.pass0 = static_cast<int>(passes.size() / 4);
+    gp.rec.slot = 2 * g.nslots + ngroups;
+    const int bundle0 = static_cast<int>(bundles.size()), cell0 = static_cast<int>(cells.size()),
+              list0 = static_cast<int>(lists_img.size()), slot0 = static_cast<int>(slots.size()),
+              rec0 = static_cast<int>(recs.size());
+    for (auto &b : gp.bundles)
+    {
+      b.group = ngroups;
+      b.cell0 += cell0;
+      b.list0 += list0;
+    }
+    for (auto &r : gp.items)
+    {
+      r.bundle += bundle0;
+      for (auto &l : r.lanes)
+        if (l.slot0 >= 0)
+        {
+          l.slot0 += slot0;
+          l.rec0 += rec0;
+        }
+    }
+    groups.push_back(gp.rec);
+    append(bundles, gp.bundles);
+    append(cells, gp.cells);
+    append(lists_img, gp.lists);
+    append(slots, gp.slots);
+    append(recs, gp.recs);
+    append(offs, gp.offs);
+    append(tabs, gp.tabs);
+    append(passes, gp.passes);
+    append(irec, gp.items);
+    gslot[gi] = ngroups++;
+    gp = group_plan();
   }
   for (int t = 0; t < T; t++)
     if (term_group[t] >= 0 && gslot[term_group[t]] < 0)
@@ -2522,14 +2574,22 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
   };
   // within a launch the largest items first (the longest-running workgroups
   // start early)
-  std::stable_sort(irec.begin(), irec.end(), [&](item_rec const &u, item_rec const &v) {
-    return cls(u) != cls(v) ? cls(u) < cls(v) : u.lds > v.lds;
-  });
+  std::vector<uint64_t> keys; // class, then LDS bytes (below 2^20) falling
+  for (auto const &r : irec)
+    keys.push_back(static_cast<uint64_t>(cls(r)) << 20 |
+                   static_cast<uint64_t>((1 << 20) - 1 - r.lds));
+  std::vector<int> item_order;
+  radix_order(keys, 26, item_order);
+  std::vector<item_rec> sorted;
+  sorted.reserve(irec.size());
+  for (int i : item_order)
+    sorted.push_back(irec[i]);
+  irec.swap(sorted);
   g.gs_launches.clear();
   g.gs_item_lds.clear();
   g.gs_side_items = 0;
   // partials of split bundles: per bundle ncell * chains of N values
-  const size_t nbundles = bundles.size() / (sizeof(gs_bundle) / sizeof(int));
+  const size_t nbundles = bundles.size();
   std::vector<int64_t> part0(nbundles, -1);
   std::vector<int> nch_of(nbundles, 0);
   int64_t nparts = 0;
@@ -2540,7 +2600,7 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     if (nch_of[bi] > 0)
     {
       part0[bi] = nparts;
-      nparts += int64_t(reinterpret_cast<const gs_bundle *>(bundles.data())[bi].ncell) *
+      nparts += int64_t(bundles[bi].ncell) *
                 nch_of[bi];
     }
   if (nparts > (int64_t(1) << 31) - 1)
@@ -2552,8 +2612,8 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     cbase[Lp + 1] = cbase[Lp] + ntab_all * gs_table_values(qm0[Lp + 1] - qm0[Lp], nn);
   if (cbase[L + 1] > (int64_t(1) << 31) - 1)
     return set_error(AKM_ERR_UNSUPPORTED, "global kron: slab factor tables too large");
-  const gs_bundle *hb = reinterpret_cast<const gs_bundle *>(bundles.data());
-  const gs_group *hg = reinterpret_cast<const gs_group *>(groups.data());
+  const gs_bundle *hb = bundles.data();
+  const gs_group *hg = groups.data();
   for (size_t i = 0; i < irec.size(); i++)
   {
     const gs_bundle &bb = hb[irec[i].bundle];

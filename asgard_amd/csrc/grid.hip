@@ -266,33 +266,40 @@ void lexicographic_order(int d, int64_t num_cells, const int *elem, std::vector<
 
 void radix_order(std::vector<uint64_t> const &keys, int bits, std::vector<int> &order)
 {
-  struct item
-  {
-    uint64_t key;
-    int index;
-  };
   const size_t count = keys.size();
-  const int passes = std::max(1, (bits + 7) / 8);
-  std::vector<item> a(count), b(count);
-  std::vector<size_t> start(size_t(passes) * 256, 0);
+  int low = 0; // bits of an index
+  while (count >> low != 0)
+    low++;
+  order.resize(count);
+  if (bits + low > 64 || count < 64)
+  {
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return keys[a] < keys[b]; });
+    return;
+  }
+  // key and index in one word, sorted by the key's digits
+  const int digit = (count < 4096) ? 8 : 11, size = 1 << digit;
+  const int passes = std::max(1, (bits + digit - 1) / digit);
+  std::vector<uint64_t> a(count), b(count);
+  std::vector<unsigned> start(size_t(passes) * size, 0);
   for (size_t i = 0; i < count; i++)
   {
-    a[i] = item{keys[i], static_cast<int>(i)};
+    a[i] = keys[i] << low | i;
     for (int p = 0; p < passes; p++)
-      start[p * 256 + (keys[i] >> (8 * p) & 255)]++;
+      start[p * size + (keys[i] >> (digit * p) & (size - 1))]++;
   }
   for (int p = 0; p < passes; p++)
   {
-    size_t *s = start.data() + p * 256, sum = 0;
-    for (int v = 0; v < 256; v++)
+    unsigned *s = start.data() + p * size, sum = 0;
+    for (int v = 0; v < size; v++)
       sum += std::exchange(s[v], sum);
-    for (item const &it : a)
-      b[s[it.key >> (8 * p) & 255]++] = it;
+    const int shift = low + digit * p;
+    for (uint64_t w : a)
+      b[s[w >> shift & (size - 1)]++] = w;
     a.swap(b);
   }
-  order.resize(count);
   for (size_t i = 0; i < count; i++)
-    order[i] = a[i].index;
+    order[i] = static_cast<int>(a[i] & ((uint64_t(1) << low) - 1));
 }
 
 void order_by_dims(int d, int64_t cells, const int *elem, std::vector<int> const &dims, int M,
