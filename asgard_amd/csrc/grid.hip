@@ -374,32 +374,38 @@ int device_sparse_pattern(int d, int64_t num_cells, const int *table_host,
 int device_sparse_pattern(int d, std::vector<uint64_t> const &pack, int max_level,
                           std::vector<int> const &c1_pntr, std::vector<int> const &c1_indx,
                           std::vector<int> const &order_host, std::vector<int64_t> &pntr,
-                          dev_buffer<int> &indx_dev)
+                          dev_buffer<int64_t> &pntr_dev, dev_buffer<int> &indx_dev)
 {
   const int64_t cells = static_cast<int64_t>(pack.size());
   const int M = 1 << max_level, words = (M + 31) / 32;
-  std::vector<unsigned> bits(size_t(M) * words, 0u);
+  // one upload: the cells' words by row and in column order, the column ids,
+  // the connection bits
+  const int64_t nbits = int64_t(M) * words;
+  std::vector<uint64_t> in(2 * cells + (cells + 1) / 2 + (nbits + 1) / 2, 0);
+  int *order = reinterpret_cast<int *>(in.data() + 2 * cells);
+  unsigned *bits = reinterpret_cast<unsigned *>(in.data() + 2 * cells + (cells + 1) / 2);
+  for (int64_t i = 0; i < cells; i++)
+  {
+    in[i] = pack[i];
+    in[cells + i] = pack[order_host[i]];
+    order[i] = order_host[i];
+  }
   for (int r = 0; r < M; r++)
     for (int j = c1_pntr[r]; j < c1_pntr[r + 1]; j++)
       bits[size_t(r) * words + c1_indx[j] / 32] |= 1u << (c1_indx[j] % 32);
-  std::vector<uint64_t> cols(cells);
-  for (int64_t i = 0; i < cells; i++)
-    cols[i] = pack[order_host[i]];
-  dev_buffer<uint64_t> pack_dev, cols_dev;
-  dev_buffer<int> order_dev;
-  dev_buffer<unsigned> bits_dev;
-  dev_buffer<int64_t> counts, pntr_dev;
-  AKM_TRY(pack_dev.upload(pack.data(), cells));
-  AKM_TRY(cols_dev.upload(cols.data(), cells));
-  AKM_TRY(order_dev.upload(order_host.data(), cells));
-  AKM_TRY(bits_dev.upload(bits.data(), int64_t(bits.size())));
+  dev_buffer<uint64_t> in_dev;
+  dev_buffer<int64_t> counts;
+  AKM_TRY(in_dev.upload(in.data(), int64_t(in.size())));
   AKM_TRY(counts.allocate(cells));
+  const uint64_t *rows_at = in_dev.data(), *cols_at = rows_at + cells;
+  const int *order_at = reinterpret_cast<const int *>(cols_at + cells);
+  const unsigned *bits_at = reinterpret_cast<const unsigned *>(cols_at + cells + (cells + 1) / 2);
   auto scan = [&](const int64_t *starts, int *indx) -> int {
     const unsigned blocks = static_cast<unsigned>((cells + 3) / 4);
     const size_t lds = sizeof(unsigned) * 4 * d * words;
     auto go = [&](auto kern) {
-      kern<<<blocks, 256, lds>>>(cells, pack_dev.data(), cols_dev.data(), order_dev.data(),
-                                 bits_dev.data(), words, counts.data(), starts, indx);
+      kern<<<blocks, 256, lds>>>(cells, rows_at, cols_at, order_at, bits_at, words,
+                                 counts.data(), starts, indx);
       return check_launch("sparse pattern scan");
     };
     switch (d)

@@ -36,11 +36,12 @@ int device_sparse_pattern(int d, int64_t num_cells, const int *table_host,
 
 //! The same for valid cells below level 11, given by their packed 1D indices
 //! (10 bits a dimension) and connect_1d(max_level); each row's columns in the
-//! order of order_host, a permutation of the cells.
+//! order of order_host, a permutation of the cells.  The row starts stay on
+//! the device, too.
 int device_sparse_pattern(int d, std::vector<uint64_t> const &pack, int max_level,
                           std::vector<int> const &c1_pntr, std::vector<int> const &c1_indx,
                           std::vector<int> const &order_host, std::vector<int64_t> &pntr,
-                          dev_buffer<int> &indx_dev);
+                          dev_buffer<int64_t> &pntr_dev, dev_buffer<int> &indx_dev);
 
 //! The cells 0 .. cells-1 ordered by their 1D indices in `dims` (the first
 //! the most significant), ties by cell id; 1D indices are below M.

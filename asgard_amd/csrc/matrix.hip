@@ -75,7 +75,8 @@ static int build_schedule(akm_matrix_s &m)
     for (int r = 0; r < m.rows; r++)
       keys[r] = static_cast<uint64_t>(longest - (m.pntr[r + 1] - m.pntr[r]));
     radix_order(keys, bits, order);
-    AKM_TRY(m.pntr_dev.upload(m.pntr.data(), int64_t(m.pntr.size()), m.stream));
+    if (m.pntr_dev.size() == 0)
+      AKM_TRY(m.pntr_dev.upload(m.pntr.data(), int64_t(m.pntr.size()), m.stream));
   }
   AKM_TRY(m.row_order.upload(order.data(), int64_t(order.size()), m.stream));
   return AKM_SUCCESS;
@@ -410,7 +411,8 @@ akm_status akm_create_sparse_grid(int d, int n, int64_t num_cells, const int *ta
     for (int64_t c = 0; c < num_cells; c++)
       for (int k = 0; k < d; k++)
         pack[c] |= static_cast<uint64_t>(elem[c * d + k]) << (10 * k);
-    AKM_TRY(device_sparse_pattern(d, pack, max_level, p1, i1, lex, m->pntr, m->indx));
+    AKM_TRY(device_sparse_pattern(d, pack, max_level, p1, i1, lex, m->pntr, m->pntr_dev,
+                                  m->indx));
   }
   else
     AKM_TRY(device_sparse_pattern(d, num_cells, table, m->pntr, m->indx, lex.data()));

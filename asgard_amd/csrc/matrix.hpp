@@ -61,11 +61,9 @@ struct akm_matrix_s
   akm::dev_buffer<unsigned char> xws, yws;
 
   // operator update on the device: connect_1d (rows, then columns) in vA
-  // order, and the device copy of the caller's operator pointers
+  // order and the scan's findings, and the device copy of the caller's operator pointers
   akm::dev_buffer<int> op_conn;
-  // the last scan of the stored factors: its number, and its findings
-  int op_scan = 0;
-  akm::dev_buffer<int> op_flags;
+  int op_scan = 0; // number of the last scan of the stored factors
   akm::dev_buffer<const void *> op_ptrs;
   // IMEX step vectors (four of output_size), on the implicit handle
   akm::dev_buffer<double> imex_ws;

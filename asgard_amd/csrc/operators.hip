@@ -126,7 +126,7 @@ static int update_operators_typed(akm_matrix_s &m, const void *const *ops_dev, i
     }
     return AKM_SUCCESS;
   }
-  const int64_t nconn = m.op_conn.size() / 2;
+  const int64_t nconn = (m.op_conn.size() - T * d - 1) / 2;
   P *vA = reinterpret_cast<P *>(m.vA.data());
   gather_grid_blocks<P><<<op_blocks(m.num_vA), op_threads, 0, m.stream>>>(
       ops, lda, m.op_conn.data(), m.op_conn.data() + nconn, nconn, T, d, n, vA);
@@ -141,7 +141,8 @@ static int update_operators_typed(akm_matrix_s &m, const void *const *ops_dev, i
   return AKM_SUCCESS;
 }
 
-//! connect_1d on the device as (row, column) per connection, in vA order.
+//! connect_1d on the device as (row, column) per connection, in vA order, and
+//! after it the flags of scan_factors.
 static int need_connections(akm_matrix_s &m)
 {
   if (m.op_conn.size() > 0)
@@ -152,14 +153,15 @@ static int need_connections(akm_matrix_s &m)
   const int64_t nconn = static_cast<int64_t>(i1.size());
   if (nconn * m.T * m.d * m.n * m.n != m.num_vA)
     return set_error(AKM_ERR_INVALID, "operator update: stored blocks do not match connect_1d");
-  std::vector<int> rc(2 * nconn);
+  std::vector<int> rc(2 * nconn + m.T * m.d + 1, 0);
   for (int r = 0; r + 1 < static_cast<int>(p1.size()); r++)
     for (int j = p1[r]; j < p1[r + 1]; j++)
     {
       rc[j] = r;
       rc[nconn + j] = i1[j];
     }
-  return m.op_conn.upload(rc.data(), 2 * nconn, m.stream);
+  m.op_scan = 0;
+  return m.op_conn.upload(rc.data(), int64_t(rc.size()), m.stream);
 }
 
 //! flags[t*d + k] = scan for a factor that is not exactly the identity (0 off
@@ -197,12 +199,12 @@ __global__ void __launch_bounds__(op_threads)
 int stored_factors(akm_matrix_s &m, std::vector<int> &mask, bool &finite)
 {
   AKM_TRY(need_connections(m));
-  const int64_t nconn = m.op_conn.size() / 2;
   const int pairs = m.T * m.d;
-  if (m.op_flags.size() == 0 || m.op_scan == std::numeric_limits<int>::max())
+  const int64_t nconn = (m.op_conn.size() - pairs - 1) / 2;
+  int *flags = m.op_conn.data() + 2 * nconn;
+  if (m.op_scan == std::numeric_limits<int>::max())
   {
-    const std::vector<int> none(pairs + 1, 0);
-    AKM_TRY(m.op_flags.upload(none.data(), pairs + 1, m.stream));
+    AKM_HIP(hipMemsetAsync(flags, 0, sizeof(int) * (pairs + 1), m.stream));
     m.op_scan = 0;
   }
   const int scan = ++m.op_scan;
@@ -212,16 +214,14 @@ int stored_factors(akm_matrix_s &m, std::vector<int> &mask, bool &finite)
   const int *row = m.op_conn.data(), *col = row + nconn;
   if (m.prec == AKM_F64)
     scan_factors<double><<<grid, op_threads, 0, m.stream>>>(
-        reinterpret_cast<const double *>(m.vA.data()), row, col, nconn, pairs, m.n, scan,
-        m.op_flags.data());
+        reinterpret_cast<const double *>(m.vA.data()), row, col, nconn, pairs, m.n, scan, flags);
   else
     scan_factors<float><<<grid, op_threads, 0, m.stream>>>(
-        reinterpret_cast<const float *>(m.vA.data()), row, col, nconn, pairs, m.n, scan,
-        m.op_flags.data());
+        reinterpret_cast<const float *>(m.vA.data()), row, col, nconn, pairs, m.n, scan, flags);
   AKM_TRY(check_launch("factor scan"));
   mask.resize(pairs + 1);
-  AKM_HIP(hipMemcpyAsync(mask.data(), m.op_flags.data(), sizeof(int) * (pairs + 1),
-                         hipMemcpyDeviceToHost, m.stream));
+  AKM_HIP(hipMemcpyAsync(mask.data(), flags, sizeof(int) * (pairs + 1), hipMemcpyDeviceToHost,
+                         m.stream));
   AKM_HIP(hipStreamSynchronize(m.stream));
   for (int &f : mask)
     f = (f == scan) ? 1 : 0;
