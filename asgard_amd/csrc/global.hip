@@ -528,7 +528,7 @@ struct gs_item
   int nd;           // slab dimensions (1 or 2)
   int str[2];       // their strides in the cell tensor
   int off;          // first of the chunk's C entries in gs_args::offs
-  int tab0, ntab;   // the group's factor tables in gs_args::tabs
+  int ntab;         // the group's factor tables
   int pass0, npass; // the group's passes in gs_args::passes
   int slot;         // work-buffer slot of the group's sum
   // a split item (one chain of a large slab): its chain of the bundle's nch
@@ -2632,7 +2632,6 @@ static int build_slabs(akm_matrix_s &m, akm_global_s &g)
     it.str[0] = gg.str[0];
     it.str[1] = gg.str[1];
     it.off = gg.off0 + irec[i].h * bb.C;
-    it.tab0 = gg.tab0;
     it.ntab = gg.ntab;
     const bool split = irec[i].chain >= 0;
     it.pass0 = gg.pass0;

@@ -701,7 +701,7 @@ struct akm_mlp_s final : akm_precond_s
   {
     if (B <= batch)
       return AKM_SUCCESS;
-    batch = B;
+    batch = 0; // nothing to rely on until everything is there
     AKM_TRY(Xb.allocate(int64_t(B) * K1));
     AKM_TRY(Tb.allocate(int64_t(B) * N3));
     AKM_TRY(H1.allocate(int64_t(B) * H));
@@ -715,6 +715,7 @@ struct akm_mlp_s final : akm_precond_s
       AKM_HIP(hipHostMalloc(reinterpret_cast<void **>(&host_loss), sizeof(double),
                             hipHostMallocDefault));
     AKM_TRY(parts.allocate(row_parts(B) * num_params));
+    batch = B;
     return AKM_SUCCESS;
   }
 
