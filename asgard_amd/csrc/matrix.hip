@@ -135,9 +135,10 @@ int64_t akm_matrix_s::flops() const
 namespace akm
 {
 
+//! Pair by pair, with the handle's shape of the kernels or a given one.
 template<typename P>
 static int apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y, P gamma,
-                       const P *xg)
+                       const P *xg, int waves, int family)
 {
   if (m.T == 0 || alpha == P{0} || m.rows == 0)
     return launch_scale<P>(m.output_size(), beta, y, gamma, xg, m.stream);
@@ -148,8 +149,8 @@ static int apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y, P gam
   a.alpha = alpha;
   a.beta = beta;
   a.gamma = gamma;
-  return launch_kronmult<P>(m.d, m.n, m.mode, a, m.rows, waves_per_row(m), m.force_generic,
-                            m.stream);
+  a.family = family;
+  return launch_kronmult<P>(m.d, m.n, m.mode, a, m.rows, waves, m.force_generic, m.stream);
 }
 
 void use_stream(akm_matrix_s &m, hipStream_t stream)
@@ -191,21 +192,37 @@ int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void
     return set_error(AKM_ERR_INVALID, "identity term needs a square operator");
   if (m.mode == mode_global)
     return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
-  // A captured apply is replayed whenever its owner likes, beside other applies
-  // and after new factors of another form: it takes the pair kernels, which
-  // read nothing but x and the stored factors, at addresses that stay.
-  if (m.factored && !m.pair_kernels && !m.pair_tuned && !capturing(m.stream))
+  int waves = waves_per_row(m), family = m.family;
+  if (m.factored && !m.pair_kernels && !m.pair_tuned)
   {
-    std::lock_guard<std::mutex> lock(m.factored_mtx);
-    return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
+    if (!capturing(m.stream))
+    {
+      std::lock_guard<std::mutex> lock(m.factored_mtx);
+      return global_apply(m, alpha, x, beta, y, gamma, xg, false, 0.0);
+    }
+    // A captured apply is replayed whenever its owner likes, beside other
+    // applies and after new factors of another form: it takes the pair
+    // kernels, which read nothing but x and the stored factors, at addresses
+    // that stay.  No shape of theirs has been timed on this handle; four
+    // wavefronts a row, and at d = 6 n = 2 in FP64 the matrix cores with 16,
+    // are at or near the best everywhere (Vlasov levels 3 / 5 / 7 13 / 452 /
+    // 31,200 us, four wavefronts 24 / 576 / 56,800, the default shape 22 /
+    // 707 / 223,700; d = 4 n = 2 levels 4 / 7 7.2 / 401, matrix cores 13 /
+    // 1,014).
+    family = (m.prec == AKM_F64 && m.d == 6 &&
+              mfma_family_applies(m.d, m.n, m.mode, m.T, m.epack.data() != nullptr))
+                 ? 1
+                 : 0;
+    waves = (family == 1) ? 16 : 4;
   }
   if (m.prec == AKM_F64)
     return apply_typed<double>(m, alpha, static_cast<const double *>(x), beta,
                                static_cast<double *>(y), gamma,
-                               static_cast<const double *>(xg));
+                               static_cast<const double *>(xg), waves, family);
   return apply_typed<float>(m, static_cast<float>(alpha), static_cast<const float *>(x),
                             static_cast<float>(beta), static_cast<float *>(y),
-                            static_cast<float>(gamma), static_cast<const float *>(xg));
+                            static_cast<float>(gamma), static_cast<const float *>(xg), waves,
+                            family);
 }
 
 //! The caller's choice between the pair kernels and the automatic one, which
