@@ -1044,12 +1044,13 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     ++stats.applies_f64;
     return apply_device(m64, -dt, v, 0.0, w, 1.0, v);
   };
-  double beta = 0; // |r| of the current cycle
+  double bnorm = 0, beta = 0; // |b|, and |r| of the current cycle
   std::function<int(const double *, double *)> op32 = [&](const double *v, double *w) -> int {
     ++stats.applies_f32;
-    // V_0 is the residual itself, at the scale of b; the other vectors of the
-    // cycle have the norms of their steps
-    const double scale = (cyc.lazy && v == V) ? f32_scale(beta) : 1.0;
+    // V_0 is the residual itself, at the scale of b, as the guess is taken to
+    // be; the other vectors of a cycle have the norms of their steps
+    const double scale = (v == x) ? f32_scale(bnorm)
+                                  : ((cyc.lazy && v == V) ? f32_scale(beta) : 1.0);
     if (scale == 1.0 && apply_f32_between(*m32, v, -dt, w))
       return check_launch("gmres fp32 apply");
     gm_to_f32<<<sblocks, gm_threads, 0, s>>>(n, v, scale, ws.v32.data());
@@ -1071,7 +1072,6 @@ static int gmres_mixed(akm_matrix_s &m64, akm_matrix_s *m32, akm_precond_s *pre,
     return cyc.start(norm);
   };
 
-  double bnorm = 0;
   AKM_TRY(cyc.norm(b, bnorm));
   stats.rhs_norm = bnorm;
   if (bnorm == 0.0)
