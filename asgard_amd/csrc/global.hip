@@ -1796,6 +1796,12 @@ int global_layout(akm_matrix_s const &m)
 
 int global_stages(akm_matrix_s const &m) { return m.gk ? m.gk->max_stages : 0; }
 
+bool global_shares_work(akm_matrix_s const &m)
+{
+  // (a global handle's apply in place runs in the chain layout)
+  return m.gk && (!m.gk->pair || m.gk->slab || m.gk->fl.vectors > 0);
+}
+
 int global_set_layout(akm_matrix_s &m, int layout)
 {
   if (!m.gk)

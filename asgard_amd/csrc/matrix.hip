@@ -153,26 +153,6 @@ static int apply_typed(akm_matrix_s &m, P alpha, const P *x, P beta, P *y, P gam
   return launch_kronmult<P>(m.d, m.n, m.mode, a, m.rows, waves, m.force_generic, m.stream);
 }
 
-void use_stream(akm_matrix_s &m, hipStream_t stream)
-{
-  const hipStream_t old = m.stream;
-  m.stream = stream;
-  if (old == stream || !m.gk)
-    return;
-  hipStreamCaptureStatus a = hipStreamCaptureStatusNone, b = hipStreamCaptureStatusNone;
-  hipEvent_t e = nullptr;
-  if (hipStreamIsCapturing(old, &a) == hipSuccess &&
-      hipStreamIsCapturing(stream, &b) == hipSuccess && a == hipStreamCaptureStatusNone &&
-      b == hipStreamCaptureStatusNone &&
-      hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess)
-  {
-    if (hipEventRecord(e, old) == hipSuccess)
-      (void)hipStreamWaitEvent(stream, e, 0);
-    (void)hipEventDestroy(e);
-  }
-  (void)hipGetLastError(); // a destroyed old stream has no work left
-}
-
 //! True while work enqueued on the stream is recorded into a graph (the null
 //! stream cannot be captured).
 static bool capturing(hipStream_t stream)
@@ -183,6 +163,22 @@ static bool capturing(hipStream_t stream)
   if (hipStreamIsCapturing(stream, &status) != hipSuccess)
     (void)hipGetLastError();
   return status != hipStreamCaptureStatusNone;
+}
+
+void use_stream(akm_matrix_s &m, hipStream_t stream)
+{
+  const hipStream_t old = m.stream;
+  m.stream = stream;
+  if (old == stream || !global_shares_work(m) || capturing(stream) || capturing(old))
+    return;
+  hipEvent_t e = nullptr;
+  if (hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess)
+  {
+    if (hipEventRecord(e, old) == hipSuccess)
+      (void)hipStreamWaitEvent(stream, e, 0);
+    (void)hipEventDestroy(e);
+  }
+  (void)hipGetLastError(); // a destroyed old stream has no work left
 }
 
 int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void *y,

@@ -99,9 +99,9 @@ namespace akm
 int apply_device(akm_matrix_s &m, double alpha, const void *x, double beta, void *y,
                  double gamma, const void *xg);
 
-//! Moves the handle to `stream`.  Work of a one-dimension-at-a-time operator
-//! still running on the old stream uses the handle's work vectors, so the new
-//! stream waits for it (unless either is being captured).
+//! Moves the handle to `stream`.  Where applies share work vectors of the
+//! handle, the new stream waits for what still runs on the old one (unless
+//! either is being captured).
 void use_stream(akm_matrix_s &m, hipStream_t stream);
 
 //! Wavefronts per row workgroup used for the matrix (explicit or automatic).
@@ -150,6 +150,9 @@ int64_t global_flops(akm_matrix_s const &m);
 int global_layout(akm_matrix_s const &m);
 //! Dependent products of its longest chain.
 int global_stages(akm_matrix_s const &m);
+//! True when its applies write work vectors of the handle, so that two of them
+//! must not run at once.
+bool global_shares_work(akm_matrix_s const &m);
 //! Global operator: times the layouts on the operator and keeps the fastest;
 //! best_ms = its time per apply.
 int global_autotune(akm_matrix_s &m, const void *x, void *y, double &best_ms);

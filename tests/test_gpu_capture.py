@@ -29,14 +29,19 @@ def factors(rng, d, n, level, active):
             for dims in active for k in range(d)]
 
 
-def capture(m, x, y):
-    """A graph of y = A x; the handle is on the null stream again after it."""
+def capture(m, x, y, inside=False):
+    """A graph of y = A x; the handle is on the null stream again after it.
+    `inside`: it moves to the captured stream and back while that is captured."""
     s = torch.cuda.Stream()
     torch.cuda.synchronize()
-    m.set_stream(s.cuda_stream)
+    if not inside:
+        m.set_stream(s.cuda_stream)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=s):
+        m.set_stream(s.cuda_stream)
         m.apply(1.0, x, 0.0, y)
+        if inside:
+            m.set_stream(0)
     m.set_stream(0)
     return graph
 
@@ -112,7 +117,7 @@ def test_replays_beside_applies_on_other_streams():
     for x, want in zip(xs, wants):
         m.apply(1.0, x, 0.0, want)
     m.set_tuning()
-    graphs = [capture(m, x, y) for x, y in zip(xs[:2], ys[:2])]
+    graphs = [capture(m, x, y, inside) for x, y, inside in zip(xs, ys, (False, True))]
     streams = [torch.cuda.Stream() for _ in graphs]
     own = torch.cuda.Stream()
     m.set_stream(own.cuda_stream)
@@ -127,8 +132,9 @@ def test_replays_beside_applies_on_other_streams():
     m.set_stream(0)
 
 
+@pytest.mark.parametrize("inside", [False, True])
 @pytest.mark.parametrize("layout", [0, 6, 8])
-def test_global_apply_follows_updates(layout):
+def test_global_apply_follows_updates(layout, inside):
     rng = np.random.default_rng(31)
     d, n, level, active, T = 3, 2, 5, [(0, 1), (2,)], 2
     table, _ = grid.element_table([level] * d)
@@ -142,7 +148,7 @@ def test_global_apply_follows_updates(layout):
     m.set_tuning(waves_per_row=layout)
     x = torch.from_numpy(rng.uniform(-1, 1, m.input_size())).cuda()
     y = torch.zeros_like(x)
-    graph = capture(m, x, y)
+    graph = capture(m, x, y, inside)
     for step in range(3):
         if step:
             ops = factors(rng, d, n, level, active)
