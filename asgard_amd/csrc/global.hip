@@ -2789,7 +2789,8 @@ static int need_slabs(akm_matrix_s &m, akm_global_s &g)
 //! (make_global_kron_matrix, src/asgard_kronmult_matrix.cpp:1198-1334).  With
 //! `pair` (the operator of a sparse-grid handle, whose cells need no padding)
 //! only what the fibre walk and the slab layout use.  `repeated` = the first
-//! cell that equals an earlier one (nothing is built then), or -1.
+//! cell that equals an earlier one (nothing is built then), or -1.  Its
+//! layout is the caller's to set with `pair`, else the default one.
 static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
                         const int *active_mask, const int *flux_dim, bool pair,
                         int64_t &repeated)
@@ -3016,10 +3017,7 @@ static int build_global(akm_matrix_s &m, const std::vector<int> &elem_active,
       if (active_mask == nullptr || active_mask[t * d + k] != 0)
         g->flops += 2 * nnz_dim[k];
   m.gk = std::move(g);
-  const int layout = default_layout(m, *m.gk);
-  if (layout < 0)
-    return AKM_SUCCESS;
-  return global_set_layout(m, layout);
+  return pair ? AKM_SUCCESS : global_set_layout(m, default_layout(m, *m.gk));
 }
 
 int factored_build(akm_matrix_s &m, std::vector<int> const &elem)
@@ -3083,30 +3081,29 @@ int factored_build_mask(akm_matrix_s &m, std::vector<int> const &elem, std::vect
   if (widest > 1 && !whole_level_grid(m.d, m.rows, elem.data()))
     return AKM_SUCCESS;
   int64_t repeated = -1;
-  if (build_global(m, elem, mask.data(), nullptr, true, repeated) != AKM_SUCCESS)
+  int layout = -1;
+  if (build_global(m, elem, mask.data(), nullptr, true, repeated) == AKM_SUCCESS && m.gk)
+    layout = default_layout(m, *m.gk);
+  // too large for the lists or for memory, or a cell repeated: the pair
+  // kernels need neither
+  if (layout < 0)
   {
-    // too large for the lists or for memory: the pair kernels need neither
     (void)hipGetLastError();
     m.gk.reset();
     return AKM_SUCCESS;
   }
-  if (!m.gk)
-    return AKM_SUCCESS; // a cell is repeated
   const akm_global_s &g = *m.gk;
-  const int layout = default_layout(m, g);
-  if (layout < 0)
-  {
-    m.gk.reset();
-    return AKM_SUCCESS;
-  }
   // Estimated times: the pair kernels' fixed part and rate, the fibre walk's
   // per launch and per step (the slab layout is taken where it is faster
   // than that).
   const double pair_us = 4.0 + double(m.flops()) / (m.prec == AKM_F64 ? 25e6 : 50e6);
   const double walk_us = 1.0 + 3.0 * std::max(g.max_stages, 1) + double(g.fl_lanes) / 0.6e6;
-  m.factored = walk_us < pair_us;
+  m.factored = walk_us < pair_us && global_set_layout(m, layout) == AKM_SUCCESS;
   if (!m.factored)
+  {
+    (void)hipGetLastError();
     m.gk.reset();
+  }
   return AKM_SUCCESS;
 }
 } // namespace akm
