@@ -184,8 +184,8 @@ __global__ void __launch_bounds__(256) pattern_scan(int64_t num_cells, const int
 //! pattern_scan on packed 1D indices: a column is one coalesced word and D
 //! bits of the row's connect_1d rows, which the wavefront keeps in LDS (dynamic:
 //! 4 * D * words).  cols holds the columns in output order.  The
-//! supports' arithmetic and 12 strided ints a column took 0.95 (count) and
-//! 1.1 ms (fill) for 16,172 cells at d = 6, this 0.16 and 0.42.
+//! supports' arithmetic and 12 strided ints a column take 0.95 ms a pass for
+//! 16,172 cells at d = 6, this 0.28 (count) and 0.43 (fill: 0.9 GB written).
 template<int D>
 __global__ void __launch_bounds__(256)
     pattern_scan_bits(int64_t num_cells, const uint64_t *__restrict__ pack,

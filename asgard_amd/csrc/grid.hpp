@@ -20,7 +20,7 @@ int build_offset_table(int max_level, std::vector<int> const &pntr, std::vector<
 
 //! The indices 0 .. keys.size()-1 ordered by key (the lowest `bits` bits hold
 //! it), equal keys by index, by radix passes (handles are built at every
-//! regrid; 16,172 cells in 42 bits 0.06 ms, a comparison sort 0.6).
+//! regrid; 16,172 cells in 42 bits 0.12 ms with the keys, a comparison sort 0.6).
 void radix_order(std::vector<uint64_t> const &keys, int bits, std::vector<int> &order);
 
 //! elem[c*d + k] = 1D index of cell c in dimension k (0 for level 0, else

@@ -184,6 +184,20 @@ def test_sparse_pattern_bit_exact_d4_l7():
     assert np.array_equal(p, po) and np.array_equal(i, io)
 
 
+@pytest.mark.parametrize("d,L", [(1, 1), (1, 6), (1, 10), (2, 10), (3, 5), (6, 2), (1, 11)])
+def test_handle_pattern_at_word_edges(d, L):
+    """The pattern a handle builds (words of 32 connection bits up to level 10,
+    the supports past it) through the pair kernels: the rows' lengths and, by
+    the apply, their columns."""
+    c = sparse_grid_case(d, 2, L, 1, seed=4)
+    m = asgard_amd.KronmultMatrix.sparse_grid(d, 2, c["table"], L, 1, c["vA"])
+    m.set_tuning(waves_per_row=4)
+    assert m.num_pairs() == c["pntr"][-1]
+    y = dev(c["y"])
+    m.apply(1.0, dev(c["x"]), 0.0, y)
+    assert rel(host(y), oracle_apply(c, 1.0, 0.0)) < TOL64
+
+
 # ------------------------------------------------ benchmark sparse grids ---
 
 @pytest.mark.parametrize("d,n,L,T,dist", [(2, 2, 5, 2, "uniform"), (3, 3, 6, 3, "normal"),
